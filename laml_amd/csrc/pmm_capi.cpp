@@ -587,10 +587,9 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   int16_t* labels;
   laml::Coef* coef;
   double2* beta;
-  int32_t *bE, *aE, *LE;
-  double4* alpha;
-  int16_t* aG;
-  double *iLm, *site_llh, *rt_part, *cpart, *nu_a, *nu_b, *nu_d, *nu_part;
+  int32_t* bE;
+  double2* alpha;
+  double *pS, *site_llh, *rt_part, *cpart, *nu_a, *nu_b, *nu_d, *nu_part;
   laml::NuState* nu_state;
   AL(labels, int16_t, int_rows);
   // prior-weight rows: read by the chain kernels only, which need 64-site
@@ -617,11 +616,8 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
     bE = static_cast<int32_t*>(q);
     f->beta_rows = int_rows;
   }
-  AL(alpha, double4, int_rows);
-  AL(aE, int32_t, int_rows);
-  AL(aG, int16_t, int_rows);
-  AL(iLm, double, S);
-  AL(LE, int32_t, S);
+  AL(alpha, double2, int_rows);
+  AL(pS, double, int_rows);
   AL(site_llh, double, S);
   AL(rt_part, double, (size_t)N * F.max_chunks);
   AL(cpart, double, (size_t)N * F.max_chunks * 5);
@@ -699,10 +695,7 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   F.beta = beta;
   F.bE = bE;
   F.alpha = alpha;
-  F.aE = aE;
-  F.aG = aG;
-  F.iLm = iLm;
-  F.LE = LE;
+  F.pS = pS;
   F.site_llh = site_llh;
   F.rt_part = rt_part;
   F.cpart = cpart;

@@ -94,9 +94,12 @@ __device__ __forceinline__ void leaf_beta(int code, double phi, int& lab, double
 // eps(0) = e0 2^e = P(D_c | parent 0); eps(alpha) = eA 2^e = P(D_c | parent in
 // the child's edit state) ('?' child: any edit state).  The child's inside
 // vector is (b0, bA) 2^E with beta(-1) = 1 for '?' children; q is the prior
-// of the child's specific state.  Branch-free over the three label kinds.
+// of the child's specific state.  s0 = 2^(E - e) and s1 = P(-> -1) 2^-e (0
+// unless the child is '?') bring values on the child's exponent and the
+// silencing term to e.  Branch-free over the three label kinds.
 struct Eps {
   double e0, eA;
+  double s0, s1;
   int e;
 };
 __device__ __forceinline__ Eps edge(int lab, double b0, double bA, int E, double q, const Coef& c) {
@@ -110,6 +113,8 @@ __device__ __forceinline__ Eps edge(int lab, double b0, double bA, int E, double
   Eps r;
   r.e0 = fma(t0, s0, s1);
   r.eA = fma(tA, s0, s1);
+  r.s0 = s0;
+  r.s1 = s1;
   r.e = e;
   return r;
 }
@@ -119,7 +124,6 @@ __device__ __forceinline__ Eps edge(int lab, double b0, double bA, int E, double
 // the non-temporal hint and leave the caches to the per-site tables (priors,
 // site offsets, likelihoods) that every node of a tree reads.
 typedef double nt_double2 __attribute__((ext_vector_type(2)));
-typedef double nt_double4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ double2 load_stream(const double2* p) {
   const nt_double2 v = __builtin_nontemporal_load(reinterpret_cast<const nt_double2*>(p));
   return make_double2(v.x, v.y);
@@ -128,16 +132,20 @@ __device__ __forceinline__ void store_stream(double2* p, const double2& a) {
   const nt_double2 v = {a.x, a.y};
   __builtin_nontemporal_store(v, reinterpret_cast<nt_double2*>(p));
 }
-__device__ __forceinline__ void store_stream(double4* p, const double4& a) {
-  const nt_double4 v = {a.x, a.y, a.z, a.w};
-  __builtin_nontemporal_store(v, reinterpret_cast<nt_double4*>(p));
-}
 
 // binary exponent x of m (m in [2^(x-1), 2^x)); 0 for m == 0
 __device__ __forceinline__ int exp_of(double m) {
   int ex;
   (void)frexp(m, &ex);
   return ex;
+}
+
+// 1 / x for x in [0.5, 1): the hardware estimate and two Newton steps (no
+// scaling for extreme arguments)
+__device__ __forceinline__ double rcp_unit(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
 }
 
 // 64-bit DPP move of a double (rows not in ROW_MASK read 0)

@@ -6,8 +6,8 @@
 //    (int16 codes) and internal rows (beta, alpha, labels) are packed
 //    separately, row_off[v] giving the row start in the matching array.
 //  - internal rows hold beta = (b0, bA) mantissas with a shared exponent bE
-//    (inside, below the node), alpha = (o0, oS, Y, Z) with exponent aE and
-//    specific state aG (outside at the node), and the az-partition label.
+//    (inside, below the node), the az-partition label, and the outside state
+//    alpha = (a0, aX), conditional on all data (see cond_post).
 //
 // A segment of W lanes handles one node and strides over its K sites, so
 // per-node reductions over sites are segment shuffles.
@@ -751,26 +751,22 @@ __device__ __forceinline__ void root_chunk(const DevForest& F, int t, int chunk,
     const int ex = exp_of(er.e0);
     const double Lm = ldexp(er.e0, -ex);
     const int LE = er.e + ex;
-    F.iLm[sb + k] = 1.0 / Lm;
-    F.LE[sb + k] = LE;
     const double sl = log(Lm) + (double)LE * 0.69314718055994530942;
     F.site_llh[sb + k] = sl;
     if (site_llh_out) site_llh_out[sb + k] = sl;
+    // the stem starts unedited: given the data, its top is unedited with
+    // probability 1, as below a node with label 'z'
+    const double A = 1.0 / er.e0;
+    const double a0 = cf.p1n * A * er.s0;
+    const double m = cf.mut * q * A * er.s0;
+    const double sil = lab < 0 ? er.s1 * A : 0.0;
     if (!leaf) {
-      // outside state at the root: the stem starts unedited
-      F.alpha[rr + k] = make_double4(cf.p1n, ldexp(cf.msil, cf.esil), cf.mut, 0.0);
-      F.aE[rr + k] = 0;
-      F.aG[rr + k] = 0;
+      F.alpha[rr + k] = make_double2(a0, m);
+      if (lab < 0) F.pS[rr + k] = sil;
     }
-    if (lab == 0) {
-      acc0 = 1.0;
-    } else {
-      const double iL = 1.0 / Lm;
-      const double f1 = ldexp(iL, min(E - LE, 1000));
-      acc0 = cf.p1n * b0 * f1;
-      acc1 = cf.mut * q * bA * f1;
-      if (lab < 0) acc2 = ldexp(iL * cf.msil, min(cf.esil - LE, 1000));
-    }
+    acc0 = lab == 0 ? 1.0 : a0 * b0;
+    if (lab != 0) acc1 = m * bA;
+    acc2 = sil;
   }
   acc0 = seg_sum_last<W>(acc0);
   acc1 = seg_sum_last<W>(acc1);
@@ -808,14 +804,11 @@ struct OutNode {
   int kind[2];
   Coef cf[2];
   ChildRows c[2];
-  double4* ca[2];        // children's outside rows (internal children)
-  int32_t* caE[2];
-  int16_t* caG[2];
-  const double4* a;      // the node's outside row
-  const int32_t* aE;
-  const int16_t* aG;
-  const double* iLm;     // the tree's site likelihoods (1 / mantissa, exponent)
-  const int32_t* LE;
+  double2* ca[2];        // children's outside rows (internal children)
+  double* cS[2];         // children's silenced posteriors (internal children)
+  const int16_t* lab;    // the node's labels
+  const double2* a;      // the node's outside row
+  const double* aS;      // the node's silenced posteriors ('?' sites)
   const int32_t* qoff;
   const double* qsum;
   double phi;
@@ -834,16 +827,13 @@ __device__ __forceinline__ void out_node_load(const DevForest& F, int u, int t, 
     n.c[i] = child_rows(F, c, n.kind[i]);
     const int64_t rc = F.row_off[c];
     n.ca[i] = F.alpha + rc;
-    n.caE[i] = F.aE + rc;
-    n.caG[i] = F.aG + rc;
+    n.cS[i] = F.pS + rc;
   }
   const int64_t ru = F.row_off[u];
+  n.lab = F.labels + ru;
   n.a = F.alpha + ru;
-  n.aE = F.aE + ru;
-  n.aG = F.aG + ru;
+  n.aS = F.pS + ru;
   const int sb = F.tree_site_base[t];
-  n.iLm = F.iLm + sb;
-  n.LE = F.LE + sb;
   n.qoff = F.site_qoff + sb;
   n.qsum = F.site_qsum + sb;
   n.phi = F.phi[p];
@@ -867,96 +857,95 @@ __device__ __forceinline__ void out_node_rec(const DevForest& F, const NodeRec& 
     n.c[i].code2 = nullptr;
     n.c[i].gc[0] = n.c[i].gc[1] = -1;
     n.ca[i] = F.alpha + ro[i];
-    n.caE[i] = F.aE + ro[i];
-    n.caG[i] = F.aG + ro[i];
+    n.cS[i] = F.pS + ro[i];
   }
+  n.lab = F.labels + r.ro;
   n.a = F.alpha + r.ro;
-  n.aE = F.aE + r.ro;
-  n.aG = F.aG + r.ro;
-  n.iLm = F.iLm + r.sb;
-  n.LE = F.LE + r.sb;
+  n.aS = F.pS + r.ro;
   n.qoff = F.site_qoff + r.sb;
   n.qsum = F.site_qsum + r.sb;
   n.phi = uniform_load(F.phi + r.p);
   n.stream = F.stream_rows != 0;
 }
 
-// The posterior step of one node at one site.  In: the node's outside state
-// au 2^Eo with specific state gu, 1/L 2^-LE of the site, and for both
-// children their inside state (lab, b0, bA, E), leaf code, prior q, edge
-// values ep and branch coefficients cf.  Adds the counts of both child
-// branches to acc and the dropout responsibility of missing leaf children to
-// rt, and hands every non-leaf child's outside state to sink(i, quad, ec, gg)
-// (the quad carries 2^ec; gg is the specific state).
-template <typename Sink>
-__device__ __forceinline__ void post_site(const double4& au, int Eo, int gu, double iL, int LE, double qs,
-                                          double phi, const int (&lab)[2], const double (&b0)[2],
-                                          const double (&bA)[2], const int (&E)[2], const int (&code)[2],
-                                          const double (&q)[2], const Eps (&ep)[2], const Coef (&cfs)[2],
-                                          const bool (&lf)[2], double (&acc)[2][5], double& rt, Sink&& sink) {
+// The posterior step of one node u at one site.
+//
+// Outside states are kept conditional on all the data and on the scale of the
+// node's own inside vector: with beta_u = (b0, bA) 2^E and the site
+// likelihood L, u's state is
+//   a0 = alpha_u(0) 2^E / L,  aX = sum over the edit states a that the data
+//   below u allow (the label's state, or any state of a '?' node) of
+//   alpha_u(a) 2^E / L,
+// so a0 b0 = P(u unedited | D) and aX bA = P(u edited | D) and no exponent or
+// site likelihood is carried.  Two facts make the pair enough.  The posterior
+// counts and the states below need no other part of alpha_u (its silenced
+// part enters only P(u silenced | D), kept beside where '?' nodes need it).
+// And a node with label 'z' is unedited given the data below it: a0 = 1 / b0
+// and aX = 0 whatever lies outside, so its row is not read (and may hold
+// anything).
+// A row is 16 bytes where the unconditional state (three more values, an
+// exponent and a specific state) took 38, and a step needs about half the
+// arithmetic: on 16 trees of 10,000 leaves x 300 sites the chain rounds below
+// level 10 went from 0.66 to 0.52 ms a pass (114 -> 87 VGPRs, 5 wavefronts a
+// SIMD), an EM step from 1.79 to 1.61 ms.
+//
+// In: u's label lu and state (a0, aX), silenced posterior pSu (read where
+// lu < 0), and for both children their label, inside mantissas, prior weight
+// q (the site's prior mass for '?'), edge values ep, branch coefficients and
+// leaf code.  Out: the children's states ca, silenced posteriors cS (kS), the
+// counts S of both child branches, and the dropout responsibility rt of
+// missing leaf children.
+struct PostOut {
+  double a0[2], aX[2], pS[2];
+  double S[2][5];
+  double rt;
+};
+template <bool kS>
+__device__ __forceinline__ void cond_post(int lu, double a0, double aX, double pSu, double phi, const int (&lab)[2],
+                                          const double (&b0)[2], const double (&bA)[2], const double (&q)[2],
+                                          const Eps (&ep)[2], const Coef (&cfs)[2], const bool (&lf)[2],
+                                          const int (&code)[2], PostOut& o) {
+  // every pass kernel gives the same bits: fused operations are written out
+#pragma clang fp contract(off)
+  const bool z = lu == 0;
+  const double B0 = ep[0].e0 * ep[1].e0;
+  const double BA = z ? 0.0 : ep[0].eA * ep[1].eA;
+  // the power of two that the inside pass scaled u's vector by
+  const double sc = ldexp(1.0, min(-exp_of(fmax(B0, BA)), 1000));
+  const double f0 = z ? rcp_unit(B0 * sc) * sc : a0 * sc;
+  const double fX = z ? 0.0 : aX * sc;
+  o.rt = 0.0;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int w = 1 - i;
-    const int lw = lab[w];
     const Coef& cf = cfs[i];
-    // values below share the exponent ea = Eo + e_w:
-    // A = alpha_u(0) eps_w(0) (joint of the data outside v with u = 0);
-    // G(a) = alpha_u(a) eps_w(a) = q_a Gy + [a = gg] Gz
-    const double A = au.x * ep[w].e0;
-    const double Gy = lw < 0 ? au.z * ep[w].eA : 0.0;
-    const double Gz = lw < 0 ? au.w * ep[w].eA
-                             : (lw > 0 ? fma(q[w], au.z, lw == gu ? au.w : 0.0) * ep[w].eA : 0.0);
-    const int gg = lw < 0 ? gu : (lw > 0 ? lw : 0);
-    const int ea = Eo + ep[w].e;
-    // sum over edit states a of G(a) = q_a Gy + [a = gg] Gz
-    const double sumG = fma(qs, Gy, Gz);
-    const double av0 = A * cf.p1n;
-    const double base = A * cf.mut;
-    const double Yv = fma(cf.pn, Gy, base);
-    const double Zv = cf.pn * Gz;
-    if (!lf[i]) {
-      // alpha_v(-1) = GS 2^Eo + sil (A + sumG) 2^ea, GS = alpha_u(-1) eps_w(-1).
-      // The stored exponent comes from the largest value of either term
-      // group (GS is often zero), so the quad is normalised in one step.
-      const double GS = lw < 0 ? au.y : 0.0;
-      const double T = ldexp(cf.msil * (A + sumG), cf.esil);
-      const double mx = fmax(fmax(av0, T), fmax(Yv, Zv));
-      const int ta = exp_of(mx);
-      const int tg = GS != 0.0 ? Eo + exp_of(GS) : kZeroTop;
-      int ec = max(mx != 0.0 ? ea + ta : kZeroTop, tg);
-      if (ec == kZeroTop) ec = Eo;
-      const double sa = ldexp(1.0, min(ea - ec, 1000));
-      const double sg = ldexp(1.0, min(Eo - ec, 1000));
-      sink(i, make_double4(av0 * sa, fma(GS, sg, T * sa), Yv * sa, Zv * sa), ec, gg);
-    }
-    const int lv = lab[i];
-    if (lv == 0) {
-      acc[i][0] += 1.0;
-    } else {
-      // S0, S1, S3 carry 2^(ea + E_v) / L; S2, S4 carry sil 2^ea / L
-      const double f1 = ldexp(iL, min(ea + E[i] - LE, 1000));
-      acc[i][0] = fma(av0 * b0[i], f1, acc[i][0]);
-      acc[i][1] = fma(base * (q[i] * bA[i]), f1, acc[i][1]);
-      const double t3 = lv > 0 ? fma(q[i], Gy, lv == gg ? Gz : 0.0) : sumG;
-      acc[i][3] = fma(t3 * (cf.pn * bA[i]), f1, acc[i][3]);
-      if (lv < 0) {
-        const double f2 = ldexp(iL * cf.msil, min(ea + cf.esil - LE, 1000));
-        acc[i][2] = fma(A, f2, acc[i][2]);
-        acc[i][4] = fma(sumG, f2, acc[i][4]);
-        if (lf[i] && code[i] == -1)
-          rt = fma(phi * (av0 + fma(qs, Yv, Zv)), ldexp(iL, min(ea - LE, 1000)), rt);
-      }
-    }
+    // A, G: the data outside the child's branch joint with u unedited / in
+    // an allowed edit state, over L and on the child's edge exponent
+    const double A = f0 * ep[w].e0;
+    const double G = fX * ep[w].eA;
+    const double As = A * ep[i].s0, Gs = G * ep[i].s0;
+    const double m = cf.mut * q[i] * As;
+    const double pg = cf.pn * Gs;
+    o.a0[i] = cf.p1n * As;
+    o.aX[i] = fma(cf.pn, Gs, m);
+    const bool cz = lab[i] == 0;
+    o.S[i][0] = cz ? 1.0 : o.a0[i] * b0[i];
+    o.S[i][1] = m * bA[i];  // bA = 0 at 'z' nodes, s1 = 0 but at '?' nodes
+    o.S[i][2] = ep[i].s1 * A;
+    o.S[i][3] = pg * bA[i];
+    o.S[i][4] = ep[i].s1 * G;
+    if (kS) o.pS[i] = o.S[i][2] + o.S[i][4] + (lu < 0 ? pSu : 0.0);
+    if (lf[i]) o.rt = fma(code[i] == -1 ? phi : 0.0, o.a0[i] + o.aX[i], o.rt);
   }
 }
 
 // The posterior step a fused cherry's own node would run at site k, from the
-// outside state its parent just formed (au 2^Eo, gu): counts of its two leaf
+// state (a0, aX) its parent just formed and its label: counts of its two leaf
 // branches into cacc, dropout responsibility of its missing leaves into crt.
-__device__ __forceinline__ void cherry_post(const DevForest& F, const ChildRows& r, int k, const double4& au, int Eo,
-                                            int gu, double iL, int LE, int qo, double qs, double phi,
-                                            double (&cacc)[2][5], double& crt) {
-  int lab[2], E[2] = {0, 0}, code[2];
+__device__ __forceinline__ void cherry_post(const DevForest& F, const ChildRows& r, int k, int lu, double a0,
+                                            double aX, int qo, double qs, double phi, double (&cacc)[2][5],
+                                            double& crt) {
+  int lab[2], code[2];
   double b0[2], bA[2], q[2];
   Eps ep[2];
   code[0] = row_at(r.code, k);
@@ -968,16 +957,22 @@ __device__ __forceinline__ void cherry_post(const DevForest& F, const ChildRows&
     ep[j] = edge(lab[j], b0[j], bA[j], 0, q[j], r.g[j]);
   }
   const bool lf[2] = {true, true};
-  post_site(au, Eo, gu, iL, LE, qs, phi, lab, b0, bA, E, code, q, ep, r.g, lf, cacc, crt,
-            [](int, const double4&, int, int) {});
+  PostOut o;
+  cond_post<false>(lu, a0, aX, 0.0, phi, lab, b0, bA, q, ep, r.g, lf, code, o);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int m = 0; m < 5; ++m) cacc[j][m] += o.S[j][m];
+  crt += o.rt;
 }
 
 // The outside step of one site in three phases: row loads, prior gathers,
 // then arithmetic and stores.
 struct OutSite {
-  double4 au;
-  int Eo, gu, LE, qo;
-  double iL, qs;
+  double2 au;
+  double pS;
+  int lu, qo;
+  double qs;
   int lab[2], E[2], code[2];
   double b0[2], bA[2], q[2];
 };
@@ -994,10 +989,9 @@ __device__ __forceinline__ void outside_load_children(const DevForest& F, const 
 template <int K0, int K1>
 __device__ __forceinline__ void outside_load(const DevForest& F, const OutNode& n, int k, OutSite& x) {
   x.au = row_at(n.a, k);
-  x.Eo = row_at(n.aE, k);
-  x.gu = row_at(n.aG, k);
-  x.iL = row_at(n.iLm, k);
-  x.LE = row_at(n.LE, k);
+  x.lu = row_at(n.lab, k);
+  x.pS = 0.0;
+  if (x.lu < 0) x.pS = row_at(n.aS, k);
   x.qo = row_at(n.qoff, k) - 1;
   x.qs = row_at(n.qsum, k);
   outside_load_children<K0, K1>(F, n, k, x);
@@ -1019,23 +1013,27 @@ __device__ __forceinline__ void outside_finish(const DevForest& F, const OutNode
                                                double (&crt)[2]) {
   const int kind[2] = {resolve_kind<K0>(n.kind[0]), resolve_kind<K1>(n.kind[1])};
   const bool lf[2] = {kind[0] == kLeaf, kind[1] == kLeaf};
-  const double iL = x.iL;
   Eps ep[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) ep[i] = edge(x.lab[i], x.b0[i], x.bA[i], x.E[i], x.q[i], n.cf[i]);
-  post_site(x.au, x.Eo, x.gu, iL, x.LE, x.qs, n.phi, x.lab, x.b0, x.bA, x.E, x.code, x.q, ep, n.cf, lf, acc, rt,
-            [&](int i, const double4& a, int ec, int gg) {
-              if (kind[i] == kCherry) {
-                cherry_post(F, n.c[i], k, a, ec, gg, iL, x.LE, x.qo, x.qs, n.phi, cacc[i], crt[i]);
-              } else {
-                if (n.stream)
-                  store_stream(&row_at(n.ca[i], k), a);
-                else
-                  row_at(n.ca[i], k) = a;
-                row_at(n.caE[i], k) = ec;
-                row_at(n.caG[i], k) = (int16_t)gg;
-              }
-            });
+  PostOut o;
+  cond_post<true>(x.lu, x.au.x, x.au.y, x.pS, n.phi, x.lab, x.b0, x.bA, x.q, ep, n.cf, lf, x.code, o);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+#pragma unroll
+    for (int m = 0; m < 5; ++m) acc[i][m] += o.S[i][m];
+    if (kind[i] == kCherry) {
+      cherry_post(F, n.c[i], k, x.lab[i], o.a0[i], o.aX[i], x.qo, x.qs, n.phi, cacc[i], crt[i]);
+    } else if (kind[i] != kLeaf) {
+      const double2 a = make_double2(o.a0[i], o.aX[i]);
+      if (n.stream)
+        store_stream(&row_at(n.ca[i], k), a);
+      else
+        row_at(n.ca[i], k) = a;
+      if (x.lab[i] < 0) row_at(n.cS[i], k) = o.pS[i];
+    }
+  }
+  rt += o.rt;
 }
 
 template <int K0, int K1>
@@ -1293,16 +1291,15 @@ typedef const __attribute__((address_space(1))) void glb_void;
 // One wavefront's LDS slice: the next step's inside rows of both children,
 // both children's prior weights, both children's branch coefficients (10
 // words each), both children's codes (the aligned 32-bit word holding each
-// lane's 16-bit code), and in a pack the next head's outside state.
+// lane's 16-bit code), and in a pack the next head's outside state and labels.
 constexpr int kChainLdsBeta = 0;       // [2][64] double2
 constexpr int kChainLdsBE = 2048;      // [2][64] int32
 constexpr int kChainLdsQ = 2560;       // [2][64] double
 constexpr int kChainLdsCoef = 3584;    // [64] uint32 (20 used)
 constexpr int kChainLdsCode = 3840;    // [2][64] uint32
-constexpr int kChainLdsHeadA = 4352;   // [2 halves][64] 16 bytes: a head's outside quad
-constexpr int kChainLdsHeadE = 6400;   // [64] int32: its exponent
-constexpr int kChainLdsHeadG = 6656;   // [64] uint32: the word holding its specific state
-constexpr int kChainLdsBytes = 6912;
+constexpr int kChainLdsHeadA = 4352;   // [64] double2: a head's outside state
+constexpr int kChainLdsHeadL = 5376;   // [64] uint32: the word holding its label
+constexpr int kChainLdsBytes = 5632;
 
 // copy `size` (4 or 16) bytes at src (per lane) to dst + size * lane; rows
 // read once per pass carry the non-temporal hint, so that the per-site
@@ -1385,26 +1382,22 @@ __device__ __forceinline__ void chain_stage(const DevForest& F, const ChainStep&
   }
 }
 
-// Copy the stored outside state (quad, exponent, specific state) of the node
-// whose rows start at ru: the head of the next chain of a pack.
+// Copy the stored outside state and the labels of the node whose rows start
+// at ru: the head of the next chain of a pack.
 __device__ __forceinline__ void chain_stage_head(const DevForest& F, int64_t ru, unsigned kk, char* lds) {
-  const char* a = reinterpret_cast<const char*>(&row_at(F.alpha + ru, kk));
-  to_lds(a, lds + kChainLdsHeadA, 16, true);
-  to_lds(a + 16, lds + kChainLdsHeadA + 1024, 16, true);
-  to_lds(&row_at(F.aE + ru, kk), lds + kChainLdsHeadE, 4, true);
-  to_lds(F.aG + ru + (kk & ~1u), lds + kChainLdsHeadG, 4, true);
+  to_lds(&row_at(F.alpha + ru, kk), lds + kChainLdsHeadA, 16, true);
+  to_lds(F.labels + ru + (kk & ~1u), lds + kChainLdsHeadL, 4, true);
 }
 
 // One chain step at one site, on registers: the children's raw row values
 // (leaf codes or labels), prior weights, inside rows (ignored for leaves)
-// and branch coefficients.  The heavy child's outside state replaces (au,
-// Eo, gu); the light internal child's is stored at row ro[light].
+// and branch coefficients.  The heavy child's outside state and label replace
+// (a0, aX, lu); the light internal child's state is stored at row ro[light].
 template <int K0, int K1, typename Stage>
 __device__ __forceinline__ void chain_compute(const DevForest& F, const char* lds, int lane, const Coef (&cf)[2],
-                                              double phi, int hv, double iL, int LE, double qs, const int (&raw)[2],
-                                              const int64_t (&ro)[2], unsigned kk, bool on, bool stream,
-                                              Stage&& stage, double4& au, int& Eo, int& gu, double (&acc)[2][5],
-                                              double& rt) {
+                                              double phi, int hv, const int (&raw)[2], const int64_t (&ro)[2],
+                                              unsigned kk, bool on, bool stream, Stage&& stage, double& a0,
+                                              double& aX, int& lu, PostOut& o) {
   const bool lf[2] = {K0 == kLeaf, K1 == kLeaf};
   int lab[2], E[2], code[2];
   double b0[2], bA[2], q[2];
@@ -1427,27 +1420,33 @@ __device__ __forceinline__ void chain_compute(const DevForest& F, const char* ld
   // the slice is read: the next step's copies may overwrite it
   chain_wait_lgkm();
   stage();
-  if (!on) return;
   Eps ep[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) ep[i] = edge(lab[i], b0[i], bA[i], E[i], q[i], cf[i]);
-  const double4 au0 = au;
-  const int Eo0 = Eo, gu0 = gu;
-  post_site(au0, Eo0, gu0, iL, LE, qs, phi, lab, b0, bA, E, code, q, ep, cf, lf, acc, rt,
-            [&](int i, const double4& a, int ec, int gg) {
-              if (i == hv) {
-                au = a;
-                Eo = ec;
-                gu = gg;
-              } else {
-                if (stream)
-                  store_stream(&row_at(F.alpha + ro[i], kk), a);
-                else
-                  row_at(F.alpha + ro[i], kk) = a;
-                row_at(F.aE + ro[i], kk) = ec;
-                row_at(F.aG + ro[i], kk) = (int16_t)gg;
-              }
-            });
+  cond_post<false>(lu, a0, aX, 0.0, phi, lab, b0, bA, q, ep, cf, lf, code, o);
+  if (!on) {
+    // lanes past the tree's sites add nothing to the counts
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int m = 0; m < 5; ++m) o.S[i][m] = 0.0;
+    o.rt = 0.0;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if (lf[i]) continue;
+    if (i == hv) {
+      a0 = o.a0[i];
+      aX = o.aX[i];
+      lu = lab[i];
+    } else if (on) {
+      const double2 a = make_double2(o.a0[i], o.aX[i]);
+      if (stream)
+        store_stream(&row_at(F.alpha + ro[i], kk), a);
+      else
+        row_at(F.alpha + ro[i], kk) = a;
+    }
+  }
 }
 
 // Packs [cbeg, cbeg + cnt) of a chain plan: pack c's steps are
@@ -1487,17 +1486,13 @@ __global__ void __launch_bounds__(256) k_outside_chain(DevForest F, const int2* 
   const int k = chunk * 64 + lane;
   const bool on = k < K;
   const unsigned kk = on ? k : K - 1;
-  const int sb = F.tree_site_base[t];
   const double phi = F.phi[p];
   const bool stream = F.stream_rows != 0;
-  const double iL = row_at(F.iLm + sb, kk);
-  const int LE = row_at(F.LE + sb, kk);
-  const double qs = row_at(F.site_qsum + sb, kk);
   const unsigned k0 = (unsigned)chunk * 64u;
   const int64_t ru = F.row_off[u0];
-  double4 au = row_at(F.alpha + ru, kk);
-  int Eo = row_at(F.aE + ru, kk);
-  int gu = row_at(F.aG + ru, kk);
+  const double2 au = row_at(F.alpha + ru, kk);
+  double a0 = au.x, aX = au.y;
+  int lu = row_at(F.labels + ru, kk);
 
   // prologue: step 0's operands and codes and step 1's codes staged
   {
@@ -1523,11 +1518,10 @@ __global__ void __launch_bounds__(256) k_outside_chain(DevForest F, const int2* 
     const bool head0 = r0.u < 0;
     const int u = head0 ? ~r0.u : r0.u;
     if (kPacked && j > 0 && head0) {
-      const double2 xy = lds_at<double2>(lds, kChainLdsHeadA + 16 * lane);
-      const double2 zw = lds_at<double2>(lds, kChainLdsHeadA + 1024 + 16 * lane);
-      au = make_double4(xy.x, xy.y, zw.x, zw.y);
-      Eo = lds_at<int>(lds, kChainLdsHeadE + 4 * lane);
-      gu = code_of_word(lds_at<uint32_t>(lds, kChainLdsHeadG + 4 * lane), kk);
+      const double2 h = lds_at<double2>(lds, kChainLdsHeadA + 16 * lane);
+      a0 = h.x;
+      aX = h.y;
+      lu = code_of_word(lds_at<uint32_t>(lds, kChainLdsHeadL + 4 * lane), kk);
     }
     // this step's operands, from the slice (wave-uniform: moved to scalar
     // registers)
@@ -1553,25 +1547,20 @@ __global__ void __launch_bounds__(256) k_outside_chain(DevForest F, const int2* 
       }
     };
     // step j
-    double acc[2][5];
-    zero_acc(acc);
-    double rt = 0.0;
+    PostOut o;
     const int hv = r0.hv;
     const int64_t ro[2] = {r0.ro0, r0.ro1};
     if (r0.ch0 < F.num_leaves) {
       if (r0.ch1 < F.num_leaves)
-        chain_compute<kLeaf, kLeaf>(F, lds, lane, cf, phi, hv, iL, LE, qs, raw, ro, kk, on, stream, stage, au, Eo,
-                                    gu, acc, rt);
+        chain_compute<kLeaf, kLeaf>(F, lds, lane, cf, phi, hv, raw, ro, kk, on, stream, stage, a0, aX, lu, o);
       else
-        chain_compute<kLeaf, kInternal>(F, lds, lane, cf, phi, hv, iL, LE, qs, raw, ro, kk, on, stream, stage, au,
-                                        Eo, gu, acc, rt);
+        chain_compute<kLeaf, kInternal>(F, lds, lane, cf, phi, hv, raw, ro, kk, on, stream, stage, a0, aX, lu, o);
     } else {
       if (r0.ch1 < F.num_leaves)
-        chain_compute<kInternal, kLeaf>(F, lds, lane, cf, phi, hv, iL, LE, qs, raw, ro, kk, on, stream, stage, au,
-                                        Eo, gu, acc, rt);
+        chain_compute<kInternal, kLeaf>(F, lds, lane, cf, phi, hv, raw, ro, kk, on, stream, stage, a0, aX, lu, o);
       else
-        chain_compute<kInternal, kInternal>(F, lds, lane, cf, phi, hv, iL, LE, qs, raw, ro, kk, on, stream, stage,
-                                            au, Eo, gu, acc, rt);
+        chain_compute<kInternal, kInternal>(F, lds, lane, cf, phi, hv, raw, ro, kk, on, stream, stage, a0, aX, lu,
+                                            o);
     }
     // partial counts: one butterfly sum of the eleven values; lane 16r + i
     // (i < 3) holds total 3r + i (counts 0..4 of child 0, of child 1, the
@@ -1579,10 +1568,10 @@ __global__ void __launch_bounds__(256) k_outside_chain(DevForest F, const int2* 
     double v[12];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
-      v[m] = acc[0][m];
-      v[5 + m] = acc[1][m];
+      v[m] = o.S[0][m];
+      v[5 + m] = o.S[1][m];
     }
-    v[10] = rt;
+    v[10] = o.rt;
     v[11] = 0.0;
     wave_sum12(v);
     {
@@ -2475,69 +2464,47 @@ __global__ void __launch_bounds__(kUltraThreads) k_ultra(DevForest F, UltraDev U
 // ---------------------------------------------------------------------------
 namespace {
 
-struct QTop {            // data outside a child branch, at its parent's side
-  double A, Gy, Gz, GS, sumG;
-  int ea, Eo, gg;
+// Data outside a branch joint with its top unedited (A) / in an edit state
+// that the data below allow (G), over the site likelihood and on a power of
+// two of the caller's choice (cond_post's A and G).
+struct QTop {
+  double A, G;
 };
 
-struct QAlpha {          // outside state at a node: (o0, oS, Y, Z) 2^E, state g
-  double x, y, z, w;
-  int E, g;
-};
-
-__device__ __forceinline__ QTop q_top(const QAlpha& au, const Eps& ew, int lw, double qw, double qs) {
-  QTop t;
-  t.A = au.x * ew.e0;
-  t.Gy = lw < 0 ? au.z * ew.eA : 0.0;
-  t.Gz = lw < 0 ? au.w * ew.eA : (lw > 0 ? fma(qw, au.z, lw == au.g ? au.w : 0.0) * ew.eA : 0.0);
-  t.gg = lw < 0 ? au.g : (lw > 0 ? lw : 0);
-  t.ea = au.E + ew.e;
-  t.GS = lw < 0 ? au.y : 0.0;
-  t.sumG = fma(qs, t.Gy, t.Gz);
-  t.Eo = au.E;
-  return t;
-}
-
-__device__ __forceinline__ QAlpha q_child_alpha(const QTop& t, const Coef& cf) {
-  const double av0 = t.A * cf.p1n;
-  const double Yv = fma(cf.pn, t.Gy, t.A * cf.mut);
-  const double Zv = cf.pn * t.Gz;
-  const double T = ldexp(cf.msil * (t.A + t.sumG), cf.esil);
-  const double mx = fmax(fmax(av0, T), fmax(Yv, Zv));
-  const int tg = t.GS != 0.0 ? t.Eo + exp_of(t.GS) : kZeroTop;
-  int ec = max(mx != 0.0 ? t.ea + exp_of(mx) : kZeroTop, tg);
-  if (ec == kZeroTop) ec = t.Eo;
-  const double sa = ldexp(1.0, min(t.ea - ec, 1000));
-  const double sg = ldexp(1.0, min(t.Eo - ec, 1000));
-  QAlpha a;
-  a.x = av0 * sa;
-  a.y = fma(t.GS, sg, T * sa);
-  a.z = Yv * sa;
-  a.w = Zv * sa;
-  a.E = ec;
-  a.g = t.gg;
-  return a;
-}
-
-// posterior counts of the branch above a node with label lv and inside
-// (b0, bA) 2^E, prior q of its state (qs for '?'), given the top of the
-// branch and 1/L = iL 2^-LE
-__device__ __forceinline__ void q_post(const QTop& t, const Coef& cf, int lv, double b0, double bA, int E, double q,
-                                       double iL, int LE, double* S) {
+// posterior counts of the branch above a node with inside mantissas (b0, bA),
+// prior weight q and edge values ep (t on the scale of ep, over the candidate's
+// site likelihood)
+__device__ __forceinline__ void q_post(const QTop& t, const Coef& cf, int lv, double b0, double bA, double q,
+                                       const Eps& ep, double* S) {
   if (lv == 0) {
     S[0] += 1.0;
     return;
   }
-  const double f1 = ldexp(iL, min(t.ea + E - LE, 1000));
-  S[0] = fma(t.A * cf.p1n * b0, f1, S[0]);
-  S[1] = fma(t.A * cf.mut * (q * bA), f1, S[1]);
-  const double t3 = lv > 0 ? fma(q, t.Gy, lv == t.gg ? t.Gz : 0.0) : t.sumG;
-  S[3] = fma(t3 * (cf.pn * bA), f1, S[3]);
-  if (lv < 0) {
-    const double f2 = ldexp(iL * cf.msil, min(t.ea + cf.esil - LE, 1000));
-    S[2] = fma(t.A, f2, S[2]);
-    S[4] = fma(t.sumG, f2, S[4]);
-  }
+  const double A = t.A, G = t.G;
+  S[0] = fma(cf.p1n * A * ep.s0, b0, S[0]);
+  S[1] = fma(cf.mut * q * A * ep.s0, bA, S[1]);
+  S[2] = fma(ep.s1, A, S[2]);
+  S[3] = fma(cf.pn * G * ep.s0, bA, S[3]);
+  S[4] = fma(ep.s1, G, S[4]);
+}
+
+// outside state (a0, aX) at the node below a branch, on the scale of its
+// inside mantissas; aX = 0 at 'z' nodes
+__device__ __forceinline__ QTop q_node(const QTop& t, const Coef& cf, int lv, double q, const Eps& ep) {
+  QTop a;
+  const double A = t.A * ep.s0, G = t.G * ep.s0;
+  a.A = cf.p1n * A;
+  a.G = lv == 0 ? 0.0 : fma(cf.pn, G, cf.mut * q * A);
+  return a;
+}
+
+// top of a child's branch from its parent's state (scaled by sc, the power
+// of two the parent's vector was scaled by) and the sibling's edge values
+__device__ __forceinline__ QTop q_top(const QTop& a, double sc, const Eps& ew) {
+  QTop t;
+  t.A = a.A * sc * ew.e0;
+  t.G = a.G * sc * ew.eA;
+  return t;
 }
 
 __device__ __forceinline__ Coef q_coef(double d, double nu) {
@@ -2552,9 +2519,10 @@ __device__ __forceinline__ Coef q_coef(double d, double nu) {
   return c;
 }
 
-// inside of a node from its two children's edge values; returns the label
+// inside of a node from its two children's edge values, and the power of two
+// sc that it was scaled by; returns the label
 __device__ __forceinline__ int q_combine(int la, int lb, const Eps& ea, const Eps& eb, double& B0, double& BA,
-                                         int& E) {
+                                         int& E, double& scale) {
   const int lv = combine_label(la, lb);
   const double b0 = ea.e0 * eb.e0;
   const double bA = lv != 0 ? ea.eA * eb.eA : 0.0;
@@ -2563,6 +2531,7 @@ __device__ __forceinline__ int q_combine(int la, int lb, const Eps& ea, const Ep
   B0 = b0 * sc;
   BA = bA * sc;
   E = ea.e + eb.e - sh;
+  scale = sc;
   return lv;
 }
 
@@ -2598,20 +2567,25 @@ __global__ void __launch_bounds__(256) k_quartet_em(DevForest F, int ncand, cons
   Coef cs{};
   ChildRows rS{};
   bool lfS = false;
-  const double4* aP = nullptr;
-  const int32_t* aEP = nullptr;
-  const int16_t* aGP = nullptr;
+  const double2* aP = nullptr;
+  const double2* bP = nullptr;
+  const int32_t* bEP = nullptr;
+  const int16_t* labP = nullptr;
+  const double* pSP = nullptr;
   if (!top_root) {
     cs = F.coef[sib];
     lfS = sib < F.num_leaves;
     rS = child_rows(F, sib, lfS);
     const int64_t rp = F.row_off[p];
     aP = F.alpha + rp;
-    aEP = F.aE + rp;
-    aGP = F.aG + rp;
+    labP = F.labels + rp;
+    pSP = F.pS + rp;
+    bP = F.beta + F.brow[p];
+    bEP = F.bE + F.brow[p];
   }
   const int32_t* qoff = F.site_qoff + sb;
   const double* qsum = F.site_qsum + sb;
+  const double* site_llh = F.site_llh + sb;
   const double kLn2 = 0.69314718055994530942;
   double llh_prev = 0.0, llh = 0.0;
   int iters = max_iter + 1;
@@ -2640,65 +2614,62 @@ __global__ void __launch_bounds__(256) k_quartet_em(DevForest F, int ncand, cons
       const Eps eW = edge(labW, b0W, bAW, EW, qW, cf[1]);
       double b0u, bAu;
       int Eu;
-      const int labU = q_combine(labA, labW, eA, eW, b0u, bAu, Eu);
+      double scU, scV;
+      const int labU = q_combine(labA, labW, eA, eW, b0u, bAu, Eu, scU);
       const double qU = labU > 0 ? row_at(F.prior, (unsigned)(qo + labU)) : qs;
       const Eps eU = edge(labU, b0u, bAu, Eu, qU, cf[2]);
       const Eps eC = edge(labC, b0C, bAC, EC, qC, cf[3]);
       double b0v, bAv;
       int Ev;
-      const int labV = q_combine(labU, labC, eU, eC, b0v, bAv, Ev);
+      const int labV = q_combine(labU, labC, eU, eC, b0v, bAv, Ev, scV);
       const double qV = labV > 0 ? row_at(F.prior, (unsigned)(qo + labV)) : qs;
-      // top of v's branch: the unedited ancestor, or p's outside state with
-      // the sibling's edge values
+      const Eps eV = edge(labV, b0v, bAv, Ev, qV, cf[4]);
+      // top of v's branch: the unedited ancestor, or p's outside state (over
+      // the likelihood L of the site before the move) with the sibling's
+      // edge values; x: the exponent of t1 below
       QTop tv;
+      double c = 0.0, base = 0.0;
+      int x = eV.e;
       if (top_root) {
         tv.A = 1.0;
-        tv.Gy = tv.Gz = tv.GS = tv.sumG = 0.0;
-        tv.ea = tv.Eo = tv.gg = 0;
+        tv.G = 0.0;
       } else {
         int labS, ES;
         double b0S, bAS;
         load_child_rows(rS, lfS, k, phi, labS, b0S, bAS, ES, code);
         const double qS = labS > 0 ? row_at(F.prior, (unsigned)(qo + labS)) : qs;
         const Eps eS = edge(labS, b0S, bAS, ES, qS, cs);
-        const double4 a4 = row_at(aP, (unsigned)k);
-        QAlpha ap;
-        ap.x = a4.x;
-        ap.y = a4.y;
-        ap.z = a4.z;
-        ap.w = a4.w;
-        ap.E = row_at(aEP, (unsigned)k);
-        ap.g = row_at(aGP, (unsigned)k);
-        tv = q_top(ap, eS, labS, qS, qs);
+        const int lp = row_at(labP, (unsigned)k);
+        const double2 ap = row_at(aP, (unsigned)k);
+        const double b0p = row_at(bP, (unsigned)k).x;
+        tv.A = (lp == 0 ? 1.0 / b0p : ap.x) * eS.e0;
+        tv.G = lp == 0 ? 0.0 : ap.y * eS.eA;
+        if (lp < 0) c = row_at(pSP, (unsigned)k);  // p silenced: free of v's branch
+        x += eS.e - row_at(bEP, (unsigned)k);
+        base = row_at(site_llh, (unsigned)k);
       }
-      const QAlpha av = q_child_alpha(tv, cf[4]);
-      // site likelihood from v's outside and inside states
-      double sumA;
-      if (labV > 0) sumA = fma(qV, av.z, labV == av.g ? av.w : 0.0);
-      else if (labV < 0) sumA = fma(qs, av.z, av.w);
-      else sumA = 0.0;
-      const double t1 = fma(av.x, b0v, sumA * bAv);
-      const double t2 = labV < 0 ? av.y : 0.0;
-      const int e1 = t1 != 0.0 ? Ev + exp_of(t1) : kZeroTop;
-      const int e2 = t2 != 0.0 ? exp_of(t2) : kZeroTop;
-      const int e = max(e1, e2);
-      double Lm = ldexp(t1, min(Ev - e, 1000)) + ldexp(t2, min(-e, 1000));
-      const int ex = exp_of(Lm);
-      Lm = ldexp(Lm, -ex);
-      const int LE = av.E + e + ex;
-      ll += log(Lm) + (double)LE * kLn2;
-      const double iL = 1.0 / Lm;
+      // site likelihood L' of the candidate: L' / L = t1 2^x + c
+      const double t1 = fma(tv.A, eV.e0, tv.G * eV.eA);
+      const int e1 = t1 != 0.0 ? x + exp_of(t1) : kZeroTop;
+      const int e = max(e1, c != 0.0 ? exp_of(c) : kZeroTop);
+      const double Lm = ldexp(t1, min(x - e, 1000)) + ldexp(c, min(-e, 1000));
+      ll += log(Lm) + (double)e * kLn2 + base;
+      // from here on over L'
+      const double iL = ldexp(1.0 / Lm, min(x - e, 1000));
+      tv.A *= iL;
+      tv.G *= iL;
       // posteriors: v's branch, then u and C below v, then A and W below u
-      q_post(tv, cf[4], labV, b0v, bAv, Ev, qV, iL, LE, S[4]);
-      const QTop tu = q_top(av, eC, labC, qC, qs);
-      q_post(tu, cf[2], labU, b0u, bAu, Eu, qU, iL, LE, S[2]);
-      const QTop tc = q_top(av, eU, labU, qU, qs);
-      q_post(tc, cf[3], labC, b0C, bAC, EC, qC, iL, LE, S[3]);
-      const QAlpha au = q_child_alpha(tu, cf[2]);
-      const QTop ta = q_top(au, eW, labW, qW, qs);
-      q_post(ta, cf[0], labA, b0A, bAA, EA, qA, iL, LE, S[0]);
-      const QTop tw = q_top(au, eA, labA, qA, qs);
-      q_post(tw, cf[1], labW, b0W, bAW, EW, qW, iL, LE, S[1]);
+      q_post(tv, cf[4], labV, b0v, bAv, qV, eV, S[4]);
+      const QTop av = q_node(tv, cf[4], labV, qV, eV);
+      const QTop tu = q_top(av, scV, eC);
+      q_post(tu, cf[2], labU, b0u, bAu, qU, eU, S[2]);
+      const QTop tc = q_top(av, scV, eU);
+      q_post(tc, cf[3], labC, b0C, bAC, qC, eC, S[3]);
+      const QTop au = q_node(tu, cf[2], labU, qU, eU);
+      const QTop ta = q_top(au, scU, eW);
+      q_post(ta, cf[0], labA, b0A, bAA, qA, eA, S[0]);
+      const QTop tw = q_top(au, scU, eA);
+      q_post(tw, cf[1], labW, b0W, bAW, qW, eW, S[1]);
     }
     ll = seg_sum_last<64>(ll);
     ll = __shfl(ll, 63, 64);
@@ -2986,8 +2957,8 @@ void run_outside_levels(const DevForest& F, const std::vector<int32_t>& lvl, int
 // Posterior state probabilities of every (node, site): P(v = 0 | D) and
 // P(v = -1 | D), the post0 / post1 of EM_solver.Estep_posterior
 // (EM_solver.py:247-300, in linear space), from the resident inside and
-// outside state.  Segments index internal nodes; a leaf child's outside
-// state is formed from its parent's as in the outside pass.  Outputs use the
+// outside state.  Segments index internal nodes; a leaf child's posteriors
+// are formed from its parent's state as in the outside pass.  Outputs use the
 // device row layout: internal node v at leaf_rows + row_off[v], leaf v at
 // row_off[v].
 template <int W>
@@ -3002,43 +2973,36 @@ __global__ void __launch_bounds__(256) k_node_post(DevForest F, int64_t leaf_row
   if (k >= K) return;
   const int sb = F.tree_site_base[t];
   const double phi = F.phi[prob];
-  const double iL = F.iLm[sb + k];
-  const int LE = F.LE[sb + k];
   const int64_t ru = F.row_off[u];
-  const double4 a4 = F.alpha[ru + k];
-  QAlpha au;
-  au.x = a4.x;
-  au.y = a4.y;
-  au.z = a4.z;
-  au.w = a4.w;
-  au.E = F.aE[ru + k];
-  au.g = F.aG[ru + k];
-  const int labu = F.labels[ru + k];
-  const int64_t bu = F.brow[u];
-  const double2 bb = F.beta[bu + k];
-  const int Eu = F.bE[bu + k];
-  p0[leaf_rows + ru + k] = au.x * bb.x * ldexp(iL, min(au.E + Eu - LE, 1000));
-  pS[leaf_rows + ru + k] = labu < 0 ? au.y * ldexp(iL, min(au.E - LE, 1000)) : 0.0;
+  const int lu = F.labels[ru + k];
+  const double2 au = F.alpha[ru + k];
+  const double b0u = F.beta[F.brow[u] + k].x;
+  const double pSu = lu < 0 ? F.pS[ru + k] : 0.0;
+  p0[leaf_rows + ru + k] = lu == 0 ? 1.0 : au.x * b0u;
+  pS[leaf_rows + ru + k] = pSu;
   const int ch[2] = {F.child0[u], F.child1[u]};
+  const bool lf[2] = {ch[0] < F.num_leaves, ch[1] < F.num_leaves};
+  if (!lf[0] && !lf[1]) return;
   const int qo = F.site_qoff[sb + k] - 1;
   const double qs = F.site_qsum[sb + k];
   int lab[2], E[2], code[2];
   double b0[2], bA[2], q[2];
   Eps ep[2];
+  const Coef cf[2] = {F.coef[ch[0]], F.coef[ch[1]]};
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    load_child(F, ch[i], ch[i] < F.num_leaves, k, phi, lab[i], b0[i], bA[i], E[i], code[i]);
+    load_child(F, ch[i], lf[i], k, phi, lab[i], b0[i], bA[i], E[i], code[i]);
     q[i] = lab[i] > 0 ? F.prior[qo + lab[i]] : qs;
-    ep[i] = edge(lab[i], b0[i], bA[i], E[i], q[i], F.coef[ch[i]]);
+    ep[i] = edge(lab[i], b0[i], bA[i], E[i], q[i], cf[i]);
   }
+  PostOut o;
+  cond_post<true>(lu, au.x, au.y, pSu, phi, lab, b0, bA, q, ep, cf, lf, code, o);
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    if (ch[i] >= F.num_leaves) continue;
-    const QTop tp = q_top(au, ep[1 - i], lab[1 - i], q[1 - i], qs);
-    const QAlpha av = q_child_alpha(tp, F.coef[ch[i]]);
+    if (!lf[i]) continue;
     const int64_t rv = F.row_off[ch[i]];
-    p0[rv + k] = av.x * b0[i] * ldexp(iL, min(av.E - LE, 1000));
-    pS[rv + k] = lab[i] < 0 ? av.y * ldexp(iL, min(av.E - LE, 1000)) : 0.0;
+    p0[rv + k] = o.S[i][0];
+    pS[rv + k] = lab[i] < 0 ? o.pS[i] : 0.0;
   }
 }
 

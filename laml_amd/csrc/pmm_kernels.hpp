@@ -89,11 +89,11 @@ struct DevForest {
   Coef* coef;       // [N]
   double2* beta;    // internal rows
   int32_t* bE;
-  double4* alpha;  // internal rows
-  int32_t* aE;
-  int16_t* aG;
-  double* iLm;  // [sites] 1 / mantissa of the site likelihood (L = 2^LE / iLm)
-  int32_t* LE;
+  // outside state (a0, aX) of internal nodes given all data, on the scale of
+  // beta (undefined where the label is 'z'), and P(silenced | D) where the
+  // label is '?'
+  double2* alpha;
+  double* pS;
   double* site_llh;
   double* rt_part;  // [N * max_chunks] dropout sums of leaf children per chunk
   double* cpart;    // [N * max_chunks * 5] per-chunk branch count partials
