@@ -96,6 +96,19 @@ struct laml_forest {
   int chain_pack = 8;
   int64_t pack_waves = laml::kPackWaves;
   bool alpha_complete = true;
+  // LDS passes: the plan of k_problem (a block per problem) where every
+  // problem fits it; taken while the launch plan is the one the forest was
+  // created with (any other plan asks for its own kernels).  They leave no
+  // rows in global memory: rows_ok says whether the rows hold the inside
+  // state of the last call.
+  bool pb_ok = false;
+  laml::LdsPlan pb{};
+  bool rows_ok = true;
+  struct {
+    int pass_mode, h_top, chains, chain_top_in, chain_top_out;
+    bool fuse;
+    std::vector<int32_t> in_cpw, out_cpw;
+  } def{};
   std::deque<laml::ChainPlan> chain_plans;  // a deque: plans stay put when more are added
   std::vector<int32_t> h_heavy;  // heavy child of each node (-1: no internal child)
   std::vector<int32_t> h_child0, h_child1;
@@ -360,6 +373,96 @@ int laml_forest_validate(const laml_forest_desc* d) {
 }
 
 static int upload_node_recs(laml_forest* f, const std::vector<int64_t>& brow);
+
+// LDS a block needs: the state of its cells, the stem's sums, the level table
+static int64_t lds_need(const laml::LdsBlk& b, const std::vector<int32_t>& lvl_base) {
+  const int64_t cells = (int64_t)b.nint * b.sb;
+  return (cells + 8) * 20 + b.sb / laml::kLdsSlotSites * 24 +
+         8 * (int64_t)(lvl_base[b.tree + 1] - lvl_base[b.tree] + 1);
+}
+
+// entries of a block's cell tables: pairs of its levels' cells, each level
+// padded to a wavefront's
+static int64_t lds_entries(const laml::LdsBlk& b, const std::vector<int32_t>& lvl_base,
+                           const std::vector<int32_t>& lvl_cnt) {
+  int64_t n = 0;
+  for (int i = lvl_base[b.tree] + 1; i < lvl_base[b.tree + 1]; ++i) n += ((int64_t)lvl_cnt[i] * b.sb + 127) / 128 * 64;
+  return n;
+}
+
+// The LDS plan whose block b runs tree blks[b].tree at its sites, a tree's
+// blocks writing one partial-count slot each.  Level tables as the tree
+// walk's.
+static int upload_lds_plan(laml_forest* f, laml::LdsPlan& L, const std::vector<laml::LdsBlk>& blks,
+                           int slots, const std::vector<int32_t>& lvl_base, const std::vector<int32_t>& lvl_beg,
+                           const std::vector<int32_t>& lvl_cnt) {
+  const int N = f->F.num_nodes, n = f->F.num_leaves, T = f->F.num_trees;
+  std::vector<int32_t> tree_sb(T, 0);  // (the same for all blocks of a tree)
+  for (const laml::LdsBlk& b : blks) tree_sb[b.tree] = b.sb;
+  std::vector<int32_t> int_base(T, 0), local(N, -1);
+  std::vector<int2> lvl_off(lvl_base[T], make_int2(0, 0));
+  int64_t recs = 0;
+  for (int t = 0; t < T; ++t) {
+    int_base[t] = (int32_t)recs;
+    int l = 0, e = 0;
+    for (int i = lvl_base[t] + 1; i < lvl_base[t + 1]; ++i) {
+      for (int j = 0; j < lvl_cnt[i]; ++j) local[lvl_beg[i] + j] = l++;
+      e += (lvl_cnt[i] * tree_sb[t] + 127) / 128 * 64;
+      lvl_off[i] = make_int2(l, e);
+    }
+    recs += l;
+  }
+  std::vector<laml::LdsRec> rec((size_t)recs);
+  for (int v = n; v < N; ++v) {
+    const int r = int_base[f->h_tree_of[v]] + local[v];
+    const int a = f->h_child0[v], b = f->h_child1[v];
+    rec[r] = laml::LdsRec{local[a], local[b], a, b, v, 0};
+  }
+  int64_t entries = 0;
+  L.lds_bytes = 0;
+  for (const laml::LdsBlk& b : blks) {
+    entries = std::max(entries, b.tab + lds_entries(b, lvl_base, lvl_cnt));
+    L.lds_bytes = (int32_t)std::max<int64_t>(L.lds_bytes, lds_need(b, lvl_base));
+  }
+  L.num_blocks = (int32_t)blks.size();
+  L.slots = slots;
+  int rc;
+  if ((rc = f->upload(&L.blk, blks.data(), blks.size())) ||
+      (rc = f->upload(&L.int_base, int_base.data(), int_base.size())) ||
+      (rc = f->upload(&L.rec, rec.data(), rec.size())) ||
+      (rc = f->upload(&L.lvl_off, lvl_off.data(), lvl_off.size())) || (rc = f->alloc(&L.lcoef, (size_t)recs)) || (rc = f->alloc(&L.w, (size_t)entries)) ||
+      (rc = f->alloc(&L.q, (size_t)entries)) || (rc = f->alloc(&L.cpart, (size_t)N * 5 * slots)) ||
+      (rc = f->alloc(&L.rt_part, (size_t)N * slots)))
+    return rc;
+  return LAML_OK;
+}
+
+// Plans the forest for k_problem where every problem fits: one tree, at most
+// kPbMaxSites sites (all of them in one block) and the state (20 bytes a node
+// and site) in a CU's LDS; and at most kPbMaxProblems of them.
+static int plan_problems(laml_forest* f, int max_k, const std::vector<int32_t>& lvl_base,
+                         const std::vector<int32_t>& lvl_beg, const std::vector<int32_t>& lvl_cnt) {
+  const int T = f->F.num_trees;
+  if (max_k > laml::kPbMaxSites || T != f->F.num_problems || T > laml::kPbMaxProblems) return LAML_OK;
+  constexpr int R = laml::kLdsSlotSites;
+  std::vector<laml::LdsBlk> blks;
+  int64_t tab = 0;
+  for (int t = 0; t < T; ++t) {
+    laml::LdsBlk b{};
+    b.tree = t;
+    b.k0 = 0;
+    b.sb = (f->tree_nsites[t] + R - 1) / R * R;
+    for (int i = lvl_base[t] + 1; i < lvl_base[t + 1]; ++i) b.nint += lvl_cnt[i];
+    if (b.nint < 1 || lds_need(b, lvl_base) > laml::kLdsMaxBytes) return LAML_OK;
+    b.tab = tab;
+    tab += lds_entries(b, lvl_base, lvl_cnt);
+    blks.push_back(b);
+  }
+  const int rc = upload_lds_plan(f, f->pb, blks, 1, lvl_base, lvl_beg, lvl_cnt);
+  if (rc) return rc;
+  f->pb_ok = true;
+  return LAML_OK;
+}
 
 int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out) {
   if (!out) return fail(LAML_EINVAL, "null output pointer");
@@ -705,6 +808,22 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   F.nu_part = nu_part;
   F.nu_state = nu_state;
   F.phi = nullptr;
+  F.cp_v = (int64_t)F.max_chunks * 5;
+  F.cp_c = 5;
+  F.rt_v = F.max_chunks;
+  F.rt_c = 1;
+  f->def.pass_mode = f->pass_mode;
+  f->def.h_top = f->h_top_default;
+  f->def.chains = f->chains;
+  f->def.chain_top_in = f->chain_top_in;
+  f->def.chain_top_out = f->chain_top_out;
+  f->def.fuse = f->fuse;
+  f->def.in_cpw = f->in_cpw;
+  f->def.out_cpw = f->out_cpw;
+  if ((rc = plan_problems(f, max_k, tw_lvl_base, tw_lvl_beg, tw_lvl_cnt))) {
+    delete f;
+    return rc;
+  }
   if (hipMemset(rt_part, 0, sizeof(double) * N * F.max_chunks) != hipSuccess ||
       hipMemset(cpart, 0, sizeof(double) * N * F.max_chunks * 5) != hipSuccess ||
       hipMemset(nu_state, 0, sizeof(laml::NuState) * P) != hipSuccess) {
@@ -741,6 +860,7 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   }
   laml::run_labels(F, f->level_off, f->W, nullptr);
   if (qleaf) laml::run_qrows(F, qleaf, qint, nullptr);
+  if (f->pb_ok) laml::run_lds_tables(F, f->pb, f->TW, nullptr);
   // every set-up copy and kernel above ran on the legacy default stream:
   // waiting for it alone leaves other threads' streams (a server's other
   // solves) running
@@ -1121,6 +1241,29 @@ static DevForest with_cherries(const laml_forest* f, const DevForest& F, bool fu
   return G;
 }
 
+// whether the passes run as k_problem: the forest was planned for it and its
+// launch plan is untouched
+static bool problem_now(const laml_forest* f) {
+  return f->pb_ok && f->ckpt_L == 0 && f->pass_mode == f->def.pass_mode && f->h_top_default == f->def.h_top &&
+         f->chains == f->def.chains && f->chain_top_in == f->def.chain_top_in &&
+         f->chain_top_out == f->def.chain_top_out && f->fuse == f->def.fuse && f->in_cpw == f->def.in_cpw &&
+         f->out_cpw == f->def.out_cpw;
+}
+
+// F with the partial counts of an LDS plan
+static DevForest lds_view(const DevForest& F, const laml::LdsPlan& L) {
+  DevForest G = F;
+  // one slot per block of a tree's sites
+  G.chunk_w = 1 << 24;
+  G.cpart = L.cpart;
+  G.rt_part = L.rt_part;
+  G.cp_v = 5;
+  G.cp_c = (int64_t)F.num_nodes * 5;
+  G.rt_v = 1;
+  G.rt_c = F.num_nodes;
+  return G;
+}
+
 // hybrid pass mode: level launches below this level, one tree-walk launch
 // (a block per tree and site chunk) for the levels from it up
 static int hybrid_split(const laml_forest* f) {
@@ -1373,18 +1516,34 @@ static void pass_outside(laml_forest* f, const DevForest& F, bool with_root, con
   f->alpha_complete = cp == nullptr;
 }
 
+// the inside rows of the last call's parameters, where it left none (its
+// branch coefficients are resident)
+static void ensure_rows(laml_forest* f, const DevForest& F, hipStream_t s) {
+  if (f->rows_ok) return;
+  pass_inside_root(f, F, nullptr, nullptr, s);
+  f->rows_ok = true;
+  f->alpha_complete = false;
+}
+
 int laml_nll(laml_forest* f, const double* d, const double* nu, const double* phi, double* nll, double* site_llh,
              void* stream) {
   if (!f || !d || !nu || !phi || !nll) return fail(LAML_EINVAL, "null argument");
   DeviceGuard guard(f->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rc = prepare_chains(f);
-  if (rc) return rc;
   DevForest F = f->F;
   F.phi = phi;
+  EmState none{};
+  if (problem_now(f)) {
+    laml::run_problem(lds_view(F, f->pb), f->pb, f->TW, const_cast<double*>(d), const_cast<double*>(nu),
+                      const_cast<double*>(phi), nll, site_llh, nullptr, none, 1, 0, 0.0, laml::kPbCoef, s);
+    f->rows_ok = f->alpha_complete = f->inside_fused = false;
+    return check_launch();
+  }
+  int rc = prepare_chains(f);
+  if (rc) return rc;
+  f->rows_ok = true;
   laml::run_coef(F, d, nu, nullptr, s);
   pass_inside_root(f, F, site_llh, nullptr, s);
-  EmState none{};
   laml::run_llh(F, nll, none, 0, 0.0, s);
   return check_launch();
 }
@@ -1396,9 +1555,20 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
   hipStream_t s = static_cast<hipStream_t>(stream);
   DevForest F = f->F;
   F.phi = phi;
+  EmState none{};
+  if (problem_now(f)) {
+    const DevForest G = lds_view(F, f->pb);
+    laml::run_problem(G, f->pb, f->TW, const_cast<double*>(d), const_cast<double*>(nu), const_cast<double*>(phi), nll,
+                      nullptr, nullptr, none, 1, 0, 0.0, laml::kPbCoef | laml::kPbOut, s);
+    f->rows_ok = f->alpha_complete = f->inside_fused = false;
+    laml::run_counts(G, counts, s);
+    laml::run_rtilde(G, rtilde, nullptr, s);
+    return check_launch();
+  }
   laml::run_coef(F, d, nu, nullptr, s);
   int rc = prepare_chains(f);
   if (rc) return rc;
+  f->rows_ok = true;
   if (f->pass_mode == 1) {
     f->inside_fused = false;
     laml::run_tree_walk(F, f->TW, f->W, 7, nullptr, nullptr, s);
@@ -1413,11 +1583,26 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
     pass_inside_root(f, F, nullptr, nullptr, s);
     pass_outside(f, F, false, nullptr, s);
   }
-  EmState none{};
   laml::run_llh(F, nll, none, 0, 0.0, s);
   laml::run_counts(F, counts, s);
   laml::run_rtilde(F, rtilde, nullptr, s);
   return check_launch();
+}
+
+// the outside pass over the state of the last call: from its rows, or with
+// the inside pass again where it left none.  Returns the view of F that holds
+// the partial counts.
+static DevForest outside_again(laml_forest* f, const DevForest& F, const double* phi, hipStream_t s) {
+  if (!f->rows_ok && problem_now(f)) {
+    const DevForest G = lds_view(F, f->pb);
+    EmState none{};
+    laml::run_problem(G, f->pb, f->TW, nullptr, nullptr, const_cast<double*>(phi), nullptr, nullptr, nullptr, none, 1,
+                      0, 0.0, laml::kPbOut, s);
+    return G;
+  }
+  ensure_rows(f, F, s);
+  pass_outside(f, F, true, nullptr, s);
+  return F;
 }
 
 int laml_outside(laml_forest* f, const double* phi, double* counts, double* rtilde, void* stream) {
@@ -1428,9 +1613,9 @@ int laml_outside(laml_forest* f, const double* phi, double* counts, double* rtil
   if (rc) return rc;
   DevForest F = f->F;
   F.phi = phi;
-  pass_outside(f, F, true, nullptr, s);
-  laml::run_counts(F, counts, s);
-  laml::run_rtilde(F, rtilde, nullptr, s);
+  const DevForest G = outside_again(f, F, phi, s);
+  laml::run_counts(G, counts, s);
+  laml::run_rtilde(G, rtilde, nullptr, s);
   return check_launch();
 }
 
@@ -1443,8 +1628,8 @@ int laml_grad(laml_forest* f, const double* d, const double* nu, const double* p
   if (rc) return rc;
   DevForest F = f->F;
   F.phi = phi;
-  pass_outside(f, F, true, nullptr, s);
-  laml::run_grad(F, d, nu, phi, grad_d, grad_nu, grad_phi, s);
+  const DevForest G = outside_again(f, F, phi, s);
+  laml::run_grad(G, d, nu, phi, grad_d, grad_nu, grad_phi, s);
   return check_launch();
 }
 
@@ -1499,8 +1684,33 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
   const int P = F.num_problems;
   EmState em = f->em;
   em.trace = trace;
+  if (problem_now(f) && !f->ultra_on) {
+    // whole problems, a block each: kPbSteps EM steps a launch, the done
+    // flags read back between launches
+    constexpr int kPbSteps = 128;
+    const DevForest G = lds_view(F, f->pb);
+    laml::run_em_reset(em, P, s);
+    std::vector<int32_t> done_h(P);
+    for (int64_t step = 0; step <= max_iter; step += kPbSteps) {
+      const int steps = (int)std::min<int64_t>(kPbSteps, (int64_t)max_iter + 1 - step);
+      laml::run_problem(G, f->pb, f->TW, d, nu, phi, nll, nullptr, iters, em, steps, max_iter, tol,
+                        laml::kPbCoef | laml::kPbOut | laml::kPbEm, s);
+      int rc = check_launch();
+      if (rc) return rc;
+      if (tol > 0.0 && step + kPbSteps <= max_iter) {
+        LAML_HIP(hipMemcpyAsync(done_h.data(), em.done, sizeof(int32_t) * P, hipMemcpyDeviceToHost, s));
+        LAML_HIP(hipStreamSynchronize(s));
+        bool all = true;
+        for (int p = 0; p < P; ++p) all = all && done_h[p];
+        if (all) break;
+      }
+    }
+    f->rows_ok = f->alpha_complete = f->inside_fused = false;
+    return LAML_OK;
+  }
   int prc = prepare_chains(f);
   if (prc) return prc;
+  f->rows_ok = true;
   laml::run_em_reset(em, P, s);
   // The EM step is captured once into a HIP graph and replayed: its kernel
   // arguments do not change between steps (the step number lives on the
@@ -1575,6 +1785,7 @@ int laml_posteriors(laml_forest* f, const double* phi, double* post0_host, doubl
   // the last outside pass kept heavy children's outside states in
   // registers: form every node's outside row again from the resident inside
   // state (one outside pass in level launches)
+  ensure_rows(f, F, s);
   if (!f->alpha_complete) pass_outside(f, F, true, nullptr, s, false);
   const int64_t rows = f->leaf_rows + f->int_rows;
   double *p0 = nullptr, *pS = nullptr;
@@ -1622,6 +1833,7 @@ int laml_posteriors_noalloc(laml_forest* f, const double* phi, double* post0_hos
   hipStream_t s = static_cast<hipStream_t>(stream);
   DevForest F = f->F;
   F.phi = phi;
+  ensure_rows(f, F, s);
   if (!f->alpha_complete) pass_outside(f, F, true, nullptr, s, false);
   double* p0 = f->post_scratch;
   double* pS = p0 + rows;
@@ -1653,11 +1865,10 @@ int laml_quartet_em(laml_forest* f, int32_t num_candidates, const int32_t* quart
                              "(laml_forest_set_fusion)");
   DeviceGuard guard(f->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (!f->alpha_complete) {
-    DevForest F = f->F;
-    F.phi = phi;
-    pass_outside(f, F, true, nullptr, s, false);
-  }
+  DevForest F = f->F;
+  F.phi = phi;
+  ensure_rows(f, F, s);
+  if (!f->alpha_complete) pass_outside(f, F, true, nullptr, s, false);
   laml::run_quartet_em(f->F, num_candidates, quartet_nodes, lengths_in, optimise, llh_const, nu, phi, max_iter, tol,
                        lengths_out, nll, iters, s);
   return check_launch();

@@ -140,9 +140,9 @@ __device__ __forceinline__ int exp_of(double m) {
   return ex;
 }
 
-// 1 / x for x in [0.5, 1): the hardware estimate and two Newton steps (no
-// scaling for extreme arguments)
-__device__ __forceinline__ double rcp_unit(double x) {
+// 1 / x where x and 1 / x are normal numbers: the hardware estimate and two
+// Newton steps (no scaling for extreme arguments)
+__device__ __forceinline__ double rcp_normal(double x) {
   double r = __builtin_amdgcn_rcp(x);
   r = fma(fma(-x, r, 1.0), r, r);
   return fma(fma(-x, r, 1.0), r, r);
@@ -221,13 +221,13 @@ __device__ __forceinline__ double bcast_last(double x) {
   return __hiloint2double(hi, lo);
 }
 
-// Sum over an aligned segment of W lanes (W = 8..64) with DPP: quad
+// Sum over an aligned segment of W lanes (W = 1..64) with DPP: quad
 // permutations, row rotations and row broadcasts.  The sum is valid in the
 // LAST lane of each segment.
 template <int W>
 __device__ __forceinline__ double seg_sum_last(double x) {
-  x += dpp_mov<0xb1>(x);  // quad_perm [1,0,3,2]
-  x += dpp_mov<0x4e>(x);  // quad_perm [2,3,0,1]
+  if (W >= 2) x += dpp_mov<0xb1>(x);  // quad_perm [1,0,3,2]
+  if (W >= 4) x += dpp_mov<0x4e>(x);  // quad_perm [2,3,0,1]
   if (W >= 8) x += dpp_mov<0x124>(x);  // row_ror:4
   if (W >= 16) x += dpp_mov<0x128>(x);  // row_ror:8
   if (W >= 32) x += dpp_mov<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3

@@ -19,14 +19,7 @@
 
 namespace laml {
 
-__global__ void k_coef(DevForest F, const double* __restrict__ d, const double* __restrict__ nu,
-                       const int32_t* __restrict__ done) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= F.num_nodes) return;
-  const int p = F.tree_prob[F.tree_of[v]];
-  if (done && done[p]) return;
-  const double dv = d[v];
-  const double nv = nu[p];
+__device__ __forceinline__ Coef branch_coef(double dv, double nv) {
   Coef c;
   c.p1n = exp(-(1.0 + nv) * dv);
   c.pn = exp(-nv * dv);
@@ -35,7 +28,16 @@ __global__ void k_coef(DevForest F, const double* __restrict__ d, const double* 
   c.msil = frexp(-expm1(-nv * dv), &es);
   c.esil = c.msil != 0.0 ? es : 0;
   c.pad = 0;
-  F.coef[v] = c;
+  return c;
+}
+
+__global__ void k_coef(DevForest F, const double* __restrict__ d, const double* __restrict__ nu,
+                       const int32_t* __restrict__ done) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= F.num_nodes) return;
+  const int p = F.tree_prob[F.tree_of[v]];
+  if (done && done[p]) return;
+  F.coef[v] = branch_coef(d[v], nu[p]);
 }
 
 // Segment mapping shared by the level kernels: a block of 256 threads holds
@@ -912,7 +914,7 @@ __device__ __forceinline__ void cond_post(int lu, double a0, double aX, double p
   const double BA = z ? 0.0 : ep[0].eA * ep[1].eA;
   // the power of two that the inside pass scaled u's vector by
   const double sc = ldexp(1.0, min(-exp_of(fmax(B0, BA)), 1000));
-  const double f0 = z ? rcp_unit(B0 * sc) * sc : a0 * sc;
+  const double f0 = z ? rcp_normal(B0 * sc) * sc : a0 * sc;
   const double fX = z ? 0.0 : aX * sc;
   o.rt = 0.0;
 #pragma unroll
@@ -1699,9 +1701,9 @@ __global__ void __launch_bounds__(256) k_counts(DevForest F, double* __restrict_
   const int v = (int)(idx / 5);
   const int j = (int)(idx - (int64_t)v * 5);
   const int C = (F.tree_nsites[F.tree_of[v]] + F.chunk_w - 1) / F.chunk_w;
-  const double* src = F.cpart + (int64_t)v * F.max_chunks * 5 + j;
+  const double* src = F.cpart + v * F.cp_v + j;
   double s = 0.0;
-  for (int c = 0; c < C; ++c) s += src[c * 5];
+  for (int c = 0; c < C; ++c) s += src[c * F.cp_c];
   counts[idx] = s;
 }
 
@@ -1766,16 +1768,16 @@ constexpr int kRedThreads = 1024;
 // to 8 chunks are loaded together before the additions
 __device__ __forceinline__ void add_node_rt(const DevForest& F, int64_t v, int C, double& s) {
   constexpr int kC = 8;
-  const double* src = F.rt_part + v * F.max_chunks;
+  const double* src = F.rt_part + v * F.rt_v;
   if (C <= kC) {
     double x[kC];
 #pragma unroll
-    for (int c = 0; c < kC; ++c) x[c] = c < C ? src[c] : 0.0;
+    for (int c = 0; c < kC; ++c) x[c] = c < C ? src[c * F.rt_c] : 0.0;
 #pragma unroll
     for (int c = 0; c < kC; ++c)
       if (c < C) s += x[c];
   } else {
-    for (int c = 0; c < C; ++c) s += src[c];
+    for (int c = 0; c < C; ++c) s += src[c * F.rt_c];
   }
 }
 
@@ -1842,26 +1844,47 @@ __device__ double solve_branch(const BranchObj& o, double dmin, double dmax, dou
   return x;
 }
 
+// the objective of a branch with expected counts s (clamped and renormalised
+// in place) over K sites
+__device__ __forceinline__ BranchObj branch_obj(double (&s)[5], double K, double nu0) {
+  double tot = 0.0;
+#pragma unroll
+  for (int j = 0; j < 5; ++j) {
+    s[j] = fmax(kEpsS, s[j]);
+    tot += s[j];
+  }
+#pragma unroll
+  for (int j = 0; j < 5; ++j) s[j] = s[j] / tot * K;
+  BranchObj o;
+  o.nu = nu0;
+  o.A = (nu0 + 1.0) * s[0] + nu0 * s[1] + nu0 * s[3];
+  o.S1 = s[1];
+  o.B = nu0 > kEpsNu ? (s[2] + s[4]) : 0.0;
+  return o;
+}
+// the new length of a free branch, and its coefficients of the nu problem
+__device__ __forceinline__ double branch_length(const DevForest& F, double (&s)[5], double K, double nu0, double d,
+                                                double& na, double& nb) {
+  const BranchObj o = branch_obj(s, K, nu0);
+  na = s[0] + s[1] + s[3];
+  nb = s[2] + s[4];
+  return solve_branch(o, F.dmin, F.dmax, d);
+}
+
 // Branch lengths of every free branch (EM_solver.py:328-366): counts are
 // clamped at eps_s and renormalised to sum K, then the per-branch concave
 // problem is solved exactly with the current nu.  Also stages the nu
 // problem's per-branch coefficients at the branch's position in its problem.
-__global__ void __launch_bounds__(64) k_branch(DevForest F, const double* __restrict__ counts,
-                                                double* __restrict__ d, const double* __restrict__ nu,
-                                                const int32_t* __restrict__ done, UltraDev U, int ultra) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= F.num_nodes) return;
-  const int t = F.tree_of[v];
-  const int p = F.tree_prob[t];
-  if (done && done[p]) return;
-  const int pos = F.node_pos[v];
+__device__ __forceinline__ void branch_update(const DevForest& F, int v, int p, int pos,
+                                              const double* __restrict__ counts, double* __restrict__ d, double nu0,
+                                              const UltraDev& U, int ultra) {
   if (!F.free_branch[v]) {
     F.nu_a[pos] = 0.0;
     F.nu_b[pos] = 0.0;
     F.nu_d[pos] = d[v];
     return;
   }
-  const int Kt = F.tree_nsites[t];
+  const int Kt = F.tree_nsites[F.tree_of[v]];
   const double K = (double)Kt;
   double s[5];
   if (counts) {
@@ -1873,22 +1896,9 @@ __global__ void __launch_bounds__(64) k_branch(DevForest F, const double* __rest
     for (int j = 0; j < 5; ++j) s[j] = 0.0;
     for (int c = 0; c < C; ++c)
 #pragma unroll
-      for (int j = 0; j < 5; ++j) s[j] += F.cpart[((int64_t)v * F.max_chunks + c) * 5 + j];
+      for (int j = 0; j < 5; ++j) s[j] += F.cpart[v * F.cp_v + c * F.cp_c + j];
   }
-  double tot = 0.0;
-#pragma unroll
-  for (int j = 0; j < 5; ++j) {
-    s[j] = fmax(kEpsS, s[j]);
-    tot += s[j];
-  }
-#pragma unroll
-  for (int j = 0; j < 5; ++j) s[j] = s[j] / tot * K;
-  const double nu0 = nu[p];
-  BranchObj o;
-  o.nu = nu0;
-  o.A = (nu0 + 1.0) * s[0] + nu0 * s[1] + nu0 * s[3];
-  o.S1 = s[1];
-  o.B = nu0 > kEpsNu ? (s[2] + s[4]) : 0.0;
+  const BranchObj o = branch_obj(s, K, nu0);
   if (ultra) {
     // the ultrametric solve needs the objective of every free branch; the
     // lengths are set by k_ultra and the nu staging refreshed after it
@@ -1907,6 +1917,16 @@ __global__ void __launch_bounds__(64) k_branch(DevForest F, const double* __rest
   F.nu_a[pos] = s[0] + s[1] + s[3];
   F.nu_b[pos] = s[2] + s[4];
   F.nu_d[pos] = dn;
+}
+
+__global__ void __launch_bounds__(64) k_branch(DevForest F, const double* __restrict__ counts,
+                                                double* __restrict__ d, const double* __restrict__ nu,
+                                                const int32_t* __restrict__ done, UltraDev U, int ultra) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= F.num_nodes) return;
+  const int p = F.tree_prob[F.tree_of[v]];
+  if (done && done[p]) return;
+  branch_update(F, v, p, F.node_pos[v], counts, d, nu[p], U, ultra);
 }
 
 // phi closed form (EM_solver.py:318-326) and nu (EM_solver.py:392-407).
@@ -1955,6 +1975,16 @@ __device__ __forceinline__ bool nu_newton_step(double x, double G, double Hs, do
   return top - lo <= 1e-12 * top;
 }
 
+// One branch's terms of h'(x) and h''(x): a = S0 + S1 + S3, b = S2 + S4 of
+// the branch, its length dv.
+__device__ __forceinline__ void nu_term(double a, double bb, double dv, double x, double& g, double& h) {
+  if (bb == 0.0) return;
+  const double en = expm1(x * dv);
+  const double ri = 1.0 / en;
+  g += dv * fma(bb, ri, -a);
+  h -= bb * dv * dv * (en + 1.0) * (ri * ri);
+}
+
 // One thread's share (stride kNuThreads from branch position i0) of h'(x)
 // and h''(x) over the branch positions [i0 - lane offset, pe) of a span.
 // Every nu kernel sums through these two functions and in the same span
@@ -1962,15 +1992,7 @@ __device__ __forceinline__ bool nu_newton_step(double x, double G, double Hs, do
 // kernel runs and whatever else the forest holds.
 __device__ __forceinline__ void nu_span_terms(const DevForest& F, int pb, int pe, int lt, double x, double& g,
                                               double& h) {
-  for (int i = pb + lt; i < pe; i += kNuThreads) {
-    const double bb = F.nu_b[i];
-    if (bb == 0.0) continue;
-    const double dv = F.nu_d[i];
-    const double en = expm1(x * dv);
-    const double ri = 1.0 / en;
-    g += dv * fma(bb, ri, -F.nu_a[i]);
-    h -= bb * dv * dv * (en + 1.0) * (ri * ri);
-  }
+  for (int i = pb + lt; i < pe; i += kNuThreads) nu_term(F.nu_a[i], F.nu_b[i], F.nu_d[i], x, g, h);
 }
 __device__ __forceinline__ void rt_span(const DevForest& F, int pb, int pe, int lt, int C, double& rt) {
   for (int i = pb + lt; i < pe; i += kNuThreads) add_node_rt(F, F.prob_nodes[i], C, rt);
@@ -2072,18 +2094,19 @@ __global__ void __launch_bounds__(kNuThreads) k_nu_eval(DevForest F, const doubl
 // The M-step status of each problem is final after this kernel.
 constexpr int kNuSolveThreads = 1024;
 constexpr int kNuSolveMaxNodes = 65536;
-constexpr int kNuGroups = kNuSolveThreads / kNuThreads;
 
 // sums over the spans of problem p in k_nu_eval's order: (h', h'') at x when
 // want_g, the dropout sum when want_rt
-__device__ void nu_eval_spans(const DevForest& F, int p, double x, bool want_g, bool want_rt, double& G, double& Hs,
-                              double& RT, double* sh) {
+template <int NT>
+__device__ __forceinline__ void nu_eval_spans(const DevForest& F, int p, double x, bool want_g, bool want_rt,
+                                              double& G, double& Hs, double& RT, double* sh) {
   const int nparts = F.prob_blk_off[p + 1] - F.prob_blk_off[p];
   const int b = F.prob_node_off[p], e = F.prob_node_off[p + 1];
   const int span = (e - b + nparts - 1) / nparts;
   const int grp = threadIdx.x / kNuThreads, lt = threadIdx.x % kNuThreads;
   const int wid = threadIdx.x >> 6;
   const int C = want_rt ? (F.tree_nsites[F.prob_tree_off[p]] + F.chunk_w - 1) / F.chunk_w : 0;
+  constexpr int kNuGroups = NT / kNuThreads;
   constexpr int kW = kNuThreads / 64;  // waves per span
   G = 0.0;
   Hs = 0.0;
@@ -2101,8 +2124,8 @@ __device__ void nu_eval_spans(const DevForest& F, int p, double x, bool want_g, 
     rt = seg_sum<64>(rt);
     if ((threadIdx.x & 63) == 0) {
       sh[wid] = g;
-      sh[kNuSolveThreads / 64 + wid] = h;
-      sh[2 * (kNuSolveThreads / 64) + wid] = rt;
+      sh[NT / 64 + wid] = h;
+      sh[2 * (NT / 64) + wid] = rt;
     }
     __syncthreads();
     for (int j = 0; j < kNuGroups && q0 + j < nparts; ++j) {
@@ -2110,8 +2133,8 @@ __device__ void nu_eval_spans(const DevForest& F, int p, double x, bool want_g, 
 #pragma unroll
       for (int w = 0; w < kW; ++w) {
         sg += sh[j * kW + w];
-        shh += sh[kNuSolveThreads / 64 + j * kW + w];
-        sr += sh[2 * (kNuSolveThreads / 64) + j * kW + w];
+        shh += sh[NT / 64 + j * kW + w];
+        sr += sh[2 * (NT / 64) + j * kW + w];
       }
       G += sg;
       Hs += shh;
@@ -2121,15 +2144,13 @@ __device__ void nu_eval_spans(const DevForest& F, int p, double x, bool want_g, 
   }
 }
 
-__global__ void __launch_bounds__(kNuSolveThreads) k_nu_solve(DevForest F, const double* __restrict__ rtilde_in,
-                                                             double* __restrict__ nu, double* __restrict__ phi,
-                                                             const int32_t* __restrict__ done, int resume) {
-  __shared__ double sh[3 * (kNuSolveThreads / 64)];
-  const int p = blockIdx.x;
+// Runs problem p's solve by the whole block of NT threads (sh: 3 NT / 64
+// doubles); nu and phi are also returned, the same in every thread.
+template <int NT>
+__device__ __forceinline__ void nu_solve(const DevForest& F, int p, const double* __restrict__ rtilde_in,
+                                         double* __restrict__ nu_p, double* __restrict__ phi_p, int resume, double* sh,
+                                         double& nu_io, double& phi_io) {
   NuState* st = F.nu_state + p;
-  if (done && done[p]) return;
-  // every thread reads the same flag, written by an earlier launch
-  if (resume && st->fin) return;
   const uint32_t flags = F.prob_flags[p];
   const bool opt_nu = (flags & 2u) && F.prob_nfree[p] > 0;
   int status = 0;
@@ -2137,19 +2158,20 @@ __global__ void __launch_bounds__(kNuSolveThreads) k_nu_solve(DevForest F, const
   int evals;
   bool fin = false;
   if (!resume) {
-    x = (nu[p] > 0.0 && nu[p] < 1.0) ? nu[p] : 0.5;
+    x = (nu_io > 0.0 && nu_io < 1.0) ? nu_io : 0.5;
     lo = 0.0;
     hi = 2.0;  // hi > 1: the bound x = 1 has not been evaluated
     // the first evaluation also sums the dropout responsibilities, as
     // k_nu_eval's first launch does
     const bool want_rt = (flags & 1u) && !rtilde_in;
     double G, Hs, RT;
-    nu_eval_spans(F, p, x, opt_nu, want_rt, G, Hs, RT, sh);
+    nu_eval_spans<NT>(F, p, x, opt_nu, want_rt, G, Hs, RT, sh);
     if (flags & 1u) {
       const double r = rtilde_in ? rtilde_in[p] : RT;
       double phi_star = r / (F.prob_nobs[p] + r);
       if (fabs(phi_star) < F.prob_phimin[p]) phi_star = 0.0;
-      if (threadIdx.x == 0) phi[p] = phi_star;
+      phi_io = phi_star;
+      if (threadIdx.x == 0) *phi_p = phi_star;
     }
     status = st->d_bad ? 1 : 0;
     __syncthreads();  // every thread has read d_bad before thread 0 clears it
@@ -2172,19 +2194,32 @@ __global__ void __launch_bounds__(kNuSolveThreads) k_nu_solve(DevForest F, const
   }
   for (; evals < kNuMaxEvals && !fin; ++evals) {
     double G, Hs, RT;
-    nu_eval_spans(F, p, x, true, false, G, Hs, RT, sh);
+    nu_eval_spans<NT>(F, p, x, true, false, G, Hs, RT, sh);
     double xn;
     fin = nu_newton_step(x, G, Hs, lo, hi, xn);
     x = xn;
   }
+  nu_io = x;
   if (threadIdx.x == 0) {
-    nu[p] = x;
+    *nu_p = x;
     st->x = x;
     st->lo = lo;
     st->hi = hi;
     st->fin = 1;
     st->status = status | (fin ? 0 : 2);
   }
+}
+
+__global__ void __launch_bounds__(kNuSolveThreads) k_nu_solve(DevForest F, const double* __restrict__ rtilde_in,
+                                                             double* __restrict__ nu, double* __restrict__ phi,
+                                                             const int32_t* __restrict__ done, int resume) {
+  __shared__ double sh[3 * (kNuSolveThreads / 64)];
+  const int p = blockIdx.x;
+  if (done && done[p]) return;
+  // every thread reads the same flag, written by an earlier launch
+  if (resume && F.nu_state[p].fin) return;
+  double nv = nu[p], pv = phi[p];
+  nu_solve<kNuSolveThreads>(F, p, rtilde_in, nu + p, phi + p, resume, sh, nv, pv);
 }
 
 // ---------------------------------------------------------------------------
@@ -2207,7 +2242,7 @@ __global__ void k_grad_branch(DevForest F, const double* __restrict__ d, const d
   double s[5] = {0, 0, 0, 0, 0};
   for (int c = 0; c < C; ++c)
 #pragma unroll
-    for (int j = 0; j < 5; ++j) s[j] += F.cpart[((int64_t)v * F.max_chunks + c) * 5 + j];
+    for (int j = 0; j < 5; ++j) s[j] += F.cpart[v * F.cp_v + c * F.cp_c + j];
   const double dv = d[v], x = nu[p];
   double g = -(1.0 + x) * s[0] + s[1] * (1.0 / expm1(dv) - x) - x * s[3];
   if (s[2] + s[4] != 0.0) g += (s[2] + s[4]) * x / expm1(x * dv);
@@ -2507,18 +2542,6 @@ __device__ __forceinline__ QTop q_top(const QTop& a, double sc, const Eps& ew) {
   return t;
 }
 
-__device__ __forceinline__ Coef q_coef(double d, double nu) {
-  Coef c;
-  c.p1n = exp(-(1.0 + nu) * d);
-  c.pn = exp(-nu * d);
-  c.mut = -expm1(-d) * c.pn;
-  int es;
-  c.msil = frexp(-expm1(-nu * d), &es);
-  c.esil = c.msil != 0.0 ? es : 0;
-  c.pad = 0;
-  return c;
-}
-
 // inside of a node from its two children's edge values, and the power of two
 // sc that it was scaled by; returns the label
 __device__ __forceinline__ int q_combine(int la, int lb, const Eps& ea, const Eps& eb, double& B0, double& BA,
@@ -2592,7 +2615,7 @@ __global__ void __launch_bounds__(256) k_quartet_em(DevForest F, int ncand, cons
   for (int it = 0; it <= max_iter; ++it) {
     Coef cf[5];
 #pragma unroll
-    for (int j = 0; j < 5; ++j) cf[j] = q_coef(d[j], nu);
+    for (int j = 0; j < 5; ++j) cf[j] = branch_coef(d[j], nu);
     double S[5][5];
 #pragma unroll
     for (int j = 0; j < 5; ++j)
@@ -2718,6 +2741,781 @@ void run_quartet_em(const DevForest& F, int ncand, const int32_t* qnodes, const 
   if (ncand <= 0) return;
   hipLaunchKernelGGL(k_quartet_em, dim3((ncand + 3) / 4), dim3(256), 0, s, F, ncand, qnodes, len_in, opt_mask,
                      llh_const, nu, phi, max_iter, tol, len_out, nll_out, iters_out);
+}
+
+// ---------------------------------------------------------------------------
+// LDS passes: a block keeps the state of every internal node of one tree at
+// its sites in LDS and runs the pass (inside levels, root, outside levels)
+// with barriers between levels.  A level then costs an LDS round trip and the
+// arithmetic (0.4 us inside, 0.8 us outside for narrow levels) where rows in
+// global memory cost a store, a barrier and a load through the L2, or a
+// launch.
+//
+// A thread takes two neighbouring sites of a node, kLdsCells (node, site)
+// cells a step.  What they need besides the LDS state (where the children's
+// vectors are, label flags, prior weights, branch coefficients) does not
+// depend on the level below, is laid out in the order the threads read it, and
+// is loaded one step ahead, across the barrier, into one of two register sets
+// used in turn: copying a set would wait for it.  A leaf child's vector is one
+// of four constant cells, so that leaves and internal children take the same
+// path.  The outside pass writes a child's state over its inside vector (its
+// last use is the parent's step) and a node's partial counts over its own
+// state, so that no store to global memory is pending when a step waits for
+// its loads.  Wide levels are bound by the CU's L1 and instruction issue
+// (hence two sites a thread, which share coefficients and sums, and silencing
+// terms only in wavefronts that hold a '?' cell), narrow ones by latency.
+//
+// Eight sites of a node share a partial-count slot.  Their four lanes lie in
+// the four 16-lane rows (lane 16 r + c: sites 2 r and 2 r + 1 of group c), so
+// that the eleven sums over them take two halving row swaps.
+// ---------------------------------------------------------------------------
+constexpr int kLdsThreads = 512;
+constexpr int kLdsCells = 2 * kLdsThreads;  // cells a step
+constexpr int kLdsWave = 128;               // of them a wavefront's
+// the 8 x 16 bytes of state of the sites that share a slot hold its eleven sums
+constexpr int kLdsR = kLdsSlotSites;
+
+// flags of a cell: label kinds of the node and its children, kinds of child
+enum : uint32_t {
+  kLdsUz = 1,                       // the node is 'z' (label 0)
+  kLdsZ0 = 2, kLdsZ1 = 4,           // child 0 / 1 is 'z'
+  kLdsQ0 = 8, kLdsQ1 = 16,          // child 0 / 1 is '?'
+  kLdsLeaf0 = 32, kLdsLeaf1 = 64,
+  kLdsDrop0 = 128, kLdsDrop1 = 256  // child 0 / 1 is a leaf with a missing entry
+};                                  // (the upper 16 bits: the cell's own place)
+// cells of the constant leaf vectors: unedited, edited, missing, none
+// (explicitly silenced entries, and the sites past the tree's); a cell that
+// is written and never read
+constexpr int kLdsLeafCells = 8, kLdsNoCell = 4;
+
+// Where cell c (node-major) lies: the sites of a group of eight in an order
+// that depends on the group, so that the lanes of a row (the same site of 16
+// groups) fall into different banks.
+__device__ __forceinline__ int lds_place(int c) {
+  return (c + kLdsLeafCells) ^ (((c >> 4) & 3) << 1) ^ ((c >> 6) & 1);
+}
+// the first cell of thread t's pair, of a step's cells
+__device__ __forceinline__ int lds_pair(unsigned t) {
+  return (int)((t >> 6) * kLdsWave + 8u * (t & 15u) + 2u * ((t >> 4) & 3u));
+}
+
+// every LDS access of the block so far is done; global loads and stores stay
+// in flight
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+struct LdsItem {
+  uint4 w;        // per cell: places of the children's vectors; flags and its own place
+  double2 q[2];   // per cell: prior weights of the children
+  LdsCoef cf;
+  bool on;        // whether the lane has cells
+};
+
+// one block's tree
+struct LdsCtx {
+  int sb, nint, H, k0, K;
+  unsigned magic;          // floor(i / sb) = umulhi(i, magic) for i < 2^20
+  const uint4* w;
+  const double4* q;
+  const LdsRec* rec;
+  const LdsCoef* lcoef;
+  double phi;
+  double2* st;             // LDS: the cells' vectors
+  int* sE;                 // LDS: their exponents
+  int2* lvl;               // LDS: first local number and first table entry of level h (level H: the end)
+  int2 lreg;               // lane i of a wavefront: lvl[i]
+  double* rpart;           // LDS: the stem's sums, 3 per kLdsR sites
+};
+
+// element i (wave-uniform) of an array that no kernel writes while it runs
+template <typename T>
+__device__ __forceinline__ T uniform_at(const T* p, int i) {
+  return uniform_load(p + __builtin_amdgcn_readfirstlane(i));
+}
+
+// the constant leaf vectors (as leaf_beta)
+__device__ __forceinline__ void lds_leaves(LdsCtx& x, double phi) {
+  const int t = (int)threadIdx.x;
+  x.phi = phi;
+  if (t < kLdsLeafCells) {
+    x.st[t] = make_double2(t == 0 ? 1.0 - phi : (t == 2 ? phi : 0.0), t == 1 ? 1.0 - phi : (t == 2 ? phi : 0.0));
+    x.sE[t] = 0;
+  }
+}
+
+__device__ __forceinline__ LdsCtx lds_ctx(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, const LdsBlk& B,
+                                          double phi, char* lds) {
+  LdsCtx x;
+  x.sb = B.sb;
+  x.nint = B.nint;
+  x.k0 = B.k0;
+  x.K = uniform_at(F.tree_nsites, B.tree);
+  const int lb = uniform_at(TW.lvl_base, B.tree);
+  x.H = uniform_at(TW.lvl_base, B.tree + 1) - lb;
+  const int ib = uniform_at(L.int_base, B.tree);
+  x.magic = 0xffffffffu / (unsigned)B.sb + 1u;
+  x.w = L.w + B.tab;
+  x.q = L.q + B.tab;
+  x.rec = L.rec + ib;
+  x.lcoef = L.lcoef + ib;
+  const int cells = B.nint * B.sb + kLdsLeafCells;
+  x.st = reinterpret_cast<double2*>(lds);
+  x.rpart = reinterpret_cast<double*>(x.st + cells);
+  x.lvl = reinterpret_cast<int2*>(x.rpart + 3 * (B.sb / kLdsR));
+  x.sE = reinterpret_cast<int*>(x.lvl + x.H + 1);
+  lds_leaves(x, phi);
+  for (int h = (int)threadIdx.x; h < x.H; h += kLdsThreads) x.lvl[h + 1] = L.lvl_off[lb + h];
+  lds_barrier();
+  x.lreg = x.lvl[min((int)(threadIdx.x & 63), x.H)];
+  return x;
+}
+
+// The uniform walk over a tree's steps: level h, its cells from i0 on, n in
+// all; up or down the levels.
+struct LdsStep {
+  int h, i0, n, l0, e0;  // the level's first local number and table entry
+};
+__device__ __forceinline__ void lds_level(const LdsCtx& x, int h, LdsStep& p) {
+  p.h = h;
+  p.i0 = 0;
+  int l1;
+  if (h < 63) {
+    p.l0 = __builtin_amdgcn_readlane(x.lreg.x, h);
+    p.e0 = __builtin_amdgcn_readlane(x.lreg.y, h);
+    l1 = __builtin_amdgcn_readlane(x.lreg.x, h + 1);
+  } else {
+    p.l0 = __builtin_amdgcn_readfirstlane(x.lvl[h].x);
+    p.e0 = __builtin_amdgcn_readfirstlane(x.lvl[h].y);
+    l1 = __builtin_amdgcn_readfirstlane(x.lvl[h + 1].x);
+  }
+  p.n = (l1 - p.l0) * x.sb;
+}
+// the step after p among levels 1 .. H - 1 (n = 0: none), of `width` cells;
+// whether it starts a level
+__device__ __forceinline__ bool lds_next(const LdsCtx& x, int dir, int width, const LdsStep& p, LdsStep& o) {
+  o = p;
+  o.i0 += width;
+  if (o.i0 < p.n) return false;
+  o.h = p.h + dir;
+  o.n = 0;
+  if (o.h >= 1 && o.h < x.H) lds_level(x, o.h, o);
+  return true;
+}
+
+// The wavefront's cells of step p, t the thread's number in the step: every
+// lane loads (lanes past the level's cells its last one), so that the number
+// of loads in flight is known.
+__device__ __forceinline__ void lds_fetch(const LdsCtx& x, const LdsStep& p, unsigned t, LdsItem& it) {
+  const int i = p.i0 + lds_pair(t);
+  const unsigned l = (unsigned)p.l0 + __umulhi((unsigned)min(i, p.n - 1), x.magic);
+  it.on = i < p.n;
+  const unsigned e = (unsigned)(p.e0 + p.i0 / 2) + t;
+  it.w = row_at(x.w, e);
+  const double4 q = row_at(x.q, e);
+  it.q[0] = make_double2(q.x, q.y);
+  it.q[1] = make_double2(q.z, q.w);
+  it.cf = row_at(x.lcoef, l);
+}
+__device__ __forceinline__ bool lds_any_q(const LdsItem& it) {
+  return __any(it.on && ((it.w.y | it.w.w) & (kLdsQ0 | kLdsQ1)));
+}
+
+// What a thread's two cells read from LDS: their children's vectors, loaded
+// before anything is stored (a load may not pass a store).
+struct LdsIn {
+  double2 b[2][2];
+  int E[2][2], pl[2][2];
+};
+template <bool kE>
+__device__ __forceinline__ void lds_load(const LdsCtx& x, const LdsItem& it, LdsIn& o) {
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const uint32_t w = c == 0 ? it.w.x : it.w.z;
+    o.pl[c][0] = w & 0xffffu;
+    o.pl[c][1] = w >> 16;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      o.b[c][i] = x.st[o.pl[c][i]];
+      o.E[c][i] = kE ? x.sE[o.pl[c][i]] : 0;
+    }
+  }
+}
+// Edge values of child i of a cell (edge() with the label kinds from the
+// flags: the inside vector is 0 where edge() selects 0; kQ false: no '?' cell
+// in the wavefront, s0 = 1 and s1 = 0).
+template <bool kQ>
+__device__ __forceinline__ Eps lds_edge(const LdsCoef& c, int i, uint32_t fl, const double2& b, int E, double mq) {
+#pragma clang fp contract(off)
+  Eps r;
+  r.e0 = fma(mq, b.y, c.p1n[i] * b.x);
+  r.eA = c.pn[i] * b.y;
+  r.e = E;
+  r.s0 = 1.0;
+  r.s1 = 0.0;
+  if (kQ) {
+    const int es = fl & (i == 0 ? kLdsQ0 : kLdsQ1) ? c.esil[i] : kZeroTop;
+    r.e = max(E, es);
+    r.s0 = ldexp(1.0, E - r.e);
+    r.s1 = ldexp(c.msil[i], es - r.e);
+    r.e0 = fma(r.e0, r.s0, r.s1);
+    r.eA = fma(r.eA, r.s0, r.s1);
+  }
+  return r;
+}
+
+template <bool kQ>
+__device__ __forceinline__ void lds_inside_cells(const LdsCtx& x, const LdsItem& it) {
+#pragma clang fp contract(off)
+  LdsIn in;
+  lds_load<true>(x, it, in);
+  double2 o[2];
+  int E[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const uint32_t fl = c == 0 ? it.w.y : it.w.w;
+    const Eps e0 = lds_edge<kQ>(it.cf, 0, fl, in.b[c][0], in.E[c][0], it.cf.mut[0] * it.q[c].x);
+    const Eps e1 = lds_edge<kQ>(it.cf, 1, fl, in.b[c][1], in.E[c][1], it.cf.mut[1] * it.q[c].y);
+    const double B0 = e0.e0 * e1.e0;
+    const double BA = fl & kLdsUz ? 0.0 : e0.eA * e1.eA;
+    const int sh = min(-exp_of(fmax(B0, BA)), 1000);
+    o[c] = make_double2(ldexp(B0, sh), ldexp(BA, sh));
+    E[c] = e0.e + e1.e - sh;
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int pl = (c == 0 ? it.w.y : it.w.w) >> 16;
+    x.st[pl] = o[c];
+    x.sE[pl] = E[c];
+  }
+}
+
+// (as cond_post; products that do not need the node's own state are formed
+// before it is known, which shortens the chain from a node to its children)
+template <bool kQ>
+__device__ __forceinline__ void lds_outside_cells(const LdsCtx& x, const LdsItem& it, double (&v)[12]) {
+#pragma clang fp contract(off)
+  LdsIn in;
+  const double2 a[2] = {x.st[it.w.y >> 16], x.st[it.w.w >> 16]};
+  lds_load<kQ>(x, it, in);
+  double2 o[2][2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const uint32_t fl = c == 0 ? it.w.y : it.w.w;
+    const double mq[2] = {it.cf.mut[0] * it.q[c].x, it.cf.mut[1] * it.q[c].y};
+    const Eps ep[2] = {lds_edge<kQ>(it.cf, 0, fl, in.b[c][0], in.E[c][0], mq[0]),
+                       lds_edge<kQ>(it.cf, 1, fl, in.b[c][1], in.E[c][1], mq[1])};
+    const bool z = fl & kLdsUz;
+    const double B0 = ep[0].e0 * ep[1].e0;
+    const double BA = z ? 0.0 : ep[0].eA * ep[1].eA;
+    const int sh = min(-exp_of(fmax(B0, BA)), 1000);
+    const double f0 = z ? rcp_normal(B0) : ldexp(a[c].x, sh);
+    const double fX = z ? 0.0 : ldexp(a[c].y, sh);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const Eps& ew = ep[1 - i];
+      double k0 = ew.e0, kX = ew.eA;
+      if (kQ) {
+        k0 *= ep[i].s0;
+        kX *= ep[i].s0;
+        v[5 * i + 2] = fma(f0, ep[i].s1 * ew.e0, v[5 * i + 2]);
+        v[5 * i + 4] = fma(fX, ep[i].s1 * ew.eA, v[5 * i + 4]);
+      }
+      const double a0 = f0 * (it.cf.p1n[i] * k0);
+      const double m = f0 * (mq[i] * k0);
+      const double pg = fX * (it.cf.pn[i] * kX);
+      const double aX = pg + m;
+      const bool cz = fl & (i == 0 ? kLdsZ0 : kLdsZ1);
+      v[5 * i] = fma(cz ? 1.0 : a0, cz ? 1.0 : in.b[c][i].x, v[5 * i]);
+      v[5 * i + 1] = fma(m, in.b[c][i].y, v[5 * i + 1]);
+      v[5 * i + 3] = fma(pg, in.b[c][i].y, v[5 * i + 3]);
+      if (kQ) v[10] = fma(fl & (i == 0 ? kLdsDrop0 : kLdsDrop1) ? x.phi : 0.0, a0 + aX, v[10]);
+      o[c][i] = make_double2(a0, aX);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const uint32_t fl = c == 0 ? it.w.y : it.w.w;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)  // (a leaf's state goes to a cell that nothing reads)
+      x.st[fl & (i == 0 ? kLdsLeaf0 : kLdsLeaf1) ? kLdsNoCell : in.pl[c][i]] = o[c][i];
+  }
+}
+
+template <int dir>
+__device__ __forceinline__ void lds_cells(const LdsCtx& x, const LdsItem& it) {
+  const bool any_q = lds_any_q(it);
+  if (dir > 0) {
+    if (!it.on) return;
+    if (any_q) lds_inside_cells<true>(x, it);
+    else lds_inside_cells<false>(x, it);
+    return;
+  }
+  double v[12];
+#pragma unroll
+  for (int m = 0; m < 12; ++m) v[m] = 0.0;
+  if (it.on) {
+    if (any_q) lds_outside_cells<true>(x, it, v);
+    else lds_outside_cells<false>(x, it, v);
+  }
+  // sums over the lanes of the group: row r ends with values 3 r .. 3 r + 2
+  // (as wave_sum12)
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    swap32(v[j], v[j + 6]);
+    v[j] += v[j + 6];
+  }
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    swap16(v[j], v[j + 3]);
+    v[j] += v[j + 3];
+  }
+  if (it.on) {
+    // the group's cells lie in one aligned run of 8 places
+    double* c = reinterpret_cast<double*>(x.st + ((it.w.y >> 16) & ~7u)) + 3 * ((threadIdx.x >> 4) & 3);
+    c[0] = v[0];
+    c[1] = v[1];
+    c[2] = v[2];
+  }
+}
+
+// One step on the cells in A while the next step's load into B.  Whether the
+// wavefront has cells at either step is uniform over it, and each case has
+// code of its own: where paths with and without the loads of B join, the
+// compiler would wait for B with A.
+template <int dir>
+__device__ __forceinline__ bool lds_turn(const LdsCtx& x, const LdsStep& p, LdsStep& o, int wave0, LdsItem& A,
+                                         LdsItem& B) {
+  const bool lvl = lds_next(x, dir, kLdsCells, p, o);
+  if (dir > 0 && o.n <= kLdsWave) o.n = 0;  // the narrow levels follow
+  const bool cur = p.i0 + wave0 < p.n;
+  if (o.i0 + wave0 < o.n) {
+    lds_fetch(x, o, threadIdx.x, B);
+    if (cur) lds_cells<dir>(x, A);
+  } else if (cur) {
+    lds_cells<dir>(x, A);
+  }
+  if (lvl) lds_barrier();
+  return o.n != 0;
+}
+// the same for the levels that one wavefront holds (it runs them without
+// barriers: its LDS accesses are in order)
+template <int dir>
+__device__ __forceinline__ bool lds_turn1(const LdsCtx& x, const LdsStep& p, LdsStep& o, LdsItem& A, LdsItem& B) {
+  lds_next(x, dir, kLdsWave, p, o);
+  if (dir < 0 && o.n > kLdsWave) o.n = 0;  // the wide levels follow
+  if (o.n != 0) {
+    lds_fetch(x, o, threadIdx.x & 63u, B);
+    lds_cells<dir>(x, A);
+  } else {
+    lds_cells<dir>(x, A);
+  }
+  return o.n != 0;
+}
+
+// The levels from h on, bottom up (dir 1) or top down (dir -1), two steps a
+// turn of the loop (one register set each): the wide ones by the block, those
+// of at most kLdsWave cells by the first wavefront (levels only get narrower
+// upwards).
+template <int dir>
+__device__ __forceinline__ void lds_wide(const LdsCtx& x, int h) {
+  LdsStep p, o;
+  LdsItem A, B;
+  const int wave0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * kLdsWave;
+  lds_level(x, h, p);
+  if (p.n <= kLdsWave) return;
+  if (wave0 < p.n) lds_fetch(x, p, threadIdx.x, A);
+  for (;;) {
+    if (!lds_turn<dir>(x, p, o, wave0, A, B)) break;
+    if (!lds_turn<dir>(x, o, p, wave0, B, A)) break;
+  }
+}
+template <int dir>
+__device__ __forceinline__ void lds_narrow(const LdsCtx& x, int h) {
+  LdsStep p, o;
+  LdsItem A, B;
+  lds_level(x, h, p);
+  lds_fetch(x, p, threadIdx.x & 63u, A);
+  for (;;) {
+    if (!lds_turn1<dir>(x, p, o, A, B)) break;
+    if (!lds_turn1<dir>(x, o, p, B, A)) break;
+  }
+}
+// the first narrow level (H: none)
+__device__ __forceinline__ int lds_first_narrow(const LdsCtx& x) {
+  int h = 1;
+  for (; h < x.H; ++h) {
+    LdsStep p;
+    lds_level(x, h, p);
+    if (p.n <= kLdsWave) break;
+  }
+  return h;
+}
+
+// Root step of the block's tree (as root_chunk): site log-likelihoods, the
+// root's state, the stem's counts.  Returns the log-likelihood of the
+// thread's site (0: none).
+__device__ __forceinline__ double lds_root(const DevForest& F, const LdsCtx& x, int t, double* site_llh_out) {
+  double sl = 0.0;
+  const int s = (int)threadIdx.x;
+  if (s < x.sb) {
+    const int r = uniform_at(F.tree_root, t);
+    const int pl = lds_place((x.nint - 1) * x.sb + s);
+    const int k = x.k0 + s;
+    const bool real = k < x.K;
+    const int kc = min(k, x.K - 1);
+    const int sk = uniform_at(F.tree_site_base, t) + kc;
+    const int lab = F.labels[F.row_off[r] + kc];
+    const double q = lab > 0 ? F.prior[F.site_qoff[sk] - 1 + lab] : F.site_qsum[sk];
+    const double2 b = x.st[pl];
+    const Coef cf = F.coef[r];
+    const Eps er = edge(lab, b.x, b.y, x.sE[pl], q, cf);
+    const int ex = exp_of(er.e0);
+    const double Lm = ldexp(er.e0, -ex);
+    // the sites past the tree's carry zeros
+    const double A = real ? 1.0 / er.e0 : 0.0;
+    const double a0 = cf.p1n * A * er.s0;
+    const double m = cf.mut * q * A * er.s0;
+    const double sil = lab < 0 ? er.s1 * A : 0.0;
+    x.st[pl] = make_double2(a0, m);
+    double acc[3] = {lab == 0 ? 1.0 : a0 * b.x, lab != 0 ? m * b.y : 0.0, sil};
+    if (real) {
+      sl = log(Lm) + (double)(er.e + ex) * 0.69314718055994530942;
+      F.site_llh[sk] = sl;
+      if (site_llh_out) site_llh_out[sk] = sl;
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      acc[j] = seg_sum_last<kLdsR>(real ? acc[j] : 0.0);
+      if ((s & (kLdsR - 1)) == kLdsR - 1) x.rpart[3 * (s / kLdsR) + j] = acc[j];
+    }
+  }
+  lds_barrier();
+  return sl;
+}
+
+// The block's passes: inside, root() (lds_root), outside when `out`; hn: the
+// first narrow level.
+template <typename Root>
+__device__ __forceinline__ double lds_pass(const LdsCtx& x, int hn, bool out, Root&& root) {
+  const bool first = __builtin_amdgcn_readfirstlane((int)threadIdx.x) < 64;
+  lds_wide<1>(x, 1);
+  if (hn < x.H && first) lds_narrow<1>(x, hn);
+  lds_barrier();
+  const double sl = root();
+  if (!out) return sl;
+  if (hn < x.H && first) lds_narrow<-1>(x, x.H - 1);
+  lds_barrier();
+  if (hn > 1) lds_wide<-1>(x, hn - 1);
+  return sl;
+}
+
+// Sums the block's partial counts over its sites, in site order, and leaves
+// them in the nodes' first slots: 16 threads a node, thread m its value m
+// (counts 0..4 of both child branches, the dropout sum).
+__device__ __forceinline__ double* lds_slot(const LdsCtx& x, int l, int g) {
+  return reinterpret_cast<double*>(x.st + (kLdsLeafCells + l * x.sb + kLdsR * g));
+}
+__device__ __forceinline__ void lds_fold(const LdsCtx& x) {
+  const int G = x.sb / kLdsR;
+  const int m = (int)threadIdx.x & 15;
+  for (int l = (int)threadIdx.x >> 4; l < x.nint; l += kLdsThreads / 16) {
+    if (m > 10) continue;
+    double s = lds_slot(x, l, 0)[m];
+    for (int g = 1; g < G; ++g) s += lds_slot(x, l, g)[m];
+    lds_slot(x, l, 0)[m] = s;
+  }
+  if (threadIdx.x < 3)
+    for (int g = 1; g < G; ++g) x.rpart[threadIdx.x] += x.rpart[3 * g + threadIdx.x];
+  lds_barrier();
+}
+// branch r of the block's tree: child r & 1 of internal node r / 2, the stem last
+__device__ __forceinline__ int lds_branch_node(const DevForest& F, const LdsCtx& x, int t, int r) {
+  if (r == 2 * x.nint) return F.tree_root[t];
+  return r & 1 ? x.rec[r >> 1].g1 : x.rec[r >> 1].g0;
+}
+__device__ __forceinline__ void lds_branch_counts(const LdsCtx& x, int r, double (&s)[5]) {
+  const bool stem = r == 2 * x.nint;
+  const double* c = stem ? x.rpart : lds_slot(x, r >> 1, 0) + 5 * (r & 1);
+#pragma unroll
+  for (int m = 0; m < 5; ++m) s[m] = stem && m > 2 ? 0.0 : c[m];
+}
+// the folded counts into slot `slot` of F's partials
+__device__ __forceinline__ void lds_flush(const DevForest& F, const LdsCtx& x, int t, int64_t slot) {
+  double* cp = F.cpart + slot * F.cp_c;
+  for (int r = (int)threadIdx.x; r <= 2 * x.nint; r += kLdsThreads) {
+    double s[5];
+    lds_branch_counts(x, r, s);
+    double* c = cp + lds_branch_node(F, x, t, r) * F.cp_v;
+#pragma unroll
+    for (int m = 0; m < 5; ++m) c[m] = s[m];
+    if (r < 2 * x.nint && !(r & 1)) F.rt_part[slot * F.rt_c + x.rec[r >> 1].v * F.rt_v] = lds_slot(x, r >> 1, 0)[10];
+  }
+}
+
+// coefficients of branch r of the tree with records from ib on
+__device__ __forceinline__ void lds_set_coef(const LdsPlan& L, int ib, int r, const Coef& c) {
+  LdsCoef* o = L.lcoef + ib + (r >> 1);
+  const int i = r & 1;
+  o->p1n[i] = c.p1n;
+  o->mut[i] = c.mut;
+  o->pn[i] = c.pn;
+  o->msil[i] = c.msil;
+  o->esil[i] = c.msil != 0.0 ? c.esil : kZeroTop;
+}
+
+// sums of three values over the block's threads (sh: 3 kLdsThreads / 64
+// doubles, free again after the next barrier)
+__device__ __forceinline__ void lds_sum3(double& a, double& b, double& c, double* sh) {
+  constexpr int kW = kLdsThreads / 64;
+  a = seg_sum_last<64>(a);
+  b = seg_sum_last<64>(b);
+  c = seg_sum_last<64>(c);
+  if ((threadIdx.x & 63) == 63) {
+    double* o = sh + 3 * (threadIdx.x >> 6);
+    o[0] = a;
+    o[1] = b;
+    o[2] = c;
+  }
+  lds_barrier();
+  a = b = c = 0.0;
+#pragma unroll
+  for (int i = 0; i < kW; ++i) {
+    a += sh[3 * i];
+    b += sh[3 * i + 1];
+    c += sh[3 * i + 2];
+  }
+}
+
+// Whole problems of one tree, a block each: likelihood, E-step, or the EM
+// loop, for problems of at most kPbMaxSites sites whose state fits LDS.  The
+// loop needs no launch, no host and no other block between EM steps.  A
+// thread keeps to the same branches throughout; the M-step reads their counts
+// from LDS.  One 250 x 30 problem: 46 us an EM step (inside 16, outside 19,
+// M-step 11), 101 us in the general passes' 13 launches; 200 trees of 20-200
+// leaves x 20 sites: 51 us, 187 us; one likelihood of 250 x 30: 23 us, 35 us.
+struct PbArgs {
+  DevForest F;
+  LdsPlan L;
+  TreeWalk TW;
+  double *d, *nu, *phi, *nll, *site_llh_out;
+  int32_t* iters_out;
+  EmState em;
+  int max_steps, max_iter;
+  double tol;
+  int what;
+};
+// The kernel's arguments, read where they are used: from an address that the
+// compiler cannot tell from the last one, so that it loads again instead of
+// keeping some 200 scalar registers' worth of pointers alive (spilled to
+// vector lanes) across the passes.
+__device__ __forceinline__ const PbArgs& pb_args() {
+  uintptr_t p = (uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const PbArgs*)(const __attribute__((address_space(4))) PbArgs*)p;
+}
+__global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
+  extern __shared__ __align__(16) char lds[];
+  __shared__ double sh[2][3 * (kLdsThreads / 64)];
+  const int p = (int)blockIdx.x;
+  const int t = p;  // one tree a problem
+  const int what = pb_args().what;
+  int step = 0;
+  double pre = 0.0, nv, pv;
+  LdsCtx x;
+  {
+    const PbArgs& A = pb_args();
+    if (what & kPbEm) {
+      if (A.em.done[p]) return;
+      step = A.em.step[p];
+      pre = A.em.pre[p];
+    }
+    nv = A.nu ? A.nu[p] : 0.0;
+    pv = A.phi[p];
+    x = lds_ctx(A.F, A.L, A.TW, uniform_at(A.L.blk, p), pv, lds);
+  }
+  const int hn = lds_first_narrow(x);
+  const int nbr = 2 * x.nint + 1;
+  for (int it = 0; it < pb_args().max_steps; ++it) {
+    if (what & kPbCoef) {
+      const PbArgs& A = pb_args();
+      const DevForest& F = A.F;
+      const int ib = uniform_at(A.L.int_base, t);
+      for (int r = (int)threadIdx.x; r < nbr; r += kLdsThreads) {
+        const int v = lds_branch_node(F, x, t, r);
+        const Coef c = branch_coef(A.d[v], nv);
+        F.coef[v] = c;
+        if (r < nbr - 1) lds_set_coef(A.L, ib, r, c);
+      }
+      __syncthreads();
+    }
+    const bool out = (what & kPbOut) && !((what & kPbEm) && step == pb_args().max_iter);
+    double llh = lds_pass(x, hn, out, [&] { return lds_root(pb_args().F, x, t, pb_args().site_llh_out); });
+    double z0 = 0.0, z1 = 0.0;
+    lds_sum3(llh, z0, z1, sh[0]);
+    if (out) lds_fold(x);
+    const PbArgs& A = pb_args();
+    const DevForest& F = A.F;
+    if (!(what & kPbEm)) {
+      if (threadIdx.x == 0 && A.nll) A.nll[p] = -llh;
+      if (out) lds_flush(F, x, t, 0);
+      return;
+    }
+    const EmState& em = A.em;
+    // bookkeeping of the EM loop (as k_llh; every thread decides alike)
+    const bool conv = step > 0 && A.tol > 0.0 && fabs((llh - pre) / pre) < A.tol;
+    const bool stop = conv || step >= A.max_iter;
+    if (threadIdx.x == 0) {
+      A.nll[p] = -llh;
+      if (em.trace) em.trace[(int64_t)step * F.num_problems + p] = -llh;
+      if (!conv) em.pre[p] = llh;
+      em.step[p] = step + 1;
+      if (stop) {
+        const int n = conv ? step : A.max_iter + 1;
+        em.done[p] = 1;
+        em.iters[p] = n;
+        A.iters_out[p] = n;
+      }
+    }
+    if (stop) return;
+    pre = llh;
+    ++step;
+    const uint32_t flags = uniform_at(F.prob_flags, p);
+    const bool opt_nu = (flags & 2u) && uniform_at(F.prob_nfree, p) > 0;
+    const double K = (double)x.K;
+    // M-step: branch lengths (as branch_update), the dropout sum on the way
+    double a0 = 0.0, b0 = 0.0, d0 = 0.0;  // the thread's first branch, as nu_a, nu_b, nu_d
+    double rt = 0.0, bad = 0.0;
+    for (int r = (int)threadIdx.x; r < nbr; r += kLdsThreads) {
+      const int v = lds_branch_node(F, x, t, r);
+      double s[5];
+      lds_branch_counts(x, r, s);
+      if (r < nbr - 1 && !(r & 1)) rt += lds_slot(x, r >> 1, 0)[10];
+      double dn = A.d[v], na = 0.0, nb = 0.0;
+      if (F.free_branch[v]) {
+        dn = branch_length(F, s, K, nv, dn, na, nb);
+        if (!isfinite(dn)) bad = 1.0;
+        A.d[v] = dn;
+      }
+      if (r == (int)threadIdx.x) {
+        a0 = na;
+        b0 = nb;
+        d0 = dn;
+      } else {
+        F.nu_a[F.node_pos[v]] = na;
+        F.nu_b[F.node_pos[v]] = nb;
+        F.nu_d[F.node_pos[v]] = dn;
+      }
+    }
+    // phi, then nu: bracketed Newton on h' (as nu_solve)
+    double xx = nv > 0.0 && nv < 1.0 ? nv : 0.5, lo = 0.0, hi = 2.0;
+    bool fin = !opt_nu;
+    int evals = 0;
+    for (; evals == 0 || (!fin && evals < kNuMaxEvals); ++evals) {
+      double g = 0.0, h = 0.0;
+      if (opt_nu) {
+        nu_term(a0, b0, d0, xx, g, h);
+        for (int r = (int)threadIdx.x + kLdsThreads; r < nbr; r += kLdsThreads) {
+          const int pos = F.node_pos[lds_branch_node(F, x, t, r)];
+          nu_term(F.nu_a[pos], F.nu_b[pos], F.nu_d[pos], xx, g, h);
+        }
+      }
+      double third = evals == 0 ? (bad != 0.0 ? INFINITY : rt) : 0.0;
+      lds_sum3(g, h, third, sh[1 - (evals & 1)]);
+      if (evals == 0) {
+        bad = isfinite(third) ? 0.0 : 1.0;
+        if (flags & 1u) {
+          pv = third / (F.prob_nobs[p] + third);
+          if (fabs(pv) < F.prob_phimin[p]) pv = 0.0;
+        }
+        if (!opt_nu) break;
+      }
+      double xn;
+      fin = nu_newton_step(xx, g, h, lo, hi, xn);
+      xx = xn;
+    }
+    if (opt_nu) nv = xx;
+    if (threadIdx.x == 0) {
+      NuState* st = F.nu_state + p;
+      A.phi[p] = pv;
+      A.nu[p] = nv;
+      st->x = xx;
+      st->lo = lo;
+      st->hi = hi;
+      st->fin = 1;
+      st->status = (bad != 0.0 ? 1 : 0) | (fin ? 0 : 2);
+    }
+    lds_leaves(x, pv);
+  }
+}
+
+// The cell tables of the blocks (blockIdx.y), a thread per pair of cells.
+__global__ void __launch_bounds__(256) k_lds_tables(DevForest F, LdsPlan L, TreeWalk TW) {
+  const LdsBlk B = L.blk[blockIdx.y];
+  const LdsRec* recs = L.rec + L.int_base[B.tree];
+  const int K = F.tree_nsites[B.tree], sb0 = F.tree_site_base[B.tree];
+  const int lb = TW.lvl_base[B.tree], H = TW.lvl_base[B.tree + 1] - lb;
+  for (int h = 1; h < H; ++h) {
+    const int l0 = L.lvl_off[lb + h - 1].x, e0 = L.lvl_off[lb + h - 1].y;
+    const int n = (L.lvl_off[lb + h].x - l0) * B.sb, ne = L.lvl_off[lb + h].y - e0;
+    for (int e = (int)(blockIdx.x * 256 + threadIdx.x); e < ne; e += (int)gridDim.x * 256) {
+      uint32_t w[4];
+      double q[4];
+#pragma unroll
+      for (int c2 = 0; c2 < 2; ++c2) {
+        const int i = lds_pair((unsigned)e) + c2;
+        uint32_t pl[2] = {3, 3}, fl = kLdsLeaf0 | kLdsLeaf1;
+        q[2 * c2] = q[2 * c2 + 1] = 0.0;
+        const int j = l0 + i / B.sb, s = i % B.sb, k = B.k0 + s;
+        if (i < n) {
+          const LdsRec r = recs[j];
+          int lab[2] = {0, 0};
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const int g = c == 0 ? r.g0 : r.g1, l = c == 0 ? r.l0 : r.l1;
+            if (l >= 0) {
+              pl[c] = (uint32_t)lds_place(l * B.sb + s);
+              fl &= ~(c == 0 ? kLdsLeaf0 : kLdsLeaf1);
+            }
+            if (k >= K) continue;
+            const int code = l < 0 ? F.codes[F.row_off[g] + k] : F.labels[F.row_off[g] + k];
+            lab[c] = l < 0 ? code_label(code) : code;
+            if (l < 0) {
+              pl[c] = code == 0 ? 0 : (code > 0 ? 1 : (code == -1 ? 2 : 3));
+              if (code == -1) fl |= c == 0 ? kLdsDrop0 : kLdsDrop1;
+            }
+            if (lab[c] == 0) fl |= c == 0 ? kLdsZ0 : kLdsZ1;
+            if (lab[c] < 0) fl |= c == 0 ? kLdsQ0 : kLdsQ1;
+            q[2 * c2 + c] = lab[c] > 0 ? F.prior[F.site_qoff[sb0 + k] - 1 + lab[c]] : F.site_qsum[sb0 + k];
+          }
+          if (k < K && combine_label(lab[0], lab[1]) == 0) fl |= kLdsUz;
+          fl |= (uint32_t)lds_place(j * B.sb + s) << 16;
+        }
+        w[2 * c2] = pl[0] | (pl[1] << 16);
+        w[2 * c2 + 1] = fl;
+      }
+      L.w[B.tab + e0 + e] = make_uint4(w[0], w[1], w[2], w[3]);
+      L.q[B.tab + e0 + e] = make_double4(q[0], q[1], q[2], q[3]);
+    }
+  }
+}
+
+void run_lds_tables(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, hipStream_t s) {
+  hipLaunchKernelGGL(k_lds_tables, dim3(8, L.num_blocks), dim3(256), 0, s, F, L, TW);
+}
+
+// a block may use all of a CU's LDS
+template <typename K>
+static void allow_lds(K kernel) {
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            kLdsMaxBytes);
+}
+
+void run_problem(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, double* d, double* nu, double* phi,
+                 double* nll, double* site_llh_out, int32_t* iters_out, const EmState& em, int max_steps,
+                 int max_iter, double tol, int what, hipStream_t s) {
+  static const bool once = (allow_lds(k_problem), true);
+  (void)once;
+  const PbArgs a{F, L, TW, d, nu, phi, nll, site_llh_out, iters_out, em, max_steps, max_iter, tol, what};
+  hipLaunchKernelGGL(k_problem, dim3(F.num_problems), dim3(kLdsThreads), L.lds_bytes, s, a);
 }
 
 // ---------------------------------------------------------------------------

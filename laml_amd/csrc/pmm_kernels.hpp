@@ -97,6 +97,10 @@ struct DevForest {
   double* site_llh;
   double* rt_part;  // [N * max_chunks] dropout sums of leaf children per chunk
   double* cpart;    // [N * max_chunks * 5] per-chunk branch count partials
+  // where the readers of the partials find node v's chunk c: cpart + v cp_v +
+  // c cp_c (5 values), rt_part + v rt_v + c rt_c.  The row kernels write a
+  // node's chunks side by side, the LDS kernels a chunk's nodes.
+  int64_t cp_v, cp_c, rt_v, rt_c;
   double* nu_a;     // [N] by position in prob_nodes: S0+S1+S3 of the branch
   double* nu_b;     // [N] S2+S4 (0 for fixed branches)
   double* nu_d;     // [N] new branch length
@@ -145,6 +149,43 @@ struct TreeWalk {
   const int32_t* lvl_cnt;
 };
 
+// Plan of the LDS passes (k_problem, k_lds_pass): block b runs tree
+// blk[b].tree at sites [k0, k0 + sb) (sb a multiple of the reduction width),
+// the state of every internal node at those sites in LDS.  Internal nodes are
+// numbered within their tree in level order ("local"), so the root is last.
+struct LdsBlk {
+  int32_t tree, k0, sb, nint;  // nint: internal nodes of the tree
+  int64_t tab;                 // first entry of the block's cell tables
+};
+// an internal node: its children's local numbers (-1: leaf) and node ids, its
+// own id
+struct LdsRec {
+  int32_t l0, l1, g0, g1, v, pad;
+};
+// coefficients of the branches to a record's two children (as Coef; esil
+// kZeroTop where msil is 0)
+struct LdsCoef {
+  double p1n[2], mut[2], pn[2], msil[2];
+  int32_t esil[2];
+  int32_t pad[2];
+};
+struct LdsPlan {
+  int32_t num_blocks, slots;   // slots: partial counts per node (blocks of its tree)
+  int32_t lds_bytes;           // dynamic LDS of a block
+  const LdsBlk* blk;
+  const int32_t* int_base;     // [T] first record of each tree
+  const LdsRec* rec;           // [internal nodes] by tree, then local
+  const int2* lvl_off;         // [as the tree walk's levels] local number and table entry after level h
+  LdsCoef* lcoef;              // [internal nodes] branch coefficients of both children of each record
+  // per block and pair of (node, site) cells, in the order the block's threads
+  // read them: where the children's vectors lie in LDS and label flags, and
+  // the children's prior weights; fixed for the forest's life
+  uint4* w;
+  double4* q;
+  double* cpart;               // partials, chunk-major
+  double* rt_part;
+};
+
 struct EmState {
   int32_t* done;   // [P] or nullptr outside the EM loop
   int32_t* iters;  // [P]
@@ -154,6 +195,29 @@ struct EmState {
 };
 
 int seg_width(int max_k);
+// dynamic LDS a block of the LDS passes may take (160 KiB less their static
+// arrays)
+constexpr int kLdsMaxBytes = 160 * 1024 - 1024;
+// sites of a block that share a partial-count slot in its LDS (a block's
+// sites are a multiple)
+constexpr int kLdsSlotSites = 8;
+// Forests that k_problem takes.  Sites: a block holds all sites of a problem,
+// and 64 x 120 leaves fill the LDS.  Problems: a CU's blocks run in turns, so
+// the general passes overtake it when blocks are many and tiny (EM step, block
+// / general: 256 problems of 250 x 30 89 / 308 us, 1,024 of them 308 / 658,
+// 2,048 of 100 x 20 373 / 576, 4,096 of 60 x 16 720 / 588).
+constexpr int kPbMaxSites = 64;
+constexpr int kPbMaxProblems = 2048;
+// the cell tables of an LDS plan (after run_labels)
+void run_lds_tables(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, hipStream_t s);
+// What k_problem does, a block per problem: branch coefficients from d and nu
+// (else those of the last call), the outside pass with counts (else inside
+// and likelihood alone), EM steps (at most max_steps, of the max_iter that
+// the run has in all)
+constexpr int kPbCoef = 1, kPbOut = 2, kPbEm = 4;
+void run_problem(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, double* d, double* nu, double* phi,
+                 double* nll, double* site_llh_out, int32_t* iters_out, const EmState& em, int max_steps,
+                 int max_iter, double tol, int what, hipStream_t s);
 void run_labels(const DevForest& F, const std::vector<int32_t>& lvl, int W, hipStream_t s);
 // the prior-weight rows qleaf / qint from the codes and labels (after run_labels)
 void run_qrows(const DevForest& F, double* qleaf, double* qint, hipStream_t s);
