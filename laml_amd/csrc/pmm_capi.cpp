@@ -1146,6 +1146,105 @@ int laml_forest_set_ultrametric(laml_forest* f, const laml_ultra_desc* u) {
   UA(bB, double, N);
   UA(status, int32_t, P);
 #undef UA
+  {
+    // the model by problem
+    std::vector<int32_t> cls_off(P + 1, 0), cls, lvl((size_t)P * (H + 1), 0), local(std::max(V, 1), 0), cprob(std::max(V, 1), 0);
+    std::vector<int32_t> more_off(V + 1, 0), more, inc_off(V + 1, 0), inc, br_off(P + 1, 0);
+    std::vector<int4> link(std::max(V, 1), make_int4(-1, -1, -1, 0));
+    std::vector<std::vector<int32_t>> kids(V);
+    std::vector<laml::UltraBranch> br;
+    for (int p = 0; p < P; ++p) {
+      for (int h = 0; h < H; ++h) {
+        lvl[(size_t)p * (H + 1) + h] = (int32_t)cls.size() - cls_off[p];
+        for (int c = u->level_problem_off[(int64_t)h * P + p]; c < u->level_problem_off[(int64_t)h * P + p + 1]; ++c) {
+          local[c] = (int32_t)cls.size() - cls_off[p];
+          cprob[c] = p;
+          cls.push_back(c);
+        }
+      }
+      lvl[(size_t)p * (H + 1) + H] = (int32_t)cls.size() - cls_off[p];
+      cls_off[p + 1] = (int32_t)cls.size();
+    }
+    // free branches by problem: those with a class at either end or between
+    // pinned heights (which the solve leaves where they are, but reports)
+    std::vector<int32_t> br_of(N, -1);
+    std::vector<std::vector<int32_t>> by_prob(P);
+    std::vector<uint8_t> fr(N);
+    LAML_HIP(hipMemcpy(fr.data(), f->F.free_branch, N, hipMemcpyDeviceToHost));
+    for (int v = 0; v < N; ++v)
+      if (fr[v]) by_prob[f->h_tree_prob[f->h_tree_of[v]]].push_back(v);
+    bool odd = false;  // a class that the packing cannot express
+    for (int p = 0; p < P; ++p) {
+      for (int v : by_prob[p]) {
+        laml::UltraBranch b{};
+        b.v = v;
+        const int up = u->up_cls[v], dn = u->dn_cls[v];
+        odd = odd || (up >= 0 && cprob[up] != p) || (dn >= 0 && cprob[dn] != p);
+        b.up = up >= 0 ? local[up] : -1;
+        b.dn = dn >= 0 ? local[dn] : -1;
+        b.up_off = u->up_off[v];
+        b.dn_off = u->dn_off[v];
+        br_of[v] = (int32_t)br.size() - br_off[p];
+        br.push_back(b);
+      }
+      br_off[p + 1] = (int32_t)br.size();
+    }
+    for (int c = 0; c < V; ++c) {
+      const int pc = u->cls_parent[c];
+      if (pc >= 0) kids[pc].push_back(c);
+    }
+    int64_t max_lds = 0;
+    for (int p = 0; p < P; ++p) {
+      for (int i = cls_off[p]; i < cls_off[p + 1]; ++i) {
+        const int c = cls[i];
+        const int pc = u->cls_parent[c];
+        odd = odd || (pc >= 0 && cprob[pc] != p);
+        link[i].z = pc >= 0 ? local[pc] : -1;
+        for (size_t k = 0; k < kids[c].size(); ++k) {
+          const int l = local[kids[c][k]];
+          if (k == 0) link[i].x = l;
+          else if (k == 1) link[i].y = l;
+          else more.push_back(l);
+        }
+        link[i].w = kids[c].size() > 2;
+        more_off[i + 1] = (int32_t)more.size();
+        for (int j = u->inc_off[c]; j < u->inc_off[c + 1]; ++j) {
+          const int v = u->inc_branch[j];
+          const bool below = u->inc_sign[j] > 0;
+          const int other = below ? u->dn_cls[v] : u->up_cls[v];
+          if (br_of[v] < 0) {
+            odd = true;
+            continue;
+          }
+          // the far class of a branch must be the class tree's neighbour
+          odd = odd || (other >= 0 && (below ? u->cls_parent[other] != c || u->cls_pedge[other] != v
+                                             : u->cls_parent[c] != other || u->cls_pedge[c] != v));
+          inc.push_back(br_of[v] * 4 + (below ? 0 : 2) + (other >= 0 ? 1 : 0));
+        }
+        inc_off[i + 1] = (int32_t)inc.size();
+      }
+      max_lds = std::max<int64_t>(max_lds, 8 * (11 * (int64_t)(cls_off[p + 1] - cls_off[p]) +
+                                                4 * (int64_t)(br_off[p + 1] - br_off[p])));
+    }
+    // without the packed model every solve is the barrier method's
+    if (odd) std::fill(cls_off.begin(), cls_off.end(), 0);
+    U.lds_bytes = (int32_t)std::min<int64_t>(odd ? 0 : max_lds, std::numeric_limits<int32_t>::max());
+    const bool big = U.lds_bytes > laml::kLdsMaxBytes;
+    if ((rc = f->uupload(&U.pk_cls_off, cls_off.data(), cls_off.size())) ||
+        (rc = f->uupload(&U.pk_cls, cls.data(), cls.size())) || (rc = f->uupload(&U.pk_lvl, lvl.data(), lvl.size())) ||
+        (rc = f->uupload(&U.pk_link, link.data(), link.size())) ||
+        (rc = f->uupload(&U.pk_more_off, more_off.data(), more_off.size())) ||
+        (rc = f->uupload(&U.pk_more, more.data(), more.size())) ||
+        (rc = f->uupload(&U.pk_inc_off, inc_off.data(), inc_off.size())) ||
+        (rc = f->uupload(&U.pk_inc, inc.data(), inc.size())) ||
+        (rc = f->uupload(&U.pk_br_off, br_off.data(), br_off.size())) ||
+        (rc = f->uupload(&U.pk_br, br.data(), br.size())) || (rc = f->ualloc(&U.t0, (size_t)V)) ||
+        (rc = f->ualloc(&U.pk_work, big ? 9 * (size_t)V + 4 * br.size() : 1))) {
+      f->free_ultra();
+      return rc;
+    }
+    LAML_HIP(hipMemset(U.t0, 0, sizeof(double) * (V > 0 ? V : 1)));
+  }
   LAML_HIP(hipMemset(U.status, 0, sizeof(int32_t) * P));
   LAML_HIP(hipMemset(U.t, 0, sizeof(double) * (V > 0 ? V : 1)));
   LAML_HIP(hipMemset(U.dt, 0, sizeof(double) * (V > 0 ? V : 1)));
@@ -1160,7 +1259,8 @@ int laml_forest_set_heights(laml_forest* f, const double* heights_host) {
   if (!f->ultra_on) return fail(LAML_ESTATE, "no ultrametric model set");
   DeviceGuard guard(f->device);
   if (f->U.num_classes > 0)
-    LAML_HIP(hipMemcpy(f->U.t, heights_host, sizeof(double) * f->U.num_classes, hipMemcpyHostToDevice));
+    for (double* t : {f->U.t, f->U.t0})
+      LAML_HIP(hipMemcpy(t, heights_host, sizeof(double) * f->U.num_classes, hipMemcpyHostToDevice));
   return LAML_OK;
 }
 
@@ -1647,6 +1747,15 @@ int laml_mstep(laml_forest* f, const double* counts, const double* rtilde, doubl
 // with posterior counts and the M-step
 static void em_step(laml_forest* f, const DevForest& F, const EmState& em, double* d, double* nu, double* phi,
                     double* nll, int32_t max_iter, double tol, bool last, hipStream_t s) {
+  if (problem_now(f)) {
+    // (ultrametric forests: their M-step is a launch of its own)
+    const DevForest G = lds_view(F, f->pb);
+    laml::run_problem(G, f->pb, f->TW, d, nu, phi, nullptr, nullptr, nullptr, em, 1, 0, 0.0,
+                      laml::kPbCoef | (last ? 0 : laml::kPbOut), s);
+    laml::run_llh(F, nll, em, max_iter, tol, s);
+    if (!last) laml::run_mstep(G, nullptr, nullptr, d, nu, phi, em.done, s, f->ultra_on ? &f->U : nullptr);
+    return;
+  }
   laml::run_coef(F, d, nu, em.done, s);
   if (f->pass_mode == 1 && !last) {
     // one launch for the whole E-step; the outside half of a problem that
@@ -1710,7 +1819,6 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
   }
   int prc = prepare_chains(f);
   if (prc) return prc;
-  f->rows_ok = true;
   laml::run_em_reset(em, P, s);
   // The EM step is captured once into a HIP graph and replayed: its kernel
   // arguments do not change between steps (the step number lives on the
@@ -1761,7 +1869,10 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
   }
   // a replayed step runs no host code: the outside rows are those of the
   // captured step's pass
-  if (max_iter > 0 && f->pass_mode != LAML_PASS_TREES)
+  f->rows_ok = !problem_now(f);
+  if (!f->rows_ok)
+    f->alpha_complete = f->inside_fused = false;
+  else if (max_iter > 0 && f->pass_mode != LAML_PASS_TREES)
     f->alpha_complete = !pass_chains(f, false, hybrid_split(f)) && !fuse_now(f);
   LAML_HIP(hipMemcpyAsync(iters, em.iters, sizeof(int32_t) * P, hipMemcpyDeviceToDevice, s));
   return check_launch();

@@ -2346,12 +2346,11 @@ __device__ double ult_phi(const DevForest& F, const UltraDev& U, int nb, int ne,
   return block_sum<kUltraThreads>(s, sh);
 }
 
-__global__ void __launch_bounds__(kUltraThreads) k_ultra(DevForest F, UltraDev U, double* __restrict__ d,
-                                                         const double* __restrict__ nu,
-                                                         const int32_t* __restrict__ done) {
-  __shared__ double sh[kUltraThreads / 64];
-  const int p = blockIdx.x;
-  if ((done && done[p]) || !U.has_free[p]) return;
+// The barrier method: mu falls tenfold a round, each round a damped Newton
+// solve (60 to 135 Newton systems a solve, more where the warm start lies at
+// the bounds).  Solves that the primal-dual method below does not finish.
+__device__ void ultra_barrier(const DevForest& F, const UltraDev& U, double* __restrict__ d,
+                              const double* __restrict__ nu, int p, double* sh) {
   const int P = F.num_problems;
   const int nb = F.prob_node_off[p], ne = F.prob_node_off[p + 1];
   const double nu0 = nu[p];
@@ -3323,8 +3322,8 @@ __global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
   LdsCtx x;
   {
     const PbArgs& A = pb_args();
+    if (A.em.done && A.em.done[p]) return;
     if (what & kPbEm) {
-      if (A.em.done[p]) return;
       step = A.em.step[p];
       pre = A.em.pre[p];
     }
@@ -3516,6 +3515,275 @@ void run_problem(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, doubl
   (void)once;
   const PbArgs a{F, L, TW, d, nu, phi, nll, site_llh_out, iters_out, em, max_steps, max_iter, tol, what};
   hipLaunchKernelGGL(k_problem, dim3(F.num_problems), dim3(kLdsThreads), L.lds_bytes, s, a);
+}
+
+// Primal-dual interior-point solve of the same problem.  With duals zl, zh of
+// the bounds (zl (d - dmin) -> mu, zh (dmax - d) -> mu) a Newton step is the
+// same Laplacian system with branch weights -f'' + zl / (d - dmin) + zh /
+// (dmax - d); mu follows the complementarity down superlinearly, and no line
+// search is needed: 8 to 15 systems a solve against the barrier's 60 to 135,
+// ending at the same point (mu_end is the same).  It starts from the last
+// solution drawn a tenth towards the strictly interior heights that the
+// caller set, since a start at the bounds costs the barrier method one
+// doubling of the distance a step.
+//
+// A system's two level sweeps are latency: everything they do not need is
+// formed before (branch derivatives, each class's own sums), a class passes
+// up the two values its parent adds (cG, cR) and down one fma, state is in
+// LDS where it fits, and levels of at most 64 classes are the first
+// wavefront's, without barriers.  250 leaves x 30 sites: 210 us a solve,
+// the barrier method 7,750.
+constexpr int kUltraIters = 60;
+
+// LDS or global arrays of one problem's solve
+struct UltraWork {
+  double *t, *dt, *gg, *G0, *wup, *cG, *cR, *f, *u;  // classes
+  double *w, *gp, *zl, *zh;                          // free branches
+  const int4* link;  // classes: two child classes and the parent class (-1: none), whether there are more children
+};
+constexpr int kUltraClsDoubles = 9, kUltraBrDoubles = 4;
+
+template <bool kLds>
+__device__ __forceinline__ void ultra_sync() {
+  if (kLds) lds_barrier(); else __syncthreads();
+}
+
+// the block's minimum of a and b, maximum of c
+__device__ __forceinline__ void ultra_reduce(double& a, double& b, double& c, double* sh) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    a = fmin(a, __shfl_xor(a, off, 64));
+    b = fmin(b, __shfl_xor(b, off, 64));
+    c = fmax(c, __shfl_xor(c, off, 64));
+  }
+  const int wid = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    sh[3 * wid] = a;
+    sh[3 * wid + 1] = b;
+    sh[3 * wid + 2] = c;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kUltraThreads / 64; ++i) {
+    a = fmin(a, sh[3 * i]);
+    b = fmin(b, sh[3 * i + 1]);
+    c = fmax(c, sh[3 * i + 2]);
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ void ultra_up(const UltraDev& U, const UltraWork& W, int c0, int c, int nc) {
+  if (c >= nc) return;
+  const int4 link = W.link[c];
+  double G = W.G0[c], r = W.gg[c];
+  if (link.x >= 0) {
+    G += W.cG[link.x];
+    r += W.cR[link.x];
+  }
+  if (link.y >= 0) {
+    G += W.cG[link.y];
+    r += W.cR[link.y];
+  }
+  if (link.w)
+    for (int j = U.pk_more_off[c0 + c]; j < U.pk_more_off[c0 + c + 1]; ++j) {
+      G += W.cG[U.pk_more[j]];
+      r += W.cR[U.pk_more[j]];
+    }
+  const double iD = 1.0 / (G + W.wup[c]);
+  const double f = W.wup[c] * iD;
+  W.f[c] = f;
+  W.u[c] = r * iD;
+  W.cG[c] = f * G;
+  W.cR[c] = f * r;
+}
+__device__ __forceinline__ void ultra_down(const UltraWork& W, int c, int nc) {
+  if (c >= nc) return;
+  const int pc = W.link[c].z;
+  W.dt[c] = pc < 0 ? W.u[c] : fma(W.f[c], W.dt[pc], W.u[c]);
+}
+
+// Returns whether the solve converged (d, nu_d, heights and status written);
+// nothing is written otherwise.
+template <bool kLds>
+__device__ bool ultra_pd(const DevForest& F, const UltraDev& U, double* __restrict__ d, double nu0, int p,
+                         const UltraWork& W, double* sh) {
+  const int tid = (int)threadIdx.x;
+  const int c0 = uniform_at(U.pk_cls_off, p), V = uniform_at(U.pk_cls_off, p + 1) - c0;
+  const int b0 = uniform_at(U.pk_br_off, p), B = uniform_at(U.pk_br_off, p + 1) - b0;
+  const int H = U.num_levels;
+  const int* lo_ = U.pk_lvl + p * (H + 1);
+  const double dmin = F.dmin, dmax = F.dmax;
+  const double K = (double)uniform_at(F.tree_nsites, uniform_at(F.prob_tree_off, p));
+  const double mu_end = 1e-13 * K;
+  double mu = 1e-2 * K;
+  // the narrow levels (at most 64 classes; levels only get narrower)
+  int hn = H;
+  if (kLds) {
+    hn = 0;
+    for (int h = 0; h < H; ++h)
+      if (uniform_at(lo_, h + 1) - uniform_at(lo_, h) > 64) hn = h + 1;
+  }
+  for (int c = tid; c < V; c += kUltraThreads) {
+    const int g = U.pk_cls[c0 + c];
+    W.t[c] = fma(0.9, U.t[g], 0.1 * U.t0[g]);
+  }
+  ultra_sync<kLds>();
+  auto height = [&](const double* t, int cls, double off) { return cls >= 0 ? t[cls] + off : off; };
+  auto diff = [&](const double* t, int cls) { return cls >= 0 ? t[cls] : 0.0; };
+  double bad = 0.0;
+  for (int i = tid; i < B; i += kUltraThreads) {
+    const UltraBranch br = U.pk_br[b0 + i];
+    const double x = height(W.t, br.up, br.up_off) - height(W.t, br.dn, br.dn_off);
+    const double lo = x - dmin, hi = dmax - x;
+    if (!(lo > 0.0 && hi > 0.0)) bad = 1.0;
+    W.zl[i] = mu / lo;
+    W.zh[i] = mu / hi;
+  }
+  {
+    double a = 0.0, b = 0.0;
+    ultra_reduce(a, b, bad, sh);
+  }
+  if (bad != 0.0) return false;
+  double last = INFINITY;
+  bool ok = false;
+  for (int it = 0; it < kUltraIters; ++it) {
+    for (int i = tid; i < B; i += kUltraThreads) {
+      const UltraBranch br = U.pk_br[b0 + i];
+      const double x = height(W.t, br.up, br.up_off) - height(W.t, br.dn, br.dn_off);
+      const double il = 1.0 / (x - dmin), ih = 1.0 / (dmax - x);
+      const double S1 = U.bS1[br.v], Bq = U.bB[br.v];
+      const double r1 = 1.0 / expm1(x);
+      double g = fma(S1, r1, -U.bA[br.v]), w = S1 * r1 * (1.0 + r1);
+      if (Bq > 0.0) {
+        const double rn = nu0 / expm1(nu0 * x);
+        g = fma(Bq, rn, g);
+        w = fma(Bq * rn, nu0 + rn, w);
+      }
+      W.gp[i] = g + mu * (il - ih);
+      W.w[i] = w + W.zl[i] * il + W.zh[i] * ih;
+    }
+    ultra_sync<kLds>();
+    for (int c = tid; c < V; c += kUltraThreads) {
+      double gg = 0.0, G = 0.0, wup = 0.0;
+      for (int j = U.pk_inc_off[c0 + c]; j < U.pk_inc_off[c0 + c + 1]; ++j) {
+        // branch, and its kind here: 0 below the class, to a pinned height; 1
+        // below, to a child class; 2 above, from a pinned height; 3 above,
+        // from the parent class
+        const int e = U.pk_inc[j], i = e >> 2, k = e & 3;
+        gg += k < 2 ? W.gp[i] : -W.gp[i];
+        if (k == 0 || k == 2) G += W.w[i];
+        if (k == 3) wup += W.w[i];
+      }
+      W.gg[c] = gg;
+      W.G0[c] = G;
+      W.wup[c] = wup;
+    }
+    ultra_sync<kLds>();
+    for (int h = 0; h < hn; ++h) {
+      const int e = uniform_at(lo_, h + 1);
+      for (int c = uniform_at(lo_, h) + tid; c < e; c += kUltraThreads) ultra_up(U, W, c0, c, e);
+      ultra_sync<kLds>();
+    }
+    if (kLds && tid < 64) {
+      for (int h = hn; h < H; ++h) ultra_up(U, W, c0, uniform_at(lo_, h) + tid, uniform_at(lo_, h + 1));
+      for (int h = H - 1; h >= hn; --h) ultra_down(W, uniform_at(lo_, h) + tid, uniform_at(lo_, h + 1));
+    }
+    ultra_sync<kLds>();
+    for (int h = hn - 1; h >= 0; --h) {
+      const int e = uniform_at(lo_, h + 1);
+      for (int c = uniform_at(lo_, h) + tid; c < e; c += kUltraThreads) ultra_down(W, c, e);
+      ultra_sync<kLds>();
+    }
+    // step lengths that keep the lengths and the duals inside
+    const double tau = fmin(0.9999, fmax(0.99, 1.0 - mu / K));
+    double ap = 1.0, ad = 1.0, step = 0.0;
+    for (int c = tid; c < V; c += kUltraThreads) {
+      const double s = fabs(W.dt[c]) / (1.0 + fabs(W.t[c]));
+      step = s >= 0.0 ? fmax(step, s) : INFINITY;  // (NaN: not a step)
+    }
+    for (int i = tid; i < B; i += kUltraThreads) {
+      const UltraBranch br = U.pk_br[b0 + i];
+      const double x = height(W.t, br.up, br.up_off) - height(W.t, br.dn, br.dn_off);
+      const double dx = diff(W.dt, br.up) - diff(W.dt, br.dn);
+      const double lo = x - dmin, hi = dmax - x, zl = W.zl[i], zh = W.zh[i];
+      const double dzl = (mu - zl * dx) / lo - zl, dzh = (mu + zh * dx) / hi - zh;
+      if (dx < 0.0) ap = fmin(ap, tau * lo / -dx);
+      if (dx > 0.0) ap = fmin(ap, tau * hi / dx);
+      if (dzl < 0.0) ad = fmin(ad, tau * zl / -dzl);
+      if (dzh < 0.0) ad = fmin(ad, tau * zh / -dzh);
+    }
+    ultra_reduce(ap, ad, step, sh);
+    if (!isfinite(step)) return false;
+    double comp = 0.0;
+    for (int i = tid; i < B; i += kUltraThreads) {
+      const UltraBranch br = U.pk_br[b0 + i];
+      const double x = height(W.t, br.up, br.up_off) - height(W.t, br.dn, br.dn_off);
+      const double dx = diff(W.dt, br.up) - diff(W.dt, br.dn);
+      const double lo = x - dmin, hi = dmax - x;
+      const double zl = fma(ad, (mu - W.zl[i] * dx) / lo - W.zl[i], W.zl[i]);
+      const double zh = fma(ad, (mu + W.zh[i] * dx) / hi - W.zh[i], W.zh[i]);
+      W.zl[i] = zl;
+      W.zh[i] = zh;
+      comp += zl * fma(ap, dx, lo) + zh * fma(-ap, dx, hi);
+    }
+    comp = block_sum<kUltraThreads>(comp, sh) / (2.0 * B);  // (all have read t)
+    for (int c = tid; c < V; c += kUltraThreads) W.t[c] = fma(ap, W.dt[c], W.t[c]);
+    ultra_sync<kLds>();
+    step *= ap;
+    if (mu <= mu_end) {
+      // at the rounding floor of the steps where they stop falling
+      if (step <= 1e-15 || (step <= 1e-12 && step > 0.25 * last)) {
+        ok = true;
+        break;
+      }
+      last = step;
+    }
+    mu = fmax(mu_end, fmin(mu, comp * fmax(0.1 * (1.0 - fmin(ap, ad)), fmin(0.1, comp / K))));
+  }
+  if (!ok) return false;
+  for (int c = tid; c < V; c += kUltraThreads) U.t[U.pk_cls[c0 + c]] = W.t[c];
+  for (int i = tid; i < B; i += kUltraThreads) {
+    const UltraBranch br = U.pk_br[b0 + i];
+    const double x = height(W.t, br.up, br.up_off) - height(W.t, br.dn, br.dn_off);
+    d[br.v] = x;
+    F.nu_d[F.node_pos[br.v]] = x;
+  }
+  if (tid == 0) U.status[p] = 0;
+  return true;
+}
+
+template <bool kLds>
+__global__ void __launch_bounds__(kUltraThreads) k_ultra(DevForest F, UltraDev U, double* __restrict__ d,
+                                                         const double* __restrict__ nu,
+                                                         const int32_t* __restrict__ done) {
+  extern __shared__ __align__(16) char lds[];
+  __shared__ double sh[3 * (kUltraThreads / 64)];
+  const int p = blockIdx.x;
+  if ((done && done[p]) || !U.has_free[p]) return;
+  const int c0 = U.pk_cls_off[p], V = U.pk_cls_off[p + 1] - c0;
+  const int b0 = U.pk_br_off[p], B = U.pk_br_off[p + 1] - b0;
+  // (16-byte records first, the doubles after them)
+  double* base = kLds ? reinterpret_cast<double*>(lds) + 2 * V
+                      : U.pk_work + (int64_t)kUltraClsDoubles * c0 + (int64_t)kUltraBrDoubles * b0;
+  double* bb = base + (int64_t)kUltraClsDoubles * V;
+  const UltraWork W{base,         base + V,     base + 2 * V, base + 3 * V, base + 4 * V, base + 5 * V, base + 6 * V,
+                    base + 7 * V, base + 8 * V, bb,           bb + B,       bb + 2 * B,   bb + 3 * B,
+                    kLds ? reinterpret_cast<const int4*>(lds) : U.pk_link + c0};
+  if (kLds)
+    for (int c = (int)threadIdx.x; c < V; c += kUltraThreads) reinterpret_cast<int4*>(lds)[c] = U.pk_link[c0 + c];
+  if (V > 0 && ultra_pd<kLds>(F, U, d, nu[p], p, W, sh)) return;
+  __syncthreads();
+  ultra_barrier(F, U, d, nu, p, sh);
+}
+
+void run_ultra(const DevForest& F, const UltraDev& U, double* d, const double* nu, const int32_t* done,
+               hipStream_t s) {
+  static const bool once = (allow_lds(k_ultra<true>), true);
+  (void)once;
+  if (U.lds_bytes <= kLdsMaxBytes)
+    hipLaunchKernelGGL(k_ultra<true>, dim3(F.num_problems), dim3(kUltraThreads), U.lds_bytes, s, F, U, d, nu, done);
+  else
+    hipLaunchKernelGGL(k_ultra<false>, dim3(F.num_problems), dim3(kUltraThreads), 0, s, F, U, d, nu, done);
 }
 
 // ---------------------------------------------------------------------------
@@ -3904,7 +4172,7 @@ void run_mstep(const DevForest& F, const double* counts, const double* rtilde, d
   hipLaunchKernelGGL(k_branch, dim3((F.num_nodes + 63) / 64), dim3(64), 0, s, F, counts, d, nu, done,
                      U ? *U : none, U ? 1 : 0);
   if (U)
-    hipLaunchKernelGGL(k_ultra, dim3(F.num_problems), dim3(kUltraThreads), 0, s, F, *U, d, nu, done);
+    run_ultra(F, *U, d, nu, done, s);
   // one launch when the problems keep enough blocks busy; otherwise split
   // each problem's branches over several blocks per evaluation
   if (F.max_prob_nodes <= kNuSolveMaxNodes && F.num_problems >= 8) {

@@ -108,6 +108,13 @@ struct DevForest {
   NuState* nu_state;  // [P]
 };
 
+// a free branch of the ultrametric solve: its node, and the class (numbered
+// within the problem, -1: pinned) and offset of its upper and lower end
+struct UltraBranch {
+  int32_t v, up, dn, pad;
+  double up_off, dn_off;
+};
+
 // Height-class model of the ultrametric constraint (one per forest)
 struct UltraDev {
   int32_t num_classes, num_levels;
@@ -134,6 +141,21 @@ struct UltraDev {
   double* bS1;
   double* bB;
   int32_t* status;           // [P] 0 ok, 1 line search stalled, 2 singular Newton system
+  double* t0;                // [V] the strictly interior heights that the caller set
+  // the same model by problem (classes and branches numbered within it,
+  // classes in level order), for the primal-dual solve
+  int32_t lds_bytes;         // state of the largest problem's solve
+  const int32_t* pk_cls_off; // [P + 1] into the class arrays below
+  const int32_t* pk_cls;     // the class's number in t
+  const int32_t* pk_lvl;     // [P][num_levels + 1] first class of each level
+  const int4* pk_link;       // the first two child classes, the parent class (-1: none), whether there are more
+  const int32_t* pk_more_off;  // further child classes
+  const int32_t* pk_more;
+  const int32_t* pk_inc_off; // incident branches: 4 * branch + kind (see ultra_pd)
+  const int32_t* pk_inc;
+  const int32_t* pk_br_off;  // [P + 1] into pk_br
+  const UltraBranch* pk_br;
+  double* pk_work;           // state of the solves that do not fit LDS
 };
 
 // Tree-walk launch plan: block b runs tree blk_tree[b] at site chunk
@@ -314,6 +336,8 @@ void run_quartet_em(const DevForest& F, int ncand, const int32_t* qnodes, const 
 void run_rtilde(const DevForest& F, double* rtilde, const int32_t* done, hipStream_t s);
 void run_grad(const DevForest& F, const double* d, const double* nu, const double* phi, double* grad_d,
               double* grad_nu, double* grad_phi, hipStream_t s);
+void run_ultra(const DevForest& F, const UltraDev& U, double* d, const double* nu, const int32_t* done,
+               hipStream_t s);
 void run_mstep(const DevForest& F, const double* counts, const double* rtilde, double* d, double* nu, double* phi,
                const int32_t* done, hipStream_t s, const UltraDev* U = nullptr);
 
