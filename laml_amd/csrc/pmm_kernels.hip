@@ -161,6 +161,9 @@ __device__ __forceinline__ T uniform_load(const T* p) {
   return out;
 }
 
+// the wavefront's LDS stores so far are done and visible to its own loads
+__device__ __forceinline__ void lds_wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // Kinds of child a pass kernel meets.  A *cherry* is an internal node whose
 // children are both leaves; when the pass fuses cherries (F.cherry_end >
 // F.num_leaves: nodes [num_leaves, cherry_end) are exactly the cherries, the
@@ -1806,38 +1809,98 @@ __global__ void __launch_bounds__(kRedThreads) k_rtilde(DevForest F, double* __r
 constexpr double kEpsNu = 1e-5;   // EM_solver.py:307 eps_nu
 constexpr double kEpsS = 1e-6;    // EM_solver.py:307 eps_s
 
+// The branch and nu solves look for the root of a decreasing function g of
+// x > 0 that behaves like S/x - A for small x, through G(x) = x g(x), which is
+// nearly linear.  From g and its first three derivatives at x: the root of G's
+// cubic Taylor polynomial, as a step from x (a plain Newton step where the
+// polynomial gives none near).  The step's own error is of the fourth order:
+// one of at most kTaylorDone x ends a solve (the functions vary on the scale
+// of 2 pi in d and in nu d, so the error is below 1e-15 x).  A warm-started
+// solve takes one or two evaluations where Newton steps to 1e-13 x took four
+// to seven.
+constexpr double kTaylorDone = 1e-4;
+__device__ __forceinline__ double taylor_step(double x, double g, double g1, double g2, double g3) {
+  const double c0 = x * g, c1 = fma(x, g1, g), c2 = fma(0.5 * x, g2, g1), c3 = fma(x * (1.0 / 6.0), g3, 0.5 * g2);
+  const double t0 = -c0 / c1;
+  double t = t0;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const double p = fma(fma(fma(c3, t, c2), t, c1), t, c0);
+    const double q = fma(fma(3.0 * c3, t, 2.0 * c2), t, c1);
+    t -= p * rcp_normal(q);
+  }
+  return fabs(t - t0) <= 0.5 * fabs(t0) ? t : t0;
+}
+
 struct BranchObj {
   double A, S1, B, nu;  // f'(d) = -A + S1/expm1(d) + B nu/expm1(nu d)
 };
-__device__ __forceinline__ void branch_g(const BranchObj& o, double d, double& g, double& h) {
-  const double em = expm1(d);
-  g = -o.A + o.S1 / em;
-  h = -o.S1 * (em + 1.0) / (em * em);
+// the derivative of the branch objective, g, and its own first three: with
+// r = 1 / expm1(y) and s = r (1 + r), r' = -s, s' = -s (1 + 2 r) and
+// (s (1 + 2 r))' = -s (1 + 6 s)
+struct BranchG {
+  double g, g1, g2, g3;
+};
+__device__ __forceinline__ BranchG branch_g(const BranchObj& o, double d) {
+  const double r = rcp_normal(expm1(d));
+  const double s = r * (1.0 + r);
+  BranchG b;
+  b.g = fma(o.S1, r, -o.A);
+  b.g1 = -o.S1 * s;
+  b.g2 = o.S1 * s * fma(2.0, r, 1.0);
+  b.g3 = -o.S1 * s * fma(6.0, s, 1.0);
   if (o.B > 0.0) {
-    const double en = expm1(o.nu * d);
-    g += o.B * o.nu / en;
-    h -= o.B * o.nu * o.nu * (en + 1.0) / (en * en);
+    const double rn = rcp_normal(expm1(o.nu * d));
+    const double sn = rn * (1.0 + rn);
+    const double B1 = o.B * o.nu, B2 = B1 * o.nu * sn, B3 = B2 * o.nu;
+    b.g = fma(B1, rn, b.g);
+    b.g1 -= B2;
+    b.g2 = fma(B3, fma(2.0, rn, 1.0), b.g2);
+    b.g3 = fma(-B3 * o.nu, fma(6.0, sn, 1.0), b.g3);
   }
+  return b;
 }
-// argmax over [dmin, dmax] of the strictly concave branch objective.  Its
-// derivative g behaves like S/d - A for small d, so Newton runs on the nearly
-// linear d*g(d) (same root and sign), safeguarded by a bracket.
+// argmax over [dmin, dmax] of the strictly concave branch objective, kept in
+// a bracket.  From a start inside the box the bounds are evaluated only when
+// a step reaches for them.
 __device__ double solve_branch(const BranchObj& o, double dmin, double dmax, double x0) {
-  double g, h;
-  branch_g(o, dmin, g, h);
-  if (!(g > 0.0)) return dmin;
-  branch_g(o, dmax, g, h);
-  if (!(g < 0.0)) return dmax;
   double lo = dmin, hi = dmax;
-  double x = (x0 > lo && x0 < hi) ? x0 : 0.5 * (lo + hi);
+  bool lo_known = false, hi_known = false;  // whether g(lo) > 0, g(hi) < 0 are known
+  double x = x0;
+  if (!(x0 > lo && x0 < hi)) {
+    if (!(branch_g(o, dmin).g > 0.0)) return dmin;
+    if (!(branch_g(o, dmax).g < 0.0)) return dmax;
+    lo_known = hi_known = true;
+    x = 0.5 * (lo + hi);
+  }
   for (int it = 0; it < 100; ++it) {
-    branch_g(o, x, g, h);
-    if (g > 0.0) lo = x; else if (g < 0.0) hi = x; else return x;
-    const double step = x * g / (g + x * h);
-    // stop once the Newton step is at the rounding-noise level of g
-    if (fabs(step) <= 1e-13 * x) return fmin(fmax(x - step, dmin), dmax);
-    double xn = x - step;
-    if (!(xn > lo && xn < hi)) xn = 0.5 * (lo + hi);
+    const BranchG b = branch_g(o, x);
+    if (b.g > 0.0) {
+      lo = x;
+      lo_known = true;
+    } else if (b.g < 0.0) {
+      hi = x;
+      hi_known = true;
+    } else if (b.g == 0.0) {
+      return x;
+    } else {
+      return dmin;  // not a number: as at the lower bound
+    }
+    const double step = taylor_step(x, b.g, b.g1, b.g2, b.g3);
+    double xn = x + step;
+    if (fabs(step) <= kTaylorDone * x && xn >= dmin && xn <= dmax) return xn;
+    if (!(xn > lo && xn < hi)) {
+      // out of the bracket: the optimum is at a bound whose slope points out
+      if (!lo_known) {
+        if (!(branch_g(o, dmin).g > 0.0)) return dmin;
+        lo_known = true;
+      }
+      if (!hi_known) {
+        if (!(branch_g(o, dmax).g < 0.0)) return dmax;
+        hi_known = true;
+      }
+      xn = 0.5 * (lo + hi);
+    }
     if (hi - lo <= 1e-13 * hi) return xn;
     x = xn;
   }
@@ -2510,16 +2573,13 @@ struct QTop {
 // site likelihood)
 __device__ __forceinline__ void q_post(const QTop& t, const Coef& cf, int lv, double b0, double bA, double q,
                                        const Eps& ep, double* S) {
-  if (lv == 0) {
-    S[0] += 1.0;
-    return;
-  }
-  const double A = t.A, G = t.G;
-  S[0] = fma(cf.p1n * A * ep.s0, b0, S[0]);
-  S[1] = fma(cf.mut * q * A * ep.s0, bA, S[1]);
-  S[2] = fma(ep.s1, A, S[2]);
-  S[3] = fma(cf.pn * G * ep.s0, bA, S[3]);
-  S[4] = fma(ep.s1, G, S[4]);
+  // ('z': bA = 0 and s1 = 0)
+  const double A = t.A * ep.s0, G = t.G * ep.s0;
+  S[0] = lv == 0 ? 1.0 : cf.p1n * A * b0;
+  S[1] = cf.mut * q * A * bA;
+  S[2] = ep.s1 * t.A;
+  S[3] = cf.pn * G * bA;
+  S[4] = ep.s1 * t.G;
 }
 
 // outside state (a0, aX) at the node below a branch, on the scale of its
@@ -2559,143 +2619,219 @@ __device__ __forceinline__ int q_combine(int la, int lb, const Eps& ea, const Ep
 
 }  // namespace
 
-__global__ void __launch_bounds__(256) k_quartet_em(DevForest F, int ncand, const int32_t* __restrict__ qnodes,
-                                                    const double* __restrict__ len_in,
-                                                    const uint8_t* __restrict__ opt_mask,
-                                                    const double* __restrict__ llh_const,
-                                                    const double* __restrict__ nu_p,
-                                                    const double* __restrict__ phi_p, int max_iter, double tol,
-                                                    double* __restrict__ len_out, double* __restrict__ nll_out,
-                                                    int32_t* __restrict__ iters_out) {
-  const int c = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-  if (c >= ncand) return;
-  const int lane = threadIdx.x & 63;
-  const int p = qnodes[c * 5 + 0], sib = qnodes[c * 5 + 1];
-  const int nA = qnodes[c * 5 + 2], nW = qnodes[c * 5 + 3], nC = qnodes[c * 5 + 4];
-  const int t = F.tree_of[nA];
+// What a candidate's EM needs of one site and does not change: the moved
+// subtrees' inside state and prior weights, labels and prior weights of u and
+// v, the data outside v's branch over the likelihood before the move (top,
+// with exponent x0), the part c of the likelihood free of v's branch, and the
+// log-likelihood before the move.
+struct QSite {
+  double b0[3], bA[3], q[3];  // A, W, C
+  double qU, qV, topA, topG, c, base;
+  int lab[3], E[3], labU, labV, x0;
+};
+
+struct QCand {
+  ChildRows r[3], rS;
+  bool lf[3], lfS, top_root;
+  Coef cs;
+  const double2 *aP, *bP;
+  const int32_t* bEP;
+  const int16_t* labP;
+  const double *pSP, *qsum, *site_llh;
+  const int32_t* qoff;
+  double phi;
+};
+
+__device__ __forceinline__ void q_load(const DevForest& F, const QCand& n, int k, QSite& x) {
+  const int qo = row_at(n.qoff, (unsigned)k) - 1;
+  const double qs = row_at(n.qsum, (unsigned)k);
+  auto weight = [&](int lab) { return lab > 0 ? row_at(F.prior, (unsigned)(qo + lab)) : qs; };
+  int code;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    load_child_rows(n.r[i], n.lf[i], k, n.phi, x.lab[i], x.b0[i], x.bA[i], x.E[i], code);
+    x.q[i] = weight(x.lab[i]);
+  }
+  x.labU = combine_label(x.lab[0], x.lab[1]);
+  x.labV = combine_label(x.labU, x.lab[2]);
+  x.qU = weight(x.labU);
+  x.qV = weight(x.labV);
+  x.c = x.base = 0.0;
+  if (n.top_root) {
+    // the unedited ancestor
+    x.topA = 1.0;
+    x.topG = 0.0;
+    x.x0 = 0;
+    return;
+  }
+  int labS, ES;
+  double b0S, bAS;
+  load_child_rows(n.rS, n.lfS, k, n.phi, labS, b0S, bAS, ES, code);
+  const Eps eS = edge(labS, b0S, bAS, ES, weight(labS), n.cs);
+  const int lp = row_at(n.labP, (unsigned)k);
+  const double2 ap = row_at(n.aP, (unsigned)k);
+  const double b0p = row_at(n.bP, (unsigned)k).x;
+  x.topA = (lp == 0 ? 1.0 / b0p : ap.x) * eS.e0;
+  x.topG = lp == 0 ? 0.0 : ap.y * eS.eA;
+  if (lp < 0) x.c = row_at(n.pSP, (unsigned)k);  // p silenced: free of v's branch
+  x.x0 = eS.e - row_at(n.bEP, (unsigned)k);
+  x.base = row_at(n.site_llh, (unsigned)k);
+}
+
+// One site's log-likelihood and posterior counts of the five branches.  Each
+// branch's five counts go to emit(branch, S) as soon as they are formed (v,
+// u, C, A, W), so that few are held at a time.
+template <typename Emit>
+__device__ __forceinline__ double q_eval(const QSite& x, const Coef (&cf)[5], Emit&& emit) {
+  const Eps eA = edge(x.lab[0], x.b0[0], x.bA[0], x.E[0], x.q[0], cf[0]);
+  const Eps eW = edge(x.lab[1], x.b0[1], x.bA[1], x.E[1], x.q[1], cf[1]);
+  double b0u, bAu, b0v, bAv, scU, scV;
+  int Eu, Ev;
+  q_combine(x.lab[0], x.lab[1], eA, eW, b0u, bAu, Eu, scU);
+  const Eps eU = edge(x.labU, b0u, bAu, Eu, x.qU, cf[2]);
+  const Eps eC = edge(x.lab[2], x.b0[2], x.bA[2], x.E[2], x.q[2], cf[3]);
+  q_combine(x.labU, x.lab[2], eU, eC, b0v, bAv, Ev, scV);
+  const Eps eV = edge(x.labV, b0v, bAv, Ev, x.qV, cf[4]);
+  // site likelihood L' of the candidate: L' / L = t1 2^xe + c
+  const int xe = x.x0 + eV.e;
+  const double t1 = fma(x.topA, eV.e0, x.topG * eV.eA);
+  const int e1 = t1 != 0.0 ? xe + exp_of(t1) : kZeroTop;
+  const int e = max(e1, x.c != 0.0 ? exp_of(x.c) : kZeroTop);
+  const double Lm = ldexp(t1, min(xe - e, 1000)) + ldexp(x.c, min(-e, 1000));
+  // from here on over L'
+  const double iL = ldexp(rcp_normal(Lm), min(xe - e, 1000));
+  const QTop tv{x.topA * iL, x.topG * iL};
+  double S[5];
+  // v's branch, then u and C below v, then A and W below u
+  q_post(tv, cf[4], x.labV, b0v, bAv, x.qV, eV, S);
+  emit(4, S);
+  const QTop av = q_node(tv, cf[4], x.labV, x.qV, eV);
+  const QTop tu = q_top(av, scV, eC);
+  q_post(tu, cf[2], x.labU, b0u, bAu, x.qU, eU, S);
+  emit(2, S);
+  const QTop tc = q_top(av, scV, eU);
+  q_post(tc, cf[3], x.lab[2], x.b0[2], x.bA[2], x.q[2], eC, S);
+  emit(3, S);
+  const QTop au = q_node(tu, cf[2], x.labU, x.qU, eU);
+  q_post(q_top(au, scU, eW), cf[0], x.lab[0], x.b0[0], x.bA[0], x.q[0], eA, S);
+  emit(0, S);
+  q_post(q_top(au, scU, eA), cf[1], x.lab[1], x.b0[1], x.bA[1], x.q[1], eW, S);
+  emit(1, S);
+  return log(Lm) + (double)e * 0.69314718055994530942 + x.base;
+}
+
+// A block of NW wavefronts per candidate, a site a lane (more than 64 NW
+// sites: in turns, loaded anew each EM step).  The sums over sites go through
+// LDS once a step; then five lanes of the first wavefront solve the five
+// branches side by side and form their coefficients, which a wavefront per
+// candidate did one after the other in every lane (3,996 candidates on 2,000
+// leaves x 200 sites: 790 us then, 270 now).  The coefficients of a step are
+// wave-uniform and held in scalar registers.  Bound by latency: half of the
+// wave cycles wait for the step's barriers, sums and solves, 37 % of the issue
+// slots are used; three wavefronts a SIMD (168 registers) in place of two
+// measured the same.
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) k_quartet_em(DevForest F, const int32_t* __restrict__ qnodes,
+                                                        const double* __restrict__ len_in,
+                                                        const uint8_t* __restrict__ opt_mask,
+                                                        const double* __restrict__ llh_const,
+                                                        const double* __restrict__ nu_p,
+                                                        const double* __restrict__ phi_p, int max_iter, double tol,
+                                                        double* __restrict__ len_out, double* __restrict__ nll_out,
+                                                        int32_t* __restrict__ iters_out) {
+  // values 0 .. 24: counts of the branches in the order they are formed (v,
+  // u, C, A, W); 25: the log-likelihood
+  __shared__ double sh[NW][27];
+  __shared__ double tot[25];
+  __shared__ Coef scf[5];
+  const int c = (int)blockIdx.x;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int p = uniform_load(qnodes + c * 5), sib = uniform_load(qnodes + c * 5 + 1);
+  const int nd[3] = {uniform_load(qnodes + c * 5 + 2), uniform_load(qnodes + c * 5 + 3),
+                     uniform_load(qnodes + c * 5 + 4)};
+  const int t = F.tree_of[nd[0]];
   const int prob = F.tree_prob[t];
   const int K = F.tree_nsites[t];
   const int sb = F.tree_site_base[t];
-  const double nu = nu_p[prob], phi = phi_p[prob];
+  const double nu = nu_p[prob];
   const uint32_t opt = opt_mask[c];
-  double d[5];
+  QCand n;
+  n.phi = phi_p[prob];
 #pragma unroll
-  for (int j = 0; j < 5; ++j) d[j] = len_in[c * 5 + j];
-  const ChildRows rA = child_rows(F, nA, nA < F.num_leaves);
-  const ChildRows rW = child_rows(F, nW, nW < F.num_leaves);
-  const ChildRows rC = child_rows(F, nC, nC < F.num_leaves);
-  const bool lfA = nA < F.num_leaves, lfW = nW < F.num_leaves, lfC = nC < F.num_leaves;
-  const bool top_root = p < 0;
-  Coef cs{};
-  ChildRows rS{};
-  bool lfS = false;
-  const double2* aP = nullptr;
-  const double2* bP = nullptr;
-  const int32_t* bEP = nullptr;
-  const int16_t* labP = nullptr;
-  const double* pSP = nullptr;
-  if (!top_root) {
-    cs = F.coef[sib];
-    lfS = sib < F.num_leaves;
-    rS = child_rows(F, sib, lfS);
-    const int64_t rp = F.row_off[p];
-    aP = F.alpha + rp;
-    labP = F.labels + rp;
-    pSP = F.pS + rp;
-    bP = F.beta + F.brow[p];
-    bEP = F.bE + F.brow[p];
+  for (int i = 0; i < 3; ++i) {
+    n.lf[i] = nd[i] < F.num_leaves;
+    n.r[i] = child_rows(F, nd[i], n.lf[i]);
   }
-  const int32_t* qoff = F.site_qoff + sb;
-  const double* qsum = F.site_qsum + sb;
-  const double* site_llh = F.site_llh + sb;
-  const double kLn2 = 0.69314718055994530942;
+  n.top_root = p < 0;
+  n.qoff = F.site_qoff + sb;
+  n.qsum = F.site_qsum + sb;
+  n.site_llh = F.site_llh + sb;
+  if (!n.top_root) {
+    n.cs = F.coef[sib];
+    n.lfS = sib < F.num_leaves;
+    n.rS = child_rows(F, sib, n.lfS);
+    const int64_t rp = F.row_off[p];
+    n.aP = F.alpha + rp;
+    n.labP = F.labels + rp;
+    n.pSP = F.pS + rp;
+    n.bP = F.beta + F.brow[p];
+    n.bEP = F.bE + F.brow[p];
+  }
+  // lane j < 5 of the first wavefront owns branch j
+  double d = tid < 5 ? len_in[c * 5 + tid] : 0.0;
+  if (tid < 5) scf[tid] = branch_coef(d, nu);
+  __syncthreads();
+  QSite x{};  // (a lane without a site evaluates zeros, which count for nothing)
   double llh_prev = 0.0, llh = 0.0;
   int iters = max_iter + 1;
   for (int it = 0; it <= max_iter; ++it) {
+    // wave-uniform: in scalar registers
     Coef cf[5];
 #pragma unroll
-    for (int j = 0; j < 5; ++j) cf[j] = branch_coef(d[j], nu);
-    double S[5][5];
-#pragma unroll
-    for (int j = 0; j < 5; ++j)
-#pragma unroll
-      for (int m = 0; m < 5; ++m) S[j][m] = 0.0;
-    double ll = 0.0;
-    for (int k = lane; k < K; k += 64) {
-      const int qo = row_at(qoff, (unsigned)k) - 1;
-      const double qs = row_at(qsum, (unsigned)k);
-      int labA, labW, labC, EA, EW, EC, code;
-      double b0A, bAA, b0W, bAW, b0C, bAC;
-      load_child_rows(rA, lfA, k, phi, labA, b0A, bAA, EA, code);
-      load_child_rows(rW, lfW, k, phi, labW, b0W, bAW, EW, code);
-      load_child_rows(rC, lfC, k, phi, labC, b0C, bAC, EC, code);
-      const double qA = labA > 0 ? row_at(F.prior, (unsigned)(qo + labA)) : qs;
-      const double qW = labW > 0 ? row_at(F.prior, (unsigned)(qo + labW)) : qs;
-      const double qC = labC > 0 ? row_at(F.prior, (unsigned)(qo + labC)) : qs;
-      const Eps eA = edge(labA, b0A, bAA, EA, qA, cf[0]);
-      const Eps eW = edge(labW, b0W, bAW, EW, qW, cf[1]);
-      double b0u, bAu;
-      int Eu;
-      double scU, scV;
-      const int labU = q_combine(labA, labW, eA, eW, b0u, bAu, Eu, scU);
-      const double qU = labU > 0 ? row_at(F.prior, (unsigned)(qo + labU)) : qs;
-      const Eps eU = edge(labU, b0u, bAu, Eu, qU, cf[2]);
-      const Eps eC = edge(labC, b0C, bAC, EC, qC, cf[3]);
-      double b0v, bAv;
-      int Ev;
-      const int labV = q_combine(labU, labC, eU, eC, b0v, bAv, Ev, scV);
-      const double qV = labV > 0 ? row_at(F.prior, (unsigned)(qo + labV)) : qs;
-      const Eps eV = edge(labV, b0v, bAv, Ev, qV, cf[4]);
-      // top of v's branch: the unedited ancestor, or p's outside state (over
-      // the likelihood L of the site before the move) with the sibling's
-      // edge values; x: the exponent of t1 below
-      QTop tv;
-      double c = 0.0, base = 0.0;
-      int x = eV.e;
-      if (top_root) {
-        tv.A = 1.0;
-        tv.G = 0.0;
-      } else {
-        int labS, ES;
-        double b0S, bAS;
-        load_child_rows(rS, lfS, k, phi, labS, b0S, bAS, ES, code);
-        const double qS = labS > 0 ? row_at(F.prior, (unsigned)(qo + labS)) : qs;
-        const Eps eS = edge(labS, b0S, bAS, ES, qS, cs);
-        const int lp = row_at(labP, (unsigned)k);
-        const double2 ap = row_at(aP, (unsigned)k);
-        const double b0p = row_at(bP, (unsigned)k).x;
-        tv.A = (lp == 0 ? 1.0 / b0p : ap.x) * eS.e0;
-        tv.G = lp == 0 ? 0.0 : ap.y * eS.eA;
-        if (lp < 0) c = row_at(pSP, (unsigned)k);  // p silenced: free of v's branch
-        x += eS.e - row_at(bEP, (unsigned)k);
-        base = row_at(site_llh, (unsigned)k);
-      }
-      // site likelihood L' of the candidate: L' / L = t1 2^x + c
-      const double t1 = fma(tv.A, eV.e0, tv.G * eV.eA);
-      const int e1 = t1 != 0.0 ? x + exp_of(t1) : kZeroTop;
-      const int e = max(e1, c != 0.0 ? exp_of(c) : kZeroTop);
-      const double Lm = ldexp(t1, min(x - e, 1000)) + ldexp(c, min(-e, 1000));
-      ll += log(Lm) + (double)e * kLn2 + base;
-      // from here on over L'
-      const double iL = ldexp(1.0 / Lm, min(x - e, 1000));
-      tv.A *= iL;
-      tv.G *= iL;
-      // posteriors: v's branch, then u and C below v, then A and W below u
-      q_post(tv, cf[4], labV, b0v, bAv, qV, eV, S[4]);
-      const QTop av = q_node(tv, cf[4], labV, qV, eV);
-      const QTop tu = q_top(av, scV, eC);
-      q_post(tu, cf[2], labU, b0u, bAu, qU, eU, S[2]);
-      const QTop tc = q_top(av, scV, eU);
-      q_post(tc, cf[3], labC, b0C, bAC, qC, eC, S[3]);
-      const QTop au = q_node(tu, cf[2], labU, qU, eU);
-      const QTop ta = q_top(au, scU, eW);
-      q_post(ta, cf[0], labA, b0A, bAA, qA, eA, S[0]);
-      const QTop tw = q_top(au, scU, eA);
-      q_post(tw, cf[1], labW, b0W, bAW, qW, eW, S[1]);
+    for (int j = 0; j < 5; ++j) {
+      cf[j].p1n = uniform_double(scf[j].p1n);
+      cf[j].mut = uniform_double(scf[j].mut);
+      cf[j].pn = uniform_double(scf[j].pn);
+      cf[j].msil = uniform_double(scf[j].msil);
+      cf[j].esil = __builtin_amdgcn_readfirstlane(scf[j].esil);
     }
-    ll = seg_sum_last<64>(ll);
-    ll = __shfl(ll, 63, 64);
-    llh = ll + llh_const[c];
+    const int r = lane >> 4, i = lane & 15;
+    for (int k0 = 0; k0 < K; k0 += 64 * NW) {
+      const int k = k0 + tid;
+      const bool on = k < K;
+      if (on && (it == 0 || K > 64 * NW)) q_load(F, n, k, x);
+      // totals over the wavefront, a dozen values at a time: row r gets
+      // values 3 r .. 3 r + 2; added to the earlier turns'
+      double v[12];
+      int nv = 0, base = 0;
+      auto put = [&](double s) {
+        v[nv++] = on ? s : 0.0;
+        if (nv < 12) return;
+        wave_sum12(v);
+        if (i < 3) {
+          double* o = &sh[wave][base + 3 * r + i];
+          const double y = i == 0 ? v[0] : (i == 1 ? v[1] : v[2]);
+          *o = k0 == 0 ? y : *o + y;
+        }
+        nv = 0;
+        base += 12;
+      };
+      double ll = q_eval(x, cf, [&](int, const double(&S)[5]) {
+#pragma unroll
+        for (int m = 0; m < 5; ++m) put(S[m]);
+      });
+      const double s24 = seg_sum_last<64>(v[0]);
+      ll = seg_sum_last<64>(on ? ll : 0.0);
+      if (lane == 63) {
+        sh[wave][24] = k0 == 0 ? s24 : sh[wave][24] + s24;
+        sh[wave][25] = k0 == 0 ? ll : sh[wave][25] + ll;
+      }
+    }
+    __syncthreads();
+    double lsum = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) lsum += sh[w][25];
+    llh = lsum + llh_const[c];
     // EM_solver.py:483-512: stop when the relative change is below tol, or
     // after max_iter M-steps (iteration count max_iter + 1)
     if (it > 0 && tol > 0.0 && fabs((llh - llh_prev) / llh_prev) < tol) {
@@ -2705,41 +2841,46 @@ __global__ void __launch_bounds__(256) k_quartet_em(DevForest F, int ncand, cons
     if (it == max_iter) break;
     llh_prev = llh;
     // M-step of the free branches (EM_solver.py:339-366 for one branch)
+    if (wave == 0) {
+      if (lane < 25) {
+        double s = 0.0;
 #pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      double sj[5];
-      double tot = 0.0;
-#pragma unroll
-      for (int m = 0; m < 5; ++m) {
-        const double x = seg_sum_last<64>(S[j][m]);
-        sj[m] = fmax(kEpsS, __shfl(x, 63, 64));
-        tot += sj[m];
+        for (int w = 0; w < NW; ++w) s += sh[w][lane];
+        tot[lane] = s;
       }
-      if (!((opt >> j) & 1u)) continue;
+      lds_wave_sync();
+      if (lane < 5 && ((opt >> lane) & 1u)) {
+        double sj[5];
 #pragma unroll
-      for (int m = 0; m < 5; ++m) sj[m] = sj[m] / tot * (double)K;
-      BranchObj o;
-      o.nu = nu;
-      o.A = (nu + 1.0) * sj[0] + nu * sj[1] + nu * sj[3];
-      o.S1 = sj[1];
-      o.B = nu > kEpsNu ? (sj[2] + sj[4]) : 0.0;
-      d[j] = solve_branch(o, F.dmin, F.dmax, d[j]);
+        for (int m = 0; m < 5; ++m) sj[m] = tot[5 * (lane == 4 ? 0 : (lane == 2 ? 1 : (lane == 3 ? 2 : lane + 3))) + m];
+        d = solve_branch(branch_obj(sj, (double)K, nu), F.dmin, F.dmax, d);
+        scf[lane] = branch_coef(d, nu);
+      }
     }
+    __syncthreads();
   }
-  if (lane == 0) {
-#pragma unroll
-    for (int j = 0; j < 5; ++j) len_out[c * 5 + j] = d[j];
+  if (tid < 5) len_out[c * 5 + tid] = d;
+  if (tid == 0) {
     nll_out[c] = -llh;
     iters_out[c] = iters;
   }
 }
 
+// the wavefronts a candidate takes: one per 64 sites of the longest row, up
+// to 8
 void run_quartet_em(const DevForest& F, int ncand, const int32_t* qnodes, const double* len_in,
                     const uint8_t* opt_mask, const double* llh_const, const double* nu, const double* phi,
                     int max_iter, double tol, double* len_out, double* nll_out, int32_t* iters_out, hipStream_t s) {
   if (ncand <= 0) return;
-  hipLaunchKernelGGL(k_quartet_em, dim3((ncand + 3) / 4), dim3(256), 0, s, F, ncand, qnodes, len_in, opt_mask,
-                     llh_const, nu, phi, max_iter, tol, len_out, nll_out, iters_out);
+  const int waves = F.chunk_w < 64 ? 1 : F.max_chunks;
+#define LAML_QUARTET(NW)                                                                                       \
+  hipLaunchKernelGGL(k_quartet_em<NW>, dim3(ncand), dim3(64 * NW), 0, s, F, qnodes, len_in, opt_mask, llh_const, \
+                     nu, phi, max_iter, tol, len_out, nll_out, iters_out)
+  if (waves <= 1) LAML_QUARTET(1);
+  else if (waves == 2) LAML_QUARTET(2);
+  else if (waves <= 4) LAML_QUARTET(4);
+  else LAML_QUARTET(8);
+#undef LAML_QUARTET
 }
 
 // ---------------------------------------------------------------------------
