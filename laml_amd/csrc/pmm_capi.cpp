@@ -348,12 +348,10 @@ int validate(const laml_forest_desc* d, Derived& D) {
     D.prob_int_off[p] = i;
     for (int j = prob_node_off[p]; j < prob_node_off[p + 1]; ++j) D.prob_nfree[p] += d->free_branch[prob_nodes[j]] ? 1 : 0;
   }
-  // nu-solve blocks: about 2048 branches per block, at most 64 per problem
   D.prob_blk_off.assign(P + 1, 0);
   for (int p = 0; p < P; ++p) {
     const int nb = prob_node_off[p + 1] - prob_node_off[p];
-    const int blocks = std::max(1, std::min(64, (nb + 2047) / 2048));
-    D.prob_blk_off[p + 1] = D.prob_blk_off[p] + blocks;
+    D.prob_blk_off[p + 1] = D.prob_blk_off[p] + std::max(1, (nb + laml::kNuSpan - 1) / laml::kNuSpan);
   }
   if (!(d->dmin > 0.0) || !(d->dmax > d->dmin)) return fail(LAML_EINVAL, "bad branch-length box");
   return LAML_OK;
@@ -638,9 +636,6 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   UP(node_pos, D.node_pos.data(), N);
   UP(prob_blk_off, D.prob_blk_off.data(), P + 1);
   F.num_nu_blocks = D.prob_blk_off[P];
-  F.max_prob_nodes = 0;
-  for (int p = 0; p < P; ++p)
-    F.max_prob_nodes = std::max(F.max_prob_nodes, D.prob_node_off[p + 1] - D.prob_node_off[p]);
   UP(prob_flags, d->problem_flags, P);
   UP(prob_nobs, d->problem_nobs, P);
   UP(prob_phimin, d->problem_phimin, P);
@@ -693,7 +688,7 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   int32_t* bE;
   double2* alpha;
   double *pS, *site_llh, *rt_part, *cpart, *nu_a, *nu_b, *nu_d, *nu_part;
-  laml::NuState* nu_state;
+  int32_t* mstep_status;
   AL(labels, int16_t, int_rows);
   // prior-weight rows: read by the chain kernels only, which need 64-site
   // segments
@@ -727,8 +722,8 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   AL(nu_a, double, N);
   AL(nu_b, double, N);
   AL(nu_d, double, N);
-  AL(nu_part, double, (size_t)F.num_nu_blocks * 3);
-  AL(nu_state, laml::NuState, P);
+  AL(nu_part, double, (size_t)F.num_nu_blocks * 12);
+  AL(mstep_status, int32_t, P);
   AL(f->counts, double, (size_t)N * 5);
   AL(f->rtilde, double, P);
   AL(f->phi_buf, double, P);
@@ -806,7 +801,7 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   F.nu_b = nu_b;
   F.nu_d = nu_d;
   F.nu_part = nu_part;
-  F.nu_state = nu_state;
+  F.mstep_status = mstep_status;
   F.phi = nullptr;
   F.cp_v = (int64_t)F.max_chunks * 5;
   F.cp_c = 5;
@@ -826,7 +821,7 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   }
   if (hipMemset(rt_part, 0, sizeof(double) * N * F.max_chunks) != hipSuccess ||
       hipMemset(cpart, 0, sizeof(double) * N * F.max_chunks * 5) != hipSuccess ||
-      hipMemset(nu_state, 0, sizeof(laml::NuState) * P) != hipSuccess) {
+      hipMemset(mstep_status, 0, sizeof(int32_t) * P) != hipSuccess) {
     delete f;
     return fail(LAML_EDEVICE, "hipMemset failed");
   }
@@ -1278,15 +1273,15 @@ int laml_forest_mstep_status(laml_forest* f, int32_t* status_host) {
   if (!f || !status_host) return fail(LAML_EINVAL, "null argument");
   DeviceGuard guard(f->device);
   const int P = f->F.num_problems;
-  std::vector<laml::NuState> st(P);
-  LAML_HIP(hipMemcpy(st.data(), f->F.nu_state, sizeof(laml::NuState) * P, hipMemcpyDeviceToHost));
+  std::vector<int32_t> st(P);
+  LAML_HIP(hipMemcpy(st.data(), f->F.mstep_status, sizeof(int32_t) * P, hipMemcpyDeviceToHost));
   std::vector<int32_t> us;
   if (f->ultra_on) {
     us.resize(P);
     LAML_HIP(hipMemcpy(us.data(), f->U.status, sizeof(int32_t) * P, hipMemcpyDeviceToHost));
   }
   for (int p = 0; p < P; ++p) {
-    int32_t s = st[p].status & 3;
+    int32_t s = st[p] & 3;
     // a singular Newton system of the ultrametric branch solve is a failed
     // branch solve; a stalled line search ends at the best point found
     if (f->ultra_on && us[p] == 2) s |= LAML_MSTEP_FAILED_D;

@@ -1934,355 +1934,295 @@ __device__ __forceinline__ double branch_length(const DevForest& F, double (&s)[
   return solve_branch(o, F.dmin, F.dmax, d);
 }
 
-// Branch lengths of every free branch (EM_solver.py:328-366): counts are
-// clamped at eps_s and renormalised to sum K, then the per-branch concave
-// problem is solved exactly with the current nu.  Also stages the nu
-// problem's per-branch coefficients at the branch's position in its problem.
-__device__ __forceinline__ void branch_update(const DevForest& F, int v, int p, int pos,
-                                              const double* __restrict__ counts, double* __restrict__ d, double nu0,
-                                              const UltraDev& U, int ultra) {
-  if (!F.free_branch[v]) {
-    F.nu_a[pos] = 0.0;
-    F.nu_b[pos] = 0.0;
-    F.nu_d[pos] = d[v];
-    return;
-  }
-  const int Kt = F.tree_nsites[F.tree_of[v]];
-  const double K = (double)Kt;
-  double s[5];
-  if (counts) {
-#pragma unroll
-    for (int j = 0; j < 5; ++j) s[j] = counts[(int64_t)v * 5 + j];
-  } else {
-    const int C = (Kt + F.chunk_w - 1) / F.chunk_w;
-#pragma unroll
-    for (int j = 0; j < 5; ++j) s[j] = 0.0;
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-      for (int j = 0; j < 5; ++j) s[j] += F.cpart[v * F.cp_v + c * F.cp_c + j];
-  }
-  const BranchObj o = branch_obj(s, K, nu0);
-  if (ultra) {
-    // the ultrametric solve needs the objective of every free branch; the
-    // lengths are set by k_ultra and the nu staging refreshed after it
-    U.bA[v] = o.A;
-    U.bS1[v] = o.S1;
-    U.bB[v] = o.B;
-    F.nu_a[pos] = s[0] + s[1] + s[3];
-    F.nu_b[pos] = s[2] + s[4];
-    return;
-  }
-  const double dn = solve_branch(o, F.dmin, F.dmax, d[v]);
-  // non-finite counts give a non-finite length: reported as the reference's
-  // failed branch solve (EM_solver.py:415-418,450-459)
-  if (!isfinite(dn)) F.nu_state[p].d_bad = 1;
-  d[v] = dn;
-  F.nu_a[pos] = s[0] + s[1] + s[3];
-  F.nu_b[pos] = s[2] + s[4];
-  F.nu_d[pos] = dn;
-}
-
-__global__ void __launch_bounds__(64) k_branch(DevForest F, const double* __restrict__ counts,
-                                                double* __restrict__ d, const double* __restrict__ nu,
-                                                const int32_t* __restrict__ done, UltraDev U, int ultra) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= F.num_nodes) return;
-  const int p = F.tree_prob[F.tree_of[v]];
-  if (done && done[p]) return;
-  branch_update(F, v, p, F.node_pos[v], counts, d, nu[p], U, ultra);
-}
-
-// phi closed form (EM_solver.py:318-326) and nu (EM_solver.py:392-407).
 // nu maximises a concave function of one variable over [0, 1] given the new
-// branch lengths; its derivative h'(x) = sum_v d_v (b_v / expm1(x d_v) - a_v)
-// sums over every branch of the problem.  Each problem's branches are split
-// over several blocks; one launch = one Newton evaluation: every block writes
-// its partial (h', h''), and the last block of the problem to arrive reduces
-// the partials in block order (deterministic) and takes a bracketed Newton
-// step.  The first launch also sums the dropout responsibilities for phi.
-// A problem still unconverged after the last of these launches is finished
-// by k_nu_solve in resume mode (one block per problem).
-constexpr int kNuThreads = 256;
-constexpr int kNuIters = 5;
+// branch lengths (EM_solver.py:392-407); its derivative
+// h'(x) = sum_v d_v (b_v / expm1(x d_v) - a_v) sums over every branch of the
+// problem.  Warm-started solves take one evaluation of h' and its derivatives,
+// two when nu moves by more than kTaylorDone (Newton steps to 1e-12 took three
+// to five).  Each problem's branches are split into spans of kNuThreads, a
+// block each, in two launches of an evaluation each, which write their spans'
+// sums; the next kernel's blocks all add the sums of their problem (in an
+// order set by the problem alone) and take the step.  So the kernels need no
+// fence between blocks: one with a last block that adds the sums took 80 us
+// for 16 problems of 20k branches, 30 us of it in the write-back that the
+// fence asks of the L2 caches.  The first evaluation follows the branch solves
+// in the same kernel and also sums the dropout responsibilities, for phi in
+// closed form (EM_solver.py:318-326).  k_nu_finish, a block per problem, takes
+// the last step and goes on alone where the solve is still open.
+constexpr int kNuThreads = kNuSpan;
 // evaluations a nu solve may take in all before its M-step reports failure:
 // the bracket halves at least every other evaluation, so this is far more
 // than [0, 1] needs to close to 1e-12 relative at any optimum the clamped
 // counts allow (nu* >= ~1e-12)
 constexpr int kNuMaxEvals = 200;
+constexpr int kNuFinishThreads = 512;
 
-// One bracketed Newton step on x h'(x), which is nearly linear in x, from the
-// evaluation (G, Hs) = (h'(x), h''(x)).  [lo, hi] brackets the root of h'
-// (hi > 1 until the bound x = 1 has been evaluated).  Returns true when the
-// solve has converged; xn is the next iterate (the answer when converged).
-__device__ __forceinline__ bool nu_newton_step(double x, double G, double Hs, double& lo, double& hi, double& xn) {
-  if (G > 0.0) lo = x; else if (G < 0.0) hi = x;
-  if (G > 0.0 && x >= 1.0) {
+// h'(x) and its first three derivatives
+struct NuSum {
+  double g, g1, g2, g3;
+};
+
+// One bracketed step towards the root of h' from its evaluation at x.
+// [lo, hi] brackets the root (hi > 1 until the bound x = 1 has been
+// evaluated).  Returns true when the solve has converged; xn is the next
+// iterate (the answer when converged).
+__device__ __forceinline__ bool nu_step(double x, const NuSum& n, double& lo, double& hi, double& xn) {
+  if (n.g > 0.0) lo = x; else if (n.g < 0.0) hi = x;
+  if (n.g > 0.0 && x >= 1.0) {
     xn = 1.0;  // optimum at the upper bound
     return true;
   }
-  if (G == 0.0) {
+  if (n.g == 0.0) {
     xn = x;
     return true;
   }
-  const double step = x * G / (G + x * Hs);
+  const double step = taylor_step(x, n.g, n.g1, n.g2, n.g3);
   const double top = fmin(hi, 1.0);
-  // the sum over branches carries ~1e-14 relative rounding noise near the
-  // root; a Newton step below 1e-12 x is converged
-  if (fabs(step) <= 1e-12 * x) {
-    xn = fmin(fmax(x - step, 0.0), 1.0);
+  xn = x + step;
+  if (fabs(step) <= kTaylorDone * x) {
+    xn = fmin(fmax(xn, 0.0), 1.0);
     return true;
   }
-  xn = x - step;
   if (xn >= 1.0 && hi > 1.0) xn = 1.0;
   else if (!(xn > lo && xn < top)) xn = 0.5 * (lo + top);
   return top - lo <= 1e-12 * top;
 }
 
-// One branch's terms of h'(x) and h''(x): a = S0 + S1 + S3, b = S2 + S4 of
-// the branch, its length dv.
-__device__ __forceinline__ void nu_term(double a, double bb, double dv, double x, double& g, double& h) {
+// One branch's terms: a = S0 + S1 + S3, b = S2 + S4 of the branch, its length
+// dv (derivatives of 1 / expm1 as in branch_g).
+__device__ __forceinline__ void nu_term(double a, double bb, double dv, double x, NuSum& n) {
   if (bb == 0.0) return;
-  const double en = expm1(x * dv);
-  const double ri = 1.0 / en;
-  g += dv * fma(bb, ri, -a);
-  h -= bb * dv * dv * (en + 1.0) * (ri * ri);
+  const double r = rcp_normal(expm1(x * dv));
+  const double s = r * (1.0 + r);
+  const double b2 = bb * dv * dv * s, b3 = b2 * dv;
+  n.g = fma(dv, fma(bb, r, -a), n.g);
+  n.g1 -= b2;
+  n.g2 = fma(b3, fma(2.0, r, 1.0), n.g2);
+  n.g3 = fma(-b3 * dv, fma(6.0, s, 1.0), n.g3);
 }
 
-// One thread's share (stride kNuThreads from branch position i0) of h'(x)
-// and h''(x) over the branch positions [i0 - lane offset, pe) of a span.
-// Every nu kernel sums through these two functions and in the same span
-// order, so all of them give a problem the same nu bit for bit, whichever
-// kernel runs and whatever else the forest holds.
-__device__ __forceinline__ void nu_span_terms(const DevForest& F, int pb, int pe, int lt, double x, double& g,
-                                              double& h) {
-  for (int i = pb + lt; i < pe; i += kNuThreads) nu_term(F.nu_a[i], F.nu_b[i], F.nu_d[i], x, g, h);
-}
-__device__ __forceinline__ void rt_span(const DevForest& F, int pb, int pe, int lt, int C, double& rt) {
-  for (int i = pb + lt; i < pe; i += kNuThreads) add_node_rt(F, F.prob_nodes[i], C, rt);
+// Sums over the block in every thread, in one pass through LDS (sh: 6 NT / 64
+// doubles).
+template <int NT>
+__device__ __forceinline__ void nu_block_sum(NuSum& n, double& rt, double& bad, double* sh) {
+  double v[6] = {n.g, n.g1, n.g2, n.g3, rt, bad};
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    v[j] = seg_sum_last<64>(v[j]);
+    if ((threadIdx.x & 63) == 63) sh[(threadIdx.x >> 6) * 6 + j] = v[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    v[j] = 0.0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) v[j] += sh[w * 6 + j];
+  }
+  __syncthreads();
+  n = NuSum{v[0], v[1], v[2], v[3]};
+  rt = v[4];
+  bad = v[5];
 }
 
-__global__ void __launch_bounds__(kNuThreads) k_nu_eval(DevForest F, const double* __restrict__ rtilde_in,
-                                                        double* __restrict__ nu, double* __restrict__ phi,
-                                                        const int32_t* __restrict__ done, int iter) {
-  __shared__ double sh[kNuThreads / 64];
-  __shared__ int s_last;
-  const int blk = blockIdx.x;
-  // block -> (problem, part) by binary search over prob_blk_off
+// the sums of the span of block blk, evaluation e
+__device__ __forceinline__ double* nu_span(const DevForest& F, int e, int blk) {
+  return F.nu_part + ((int64_t)e * F.num_nu_blocks + blk) * 6;
+}
+__device__ __forceinline__ void nu_store(const DevForest& F, int e, NuSum n, double rt, double bad, double* sh) {
+  nu_block_sum<kNuThreads>(n, rt, bad, sh);
+  if (threadIdx.x != 0) return;
+  double* o = nu_span(F, e, (int)blockIdx.x);
+  o[0] = n.g;
+  o[1] = n.g1;
+  o[2] = n.g2;
+  o[3] = n.g3;
+  if (e != 0) return;
+  o[4] = rt;
+  o[5] = bad;
+}
+
+// the sums of evaluation e of problem p in every thread (the same bits for
+// every NT)
+template <int NT>
+__device__ __forceinline__ void nu_load(const DevForest& F, int p, int e, NuSum& n, double& rt, double& bad,
+                                        double* sh) {
+  const int b0 = F.prob_blk_off[p], nparts = F.prob_blk_off[p + 1] - b0;
+  n = NuSum{0.0, 0.0, 0.0, 0.0};
+  rt = bad = 0.0;
+  if ((int)threadIdx.x < kNuThreads)
+    for (int q = (int)threadIdx.x; q < nparts; q += kNuThreads) {
+      const double* o = nu_span(F, e, b0 + q);
+      n.g += o[0];
+      n.g1 += o[1];
+      n.g2 += o[2];
+      n.g3 += o[3];
+      rt += o[4];
+      bad += o[5];
+    }
+  nu_block_sum<NT>(n, rt, bad, sh);
+}
+
+// the first evaluation point: the current nu, or 1/2 when outside (0, 1)
+__device__ __forceinline__ double nu_start(double nu) { return nu > 0.0 && nu < 1.0 ? nu : 0.5; }
+
+// the problem whose spans hold block blk, by binary search over prob_blk_off
+__device__ __forceinline__ int nu_problem(const DevForest& F, int blk) {
   int lo_p = 0, hi_p = F.num_problems;
   while (hi_p - lo_p > 1) {
     const int mid = (lo_p + hi_p) >> 1;
     if (F.prob_blk_off[mid] <= blk) lo_p = mid; else hi_p = mid;
   }
-  const int p = lo_p;
-  NuState* st = F.nu_state + p;
-  if (iter > 0) {
-    // set by the first evaluation for problems that are done or keep nu
-    // fixed, and by the evaluation that converges: the remaining launches of
-    // a captured M-step cost one load
-    if (st->fin) return;
-  } else if (done && done[p]) {
-    if (blk == F.prob_blk_off[p] && threadIdx.x == 0) st->fin = 1;
-    return;
-  }
-  const uint32_t flags = F.prob_flags[p];
-  const bool opt_nu = (flags & 2u) && F.prob_nfree[p] > 0;
-  const int part = blk - F.prob_blk_off[p];
-  const int nparts = F.prob_blk_off[p + 1] - F.prob_blk_off[p];
-  const int b = F.prob_node_off[p], e = F.prob_node_off[p + 1];
-  const int span = (e - b + nparts - 1) / nparts;
-  const int pb = b + part * span, pe = min(e, pb + span);
-  // first evaluation point: the current nu (or 1/2 when outside (0, 1))
-  const double x = (iter == 0) ? ((nu[p] > 0.0 && nu[p] < 1.0) ? nu[p] : 0.5) : st->x;
-  double g = 0.0, h = 0.0, rt = 0.0;
-  if (opt_nu) nu_span_terms(F, pb, pe, threadIdx.x, x, g, h);
-  if (iter == 0 && (flags & 1u) && !rtilde_in) {
-    const int C = (F.tree_nsites[F.prob_tree_off[p]] + F.chunk_w - 1) / F.chunk_w;
-    rt_span(F, max(pb, F.prob_int_off[p]), pe, threadIdx.x, C, rt);
-  }
-  g = block_sum<kNuThreads>(g, sh);
-  h = block_sum<kNuThreads>(h, sh);
-  rt = block_sum<kNuThreads>(rt, sh);
-  if (threadIdx.x == 0) {
-    double* pp = F.nu_part + (int64_t)blk * 3;
-    pp[0] = g;
-    pp[1] = h;
-    pp[2] = rt;
-    __threadfence();
-    const int prev = atomicAdd(&st->count, 1);
-    s_last = (prev == nparts - 1);
-  }
-  __syncthreads();
-  if (!s_last || threadIdx.x != 0) return;
-  __threadfence();
-  st->count = 0;
-  double G = 0.0, Hs = 0.0, RT = 0.0;
-  for (int q = F.prob_blk_off[p]; q < F.prob_blk_off[p + 1]; ++q) {
-    const volatile double* pp = F.nu_part + (int64_t)q * 3;
-    G += pp[0];
-    Hs += pp[1];
-    RT += pp[2];
-  }
-  if (iter == 0) {
-    double phi_star = phi[p];
-    if (flags & 1u) {
-      const double r = rtilde_in ? rtilde_in[p] : RT;
-      phi_star = r / (F.prob_nobs[p] + r);
-      if (fabs(phi_star) < F.prob_phimin[p]) phi_star = 0.0;
-    }
-    phi[p] = phi_star;
-    st->status = st->d_bad ? 1 : 0;
-    st->d_bad = 0;
-    st->lo = 0.0;
-    st->hi = 2.0;  // > 1: the bound x = 1 has not been evaluated
-    st->fin = opt_nu ? 0 : 1;
-    if (!opt_nu) return;
-  }
-  double lo = st->lo, hi = st->hi, xn;
-  const bool fin = nu_newton_step(x, G, Hs, lo, hi, xn);
-  st->lo = lo;
-  st->hi = hi;
-  st->x = xn;
-  st->fin = fin ? 1 : 0;
-  nu[p] = xn;
+  return lo_p;
 }
 
-// The same phi update and nu solve with one block per problem and every
-// Newton evaluation in one launch (forests of several problems of up to
-// kNuSolveMaxNodes branches).  The block's four groups of kNuThreads threads
-// sum four of the problem's spans (those of k_nu_eval's blocks) at a time,
-// each span exactly as a k_nu_eval block sums it, and the span sums are added
-// in span order, so the result equals k_nu_eval's bit for bit.  resume = 1
-// continues the solves that the k_nu_eval launches left unconverged (from
-// their Newton state; phi is already done) and does nothing for the others.
-// The M-step status of each problem is final after this kernel.
-constexpr int kNuSolveThreads = 1024;
-constexpr int kNuSolveMaxNodes = 65536;
-
-// sums over the spans of problem p in k_nu_eval's order: (h', h'') at x when
-// want_g, the dropout sum when want_rt
-template <int NT>
-__device__ __forceinline__ void nu_eval_spans(const DevForest& F, int p, double x, bool want_g, bool want_rt,
-                                              double& G, double& Hs, double& RT, double* sh) {
-  const int nparts = F.prob_blk_off[p + 1] - F.prob_blk_off[p];
-  const int b = F.prob_node_off[p], e = F.prob_node_off[p + 1];
-  const int span = (e - b + nparts - 1) / nparts;
-  const int grp = threadIdx.x / kNuThreads, lt = threadIdx.x % kNuThreads;
-  const int wid = threadIdx.x >> 6;
-  const int C = want_rt ? (F.tree_nsites[F.prob_tree_off[p]] + F.chunk_w - 1) / F.chunk_w : 0;
-  constexpr int kNuGroups = NT / kNuThreads;
-  constexpr int kW = kNuThreads / 64;  // waves per span
-  G = 0.0;
-  Hs = 0.0;
-  RT = 0.0;
-  for (int q0 = 0; q0 < nparts; q0 += kNuGroups) {
-    const int part = q0 + grp;
-    double g = 0.0, h = 0.0, rt = 0.0;
-    if (part < nparts) {
-      const int pb = b + part * span, pe = min(e, pb + span);
-      if (want_g) nu_span_terms(F, pb, pe, lt, x, g, h);
-      if (want_rt) rt_span(F, max(pb, F.prob_int_off[p]), pe, lt, C, rt);
-    }
-    g = seg_sum<64>(g);
-    h = seg_sum<64>(h);
-    rt = seg_sum<64>(rt);
-    if ((threadIdx.x & 63) == 0) {
-      sh[wid] = g;
-      sh[NT / 64 + wid] = h;
-      sh[2 * (NT / 64) + wid] = rt;
-    }
-    __syncthreads();
-    for (int j = 0; j < kNuGroups && q0 + j < nparts; ++j) {
-      double sg = 0.0, shh = 0.0, sr = 0.0;
+// Branch lengths of every free branch (EM_solver.py:328-366): counts are
+// clamped at eps_s and renormalised to sum K, then the per-branch concave
+// problem is solved exactly with the current nu; then the first nu
+// evaluation, at the current nu (or 1/2 when outside (0, 1)).  The branch's
+// nu coefficients are staged at its position in the problem for the later
+// evaluations.  Ultrametric forests solve their lengths together: for them
+// the objective of every branch is written instead, and k_nu_eval<true>
+// follows k_ultra.  Bound by latency (counts, then the dependent steps of the
+// solves, then the sums): 20k branches of one problem 9 us with the first nu
+// evaluation, 16 such problems 31 us; the M-step of the first with the two
+// kernels below 20 us, 58 us when nu took six Newton launches after the branch
+// solves, of the second 47 us, 111 us.
+template <bool kUltra>
+__global__ void __launch_bounds__(kNuThreads) k_branch(DevForest F, const double* __restrict__ counts,
+                                                       const double* __restrict__ rtilde_in, double* __restrict__ d,
+                                                       const double* __restrict__ nu,
+                                                       const int32_t* __restrict__ done, UltraDev U) {
+  __shared__ double sh[6 * (kNuThreads / 64)];
+  const int p = nu_problem(F, (int)blockIdx.x);
+  const int part = (int)blockIdx.x - F.prob_blk_off[p];
+  if (done && done[p]) return;
+  const int pos = F.prob_node_off[p] + part * kNuThreads + (int)threadIdx.x;
+  const double nu0 = nu[p];
+  const uint32_t flags = F.prob_flags[p];
+  double na = 0.0, nb = 0.0, dn = 0.0, rt = 0.0, bad = 0.0;
+  if (pos < F.prob_node_off[p + 1]) {
+    const int v = F.prob_nodes[pos];
+    dn = d[v];
+    const int Kt = F.tree_nsites[F.tree_of[v]];
+    const int C = (Kt + F.chunk_w - 1) / F.chunk_w;
+    if (!kUltra && (flags & 1u) && !rtilde_in && pos >= F.prob_int_off[p]) add_node_rt(F, v, C, rt);
+    if (F.free_branch[v]) {
+      double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+      if (counts) {
 #pragma unroll
-      for (int w = 0; w < kW; ++w) {
-        sg += sh[j * kW + w];
-        shh += sh[NT / 64 + j * kW + w];
-        sr += sh[2 * (NT / 64) + j * kW + w];
+        for (int j = 0; j < 5; ++j) s[j] = counts[(int64_t)v * 5 + j];
+      } else {
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+          for (int j = 0; j < 5; ++j) s[j] += F.cpart[v * F.cp_v + c * F.cp_c + j];
       }
-      G += sg;
-      Hs += shh;
-      RT += sr;
+      if (kUltra) {
+        const BranchObj o = branch_obj(s, (double)Kt, nu0);
+        U.bA[v] = o.A;
+        U.bS1[v] = o.S1;
+        U.bB[v] = o.B;
+        na = s[0] + s[1] + s[3];
+        nb = s[2] + s[4];
+      } else {
+        dn = branch_length(F, s, (double)Kt, nu0, dn, na, nb);
+        if (!isfinite(dn)) bad = 1.0;
+        d[v] = dn;
+      }
     }
-    __syncthreads();
+    F.nu_a[pos] = na;
+    F.nu_b[pos] = nb;
+    F.nu_d[pos] = dn;  // (ultrametric: of fixed branches; k_ultra sets the others)
   }
+  if (kUltra) return;
+  const bool opt_nu = (flags & 2u) && F.prob_nfree[p] > 0;
+  NuSum n{0.0, 0.0, 0.0, 0.0};
+  if (opt_nu) nu_term(na, nb, dn, nu_start(nu0), n);
+  nu_store(F, 0, n, rt, bad, sh);
 }
 
-// Runs problem p's solve by the whole block of NT threads (sh: 3 NT / 64
-// doubles); nu and phi are also returned, the same in every thread.
-template <int NT>
-__device__ __forceinline__ void nu_solve(const DevForest& F, int p, const double* __restrict__ rtilde_in,
-                                         double* __restrict__ nu_p, double* __restrict__ phi_p, int resume, double* sh,
-                                         double& nu_io, double& phi_io) {
-  NuState* st = F.nu_state + p;
+// An evaluation of the nu solves: the first one (after k_ultra), or the second
+// one of those that the first has not brought to their end.
+template <bool kFirst>
+__global__ void __launch_bounds__(kNuThreads) k_nu_eval(DevForest F, const double* __restrict__ rtilde_in,
+                                                        const double* __restrict__ nu,
+                                                        const int32_t* __restrict__ done) {
+  __shared__ double sh[6 * (kNuThreads / 64)];
+  const int p = nu_problem(F, (int)blockIdx.x);
+  if (done && done[p]) return;
   const uint32_t flags = F.prob_flags[p];
   const bool opt_nu = (flags & 2u) && F.prob_nfree[p] > 0;
-  int status = 0;
-  double x, lo, hi;
-  int evals;
-  bool fin = false;
-  if (!resume) {
-    x = (nu_io > 0.0 && nu_io < 1.0) ? nu_io : 0.5;
-    lo = 0.0;
-    hi = 2.0;  // hi > 1: the bound x = 1 has not been evaluated
-    // the first evaluation also sums the dropout responsibilities, as
-    // k_nu_eval's first launch does
-    const bool want_rt = (flags & 1u) && !rtilde_in;
-    double G, Hs, RT;
-    nu_eval_spans<NT>(F, p, x, opt_nu, want_rt, G, Hs, RT, sh);
-    if (flags & 1u) {
-      const double r = rtilde_in ? rtilde_in[p] : RT;
-      double phi_star = r / (F.prob_nobs[p] + r);
-      if (fabs(phi_star) < F.prob_phimin[p]) phi_star = 0.0;
-      phi_io = phi_star;
-      if (threadIdx.x == 0) *phi_p = phi_star;
-    }
-    status = st->d_bad ? 1 : 0;
-    __syncthreads();  // every thread has read d_bad before thread 0 clears it
-    if (threadIdx.x == 0) {
-      st->d_bad = 0;
-      st->status = status;
-      st->fin = 1;
-    }
+  const int pos = F.prob_node_off[p] + ((int)blockIdx.x - F.prob_blk_off[p]) * kNuThreads + (int)threadIdx.x;
+  const bool on = pos < F.prob_node_off[p + 1];
+  double x = nu_start(nu[p]), rt = 0.0;
+  NuSum n{0.0, 0.0, 0.0, 0.0};
+  if (!kFirst) {
     if (!opt_nu) return;
-    double xn;
-    fin = nu_newton_step(x, G, Hs, lo, hi, xn);
+    double r, b, lo = 0.0, hi = 2.0, xn;
+    nu_load<kNuThreads>(F, p, 0, n, r, b, sh);
+    const bool fin = nu_step(x, n, lo, hi, xn);
+    if (threadIdx.x == 0) {
+      // the step as k_nu_finish is to take it
+      double* o = nu_span(F, 1, (int)blockIdx.x);
+      o[4] = xn;
+      o[5] = fin ? 1.0 : 0.0;
+    }
+    if (fin) return;
     x = xn;
-    evals = 1;
-  } else {
-    x = st->x;
-    lo = st->lo;
-    hi = st->hi;
-    evals = kNuIters + 1;
-    status = st->status;
+    n = NuSum{0.0, 0.0, 0.0, 0.0};
+  } else if (on && (flags & 1u) && !rtilde_in && pos >= F.prob_int_off[p]) {
+    const int C = (F.tree_nsites[F.prob_tree_off[p]] + F.chunk_w - 1) / F.chunk_w;
+    add_node_rt(F, F.prob_nodes[pos], C, rt);
   }
-  for (; evals < kNuMaxEvals && !fin; ++evals) {
-    double G, Hs, RT;
-    nu_eval_spans<NT>(F, p, x, true, false, G, Hs, RT, sh);
-    double xn;
-    fin = nu_newton_step(x, G, Hs, lo, hi, xn);
-    x = xn;
-  }
-  nu_io = x;
-  if (threadIdx.x == 0) {
-    *nu_p = x;
-    st->x = x;
-    st->lo = lo;
-    st->hi = hi;
-    st->fin = 1;
-    st->status = status | (fin ? 0 : 2);
-  }
+  if (on && opt_nu) nu_term(F.nu_a[pos], F.nu_b[pos], F.nu_d[pos], x, n);
+  nu_store(F, kFirst ? 0 : 1, n, rt, 0.0, sh);
 }
 
-__global__ void __launch_bounds__(kNuSolveThreads) k_nu_solve(DevForest F, const double* __restrict__ rtilde_in,
-                                                             double* __restrict__ nu, double* __restrict__ phi,
-                                                             const int32_t* __restrict__ done, int resume) {
-  __shared__ double sh[3 * (kNuSolveThreads / 64)];
+// phi, the end of the nu solve and the status of the M-step, a block per
+// problem: the steps of the two evaluations, and more of them where the solve
+// is still open.
+__global__ void __launch_bounds__(kNuFinishThreads) k_nu_finish(DevForest F, const double* __restrict__ rtilde_in,
+                                                               double* __restrict__ nu, double* __restrict__ phi,
+                                                               const int32_t* __restrict__ done) {
+  __shared__ double sh[6 * (kNuFinishThreads / 64)];
   const int p = blockIdx.x;
   if (done && done[p]) return;
-  // every thread reads the same flag, written by an earlier launch
-  if (resume && F.nu_state[p].fin) return;
-  double nv = nu[p], pv = phi[p];
-  nu_solve<kNuSolveThreads>(F, p, rtilde_in, nu + p, phi + p, resume, sh, nv, pv);
+  const uint32_t flags = F.prob_flags[p];
+  const bool opt_nu = (flags & 2u) && F.prob_nfree[p] > 0;
+  double x = nu_start(nu[p]), rt, bad, lo = 0.0, hi = 2.0, xn;  // (hi > 1: x = 1 not evaluated)
+  NuSum n;
+  nu_load<kNuFinishThreads>(F, p, 0, n, rt, bad, sh);
+  bool fin = true;
+  if (opt_nu) {
+    nu_step(x, n, lo, hi, xn);
+    const double* o = nu_span(F, 1, F.prob_blk_off[p]);
+    x = o[4];
+    fin = o[5] != 0.0;
+    const int e = F.prob_node_off[p + 1];
+    for (int evals = 1; evals < kNuMaxEvals && !fin; ++evals) {
+      double z0 = 0.0, z1 = 0.0;
+      if (evals == 1) {
+        nu_load<kNuFinishThreads>(F, p, 1, n, z0, z1, sh);
+      } else {
+        n = NuSum{0.0, 0.0, 0.0, 0.0};
+        for (int i = F.prob_node_off[p] + (int)threadIdx.x; i < e; i += kNuFinishThreads)
+          nu_term(F.nu_a[i], F.nu_b[i], F.nu_d[i], x, n);
+        nu_block_sum<kNuFinishThreads>(n, z0, z1, sh);
+      }
+      fin = nu_step(x, n, lo, hi, xn);
+      x = xn;
+    }
+  }
+  if (threadIdx.x != 0) return;
+  if (opt_nu) nu[p] = x;
+  if (flags & 1u) {
+    const double r = rtilde_in ? rtilde_in[p] : rt;
+    double phi_star = r / (F.prob_nobs[p] + r);
+    if (fabs(phi_star) < F.prob_phimin[p]) phi_star = 0.0;
+    phi[p] = phi_star;
+  }
+  // a branch length came out non-finite: reported as the reference's failed
+  // branch solve (EM_solver.py:415-418,450-459)
+  F.mstep_status[p] = (bad != 0.0 ? 1 : 0) | (fin ? 0 : 2);
 }
 
 // ---------------------------------------------------------------------------
@@ -3402,26 +3342,21 @@ __device__ __forceinline__ void lds_set_coef(const LdsPlan& L, int ib, int r, co
   o->esil[i] = c.msil != 0.0 ? c.esil : kZeroTop;
 }
 
-// sums of three values over the block's threads (sh: 3 kLdsThreads / 64
-// doubles, free again after the next barrier)
-__device__ __forceinline__ void lds_sum3(double& a, double& b, double& c, double* sh) {
+// sums of kN values over the block's threads (sh: kN kLdsThreads / 64 doubles, free again after the next barrier)
+template <int kN>
+__device__ __forceinline__ void lds_sum(double (&v)[kN], double* sh) {
   constexpr int kW = kLdsThreads / 64;
-  a = seg_sum_last<64>(a);
-  b = seg_sum_last<64>(b);
-  c = seg_sum_last<64>(c);
-  if ((threadIdx.x & 63) == 63) {
-    double* o = sh + 3 * (threadIdx.x >> 6);
-    o[0] = a;
-    o[1] = b;
-    o[2] = c;
+#pragma unroll
+  for (int j = 0; j < kN; ++j) {
+    v[j] = seg_sum_last<64>(v[j]);
+    if ((threadIdx.x & 63) == 63) sh[kN * (threadIdx.x >> 6) + j] = v[j];
   }
   lds_barrier();
-  a = b = c = 0.0;
 #pragma unroll
-  for (int i = 0; i < kW; ++i) {
-    a += sh[3 * i];
-    b += sh[3 * i + 1];
-    c += sh[3 * i + 2];
+  for (int j = 0; j < kN; ++j) {
+    v[j] = 0.0;
+#pragma unroll
+    for (int i = 0; i < kW; ++i) v[j] += sh[kN * i + j];
   }
 }
 
@@ -3454,7 +3389,7 @@ __device__ __forceinline__ const PbArgs& pb_args() {
 }
 __global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
   extern __shared__ __align__(16) char lds[];
-  __shared__ double sh[2][3 * (kLdsThreads / 64)];
+  __shared__ double sh[2][5 * (kLdsThreads / 64)];
   const int p = (int)blockIdx.x;
   const int t = p;  // one tree a problem
   const int what = pb_args().what;
@@ -3488,9 +3423,9 @@ __global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
       __syncthreads();
     }
     const bool out = (what & kPbOut) && !((what & kPbEm) && step == pb_args().max_iter);
-    double llh = lds_pass(x, hn, out, [&] { return lds_root(pb_args().F, x, t, pb_args().site_llh_out); });
-    double z0 = 0.0, z1 = 0.0;
-    lds_sum3(llh, z0, z1, sh[0]);
+    double lsum[1] = {lds_pass(x, hn, out, [&] { return lds_root(pb_args().F, x, t, pb_args().site_llh_out); })};
+    lds_sum<1>(lsum, sh[0]);
+    const double llh = lsum[0];
     if (out) lds_fold(x);
     const PbArgs& A = pb_args();
     const DevForest& F = A.F;
@@ -3545,21 +3480,24 @@ __global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
         F.nu_d[F.node_pos[v]] = dn;
       }
     }
-    // phi, then nu: bracketed Newton on h' (as nu_solve)
-    double xx = nv > 0.0 && nv < 1.0 ? nv : 0.5, lo = 0.0, hi = 2.0;
+    // phi, then nu (as k_nu_finish)
+    double xx = nu_start(nv), lo = 0.0, hi = 2.0;
     bool fin = !opt_nu;
     int evals = 0;
     for (; evals == 0 || (!fin && evals < kNuMaxEvals); ++evals) {
-      double g = 0.0, h = 0.0;
+      NuSum n{0.0, 0.0, 0.0, 0.0};
       if (opt_nu) {
-        nu_term(a0, b0, d0, xx, g, h);
+        nu_term(a0, b0, d0, xx, n);
         for (int r = (int)threadIdx.x + kLdsThreads; r < nbr; r += kLdsThreads) {
           const int pos = F.node_pos[lds_branch_node(F, x, t, r)];
-          nu_term(F.nu_a[pos], F.nu_b[pos], F.nu_d[pos], xx, g, h);
+          nu_term(F.nu_a[pos], F.nu_b[pos], F.nu_d[pos], xx, n);
         }
       }
       double third = evals == 0 ? (bad != 0.0 ? INFINITY : rt) : 0.0;
-      lds_sum3(g, h, third, sh[1 - (evals & 1)]);
+      double v[5] = {n.g, n.g1, n.g2, n.g3, third};
+      lds_sum<5>(v, sh[1 - (evals & 1)]);
+      n = NuSum{v[0], v[1], v[2], v[3]};
+      third = v[4];
       if (evals == 0) {
         bad = isfinite(third) ? 0.0 : 1.0;
         if (flags & 1u) {
@@ -3569,19 +3507,14 @@ __global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
         if (!opt_nu) break;
       }
       double xn;
-      fin = nu_newton_step(xx, g, h, lo, hi, xn);
+      fin = nu_step(xx, n, lo, hi, xn);
       xx = xn;
     }
     if (opt_nu) nv = xx;
     if (threadIdx.x == 0) {
-      NuState* st = F.nu_state + p;
       A.phi[p] = pv;
       A.nu[p] = nv;
-      st->x = xx;
-      st->lo = lo;
-      st->hi = hi;
-      st->fin = 1;
-      st->status = (bad != 0.0 ? 1 : 0) | (fin ? 0 : 2);
+      F.mstep_status[p] = (bad != 0.0 ? 1 : 0) | (fin ? 0 : 2);
     }
     lds_leaves(x, pv);
   }
@@ -4309,21 +4242,16 @@ void run_rtilde(const DevForest& F, double* rtilde, const int32_t* done, hipStre
 
 void run_mstep(const DevForest& F, const double* counts, const double* rtilde, double* d, double* nu, double* phi,
                const int32_t* done, hipStream_t s, const UltraDev* U) {
-  UltraDev none{};
-  hipLaunchKernelGGL(k_branch, dim3((F.num_nodes + 63) / 64), dim3(64), 0, s, F, counts, d, nu, done,
-                     U ? *U : none, U ? 1 : 0);
-  if (U)
+  const dim3 g(F.num_nu_blocks), b(kNuThreads);
+  if (U) {
+    hipLaunchKernelGGL(k_branch<true>, g, b, 0, s, F, counts, rtilde, d, nu, done, *U);
     run_ultra(F, *U, d, nu, done, s);
-  // one launch when the problems keep enough blocks busy; otherwise split
-  // each problem's branches over several blocks per evaluation
-  if (F.max_prob_nodes <= kNuSolveMaxNodes && F.num_problems >= 8) {
-    hipLaunchKernelGGL(k_nu_solve, dim3(F.num_problems), dim3(kNuSolveThreads), 0, s, F, rtilde, nu, phi, done, 0);
-    return;
+    hipLaunchKernelGGL(k_nu_eval<true>, g, b, 0, s, F, rtilde, nu, done);
+  } else {
+    hipLaunchKernelGGL(k_branch<false>, g, b, 0, s, F, counts, rtilde, d, nu, done, UltraDev{});
   }
-  for (int it = 0; it <= kNuIters; ++it)
-    hipLaunchKernelGGL(k_nu_eval, dim3(F.num_nu_blocks), dim3(kNuThreads), 0, s, F, rtilde, nu, phi, done, it);
-  // solves the launches above left unconverged (rare): one block each
-  hipLaunchKernelGGL(k_nu_solve, dim3(F.num_problems), dim3(kNuSolveThreads), 0, s, F, rtilde, nu, phi, done, 1);
+  hipLaunchKernelGGL(k_nu_eval<false>, g, b, 0, s, F, rtilde, nu, done);
+  hipLaunchKernelGGL(k_nu_finish, dim3(F.num_problems), dim3(kNuFinishThreads), 0, s, F, rtilde, nu, phi, done);
 }
 
 }  // namespace laml

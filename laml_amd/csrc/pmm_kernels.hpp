@@ -9,16 +9,8 @@
 
 namespace laml {
 
-// Newton state of one problem's nu solve, and the status of its last M-step
-struct NuState {
-  double x, lo, hi;
-  int32_t fin;
-  int32_t count;   // blocks arrived in the current evaluation
-  int32_t status;  // last M-step: bit 0 a branch length came out non-finite,
-                   // bit 1 the nu solve did not converge (kept at its last
-                   // iterate)
-  int32_t d_bad;   // set by k_branch, folded into status by the nu solve
-};
+// branches of a problem that a block of the nu evaluations takes
+constexpr int kNuSpan = 256;
 
 // Per internal node, what the inside row kernel reads before its row loads
 // (one scalar load instead of chains of dependent ones): children, problem,
@@ -66,7 +58,6 @@ struct DevForest {
   const int32_t* node_pos;       // [N] position of each node in prob_nodes
   const int32_t* prob_blk_off;   // [P+1] blocks of the nu solve per problem
   int32_t num_nu_blocks;
-  int32_t max_prob_nodes;        // branches of the largest problem
   const uint32_t* prob_flags;
   const double* prob_nobs;
   const double* prob_phimin;
@@ -104,8 +95,9 @@ struct DevForest {
   double* nu_a;     // [N] by position in prob_nodes: S0+S1+S3 of the branch
   double* nu_b;     // [N] S2+S4 (0 for fixed branches)
   double* nu_d;     // [N] new branch length
-  double* nu_part;  // [num_nu_blocks * 3] partial sums of the nu solve
-  NuState* nu_state;  // [P]
+  double* nu_part;  // [2][num_nu_blocks][6] partial sums of the nu solve
+  int32_t* mstep_status;  // [P] last M-step: bit 0 a branch length came out non-finite, bit 1 the nu solve did
+                          // not converge (kept at its last iterate)
 };
 
 // a free branch of the ultrametric solve: its node, and the class (numbered
