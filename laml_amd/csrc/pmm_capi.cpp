@@ -109,6 +109,13 @@ struct laml_forest {
     bool fuse;
     std::vector<int32_t> in_cpw, out_cpw;
   } def{};
+  // clades of the inside pass: whether the forest takes them, and the most
+  // nodes of one (0: by the forest's size; environment LAML_CLADES, where 0
+  // turns them off)
+  bool clades = false;
+  int clade_cap = 0;
+  int64_t clade_q = 0;              // most prior weights of a 64-site chunk
+  std::deque<laml::CladePlan> clade_plans;
   std::deque<laml::ChainPlan> chain_plans;  // a deque: plans stay put when more are added
   std::vector<int32_t> h_heavy;  // heavy child of each node (-1: no internal child)
   std::vector<int32_t> h_child0, h_child1;
@@ -766,6 +773,16 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
     const int64_t units = (int64_t)(N - d->num_leaves) * ((max_k + 63) / 64);
     f->chains = env ? (atoi(env) & (LAML_CHAINS_OUTSIDE | LAML_CHAINS_INSIDE))
                     : (f->W == 64 && units >= 32768 ? LAML_CHAINS_OUTSIDE : 0);
+    const char* cenv = getenv("LAML_CLADES");
+    if (cenv) f->clade_cap = std::max(0, atoi(cenv));
+    int64_t qmax = 0;  // prior weights of a 64-site chunk
+    for (int t = 0; t < T; ++t)
+      for (int k = 0; k < d->tree_nsites[t]; k += 64) {
+        const int32_t* qo = d->site_qoff + tree_site_base[t];
+        qmax = std::max<int64_t>(qmax, qo[std::min(k + 64, d->tree_nsites[t])] - qo[k]);
+      }
+    f->clade_q = qmax;
+    f->clades = f->W == 64 && qmax * 8 <= laml::kCladeMaxQ && (cenv ? f->clade_cap > 0 : units >= laml::kCladeForest);
   }
   f->h_row_off = row_off;
   if ((rc = upload_node_recs(f, row_off))) {
@@ -1519,6 +1536,182 @@ static const laml::ChainPlan* chain_plan(laml_forest* f, int hs) {
   return &f->chain_plans.back();
 }
 
+// The clade plan of the inside pass (nullptr: it runs none): row kernels in
+// their default shapes, full inside storage, no cherry fusion, no inside
+// chains, and the plan of the current split built.
+static bool clades_now(const laml_forest* f) {
+  return f->clades && f->W == 64 && f->ckpt_L == 0 && f->pass_mode != LAML_PASS_TREES && !fuse_now(f) &&
+         !(f->chains & LAML_CHAINS_INSIDE) && f->in_cpw == f->def.in_cpw && hybrid_split(f) > 1;
+}
+static const laml::CladePlan* pass_clades(const laml_forest* f) {
+  if (clades_now(f))
+    for (const laml::CladePlan& cl : f->clade_plans)
+      if (cl.h_split == hybrid_split(f)) return &cl;
+  return nullptr;
+}
+
+// Builds the clade plan of the internal nodes below the current split, if
+// there is none yet (kept for the forest's life).  A call that is being
+// captured, or that finds no memory, runs level launches.
+static void prepare_clades(laml_forest* f, hipStream_t s) {
+  if (!clades_now(f) || pass_clades(f)) return;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return;
+  const int hs = hybrid_split(f);
+  std::lock_guard<std::mutex> legacy_lock(g_legacy_mu);  // (as chain_plan)
+  const int n = f->F.num_leaves, B = f->level_off[hs];
+  laml::CladePlan cl;
+  cl.h_split = hs;
+  // nodes of each subtree, and the pending states that its walk needs; both
+  // grow towards the root, so the subtrees within bounds are closed below
+  std::vector<int32_t> size(B, 0), need(B, 0);
+  for (int v = n; v < B; ++v) {
+    const int a = f->h_child0[v], b = f->h_child1[v];
+    const int na = need[a], nb = need[b];
+    size[v] = size[a] + size[b] + 1;
+    need[v] = a >= n && b >= n ? std::max(std::max(na, nb), std::min(na, nb) + 1) : std::max(na, nb);
+  }
+  cl.cap = f->clade_cap;
+  if (cl.cap <= 0)
+    cl.cap = (int)std::max<int64_t>(laml::kCladeMin, std::min<int64_t>(laml::kCladeCap, (int64_t)(B - n) *
+                                                                                         f->F.max_chunks /
+                                                                                         laml::kCladePairs));
+  auto in = [&](int v) { return size[v] <= cl.cap && need[v] <= laml::kCladeSlots; };
+  std::vector<int32_t> roots, round(B, -1);
+  std::vector<std::vector<int32_t>> rounds;
+  for (int v = n; v < B; ++v) {
+    if (in(v)) {
+      const int pa = f->h_parent[v];
+      if (pa < 0 || pa >= B || !in(pa)) roots.push_back(v);
+      continue;
+    }
+    const int r = std::max(round[f->h_child0[v]], round[f->h_child1[v]]) + 1;
+    round[v] = r;
+    if ((int)rounds.size() <= r) rounds.resize(r + 1);
+    rounds[r].push_back(v);
+  }
+  std::vector<int32_t> rest;
+  for (const auto& r : rounds) {
+    cl.round_off.push_back((int32_t)rest.size());
+    rest.insert(rest.end(), r.begin(), r.end());
+  }
+  cl.round_off.push_back((int32_t)rest.size());
+  // blocks of clades of one tree, the largest first
+  std::stable_sort(roots.begin(), roots.end(), [&](int a, int b) {
+    const int ta = f->h_tree_of[a], tb = f->h_tree_of[b];
+    return ta != tb ? ta < tb : size[a] > size[b];
+  });
+  std::vector<int4> blocks;
+  for (size_t i = 0; i < roots.size(); ++i) {
+    const int t = f->h_tree_of[roots[i]];
+    if (blocks.empty() || blocks.back().z != t || blocks.back().y == laml::kCladeWaves)
+      blocks.push_back(make_int4((int)i, 0, t, size[roots[i]]));
+    ++blocks.back().y;
+  }
+  std::stable_sort(blocks.begin(), blocks.end(), [](const int4& a, const int4& b) { return a.w > b.w; });
+  cl.q_bytes = (int)((f->clade_q + 2) * 8);  // (with a spare entry)
+  std::vector<int4> clades;
+  std::vector<int32_t> leaf_row;
+  std::vector<int32_t> pos(f->F.num_nodes, -1);
+  std::vector<laml::CladeStep> steps;
+  auto row_of = [&](int v) { return (int32_t)(f->h_row_off[v] >> 6); };
+  const size_t inner = (size_t)(B - n) - rest.size();
+  clades.reserve(roots.size());
+  steps.reserve(inner);
+  leaf_row.reserve(2 * inner);
+  struct Item {
+    int v, depth, push;
+    bool open;
+  };
+  std::vector<Item> stack;
+  for (const int root : roots) {
+    const int batch0 = (int)(leaf_row.size() / laml::kCladeBatch);
+    int used = laml::kCladeBatch;  // places taken of the last batch
+    clades.push_back(make_int4((int)steps.size(), size[root], batch0, 0));
+    stack.assign(1, Item{root, 0, 0, true});
+    while (!stack.empty()) {
+      const Item it = stack.back();
+      stack.pop_back();
+      int a = f->h_child0[it.v], b = f->h_child1[it.v];
+      const bool ia = a >= n, ib = b >= n;
+      if (it.open) {
+        stack.push_back(Item{it.v, it.depth, it.push, false});
+        if (ia && ib) {
+          // the needier child first; its result waits in slot `depth`
+          if (need[b] > need[a]) std::swap(a, b);
+          stack.push_back(Item{b, it.depth + 1, 0, true});
+          stack.push_back(Item{a, it.depth, it.depth + 1, true});
+        } else if (ia || ib) {
+          stack.push_back(Item{ia ? a : b, it.depth, 0, true});
+        }
+        continue;
+      }
+      laml::CladeStep r{};
+      const int kind = ia && ib ? 2 : (ia || ib ? 1 : 0);
+      // first the carried child: of two internal ones the one walked last
+      if (kind == 2 ? need[b] <= need[a] : ib) std::swap(a, b);
+      pos[a] = 2 * (int)steps.size();
+      pos[b] = 2 * (int)steps.size() + 1;
+      r.row = row_of(it.v);
+      r.flags = kind | (kind == 2 ? it.depth << 2 : 0) | it.push << 4;
+      if (kind < 2) {
+        if (used + 2 - kind > laml::kCladeBatch) {
+          // (the places left over repeat a row)
+          leaf_row.resize((leaf_row.size() / laml::kCladeBatch + 1) * laml::kCladeBatch, row_of(b));
+          used = 0;
+          r.flags |= 128;
+        }
+        int32_t* ro = &leaf_row[leaf_row.size() - laml::kCladeBatch];
+        if (kind == 0) {
+          r.flags |= used << 8;
+          ro[used++] = row_of(a);
+        }
+        r.flags |= used << 11;
+        ro[used++] = row_of(b);
+      }
+      steps.push_back(r);
+    }
+    clades.back().w = (int)(leaf_row.size() / laml::kCladeBatch) - batch0;
+  }
+  cl.num = (int)blocks.size();
+  // one allocation
+  size_t bytes = 0;
+  auto place = [&](size_t n) {
+    const size_t o = bytes;
+    bytes += (n + 255) / 256 * 256;
+    return o;
+  };
+  const size_t o[7] = {place(blocks.size() * sizeof(int4)),
+                       place(clades.size() * sizeof(int4)),
+                       place(steps.size() * sizeof(laml::CladeStep)),
+                       place(pos.size() * sizeof(int32_t)),
+                       place(leaf_row.size() * sizeof(int32_t)),
+                       place(rest.size() * sizeof(int32_t)),
+                       place(steps.size() * sizeof(laml::CladeCoef))};
+  char* m = nullptr;
+  auto up = [&](size_t at, const void* src, size_t n) {
+    return n == 0 || hipMemcpy(m + at, src, n, hipMemcpyHostToDevice) == hipSuccess;
+  };
+  if (f->alloc(&m, bytes) || !up(o[0], blocks.data(), blocks.size() * sizeof(int4)) ||
+      !up(o[1], clades.data(), clades.size() * sizeof(int4)) ||
+      !up(o[2], steps.data(), steps.size() * sizeof(laml::CladeStep)) ||
+      !up(o[3], pos.data(), pos.size() * sizeof(int32_t)) ||
+      !up(o[4], leaf_row.data(), leaf_row.size() * sizeof(int32_t)) ||
+      !up(o[5], rest.data(), rest.size() * sizeof(int32_t))) {
+    (void)hipGetLastError();
+    f->clades = false;
+    return;
+  }
+  cl.blocks = reinterpret_cast<const int4*>(m + o[0]);
+  cl.clades = reinterpret_cast<const int4*>(m + o[1]);
+  cl.steps = reinterpret_cast<const laml::CladeStep*>(m + o[2]);
+  cl.pos = reinterpret_cast<const int32_t*>(m + o[3]);
+  cl.leaf_row = reinterpret_cast<const int32_t*>(m + o[4]);
+  cl.rest = reinterpret_cast<const int32_t*>(m + o[5]);
+  cl.coef = reinterpret_cast<laml::CladeCoef*>(m + o[6]);
+  f->clade_plans.push_back(std::move(cl));
+}
+
 // the chain plan of a pass below split level hs (nullptr: that pass runs
 // no chains)
 static const laml::ChainPlan* pass_chains(laml_forest* f, bool inside, int hs) {
@@ -1529,7 +1722,7 @@ static const laml::ChainPlan* pass_chains(laml_forest* f, bool inside, int hs) {
 }
 
 // builds the chain plans the next passes use, outside any stream capture
-static int prepare_chains(laml_forest* f) {
+static int prepare_chains(laml_forest* f, hipStream_t s) {
   const int hs = hybrid_split(f);
   for (const bool inside : {true, false}) {
     if (!(chains_now(f) & (inside ? LAML_CHAINS_INSIDE : LAML_CHAINS_OUTSIDE))) continue;
@@ -1537,12 +1730,27 @@ static int prepare_chains(laml_forest* f) {
     const int top = t <= 0 ? hs : std::min(t, hs);
     if (top > 1 && !chain_plan(f, top)) return fail(LAML_ENOMEM, "chain plan");
   }
+  prepare_clades(f, s);
   return LAML_OK;
+}
+
+// the coefficients of every branch, for an inside pass in the current launch
+// plan too
+static void pass_coef(laml_forest* f, DevForest& F, const double* d, const double* nu, const int32_t* done,
+                      hipStream_t s) {
+  const laml::CladePlan* cl = pass_clades(f);
+  F.clade_coef = cl ? cl->coef : nullptr;
+  F.clade_pos = cl ? cl->pos : nullptr;
+  laml::run_coef(F, d, nu, done, s);
 }
 
 // inside levels [1, hs) of the level and hybrid passes: chains below the
 // chain region's top, level launches above it
 static void inside_below(laml_forest* f, const DevForest& F, int hs, const int32_t* done, hipStream_t s) {
+  if (const laml::CladePlan* cl = F.clade_coef ? pass_clades(f) : nullptr) {
+    laml::run_inside_clades(F, *cl, done, s);
+    return;
+  }
   const laml::ChainPlan* cp = pass_chains(f, true, hs);
   if (cp) laml::run_inside_chains(F, *cp, done, s);
   laml::run_inside_levels(F, f->level_off, f->W, cp ? cp->h_split : 1, hs, f->in_cpw, done, s);
@@ -1572,7 +1780,9 @@ static void pass_inside_root(laml_forest* f, const DevForest& F, double* site_ll
     f->inside_fused = fuse_now(f);
     const DevForest G = with_cherries(f, F, f->inside_fused);
     const laml::ChainPlan* cp = pass_chains(f, true, hybrid_split(f));
-    laml::run_inside(G, f->level_off, f->W, f->h_top, f->in_cpw, done, s, f->inside_fused ? &f->split : nullptr, cp);
+    const laml::CladePlan* cl = F.clade_coef ? pass_clades(f) : nullptr;
+    laml::run_inside(G, f->level_off, f->W, f->h_top, f->in_cpw, done, s, f->inside_fused ? &f->split : nullptr, cp,
+                     cl);
     laml::run_root(G, f->W, site_llh, done, s);
   }
 }
@@ -1612,7 +1822,7 @@ static void pass_outside(laml_forest* f, const DevForest& F, bool with_root, con
 }
 
 // the inside rows of the last call's parameters, where it left none (its
-// branch coefficients are resident)
+// branch coefficients are resident; not in a clade plan's steps: F names none)
 static void ensure_rows(laml_forest* f, const DevForest& F, hipStream_t s) {
   if (f->rows_ok) return;
   pass_inside_root(f, F, nullptr, nullptr, s);
@@ -1634,10 +1844,10 @@ int laml_nll(laml_forest* f, const double* d, const double* nu, const double* ph
     f->rows_ok = f->alpha_complete = f->inside_fused = false;
     return check_launch();
   }
-  int rc = prepare_chains(f);
+  int rc = prepare_chains(f, s);
   if (rc) return rc;
   f->rows_ok = true;
-  laml::run_coef(F, d, nu, nullptr, s);
+  pass_coef(f, F, d, nu, nullptr, s);
   pass_inside_root(f, F, site_llh, nullptr, s);
   laml::run_llh(F, nll, none, 0, 0.0, s);
   return check_launch();
@@ -1660,8 +1870,8 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
     laml::run_rtilde(G, rtilde, nullptr, s);
     return check_launch();
   }
-  laml::run_coef(F, d, nu, nullptr, s);
-  int rc = prepare_chains(f);
+  pass_coef(f, F, d, nu, nullptr, s);
+  int rc = prepare_chains(f, s);
   if (rc) return rc;
   f->rows_ok = true;
   if (f->pass_mode == 1) {
@@ -1704,7 +1914,7 @@ int laml_outside(laml_forest* f, const double* phi, double* counts, double* rtil
   if (!f || !phi || !counts || !rtilde) return fail(LAML_EINVAL, "null argument");
   DeviceGuard guard(f->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rc = prepare_chains(f);
+  int rc = prepare_chains(f, s);
   if (rc) return rc;
   DevForest F = f->F;
   F.phi = phi;
@@ -1719,7 +1929,7 @@ int laml_grad(laml_forest* f, const double* d, const double* nu, const double* p
   if (!f || !d || !nu || !phi || !grad_d || !grad_nu || !grad_phi) return fail(LAML_EINVAL, "null argument");
   DeviceGuard guard(f->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rc = prepare_chains(f);
+  int rc = prepare_chains(f, s);
   if (rc) return rc;
   DevForest F = f->F;
   F.phi = phi;
@@ -1740,7 +1950,7 @@ int laml_mstep(laml_forest* f, const double* counts, const double* rtilde, doubl
 // one EM step of every problem not yet converged: inside pass, likelihood
 // and convergence test, then (unless this is the final step) outside pass
 // with posterior counts and the M-step
-static void em_step(laml_forest* f, const DevForest& F, const EmState& em, double* d, double* nu, double* phi,
+static void em_step(laml_forest* f, DevForest F, const EmState& em, double* d, double* nu, double* phi,
                     double* nll, int32_t max_iter, double tol, bool last, hipStream_t s) {
   if (problem_now(f)) {
     // (ultrametric forests: their M-step is a launch of its own)
@@ -1751,7 +1961,7 @@ static void em_step(laml_forest* f, const DevForest& F, const EmState& em, doubl
     if (!last) laml::run_mstep(G, nullptr, nullptr, d, nu, phi, em.done, s, f->ultra_on ? &f->U : nullptr);
     return;
   }
-  laml::run_coef(F, d, nu, em.done, s);
+  pass_coef(f, F, d, nu, em.done, s);
   if (f->pass_mode == 1 && !last) {
     // one launch for the whole E-step; the outside half of a problem that
     // converges at this step is not used (its M-step is skipped)
@@ -1812,7 +2022,7 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
     f->rows_ok = f->alpha_complete = f->inside_fused = false;
     return LAML_OK;
   }
-  int prc = prepare_chains(f);
+  int prc = prepare_chains(f, s);
   if (prc) return prc;
   laml::run_em_reset(em, P, s);
   // The EM step is captured once into a HIP graph and replayed: its kernel

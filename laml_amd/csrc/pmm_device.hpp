@@ -103,9 +103,8 @@ struct Eps {
   int e;
 };
 __device__ __forceinline__ Eps edge(int lab, double b0, double bA, int E, double q, const Coef& c) {
-  const bool z = lab == 0;
-  const double t0 = fma(z ? 0.0 : c.mut * q, bA, c.p1n * b0);
-  const double tA = z ? 0.0 : c.pn * bA;
+  const double t0 = fma(c.mut * q, bA, c.p1n * b0);  // (bA = 0 at 'z' nodes)
+  const double tA = c.pn * bA;
   const int es = (lab < 0 && c.msil != 0.0) ? c.esil : kZeroTop;
   const int e = max(E, es);
   const double s0 = ldexp(1.0, E - e);

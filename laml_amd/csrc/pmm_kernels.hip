@@ -37,7 +37,20 @@ __global__ void k_coef(DevForest F, const double* __restrict__ d, const double* 
   if (v >= F.num_nodes) return;
   const int p = F.tree_prob[F.tree_of[v]];
   if (done && done[p]) return;
-  F.coef[v] = branch_coef(d[v], nu[p]);
+  const Coef c = branch_coef(d[v], nu[p]);
+  F.coef[v] = c;
+  if (F.clade_pos) {
+    const int q = F.clade_pos[v];
+    if (q >= 0) {
+      CladeCoef& r = F.clade_coef[q >> 1];
+      const int i = q & 1;
+      r.p1n[i] = c.p1n;
+      r.mut[i] = c.mut;
+      r.pn[i] = c.pn;
+      r.msil[i] = c.msil;
+      r.esil[i] = c.esil;
+    }
+  }
 }
 
 // Segment mapping shared by the level kernels: a block of 256 threads holds
@@ -710,6 +723,170 @@ __global__ void __launch_bounds__(256) k_inside_chain(DevForest F, const int2* _
     prev = v;
     v = vn;
     r = rn;
+  }
+}
+
+// Inside pass over clades: a wavefront walks a clade's nodes in postorder at
+// one 64-site chunk.  The state of the node just done stays in registers, that
+// of a finished subtree whose sibling is still to come waits in the
+// wavefront's LDS slice (children with the larger need for slots first, so
+// two slots suffice for most subtrees of a few dozen leaves).  Rows are only
+// written, never read, and nothing is gathered for internal nodes: a node's
+// label comes from its children's, and its prior weight is that of the child
+// with the same label.  A load waits for all stores before it, so the steps
+// make none: the codes of kCladeBatch leaves at a time come with one load into
+// the LDS slice, a batch ahead.  The wavefronts of a block share a tree and a
+// chunk, whose prior weights (one contiguous piece of the table) they keep in
+// LDS: gathered from global memory, every lane of a gather touches another
+// cache line, and the L1 caches hold too few of them.  Sixteen trees of 10,000
+// leaves x 300 sites: 223 us (4.7 TB/s of rows written and codes read) and 112
+// us in the rounds above, where level launches took 653 us; 50,000 x 500: 100
+// and 70 us, 351.  Bound by the row stores and the latency of a step's chain
+// (LDS reads, then the arithmetic of one node) at six wavefronts a SIMD.  The
+// same operations as the level kernels, the same bits.
+struct CladeIn {
+  int lab, E;
+  double b0, bA, q;
+};
+struct CladeCtx {
+  double2* beta;
+  int32_t* bE;
+  double phi, qs;
+  unsigned k;
+  bool on, stream;
+  const int16_t* code;  // the lane's place in the wavefront's batch of leaf codes
+  const double* q;      // q[j]: the site's weight of edit state j (LDS)
+};
+// prior weight of a label (a leaf's code does as well)
+__device__ __forceinline__ double clade_q(const CladeCtx& x, int lab) {
+  const double g = x.q[max(lab, 1)];
+  return lab > 0 ? g : x.qs;
+}
+__device__ __forceinline__ CladeIn clade_leaf(const CladeCtx& x, int slot) {
+  const int code = x.code[slot * 64];
+  CladeIn a;
+  leaf_beta(code, x.phi, a.lab, a.b0, a.bA);
+  a.E = 0;
+  a.q = clade_q(x, code);
+  return a;
+}
+// the node of children a and b
+__device__ __forceinline__ CladeIn clade_node(const CladeCtx& x, int64_t ro, const CladeCoef& r, const CladeIn& a,
+                                              const CladeIn& b) {
+  const Eps ea = edge(a.lab, a.b0, a.bA, a.E, a.q, Coef{r.p1n[0], r.mut[0], r.pn[0], r.msil[0], r.esil[0], 0});
+  const Eps eb = edge(b.lab, b.b0, b.bA, b.E, b.q, Coef{r.p1n[1], r.mut[1], r.pn[1], r.msil[1], r.esil[1], 0});
+  const int lv = combine_label(a.lab, b.lab);
+  const double B0 = ea.e0 * eb.e0;
+  const double BA = lv != 0 ? ea.eA * eb.eA : 0.0;
+  const int sh = min(-exp_of(fmax(B0, BA)), 1000);
+  const double sc = ldexp(1.0, sh);
+  CladeIn c;
+  c.q = lv > 0 ? (a.lab > 0 ? a.q : b.q) : x.qs;
+  c.lab = lv;
+  c.b0 = B0 * sc;
+  c.bA = BA * sc;
+  c.E = ea.e + eb.e - sh;
+  if (x.on) {
+    const double2 o = make_double2(c.b0, c.bA);
+    if (x.stream)
+      store_stream(&row_at(x.beta + ro, x.k), o);
+    else
+      row_at(x.beta + ro, x.k) = o;
+    row_at(x.bE + ro, x.k) = c.E;
+  }
+  return c;
+}
+
+// a block: up to kCladeWaves clades of one tree, at one chunk
+__global__ void __launch_bounds__(64 * kCladeWaves) k_inside_clade(DevForest F, const int4* __restrict__ blocks,
+                                                                   const int4* __restrict__ clades,
+                                                                   const CladeStep* __restrict__ steps,
+                                                                   const int32_t* __restrict__ leaf_row,
+                                                                   int num, const int32_t* __restrict__ done) {
+  extern __shared__ __attribute__((aligned(16))) char clade_lds[];
+  // the chunks of a block's clades, eight workgroups apart, on one XCD: its
+  // L2 cache then serves their step records
+  const int g = (int)blockIdx.x >> 3, b = g / F.max_chunks * 8 + ((int)blockIdx.x & 7), chunk = g % F.max_chunks;
+  if (b >= num) return;
+  const int4 bd = uniform_load(blocks + b);
+  const int t = bd.z, k0 = chunk * 64;
+  const int K = F.tree_nsites[t], p = F.tree_prob[t];
+  if (k0 >= K) return;
+  if (done && done[p]) return;
+  const int lane = (int)(threadIdx.x & 63);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int sb = F.tree_site_base[t];
+  CladeCtx x;
+  x.k = (unsigned)(k0 + lane);
+  x.on = k0 + lane < K;
+  // lanes past the tree's sites run on their rows' pad codes (0) and store
+  // nothing
+  const unsigned ks = (unsigned)min(k0 + lane, K - 1);
+  x.qs = row_at(F.site_qsum + sb, ks);
+  {
+    double* q = (double*)(clade_lds + kCladeWaves * kCladeLds);
+    const int q0 = uniform_load(F.site_qoff + sb + k0), q1 = uniform_load(F.site_qoff + sb + min(k0 + 64, K));
+    for (int i = (int)threadIdx.x; i < q1 - q0; i += 64 * kCladeWaves) q[i] = F.prior[q0 + i];
+    // (a site without edit states reads q[1] all the same: the piece has a
+    // spare entry)
+    x.q = q + (row_at(F.site_qoff + sb, ks) - 1 - q0);
+    __syncthreads();
+  }
+  if (wave >= bd.y) return;
+  const int4 cd = uniform_load(clades + bd.x + wave);
+  x.phi = uniform_load(F.phi + p);
+  x.beta = F.beta;
+  x.bE = F.bE;
+  x.stream = F.stream_rows != 0;
+  char* slice = clade_lds + wave * kCladeLds;
+  char* batch = slice + kCladeSlots * kCladeSlotBytes;
+  x.code = (const int16_t*)batch + lane;
+  // a batch: eight lanes a leaf, eight sites a lane
+  const int32_t* lr = leaf_row + cd.z * kCladeBatch + (lane >> 3);
+  const int16_t* codes = F.codes + k0 + (lane & 7) * 8;
+  int nb = 1;
+  uint4 w = *(const uint4*)(codes + (int64_t)lr[0] * 64);
+  int row = lr[min(1, cd.w - 1) * kCladeBatch];
+  const CladeStep* st = steps + cd.x;
+  const CladeCoef* sc = F.clade_coef + cd.x;
+  CladeStep r = uniform_load(st);
+  CladeCoef cf = uniform_load(sc);
+  CladeIn c{0, 0, 0.0, 0.0, 0.0};
+  for (int j = 1;; ++j) {
+    if (r.flags & 128) {
+      *(uint4*)(batch + lane * 16) = w;
+      lds_wave_sync();
+      w = *(const uint4*)(codes + (int64_t)row * 64);
+      nb = min(nb + 1, cd.w - 1);
+      row = lr[nb * kCladeBatch];
+    }
+    const int kind = r.flags & 3;
+    CladeIn b;
+    if (kind == 2) {
+      const char* l = slice + ((r.flags >> 2) & 3) * kCladeSlotBytes;
+      const double2 u = *(const double2*)(l + lane * 16);
+      const int2 v = *(const int2*)(l + 1024 + lane * 8);
+      b = CladeIn{v.y, v.x, u.x, u.y, clade_q(x, v.y)};
+    } else {
+      b = clade_leaf(x, (r.flags >> 11) & 7);
+      if (kind == 0) c = clade_leaf(x, (r.flags >> 8) & 7);
+    }
+    // the next step's record, once the operands are there: LDS and scalar
+    // loads share a counter
+    int jn = min(j, cd.y - 1);
+    asm volatile("" : "+s"(jn) : "v"(b.q), "v"(c.q));
+    const CladeStep rn = uniform_load(st + jn);
+    const CladeCoef cn = uniform_load(sc + jn);
+    c = clade_node(x, (int64_t)r.row * 64, cf, c, b);
+    if (j == cd.y) break;
+    const int push = (r.flags >> 4) & 7;
+    if (push) {
+      char* l = slice + (push - 1) * kCladeSlotBytes;
+      *(double2*)(l + lane * 16) = make_double2(c.b0, c.bA);
+      *(int2*)(l + 1024 + lane * 8) = make_int2(c.E, c.lab);
+    }
+    r = rn;
+    cf = cn;
   }
 }
 
@@ -3992,7 +4169,7 @@ static void split_level(bool outside, const DevForest& F, const CherrySplit& cs,
 }
 
 void run_inside(const DevForest& F, const std::vector<int32_t>& lvl, int W, int h_top, const std::vector<int32_t>& cpw,
-                const int32_t* done, hipStream_t s, const CherrySplit* cs, const ChainPlan* cp) {
+                const int32_t* done, hipStream_t s, const CherrySplit* cs, const ChainPlan* cp, const CladePlan* cl) {
   const int H = (int)lvl.size() - 1;
   if (cs) {
     // fused cherries: row kernels on every level from 2 up, no top kernel
@@ -4000,9 +4177,11 @@ void run_inside(const DevForest& F, const std::vector<int32_t>& lvl, int W, int 
     return;
   }
   const int ht = std::max(1, std::min(h_top, H));
-  // chains below the chain plan's top level, level launches from there
-  const int h0 = cp ? std::min(cp->h_split, ht) : 1;
-  if (cp) run_inside_chains(F, *cp, done, s);
+  // chains below the chain plan's top level or clades and their rounds below
+  // theirs, level launches from there
+  const int h0 = cl ? std::min(cl->h_split, ht) : (cp ? std::min(cp->h_split, ht) : 1);
+  if (cl) run_inside_clades(F, *cl, done, s);
+  else if (cp) run_inside_chains(F, *cp, done, s);
   for (int h = h0; h < ht; ++h) inside_level(F, lvl, W, cpw, h, done, s);
   if (ht < H) {
     LAML_DISPATCH_W(W, {
@@ -4050,6 +4229,18 @@ void run_outside(const DevForest& F, const std::vector<int32_t>& lvl, int W, int
   const int h0 = cp ? std::min(cp->h_split, ht) : 1;
   for (int h = ht - 1; h >= h0; --h) outside_level(F, lvl, W, cpw, h, done, s);
   if (cp) run_outside_chains(F, *cp, done, s);
+}
+
+void run_inside_clades(const DevForest& F, const CladePlan& cl, const int32_t* done, hipStream_t s) {
+  if (cl.num > 0) {
+    const dim3 g((unsigned)((cl.num + 7) / 8 * 8 * F.max_chunks)), b(64 * kCladeWaves);
+    hipLaunchKernelGGL(k_inside_clade, g, b, (size_t)kCladeWaves * kCladeLds + cl.q_bytes, s, F, cl.blocks, cl.clades,
+                       cl.steps, cl.leaf_row, cl.num, done);
+  }
+  for (size_t r = 0; r + 1 < cl.round_off.size(); ++r) {
+    const int beg = cl.round_off[r], cnt = cl.round_off[r + 1] - beg;
+    launch_inside_rows(dim3((cnt + 3) / 4, F.max_chunks), s, F, beg, cnt, 1, done, cl.rest);
+  }
 }
 
 void run_inside_chains(const DevForest& F, const ChainPlan& cp, const int32_t* done, hipStream_t s) {

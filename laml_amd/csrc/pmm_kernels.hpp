@@ -78,6 +78,10 @@ struct DevForest {
   // state
   int16_t* labels;  // internal rows
   Coef* coef;       // [N]
+  // the coefficients of the clade plan of the next inside pass (null: none),
+  // written by k_coef, and their places by branch
+  struct CladeCoef* clade_coef;
+  const int32_t* clade_pos;
   double2* beta;    // internal rows
   int32_t* bE;
   // outside state (a0, aX) of internal nodes given all data, on the scale of
@@ -290,9 +294,67 @@ struct ChainPlan {
 // only thins rounds with wavefronts to spare (16 per SIMD)
 constexpr int64_t kPackWaves = 16384;
 
-// cp: the levels below the top kernel's run as heavy-path chains
+// Clades of the inside pass (k_inside_clade): maximal subtrees below level
+// h_split of at most `cap` internal nodes whose walk keeps at most kCladeSlots
+// pending states.  A wavefront walks a clade's nodes in postorder at a 64-site
+// chunk, so that their rows are written and never read; the other nodes below
+// h_split follow in rounds of row launches (`rest`: node list, round_off: host
+// offsets), each after the rounds of its children.
+constexpr int kCladeSlots = 2;
+constexpr int kCladeBatch = 8;  // leaves whose codes a wavefront loads at a time
+constexpr int kCladeSlotBytes = 64 * 24;
+constexpr int kCladeLds = kCladeSlots * kCladeSlotBytes + kCladeBatch * 128;  // a wavefront's slice
+// One node of a clade: its row, in units of 64 sites, and bits of flags: 0-1
+// kind (0 two leaves, 1 carried and leaf, 2 carried and pending), 2-3 slot of
+// the pending state, 4-6 one more than the slot that the result goes to (0:
+// carried only), 7 the next batch of leaves comes before this step, 8-10 and
+// 11-13 place of the children's codes in the batch.
+struct CladeStep {
+  int32_t row, flags;
+};
+// The coefficients of its branches in one piece, written by k_coef (scalar
+// loads of coefficients by branch took most of the walk's time); children
+// ordered so that the first is the one whose state the wavefront carries (or
+// both are leaves).
+struct CladeCoef {
+  double p1n[2], mut[2], pn[2], msil[2];
+  int32_t esil[2];
+};
+struct CladePlan {
+  int32_t h_split = -1, cap = 0;
+  int32_t num = 0;               // blocks
+  int32_t q_bytes = 0;           // LDS for the prior weights of a chunk
+  const int4* blocks = nullptr;  // first clade, clades, tree
+  const int4* clades = nullptr;  // offset into steps, steps, first batch, batches
+  const CladeStep* steps = nullptr;
+  CladeCoef* coef = nullptr;     // by step
+  const int32_t* pos = nullptr;  // [N] place of a branch's coefficients: 2 step + child, -1 none
+  const int32_t* leaf_row = nullptr;  // [batch][kCladeBatch] code rows of the leaves, in units of 64 sites
+  const int32_t* rest = nullptr;
+  std::vector<int32_t> round_off;
+};
+constexpr int kCladeWaves = 8;  // wavefronts of a block
+// Most nodes of a clade: one per kCladePairs (internal node, 64-site chunk)
+// pairs of the forest, between kCladeMin and kCladeCap.  Longer walks read
+// fewer rows back, but the wavefronts have to fill the chip.  Likelihood of
+// 10,000 leaves x 300 (50k pairs): 95 us at 16 and 32, 105 at 64 (109 by
+// levels); sixteen such trees 425 us at 16, 365 at 64 (681).
+constexpr int64_t kCladePairs = 2048;
+constexpr int kCladeMin = 16, kCladeCap = 64;
+// Forests of at least this many pairs take clades: 2,000 x 500 (16k pairs) 61
+// us, 77 by levels; 1,000 x 500 (8k) 47 and 53, but a forest that is solved
+// once and dropped does not earn its plan back.
+constexpr int64_t kCladeForest = 12288;
+// most LDS for a chunk's prior weights: 64 sites of 62 edit states (up to 21 KB
+// three blocks fit a CU)
+constexpr int kCladeMaxQ = 31 * 1024;
+
+// cp: the levels below the top kernel's run as heavy-path chains; cl: as
+// clades
 void run_inside(const DevForest& F, const std::vector<int32_t>& lvl, int W, int h_top, const std::vector<int32_t>& cpw,
-                const int32_t* done, hipStream_t s, const CherrySplit* cs = nullptr, const ChainPlan* cp = nullptr);
+                const int32_t* done, hipStream_t s, const CherrySplit* cs = nullptr, const ChainPlan* cp = nullptr,
+                const CladePlan* cl = nullptr);
+void run_inside_clades(const DevForest& F, const CladePlan& cl, const int32_t* done, hipStream_t s);
 void run_inside_chains(const DevForest& F, const ChainPlan& cp, const int32_t* done, hipStream_t s);
 // cp: the levels below the top kernel's run as heavy-path chains
 void run_outside(const DevForest& F, const std::vector<int32_t>& lvl, int W, int h_top,
