@@ -114,6 +114,8 @@ struct laml_forest {
   // turns them off)
   bool clades = false;
   int clade_cap = 0;
+  bool out_clades = false;          // and of the outside pass
+  const laml::CladePlan* coef_plan = nullptr;  // whose coefficients are those of the last call
   int64_t clade_q = 0;              // most prior weights of a 64-site chunk
   std::deque<laml::CladePlan> clade_plans;
   std::deque<laml::ChainPlan> chain_plans;  // a deque: plans stay put when more are added
@@ -782,6 +784,7 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
         qmax = std::max<int64_t>(qmax, qo[std::min(k + 64, d->tree_nsites[t])] - qo[k]);
       }
     f->clade_q = qmax;
+    f->out_clades = !env && (cenv || units >= laml::kCladeOutForest);
     f->clades = f->W == 64 && qmax * 8 <= laml::kCladeMaxQ && (cenv ? f->clade_cap > 0 : units >= laml::kCladeForest);
   }
   f->h_row_off = row_off;
@@ -1550,6 +1553,15 @@ static const laml::CladePlan* pass_clades(const laml_forest* f) {
   return nullptr;
 }
 
+// The same for the outside pass, whose chains and shapes must be the default
+// ones as well.
+static const laml::CladePlan* out_clades(const laml_forest* f, const DevForest& F) {
+  return F.clade_coef && f->out_clades && f->chains == f->def.chains && f->chain_top_out == f->def.chain_top_out &&
+                 f->out_cpw == f->def.out_cpw
+             ? pass_clades(f)
+             : nullptr;
+}
+
 // Builds the clade plan of the internal nodes below the current split, if
 // there is none yet (kept for the forest's life).  A call that is being
 // captured, or that finds no memory, runs level launches.
@@ -1601,16 +1613,20 @@ static void prepare_clades(laml_forest* f, hipStream_t s) {
     const int ta = f->h_tree_of[a], tb = f->h_tree_of[b];
     return ta != tb ? ta < tb : size[a] > size[b];
   });
-  std::vector<int4> blocks;
-  for (size_t i = 0; i < roots.size(); ++i) {
-    const int t = f->h_tree_of[roots[i]];
-    if (blocks.empty() || blocks.back().z != t || blocks.back().y == laml::kCladeWaves)
-      blocks.push_back(make_int4((int)i, 0, t, size[roots[i]]));
-    ++blocks.back().y;
-  }
-  std::stable_sort(blocks.begin(), blocks.end(), [](const int4& a, const int4& b) { return a.w > b.w; });
+  auto group = [&](int waves) {
+    std::vector<int4> g;
+    for (size_t i = 0; i < roots.size(); ++i) {
+      const int t = f->h_tree_of[roots[i]];
+      if (g.empty() || g.back().z != t || g.back().y == waves) g.push_back(make_int4((int)i, 0, t, size[roots[i]]));
+      ++g.back().y;
+    }
+    std::stable_sort(g.begin(), g.end(), [](const int4& a, const int4& b) { return a.w > b.w; });
+    return g;
+  };
+  const std::vector<int4> blocks = group(laml::kCladeWaves), oblocks = group(laml::kCladeOutWaves);
   cl.q_bytes = (int)((f->clade_q + 2) * 8);  // (with a spare entry)
   std::vector<int4> clades;
+  std::vector<laml::CladeOut> osteps;
   std::vector<int32_t> leaf_row;
   std::vector<int32_t> pos(f->F.num_nodes, -1);
   std::vector<laml::CladeStep> steps;
@@ -1618,6 +1634,7 @@ static void prepare_clades(laml_forest* f, hipStream_t s) {
   const size_t inner = (size_t)(B - n) - rest.size();
   clades.reserve(roots.size());
   steps.reserve(inner);
+  osteps.reserve(inner);
   leaf_row.reserve(2 * inner);
   struct Item {
     int v, depth, push;
@@ -1670,10 +1687,12 @@ static void prepare_clades(laml_forest* f, hipStream_t s) {
         ro[used++] = row_of(b);
       }
       steps.push_back(r);
+      osteps.push_back(laml::CladeOut{it.v, r.flags, {a, b}, {row_of(a), row_of(b)}});
     }
     clades.back().w = (int)(leaf_row.size() / laml::kCladeBatch) - batch0;
   }
   cl.num = (int)blocks.size();
+  cl.out_num = (int)oblocks.size();
   // one allocation
   size_t bytes = 0;
   auto place = [&](size_t n) {
@@ -1681,13 +1700,15 @@ static void prepare_clades(laml_forest* f, hipStream_t s) {
     bytes += (n + 255) / 256 * 256;
     return o;
   };
-  const size_t o[7] = {place(blocks.size() * sizeof(int4)),
+  const size_t o[9] = {place(blocks.size() * sizeof(int4)),
                        place(clades.size() * sizeof(int4)),
                        place(steps.size() * sizeof(laml::CladeStep)),
                        place(pos.size() * sizeof(int32_t)),
                        place(leaf_row.size() * sizeof(int32_t)),
                        place(rest.size() * sizeof(int32_t)),
-                       place(steps.size() * sizeof(laml::CladeCoef))};
+                       place(steps.size() * sizeof(laml::CladeCoef)),
+                       place(oblocks.size() * sizeof(int4)),
+                       place(osteps.size() * sizeof(laml::CladeOut))};
   char* m = nullptr;
   auto up = [&](size_t at, const void* src, size_t n) {
     return n == 0 || hipMemcpy(m + at, src, n, hipMemcpyHostToDevice) == hipSuccess;
@@ -1697,7 +1718,9 @@ static void prepare_clades(laml_forest* f, hipStream_t s) {
       !up(o[2], steps.data(), steps.size() * sizeof(laml::CladeStep)) ||
       !up(o[3], pos.data(), pos.size() * sizeof(int32_t)) ||
       !up(o[4], leaf_row.data(), leaf_row.size() * sizeof(int32_t)) ||
-      !up(o[5], rest.data(), rest.size() * sizeof(int32_t))) {
+      !up(o[5], rest.data(), rest.size() * sizeof(int32_t)) ||
+      !up(o[7], oblocks.data(), oblocks.size() * sizeof(int4)) ||
+      !up(o[8], osteps.data(), osteps.size() * sizeof(laml::CladeOut))) {
     (void)hipGetLastError();
     f->clades = false;
     return;
@@ -1709,6 +1732,8 @@ static void prepare_clades(laml_forest* f, hipStream_t s) {
   cl.leaf_row = reinterpret_cast<const int32_t*>(m + o[4]);
   cl.rest = reinterpret_cast<const int32_t*>(m + o[5]);
   cl.coef = reinterpret_cast<laml::CladeCoef*>(m + o[6]);
+  cl.out_blocks = reinterpret_cast<const int4*>(m + o[7]);
+  cl.out_steps = reinterpret_cast<const laml::CladeOut*>(m + o[8]);
   f->clade_plans.push_back(std::move(cl));
 }
 
@@ -1739,6 +1764,7 @@ static int prepare_chains(laml_forest* f, hipStream_t s) {
 static void pass_coef(laml_forest* f, DevForest& F, const double* d, const double* nu, const int32_t* done,
                       hipStream_t s) {
   const laml::CladePlan* cl = pass_clades(f);
+  f->coef_plan = cl;
   F.clade_coef = cl ? cl->coef : nullptr;
   F.clade_pos = cl ? cl->pos : nullptr;
   laml::run_coef(F, d, nu, done, s);
@@ -1759,6 +1785,11 @@ static void inside_below(laml_forest* f, const DevForest& F, int hs, const int32
 // outside levels [1, hs) of the level and hybrid passes
 static void outside_below(laml_forest* f, const DevForest& F, int hs, const int32_t* done, hipStream_t s,
                           bool allow_chains) {
+  if (const laml::CladePlan* cl = allow_chains ? out_clades(f, F) : nullptr) {
+    laml::run_outside_clades(F, *cl, done, s);
+    f->alpha_complete = false;
+    return;
+  }
   const laml::ChainPlan* cp = allow_chains ? pass_chains(f, false, hs) : nullptr;
   laml::run_outside_levels(F, f->level_off, f->W, cp ? cp->h_split : 1, hs, f->out_cpw, done, s);
   if (cp) laml::run_outside_chains(F, *cp, done, s);
@@ -1816,9 +1847,10 @@ static void pass_outside(laml_forest* f, const DevForest& F, bool with_root, con
     f->alpha_complete = true;
     return;
   }
-  const laml::ChainPlan* cp = allow_chains ? pass_chains(f, false, hybrid_split(f)) : nullptr;
-  laml::run_outside(F, f->level_off, f->W, f->h_top, f->out_cpw, done, s, nullptr, cp);
-  f->alpha_complete = cp == nullptr;
+  const laml::CladePlan* cl = allow_chains ? out_clades(f, F) : nullptr;
+  const laml::ChainPlan* cp = allow_chains && !cl ? pass_chains(f, false, hybrid_split(f)) : nullptr;
+  laml::run_outside(F, f->level_off, f->W, f->h_top, f->out_cpw, done, s, nullptr, cp, cl);
+  f->alpha_complete = !cp && !cl;
 }
 
 // the inside rows of the last call's parameters, where it left none (its
@@ -1842,6 +1874,7 @@ int laml_nll(laml_forest* f, const double* d, const double* nu, const double* ph
     laml::run_problem(lds_view(F, f->pb), f->pb, f->TW, const_cast<double*>(d), const_cast<double*>(nu),
                       const_cast<double*>(phi), nll, site_llh, nullptr, none, 1, 0, 0.0, laml::kPbCoef, s);
     f->rows_ok = f->alpha_complete = f->inside_fused = false;
+    f->coef_plan = nullptr;
     return check_launch();
   }
   int rc = prepare_chains(f, s);
@@ -1866,6 +1899,7 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
     laml::run_problem(G, f->pb, f->TW, const_cast<double*>(d), const_cast<double*>(nu), const_cast<double*>(phi), nll,
                       nullptr, nullptr, none, 1, 0, 0.0, laml::kPbCoef | laml::kPbOut, s);
     f->rows_ok = f->alpha_complete = f->inside_fused = false;
+    f->coef_plan = nullptr;
     laml::run_counts(G, counts, s);
     laml::run_rtilde(G, rtilde, nullptr, s);
     return check_launch();
@@ -1906,7 +1940,9 @@ static DevForest outside_again(laml_forest* f, const DevForest& F, const double*
     return G;
   }
   ensure_rows(f, F, s);
-  pass_outside(f, F, true, nullptr, s);
+  DevForest G = F;
+  if (f->coef_plan && f->coef_plan == pass_clades(f)) G.clade_coef = f->coef_plan->coef;
+  pass_outside(f, G, true, nullptr, s);
   return F;
 }
 
@@ -2020,6 +2056,7 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
       }
     }
     f->rows_ok = f->alpha_complete = f->inside_fused = false;
+    f->coef_plan = nullptr;
     return LAML_OK;
   }
   int prc = prepare_chains(f, s);

@@ -31,6 +31,13 @@ __device__ __forceinline__ Coef branch_coef(double dv, double nv) {
   return c;
 }
 
+// a block may use all of a CU's LDS
+template <typename K>
+static void allow_lds(K kernel) {
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            kLdsMaxBytes);
+}
+
 __global__ void k_coef(DevForest F, const double* __restrict__ d, const double* __restrict__ nu,
                        const int32_t* __restrict__ done) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1770,6 +1777,179 @@ __global__ void __launch_bounds__(256) k_outside_chain(DevForest F, const int2* 
     }
     if (!more) break;
     ++j;
+  }
+  if (pp) *pp = pv;
+}
+
+// Outside pass over clades: the steps of k_inside_clade's walk in reverse, from
+// the clade's root, whose outside state comes from above.  The carried child's
+// state stays in registers, the other internal child's waits in the
+// wavefront's LDS slice, so that no outside row is written or read below a
+// clade's root.  The children's inside rows, labels and codes of the next step
+// are copied to the slice during the step, as in k_outside_chain; prior
+// weights come from the chunk's piece in LDS and the coefficients in walking
+// order, as in k_inside_clade.  Sixteen trees of 10,000 leaves x 300 sites: 337
+// us and 150 in the rounds above, where the chain rounds and the levels above
+// took 675 us; 50,000 x 500: 178 and 82, 325.  Bound by instruction issue (93 %
+// of the VALU cycles at six wavefronts a SIMD).
+constexpr int kOutLdsBeta = 0;     // [2][64] double2
+constexpr int kOutLdsE = 2048;     // [2][64] int32
+constexpr int kOutLdsCode = 2560;  // [2][64] int16
+constexpr int kOutLdsSlots = 2816;  // [kCladeSlots][64] double2
+constexpr int kOutLdsBytes = kOutLdsSlots + kCladeSlots * 1024;
+
+__device__ __forceinline__ void clade_stage(const DevForest& F, const CladeOut& r, unsigned k0, int lane, char* lds,
+                                            bool stream) {
+  const int kind = r.flags & 3;
+  // codes or labels of both children, a row by each half of the wavefront
+  const int16_t* c0 = (kind == 0 ? F.codes : F.labels) + (int64_t)r.row[0] * 64 + k0;
+  const int16_t* c1 = (kind == 2 ? F.labels : F.codes) + (int64_t)r.row[1] * 64 + k0;
+  to_lds((lane < 32 ? c0 : c1) + 2 * (lane & 31), lds + kOutLdsCode, 4, stream);
+  if (kind == 0) return;
+  to_lds(&row_at(F.beta + (int64_t)r.row[0] * 64 + k0, (unsigned)lane), lds + kOutLdsBeta, 16, stream);
+  to_lds(&row_at(F.bE + (int64_t)r.row[0] * 64 + k0, (unsigned)lane), lds + kOutLdsE, 4, stream);
+  if (kind == 1) return;
+  to_lds(&row_at(F.beta + (int64_t)r.row[1] * 64 + k0, (unsigned)lane), lds + kOutLdsBeta + 1024, 16, stream);
+  to_lds(&row_at(F.bE + (int64_t)r.row[1] * 64 + k0, (unsigned)lane), lds + kOutLdsE + 256, 4, stream);
+}
+
+template <int kKind, typename Stage>
+__device__ __forceinline__ void clade_out_step(const char* lds, int lane, const CladeCoef& r, double phi, double qs,
+                                               const double* q, bool on, Stage&& stage, double a0, double aX,
+                                               PostOut& o) {
+  const bool lf[2] = {kKind == 0, kKind != 2};
+  int lab[2], E[2], code[2];
+  double b0[2], bA[2], qv[2];
+  Coef cf[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    cf[i] = Coef{r.p1n[i], r.mut[i], r.pn[i], r.msil[i], r.esil[i], 0};
+    // (lanes past the tree's sites: label 0)
+    const int raw = on ? lds_at<int16_t>(lds, kOutLdsCode + 128 * i + 2 * lane) : 0;
+    const double g = q[max(raw, 1)];
+    code[i] = raw;
+    if (lf[i]) {
+      leaf_beta(raw, phi, lab[i], b0[i], bA[i]);
+      E[i] = 0;
+    } else {
+      lab[i] = raw;
+      const double2 bb = lds_at<double2>(lds, kOutLdsBeta + 1024 * i + 16 * lane);
+      b0[i] = bb.x;
+      bA[i] = bb.y;
+      E[i] = lds_at<int>(lds, kOutLdsE + 256 * i + 4 * lane);
+    }
+    qv[i] = lab[i] > 0 ? g : qs;
+  }
+  // the slice is read: the next step's copies may overwrite it
+  chain_wait_lgkm();
+  stage();
+  Eps ep[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) ep[i] = edge(lab[i], b0[i], bA[i], E[i], qv[i], cf[i]);
+  cond_post<false>(combine_label(lab[0], lab[1]), a0, aX, 0.0, phi, lab, b0, bA, qv, ep, cf, lf, code, o);
+  if (!on) {
+    // lanes past the tree's sites add nothing to the counts
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int m = 0; m < 5; ++m) o.S[i][m] = 0.0;
+    o.rt = 0.0;
+  }
+}
+
+__global__ void __launch_bounds__(64 * kCladeOutWaves)
+    k_outside_clade(DevForest F, const int4* __restrict__ blocks, const int4* __restrict__ clades,
+                    const CladeOut* __restrict__ steps, int num, const int32_t* __restrict__ done) {
+  extern __shared__ __attribute__((aligned(16))) char clade_lds[];
+  const int g = (int)blockIdx.x >> 3, b = g / F.max_chunks * 8 + ((int)blockIdx.x & 7), chunk = g % F.max_chunks;
+  if (b >= num) return;
+  const int4 bd = uniform_load(blocks + b);
+  const int t = bd.z, k0 = chunk * 64;
+  const int K = F.tree_nsites[t], p = F.tree_prob[t];
+  if (k0 >= K) return;
+  if (done && done[p]) return;
+  const int lane = (int)(threadIdx.x & 63);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int sb = F.tree_site_base[t];
+  const bool on = k0 + lane < K;
+  const unsigned ks = (unsigned)min(k0 + lane, K - 1);
+  const double qs = row_at(F.site_qsum + sb, ks);
+  double* qt = (double*)(clade_lds + kCladeOutWaves * kOutLdsBytes);
+  const int q0 = uniform_load(F.site_qoff + sb + k0), q1 = uniform_load(F.site_qoff + sb + min(k0 + 64, K));
+  for (int i = (int)threadIdx.x; i < q1 - q0; i += 64 * kCladeOutWaves) qt[i] = F.prior[q0 + i];
+  const double* q = qt + (row_at(F.site_qoff + sb, ks) - 1 - q0);
+  __syncthreads();
+  if (wave >= bd.y) return;
+  const int4 cd = uniform_load(clades + bd.x + wave);
+  const double phi = uniform_load(F.phi + p);
+  const bool stream = F.stream_rows != 0;
+  char* lds = clade_lds + wave * kOutLdsBytes;
+  int j = cd.x + cd.y - 1;
+  CladeOut r = uniform_load(steps + j);
+  CladeOut r1 = uniform_load(steps + max(j - 1, cd.x));
+  CladeCoef cf = uniform_load(F.clade_coef + j);
+  double a0, aX;
+  {
+    const double2 a = row_at(F.alpha + uniform_load(F.row_off + r.u), ks);
+    a0 = a.x;
+    aX = a.y;
+  }
+  clade_stage(F, r, (unsigned)k0, lane, lds, stream);
+  double* pp = nullptr;  // partial count held back from the previous step
+  double pv = 0.0;
+  for (;; --j) {
+    chain_wait_all();
+    if (pp) *pp = pv;
+    const int pop = (r.flags >> 4) & 7;
+    if (pop) {
+      const double2 a = lds_at<double2>(lds, kOutLdsSlots + (pop - 1) * 1024 + 16 * lane);
+      a0 = a.x;
+      aX = a.y;
+    }
+    const int kind = r.flags & 3;
+    const bool more = j > cd.x;
+    CladeOut r2;
+    CladeCoef c1;
+    auto stage = [&]() {
+      if (more) clade_stage(F, r1, (unsigned)k0, lane, lds, stream);
+      r2 = uniform_load(steps + max(j - 2, cd.x));
+      c1 = uniform_load(F.clade_coef + max(j - 1, cd.x));
+    };
+    PostOut o;
+    if (kind == 0) clade_out_step<0>(lds, lane, cf, phi, qs, q, on, stage, a0, aX, o);
+    else if (kind == 1) clade_out_step<1>(lds, lane, cf, phi, qs, q, on, stage, a0, aX, o);
+    else {
+      clade_out_step<2>(lds, lane, cf, phi, qs, q, on, stage, a0, aX, o);
+      *(double2*)(lds + kOutLdsSlots + ((r.flags >> 2) & 3) * 1024 + 16 * lane) = make_double2(o.a0[1], o.aX[1]);
+    }
+    a0 = o.a0[0];
+    aX = o.aX[0];
+    // partial counts (as in k_outside_chain)
+    double v[12];
+#pragma unroll
+    for (int m = 0; m < 5; ++m) {
+      v[m] = o.S[0][m];
+      v[5 + m] = o.S[1][m];
+    }
+    v[10] = o.rt;
+    v[11] = 0.0;
+    wave_sum12(v);
+    {
+      const int rr = lane >> 4, i = lane & 15;
+      const int vi = 3 * rr + i;
+      pv = i == 0 ? v[0] : (i == 1 ? v[1] : v[2]);
+      pp = nullptr;
+      if (i < 3 && vi < 10) {
+        const int c = vi >= 5 ? 1 : 0;
+        pp = F.cpart + ((int64_t)(c ? r.ch[1] : r.ch[0]) * F.max_chunks + chunk) * 5 + (vi - 5 * c);
+      } else if (i < 3 && vi == 10) {
+        pp = F.rt_part + (int64_t)r.u * F.max_chunks + chunk;
+      }
+    }
+    if (!more) break;
+    r = r1;
+    r1 = r2;
+    cf = c1;
   }
   if (pp) *pp = pv;
 }
@@ -3752,13 +3932,6 @@ void run_lds_tables(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, hi
   hipLaunchKernelGGL(k_lds_tables, dim3(8, L.num_blocks), dim3(256), 0, s, F, L, TW);
 }
 
-// a block may use all of a CU's LDS
-template <typename K>
-static void allow_lds(K kernel) {
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            kLdsMaxBytes);
-}
-
 void run_problem(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, double* d, double* nu, double* phi,
                  double* nll, double* site_llh_out, int32_t* iters_out, const EmState& em, int max_steps,
                  int max_iter, double tol, int what, hipStream_t s) {
@@ -4214,7 +4387,7 @@ void run_outside_ckpt(const DevForest& F, const std::vector<int32_t>& lvl, int W
 
 void run_outside(const DevForest& F, const std::vector<int32_t>& lvl, int W, int h_top,
                  const std::vector<int32_t>& cpw, const int32_t* done, hipStream_t s, const CherrySplit* cs,
-                 const ChainPlan* cp) {
+                 const ChainPlan* cp, const CladePlan* cl) {
   const int H = (int)lvl.size() - 1;
   if (cs) {
     for (int h = H - 1; h >= 2; --h) split_level(true, F, *cs, cpw, h, done, s);
@@ -4226,9 +4399,10 @@ void run_outside(const DevForest& F, const std::vector<int32_t>& lvl, int W, int
       hipLaunchKernelGGL(k_outside_top<WW>, dim3(F.max_chunks), dim3(1024), 0, s, F, ht, H, done);
     });
   }
-  const int h0 = cp ? std::min(cp->h_split, ht) : 1;
+  const int h0 = cl ? std::min(cl->h_split, ht) : (cp ? std::min(cp->h_split, ht) : 1);
   for (int h = ht - 1; h >= h0; --h) outside_level(F, lvl, W, cpw, h, done, s);
-  if (cp) run_outside_chains(F, *cp, done, s);
+  if (cl) run_outside_clades(F, *cl, done, s);
+  else if (cp) run_outside_chains(F, *cp, done, s);
 }
 
 void run_inside_clades(const DevForest& F, const CladePlan& cl, const int32_t* done, hipStream_t s) {
@@ -4241,6 +4415,19 @@ void run_inside_clades(const DevForest& F, const CladePlan& cl, const int32_t* d
     const int beg = cl.round_off[r], cnt = cl.round_off[r + 1] - beg;
     launch_inside_rows(dim3((cnt + 3) / 4, F.max_chunks), s, F, beg, cnt, 1, done, cl.rest);
   }
+}
+
+void run_outside_clades(const DevForest& F, const CladePlan& cl, const int32_t* done, hipStream_t s) {
+  for (size_t r = cl.round_off.size() - 1; r-- > 0;) {
+    const int beg = cl.round_off[r], cnt = cl.round_off[r + 1] - beg;
+    launch_outside_rows(dim3((cnt + 3) / 4, F.max_chunks), s, F, beg, cnt, 1, done, cl.rest);
+  }
+  if (cl.out_num == 0) return;
+  const size_t lds = (size_t)kCladeOutWaves * kOutLdsBytes + cl.q_bytes;
+  static const bool once = (allow_lds(k_outside_clade), true);
+  (void)once;
+  hipLaunchKernelGGL(k_outside_clade, dim3((unsigned)((cl.out_num + 7) / 8 * 8 * F.max_chunks)),
+                     dim3(64 * kCladeOutWaves), lds, s, F, cl.out_blocks, cl.clades, cl.out_steps, cl.out_num, done);
 }
 
 void run_inside_chains(const DevForest& F, const ChainPlan& cp, const int32_t* done, hipStream_t s) {

@@ -312,6 +312,12 @@ constexpr int kCladeLds = kCladeSlots * kCladeSlotBytes + kCladeBatch * 128;  //
 struct CladeStep {
   int32_t row, flags;
 };
+// The same node for the outside walk, which runs the steps in reverse: the
+// node, its children and their rows (codes of a leaf, inside row and labels of
+// an internal node).
+struct CladeOut {
+  int32_t u, flags, ch[2], row[2];
+};
 // The coefficients of its branches in one piece, written by k_coef (scalar
 // loads of coefficients by branch took most of the walk's time); children
 // ordered so that the first is the one whose state the wavefront carries (or
@@ -328,23 +334,31 @@ struct CladePlan {
   const int4* clades = nullptr;  // offset into steps, steps, first batch, batches
   const CladeStep* steps = nullptr;
   CladeCoef* coef = nullptr;     // by step
+  int32_t out_num = 0;           // blocks of the outside pass
+  const int4* out_blocks = nullptr;
+  const CladeOut* out_steps = nullptr;
   const int32_t* pos = nullptr;  // [N] place of a branch's coefficients: 2 step + child, -1 none
   const int32_t* leaf_row = nullptr;  // [batch][kCladeBatch] code rows of the leaves, in units of 64 sites
   const int32_t* rest = nullptr;
   std::vector<int32_t> round_off;
 };
-constexpr int kCladeWaves = 8;  // wavefronts of a block
+constexpr int kCladeWaves = 8;      // wavefronts of a block, inside
+constexpr int kCladeOutWaves = 12;  // and outside
 // Most nodes of a clade: one per kCladePairs (internal node, 64-site chunk)
 // pairs of the forest, between kCladeMin and kCladeCap.  Longer walks read
-// fewer rows back, but the wavefronts have to fill the chip.  Likelihood of
-// 10,000 leaves x 300 (50k pairs): 95 us at 16 and 32, 105 at 64 (109 by
-// levels); sixteen such trees 425 us at 16, 365 at 64 (681).
-constexpr int64_t kCladePairs = 2048;
+// fewer rows back, but the wavefronts have to fill the chip.  E-step of 10,000
+// leaves x 300 (50k pairs): 216 us at 16, 219 at 24, 234 at 32; of sixteen such
+// trees (800k) 1052 at 16, 929 at 32, 899 at 64.
+constexpr int64_t kCladePairs = 4096;
 constexpr int kCladeMin = 16, kCladeCap = 64;
-// Forests of at least this many pairs take clades: 2,000 x 500 (16k pairs) 61
-// us, 77 by levels; 1,000 x 500 (8k) 47 and 53, but a forest that is solved
-// once and dropped does not earn its plan back.
+// Forests of at least this many pairs take clades in the inside pass: 2,000 x
+// 500 (16k pairs) 63 us, 76 by levels; 1,000 x 500 (8k) 48 and 53, but a forest
+// that is solved once and dropped does not earn its plan back.
 constexpr int64_t kCladeForest = 12288;
+// And of at least this many in the outside pass as well: E-step of 300 trees of
+// 300 leaves x 300 (60k pairs) 172 us, 203 by chains; of 10,000 x 300 (50k) 216
+// and 221, but its gradient, whose launches are not in a graph, 291 and 267.
+constexpr int64_t kCladeOutForest = 57344;
 // most LDS for a chunk's prior weights: 64 sites of 62 edit states (up to 21 KB
 // three blocks fit a CU)
 constexpr int kCladeMaxQ = 31 * 1024;
@@ -355,11 +369,12 @@ void run_inside(const DevForest& F, const std::vector<int32_t>& lvl, int W, int 
                 const int32_t* done, hipStream_t s, const CherrySplit* cs = nullptr, const ChainPlan* cp = nullptr,
                 const CladePlan* cl = nullptr);
 void run_inside_clades(const DevForest& F, const CladePlan& cl, const int32_t* done, hipStream_t s);
+void run_outside_clades(const DevForest& F, const CladePlan& cl, const int32_t* done, hipStream_t s);
 void run_inside_chains(const DevForest& F, const ChainPlan& cp, const int32_t* done, hipStream_t s);
 // cp: the levels below the top kernel's run as heavy-path chains
 void run_outside(const DevForest& F, const std::vector<int32_t>& lvl, int W, int h_top,
                  const std::vector<int32_t>& cpw, const int32_t* done, hipStream_t s, const CherrySplit* cs = nullptr,
-                 const ChainPlan* cp = nullptr);
+                 const ChainPlan* cp = nullptr, const CladePlan* cl = nullptr);
 void run_outside_chains(const DevForest& F, const ChainPlan& cp, const int32_t* done, hipStream_t s);
 void run_outside_ckpt(const DevForest& F, const std::vector<int32_t>& lvl, int W, int L,
                       const std::vector<int32_t>& in_cpw, const std::vector<int32_t>& out_cpw, const int32_t* done,
