@@ -68,6 +68,7 @@ struct laml_forest {
   int W = 64;
   int h_top = 1 << 30;  // first level handled by the fused top-level kernels
   int h_top_default = 1 << 30;
+  int h_walk = 1 << 30;  // first level of the hybrid passes' walk, in the launch plan the forest was created with
   int ckpt_L = 0;       // level-checkpoint segment length (0: all inside vectors stored)
   // per level: 64-site chunks one wavefront of the row kernels walks (W == 64)
   std::vector<int32_t> in_cpw, out_cpw;
@@ -530,6 +531,18 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
     while (ht - 1 >= 1 && d->level_off[ht] - d->level_off[ht - 1] <= top_max) --ht;
     f->h_top = ht;
     f->h_top_default = ht;
+    // The hybrid passes' walk takes more, the levels where each of its blocks
+    // (a tree and a site chunk, 16 wavefronts) meets few nodes: it then runs a
+    // level in 2 us, a launch in 4.6.  E-step by the largest such level (nodes
+    // a tree): 10,000 x 300 220 us at 24, 225 at 48; sixteen such trees 884 at
+    // 10, 908 at 3; 50 trees of 50-500 x 100 126 at 8, 128 at 16, 154 at 1; 300
+    // of 20-200 x 100 156 at 8, 168 at 16, 177 at 1.  With more blocks than the
+    // chip holds the launches are better (3,000 trees x 20: 604 and 823).
+    int hh = d->num_levels;
+    const int64_t T = d->num_trees, chunks = (max_k + f->W - 1) / f->W;
+    const int walk_max = env || T * chunks > 1024 ? top_max : (int)std::max<int64_t>(24, 10 * T);
+    while (hh - 1 >= 1 && d->level_off[hh] - d->level_off[hh - 1] <= walk_max) --hh;
+    f->h_walk = hh;
     const char* pm = getenv("LAML_PASS_MODE");
     if (pm && (atoi(pm) == 0 || atoi(pm) == 1)) f->pass_mode = atoi(pm);
   }
@@ -1383,7 +1396,8 @@ static DevForest lds_view(const DevForest& F, const laml::LdsPlan& L) {
 // (a block per tree and site chunk) for the levels from it up
 static int hybrid_split(const laml_forest* f) {
   const int H = (int)f->level_off.size() - 1;
-  return std::max(1, std::min(f->h_top, H));
+  const bool def = f->pass_mode == LAML_PASS_HYBRID && f->h_top == f->def.h_top;
+  return std::max(1, std::min(def ? f->h_walk : f->h_top, H));
 }
 
 // which passes run the levels below their split as heavy-path chains
