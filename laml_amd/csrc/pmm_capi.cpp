@@ -116,7 +116,6 @@ struct laml_forest {
   bool clades = false;
   int clade_cap = 0;
   bool out_clades = false;          // and of the outside pass
-  const laml::CladePlan* coef_plan = nullptr;  // whose coefficients are those of the last call
   int64_t clade_q = 0;              // most prior weights of a 64-site chunk
   std::deque<laml::CladePlan> clade_plans;
   std::deque<laml::ChainPlan> chain_plans;  // a deque: plans stay put when more are added
@@ -1569,8 +1568,8 @@ static const laml::CladePlan* pass_clades(const laml_forest* f) {
 
 // The same for the outside pass, whose chains and shapes must be the default
 // ones as well.
-static const laml::CladePlan* out_clades(const laml_forest* f, const DevForest& F) {
-  return F.clade_coef && f->out_clades && f->chains == f->def.chains && f->chain_top_out == f->def.chain_top_out &&
+static const laml::CladePlan* out_clades(const laml_forest* f) {
+  return f->out_clades && f->chains == f->def.chains && f->chain_top_out == f->def.chain_top_out &&
                  f->out_cpw == f->def.out_cpw
              ? pass_clades(f)
              : nullptr;
@@ -1762,14 +1761,15 @@ static const laml::ChainPlan* pass_chains(laml_forest* f, bool inside, int hs) {
 
 // builds the chain plans the next passes use, outside any stream capture
 static int prepare_chains(laml_forest* f, hipStream_t s) {
+  prepare_clades(f, s);
   const int hs = hybrid_split(f);
   for (const bool inside : {true, false}) {
+    if (!inside && out_clades(f)) continue;
     if (!(chains_now(f) & (inside ? LAML_CHAINS_INSIDE : LAML_CHAINS_OUTSIDE))) continue;
     const int t = inside ? f->chain_top_in : f->chain_top_out;
     const int top = t <= 0 ? hs : std::min(t, hs);
     if (top > 1 && !chain_plan(f, top)) return fail(LAML_ENOMEM, "chain plan");
   }
-  prepare_clades(f, s);
   return LAML_OK;
 }
 
@@ -1778,7 +1778,6 @@ static int prepare_chains(laml_forest* f, hipStream_t s) {
 static void pass_coef(laml_forest* f, DevForest& F, const double* d, const double* nu, const int32_t* done,
                       hipStream_t s) {
   const laml::CladePlan* cl = pass_clades(f);
-  f->coef_plan = cl;
   F.clade_coef = cl ? cl->coef : nullptr;
   F.clade_pos = cl ? cl->pos : nullptr;
   laml::run_coef(F, d, nu, done, s);
@@ -1799,7 +1798,7 @@ static void inside_below(laml_forest* f, const DevForest& F, int hs, const int32
 // outside levels [1, hs) of the level and hybrid passes
 static void outside_below(laml_forest* f, const DevForest& F, int hs, const int32_t* done, hipStream_t s,
                           bool allow_chains) {
-  if (const laml::CladePlan* cl = allow_chains ? out_clades(f, F) : nullptr) {
+  if (const laml::CladePlan* cl = allow_chains && F.clade_coef ? out_clades(f) : nullptr) {
     laml::run_outside_clades(F, *cl, done, s);
     f->alpha_complete = false;
     return;
@@ -1861,7 +1860,7 @@ static void pass_outside(laml_forest* f, const DevForest& F, bool with_root, con
     f->alpha_complete = true;
     return;
   }
-  const laml::CladePlan* cl = allow_chains ? out_clades(f, F) : nullptr;
+  const laml::CladePlan* cl = allow_chains && F.clade_coef ? out_clades(f) : nullptr;
   const laml::ChainPlan* cp = allow_chains && !cl ? pass_chains(f, false, hybrid_split(f)) : nullptr;
   laml::run_outside(F, f->level_off, f->W, f->h_top, f->out_cpw, done, s, nullptr, cp, cl);
   f->alpha_complete = !cp && !cl;
@@ -1888,7 +1887,6 @@ int laml_nll(laml_forest* f, const double* d, const double* nu, const double* ph
     laml::run_problem(lds_view(F, f->pb), f->pb, f->TW, const_cast<double*>(d), const_cast<double*>(nu),
                       const_cast<double*>(phi), nll, site_llh, nullptr, none, 1, 0, 0.0, laml::kPbCoef, s);
     f->rows_ok = f->alpha_complete = f->inside_fused = false;
-    f->coef_plan = nullptr;
     return check_launch();
   }
   int rc = prepare_chains(f, s);
@@ -1913,7 +1911,6 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
     laml::run_problem(G, f->pb, f->TW, const_cast<double*>(d), const_cast<double*>(nu), const_cast<double*>(phi), nll,
                       nullptr, nullptr, none, 1, 0, 0.0, laml::kPbCoef | laml::kPbOut, s);
     f->rows_ok = f->alpha_complete = f->inside_fused = false;
-    f->coef_plan = nullptr;
     laml::run_counts(G, counts, s);
     laml::run_rtilde(G, rtilde, nullptr, s);
     return check_launch();
@@ -1955,7 +1952,13 @@ static DevForest outside_again(laml_forest* f, const DevForest& F, const double*
   }
   ensure_rows(f, F, s);
   DevForest G = F;
-  if (f->coef_plan && f->coef_plan == pass_clades(f)) G.clade_coef = f->coef_plan->coef;
+  if (const laml::CladePlan* cl = pass_clades(f)) {
+    G.clade_coef = cl->coef;
+    G.clade_pos = cl->pos;
+    // (the resident coefficients are those of any earlier call, a captured one
+    // included)
+    if (out_clades(f)) laml::run_clade_coef(G, s);
+  }
   pass_outside(f, G, true, nullptr, s);
   return F;
 }
@@ -2070,7 +2073,6 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
       }
     }
     f->rows_ok = f->alpha_complete = f->inside_fused = false;
-    f->coef_plan = nullptr;
     return LAML_OK;
   }
   int prc = prepare_chains(f, s);
@@ -2129,7 +2131,7 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
   if (!f->rows_ok)
     f->alpha_complete = f->inside_fused = false;
   else if (max_iter > 0 && f->pass_mode != LAML_PASS_TREES)
-    f->alpha_complete = !pass_chains(f, false, hybrid_split(f)) && !fuse_now(f);
+    f->alpha_complete = !out_clades(f) && !pass_chains(f, false, hybrid_split(f)) && !fuse_now(f);
   LAML_HIP(hipMemcpyAsync(iters, em.iters, sizeof(int32_t) * P, hipMemcpyDeviceToDevice, s));
   return check_launch();
 }

@@ -38,6 +38,19 @@ static void allow_lds(K kernel) {
                             kLdsMaxBytes);
 }
 
+// branch v's coefficients to its place in the steps of the clade plan
+__device__ __forceinline__ void clade_coef(const DevForest& F, int v, const Coef& c) {
+  const int q = F.clade_pos[v];
+  if (q < 0) return;
+  CladeCoef& r = F.clade_coef[q >> 1];
+  const int i = q & 1;
+  r.p1n[i] = c.p1n;
+  r.mut[i] = c.mut;
+  r.pn[i] = c.pn;
+  r.msil[i] = c.msil;
+  r.esil[i] = c.esil;
+}
+
 __global__ void k_coef(DevForest F, const double* __restrict__ d, const double* __restrict__ nu,
                        const int32_t* __restrict__ done) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
@@ -46,18 +59,13 @@ __global__ void k_coef(DevForest F, const double* __restrict__ d, const double* 
   if (done && done[p]) return;
   const Coef c = branch_coef(d[v], nu[p]);
   F.coef[v] = c;
-  if (F.clade_pos) {
-    const int q = F.clade_pos[v];
-    if (q >= 0) {
-      CladeCoef& r = F.clade_coef[q >> 1];
-      const int i = q & 1;
-      r.p1n[i] = c.p1n;
-      r.mut[i] = c.mut;
-      r.pn[i] = c.pn;
-      r.msil[i] = c.msil;
-      r.esil[i] = c.esil;
-    }
-  }
+  if (F.clade_pos) clade_coef(F, v, c);
+}
+
+// the resident coefficients into a clade plan's steps
+__global__ void k_clade_coef(DevForest F) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v < F.num_nodes) clade_coef(F, v, F.coef[v]);
 }
 
 // Segment mapping shared by the level kernels: a block of 256 threads holds
@@ -4256,6 +4264,10 @@ void run_pad_codes(const DevForest& F, const int16_t* packed, const int64_t* pac
 void run_coef(const DevForest& F, const double* d, const double* nu, const int32_t* done, hipStream_t s) {
   const int grid = (F.num_nodes + 255) / 256;
   hipLaunchKernelGGL(k_coef, dim3(grid), dim3(256), 0, s, F, d, nu, done);
+}
+
+void run_clade_coef(const DevForest& F, hipStream_t s) {
+  hipLaunchKernelGGL(k_clade_coef, dim3((F.num_nodes + 255) / 256), dim3(256), 0, s, F);
 }
 
 static void launch_inside_rows(dim3 grid, hipStream_t s, const DevForest& F, int beg, int cnt, int cpw,

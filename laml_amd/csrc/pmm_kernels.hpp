@@ -368,6 +368,7 @@ constexpr int kCladeMaxQ = 31 * 1024;
 void run_inside(const DevForest& F, const std::vector<int32_t>& lvl, int W, int h_top, const std::vector<int32_t>& cpw,
                 const int32_t* done, hipStream_t s, const CherrySplit* cs = nullptr, const ChainPlan* cp = nullptr,
                 const CladePlan* cl = nullptr);
+void run_clade_coef(const DevForest& F, hipStream_t s);
 void run_inside_clades(const DevForest& F, const CladePlan& cl, const int32_t* done, hipStream_t s);
 void run_outside_clades(const DevForest& F, const CladePlan& cl, const int32_t* done, hipStream_t s);
 void run_inside_chains(const DevForest& F, const ChainPlan& cp, const int32_t* done, hipStream_t s);

@@ -75,7 +75,10 @@ def test_clades_equal_levels(kind, n, K, P, cap, monkeypatch):
             em = [x.clone() for x in (d, nu, phi)]
             F.em(*em, 3, 0.0)
             torch.cuda.synchronize()
-            got[clades, mode] = [nll, counts, rt, enll] + [x.cpu().numpy() for x in em]
+            # every outside row again, after an E-step that kept them in registers
+            F.estep(d, nu, phi)
+            post = [x.copy() for pair in F.posteriors(phi) for x in pair]
+            got[clades, mode] = [nll, counts, rt, enll] + [x.cpu().numpy() for x in em] + post
         F.close()
     for mode in (PASS_HYBRID, PASS_LEVELS):
         for a, b in zip(got[cap, mode], got[0, mode]):
