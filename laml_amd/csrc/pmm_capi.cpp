@@ -2156,30 +2156,17 @@ int laml_posteriors(laml_forest* f, const double* phi, double* post0_host, doubl
   // state (one outside pass in level launches)
   ensure_rows(f, F, s);
   if (!f->alpha_complete) pass_outside(f, F, true, nullptr, s, false);
-  const int64_t rows = f->leaf_rows + f->int_rows;
-  double *p0 = nullptr, *pS = nullptr;
-  LAML_HIP(hipMalloc(&p0, sizeof(double) * std::max<int64_t>(rows, 1)));
-  if (hipMalloc(&pS, sizeof(double) * std::max<int64_t>(rows, 1)) != hipSuccess) {
-    (void)hipFree(p0);
+  double* p0 = nullptr;
+  if (hipMalloc(&p0, 2 * sizeof(double) * std::max<int64_t>(need, 1)) != hipSuccess)
     return fail(LAML_ENOMEM, "hipMalloc posteriors");
-  }
-  laml::run_node_post(F, f->W, f->leaf_rows, p0, pS, s);
-  std::vector<double> h0(rows), hS(rows);
+  double* pS = p0 + need;
+  laml::run_node_post(F, f->W, f->d_desc_off, f->leaf_sites, p0, pS, s);
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(h0.data(), p0, sizeof(double) * rows, hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(hS.data(), pS, sizeof(double) * rows, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess && need > 0) e = hipMemcpyAsync(post0_host, p0, sizeof(double) * need, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess && need > 0) e = hipMemcpyAsync(postS_host, pS, sizeof(double) * need, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   (void)hipFree(p0);
-  (void)hipFree(pS);
   if (e != hipSuccess) return fail(LAML_EDEVICE, std::string("posteriors: ") + hipGetErrorString(e));
-  const int N = f->F.num_nodes, n = f->F.num_leaves;
-  for (int v = 0; v < N; ++v) {
-    const int K = f->h_Kt[v];
-    const int64_t src = (v < n ? 0 : f->leaf_rows) + f->h_row_off[v];
-    const int64_t dst = (v < n ? 0 : f->leaf_sites) + f->h_desc_off[v];
-    std::memcpy(post0_host + dst, h0.data() + src, sizeof(double) * K);
-    std::memcpy(postS_host + dst, hS.data() + src, sizeof(double) * K);
-  }
   return LAML_OK;
 }
 
@@ -2189,7 +2176,7 @@ int laml_posteriors_noalloc(laml_forest* f, const double* phi, double* post0_hos
   const int64_t need = f->leaf_sites + f->int_sites;
   if (capacity < need) return fail(LAML_EINVAL, "posterior capacity too small");
   const int64_t rows = f->leaf_rows + f->int_rows;
-  // padded rows of both posteriors, then their packed copies
+  // (the limit also counts the rows' padding)
   if (2 * (rows + need) > laml::kPostScratchDoubles)
     return fail(LAML_EINVAL, "laml_posteriors_noalloc: the forest's posteriors (2 x (padded rows + entries) "
                              "doubles) exceed the fixed staging area of 8388608 doubles; use laml_posteriors");
@@ -2204,12 +2191,9 @@ int laml_posteriors_noalloc(laml_forest* f, const double* phi, double* post0_hos
   F.phi = phi;
   ensure_rows(f, F, s);
   if (!f->alpha_complete) pass_outside(f, F, true, nullptr, s, false);
-  double* p0 = f->post_scratch;
-  double* pS = p0 + rows;
-  double* o0 = pS + rows;
+  double* o0 = f->post_scratch;
   double* oS = o0 + need;
-  laml::run_node_post(F, f->W, f->leaf_rows, p0, pS, s);
-  laml::run_post_pack(F, f->d_desc_off, f->leaf_rows, f->leaf_sites, p0, pS, o0, oS, s);
+  laml::run_node_post(F, f->W, f->d_desc_off, f->leaf_sites, o0, oS, s);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && need > 0)
     e = hipMemcpyAsync(post0_host, o0, sizeof(double) * need, hipMemcpyDeviceToHost, s);
