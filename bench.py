@@ -54,22 +54,42 @@ def heavy_children(F):
     return heavy
 
 
-def algorithmic_bytes(F, fused=False, chain_split=None, in_chain_split=None):
+def clade_members(F, split):
+    """Whether each node lies in a clade of the passes' default plan: a
+    maximal subtree below level `split` of at most so many internal nodes
+    (one per 4,096 (internal node, 64-site chunk) pairs, 16 to 64) whose walk
+    keeps at most two pending states."""
+    N, n = F.num_nodes, F.num_leaves
+    B = int(F.level_off[split])
+    cap = min(64, max(16, (B - n) * -(-int(F.tree_K.max()) // 64) // 4096))
+    size, need = np.zeros(N, dtype=np.int64), np.zeros(N, dtype=np.int64)
+    for h in range(1, split):
+        v = np.arange(F.level_off[h], F.level_off[h + 1])
+        a, b = F.child0[v], F.child1[v]
+        size[v] = size[a] + size[b] + 1
+        lo, hi = np.minimum(need[a], need[b]), np.maximum(need[a], need[b])
+        need[v] = np.where((a >= n) & (b >= n), np.maximum(hi, lo + 1), hi)
+    return (np.arange(N) >= n) & (np.arange(N) < B) & (size <= cap) & (need <= 2)
+
+
+def algorithmic_bytes(F, fused=False, chain_split=None, in_chain_split=None, state=38, clade_split=None):
     """Compulsory HBM bytes of one inside pass and one outside pass.
 
     Per (internal node, site): inside reads the node's label (2 B) and each
     child's state (leaf: int16 code, 2 B; internal: label + beta pair +
     exponent, 22 B) and writes beta + exponent (20 B).  Outside reads the
-    node's outside state (alpha quad + exponent + specific state, 38 B), each
+    node's outside state (`state` bytes; 16 for the conditional pair), each
     child's inside state again (2 / 22 B) and writes each internal child's
-    outside state (38 B).  With fused cherries (nodes whose children are both
+    outside state.  With fused cherries (nodes whose children are both
     leaves) a cherry has no rows: its parent reads the two leaf codes (4 B)
     in place of its state, and the cherry's own steps move nothing else.
     With outside chains below level chain_split, a heavy child's outside
     state stays in registers: it is neither written by its parent nor read by
-    itself (38 + 38 B less per heavy child and site); with inside chains
+    itself (twice `state` less per heavy child and site); with inside chains
     below level in_chain_split its parent does not read its inside state
-    (22 B less)."""
+    (22 B less).  With clades below level clade_split no inside row of a
+    clade's inner node is read by the inside pass, nor its label, and no
+    outside row but the clade root's is read or written."""
     N, n = F.num_nodes, F.num_leaves
     K = F.tree_K[F.tree_of].astype(np.int64)
     lo, hi = (int(F.level_off[1]), int(F.level_off[2])) if fused else (n, n)
@@ -77,8 +97,9 @@ def algorithmic_bytes(F, fused=False, chain_split=None, in_chain_split=None):
     c = np.stack([F.child0[inter], F.child1[inter]])
     cherry = (c >= lo) & (c < hi)
     rc = np.where(c < n, 2, np.where(cherry, 4, 22))
-    wo = np.where((c < n) | cherry, 0, 38)
-    ra = np.full(len(inter), 38)
+    wo = np.where((c < n) | cherry, 0, state)
+    ra = np.full(len(inter), state)
+    label = np.full(len(inter), 2)
     if chain_split is not None:
         B = int(F.level_off[chain_split])
         heavy = heavy_children(F)
@@ -97,8 +118,19 @@ def algorithmic_bytes(F, fused=False, chain_split=None, in_chain_split=None):
         Bi = int(F.level_off[in_chain_split])
         heavy = heavy_children(F)
         rci = np.where((c == heavy[inter][None, :]) & (inter < Bi)[None, :], 0, rc)
+    if clade_split is not None:
+        mem = clade_members(F, clade_split)
+        par = np.full(N, -1, dtype=np.int64)
+        par[F.child0[inter]] = inter
+        par[F.child1[inter]] = inter
+        inner = mem[c] & mem[inter][None, :]  # child in its parent's clade
+        rci = np.where(inner, 0, rci)
+        wo = np.where(inner, 0, wo)
+        p = par[inter]
+        ra = np.where(mem[inter] & (p >= 0) & mem[np.maximum(p, 0)], 0, ra)
+        label = np.where(mem[inter], 0, label)
     Kv = K[inter]
-    inside = int((Kv * (2 + 20 + rci.sum(0))).sum())
+    inside = int((Kv * (label + 20 + rci.sum(0))).sum())
     outside = int((Kv * (ra + rc.sum(0) + wo.sum(0))).sum())
     return inside, outside
 
@@ -766,10 +798,13 @@ def main():
 
     plan_desc = {}
 
+    from laml_amd.autotune import current_plan
+
     def run(problems, steps, warmup, tune=False):
         specs = [sim.problem_spec(t, q, c) for (t, q, c, _) in problems]
         t0 = time.perf_counter()
         F = Forest(specs, device=0)
+        F.created_plan = current_plan(F).describe()
         torch.cuda.synchronize()
         setup = time.perf_counter() - t0
         dev = F.device
@@ -865,7 +900,18 @@ def main():
     flags = F.chains()
     _, top_in, top_out = F.get_chains()
     region = lambda t: split if t <= 0 else min(t, split)
-    inside_b, outside_b = algorithmic_bytes(F, fused=F.fusion(), chain_split=region(top_out) if flags & 1 else None,
+    # the plan the forest was created with runs the passes of a large forest
+    # over clades below the walk's level
+    pairs = (F.num_nodes - F.num_leaves) * -(-int(F.tree_K.max()) // 64)
+    clades = None
+    if current_plan(F).describe() == F.created_plan and F.tree_K.max() > 32 and pairs >= 57344:
+        sizes, T = np.diff(F.level_off), F.num_trees
+        walk = 48 if T * -(-int(F.tree_K.max()) // 64) > 1024 else max(24, 10 * T)
+        clades = F.num_levels
+        while clades > 1 and sizes[clades - 1] <= walk:
+            clades -= 1
+    inside_b, outside_b = algorithmic_bytes(F, fused=F.fusion(), state=16, clade_split=clades,
+                                            chain_split=region(top_out) if flags & 1 and clades is None else None,
                                             in_chain_split=region(top_in) if flags & 2 else None)
     F.nll(d, nu, phi)
     stream = torch.cuda.current_stream()
@@ -923,17 +969,14 @@ def main():
                      "traffic_source": PROFILE if traffic is not None else None,
                      "valu_issue_frac": valu,
                      "traffic_gbs": round(traffic / (out_ms * 1e-3) / 1e9, 1) if traffic else None,
-                     "note": "achieved counts the compulsory bytes of the algorithm the plan runs (outside chains "
-                             "keep heavy children's outside states in registers, about half the bytes of level "
-                             "launches); the chain steps read each child's prior weight from a row built at "
-                             "forest creation (8 B per child and site, streamed) instead of gathering prior-table "
-                             "entries, a line per lane: those bytes are in traffic, not in achieved; the chain "
-                             "steps are bound by instruction issue (FP64 VALU) and memory latency together, not by "
-                             "HBM bandwidth (traffic_gbs)",
+                     "note": "achieved counts the compulsory bytes of the algorithm the plan runs (walks over "
+                             "clades keep outside states in registers and LDS: only the inside rows are read); "
+                             "the walk is bound by instruction issue (FP64 VALU), the rounds above it and the "
+                             "tree walk by latency, not by HBM bandwidth (traffic_gbs)",
                      "launch_plan": "as in " + PROFILE if roof_plan is not None else "as the batch",
-                     "kernel": "outside pass (laml_outside: k_tree_walk top levels + root in the hybrid plan, "
-                               "k_outside_chain rounds below the split when the plan has chains, else "
-                               "k_outside_rows levels, k_counts, k_rtilde)",
+                     "kernel": "outside pass (laml_outside: k_clade_coef, k_tree_walk top levels + root in the hybrid "
+                               "plan, k_outside_rows rounds and k_outside_clade below the split, or chains or "
+                               "levels where the plan has them, k_counts, k_rtilde)",
                      "algorithmic_bytes": outside_b, "ms": round(out_ms, 4),
                      "inside_pass": {"algorithmic_bytes": inside_b, "ms": round(in_ms, 4)}},
     }
