@@ -561,8 +561,10 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   F.max_chunks = (max_k + f->W - 1) / f->W;
   F.cherry_end = d->num_leaves;
   {
-    // stream the rows past the caches when one pass's inside + outside rows
-    // (60 B per internal site) exceed the 256 MiB last-level cache
+    // stream the rows past the caches when one pass's rows and tables (about
+    // 60 B per internal site, 46 of them rows) exceed the 256 MiB last-level
+    // cache (10,000 x 300: 220 us an E-step, 239 streamed; 50,000 x 500: 730
+    // streamed, 834 not)
     const char* env = getenv("LAML_STREAM_ROWS");
     const double row_bytes = 60.0 * (double)int_rows;
     F.stream_rows = env ? (atoi(env) != 0) : (row_bytes > 256.0 * 1024 * 1024);
@@ -668,8 +670,7 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
     UP(site_qsum, qs.data(), qs.size());
   }
   {
-    // two entries of padding: the outside chain kernel gathers 16 bytes at a
-    // prior entry (entry 0 for labels that name no edit state)
+    // (labels that name no edit state read entry 0, so there is always one)
     std::vector<double> pr((size_t)d->site_qoff[S] + 2, 0.0);
     std::copy(d->prior, d->prior + d->site_qoff[S], pr.begin());
     UP(prior, pr.data(), pr.size());

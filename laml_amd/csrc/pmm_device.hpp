@@ -10,43 +10,8 @@
 namespace laml {
 
 // value = m * 2^e
-struct SD {
-  double m;
-  int e;
-};
-
-__device__ __forceinline__ SD sd(double m, int e) {
-  SD r;
-  r.m = m;
-  r.e = e;
-  return r;
-}
-__device__ __forceinline__ SD sd_zero() { return sd(0.0, 0); }
-__device__ __forceinline__ SD sd_mul(SD a, SD b) { return sd(a.m * b.m, a.e + b.e); }
-__device__ __forceinline__ SD sd_scale(SD a, double c) { return sd(a.m * c, a.e); }
-__device__ __forceinline__ SD sd_add(SD a, SD b) {
-  if (a.m == 0.0) return b;
-  if (b.m == 0.0) return a;
-  const int e = a.e > b.e ? a.e : b.e;
-  return sd(ldexp(a.m, a.e - e) + ldexp(b.m, b.e - e), e);
-}
-// exponent t with |value| in [2^(t-1), 2^t); a very small sentinel for zero
+// the exponent of zero: below every other
 constexpr int kZeroTop = -0x3fffffff;
-__device__ __forceinline__ int sd_top(SD a) {
-  int ex;
-  (void)frexp(a.m, &ex);
-  return a.m != 0.0 ? a.e + ex : kZeroTop;
-}
-// a / b as a plain double (used for posteriors, which are O(1))
-__device__ __forceinline__ double sd_div(SD a, SD b) {
-  if (a.m == 0.0) return 0.0;
-  return ldexp(a.m / b.m, a.e - b.e);
-}
-// the value as a plain double (used for O(1) posteriors)
-__device__ __forceinline__ double sd_val(SD a) { return ldexp(a.m, a.e); }
-__device__ __forceinline__ double sd_log(SD a) {
-  return log(a.m) + (double)a.e * 0.69314718055994530942;
-}
 
 // transition coefficients of one branch of length d (rate 1, silencing nu):
 //   p1n = P(0->0) = e^{-(1+nu)d}

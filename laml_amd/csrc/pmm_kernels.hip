@@ -2856,8 +2856,7 @@ __device__ void ultra_barrier(const DevForest& F, const UltraDev& U, double* __r
 // are fixed, so the subtrees hanging off the quartet (A and W below u, C below
 // v) keep their inside vectors and the data above v keeps its outside state.
 // A candidate's EM then needs, per site, only those inputs and the five free
-// branches: each EM step is O(K) instead of a pass over the tree.  One
-// wavefront per candidate; lanes stride over the tree's sites.
+// branches: each EM step is O(K) instead of a pass over the tree.
 //
 // Candidate c (after the move): v has children u and C, u has children A and
 // W; p is v's parent and s v's sibling (p = -1: v is the root and its branch
@@ -3729,8 +3728,8 @@ __device__ __forceinline__ void lds_sum(double (&v)[kN], double* sh) {
 // loop, for problems of at most kPbMaxSites sites whose state fits LDS.  The
 // loop needs no launch, no host and no other block between EM steps.  A
 // thread keeps to the same branches throughout; the M-step reads their counts
-// from LDS.  One 250 x 30 problem: 46 us an EM step (inside 16, outside 19,
-// M-step 11), 101 us in the general passes' 13 launches; 200 trees of 20-200
+// from LDS.  One 250 x 30 problem: 43 us an EM step (inside 16, outside 19,
+// M-step 8), 101 us in the general passes' 13 launches; 200 trees of 20-200
 // leaves x 20 sites: 51 us, 187 us; one likelihood of 250 x 30: 23 us, 35 us.
 struct PbArgs {
   DevForest F;
