@@ -4,7 +4,6 @@
 
 #include <algorithm>
 #include <deque>
-#include <tuple>
 #include <limits>
 #include <mutex>
 #include <cstdlib>
@@ -1412,8 +1411,9 @@ static int chains_now(const laml_forest* f) {
 // parent lies at hs or above, and light children; a head's round is one
 // more than its parent's chain's (0 when the state comes from above).
 static const laml::ChainPlan* chain_plan(laml_forest* f, int hs) {
+  const bool inside = f->chains & LAML_CHAINS_INSIDE;
   for (const laml::ChainPlan& cp : f->chain_plans)
-    if (cp.h_split == hs && cp.pack_cap == f->chain_pack) return &cp;
+    if (cp.h_split == hs && cp.pack_cap == f->chain_pack && (cp.inside || !inside)) return &cp;
   // a new plan is uploaded with synchronous copies: not while another
   // thread captures its EM step (the passes only look plans up: each entry
   // point builds them before any capture)
@@ -1421,7 +1421,10 @@ static const laml::ChainPlan* chain_plan(laml_forest* f, int hs) {
   const int N = f->F.num_nodes;
   const int lo = f->level_off[1], B = f->level_off[hs];
   std::vector<int32_t> chain_of(N, -1), round_of(N, 0);
-  std::vector<std::tuple<int, int, int>> heads;  // (round, -len, -head)
+  struct Head {
+    int round, len, v;
+  };
+  std::vector<Head> heads;
   for (int v = B - 1; v >= lo; --v) {
     const int pa = f->h_parent[v];
     const bool above = pa < 0 || pa >= B;
@@ -1433,13 +1436,16 @@ static const laml::ChainPlan* chain_plan(laml_forest* f, int hs) {
       ++len;
     }
     round_of[v] = r;
-    heads.emplace_back(r, -len, -v);
+    heads.push_back(Head{r, len, v});
   }
-  std::sort(heads.begin(), heads.end());
+  // by round, the longest first (heads are in descending order already)
+  std::stable_sort(heads.begin(), heads.end(), [](const Head& a, const Head& b) {
+    return a.round != b.round ? a.round < b.round : a.len > b.len;
+  });
   // inside rounds: children precede parents, so a light child's chain has
   // its final round when its parent is visited
-  std::vector<int32_t> in_round(N, 0);
-  for (int v = lo; v < B; ++v) {
+  std::vector<int32_t> in_round(inside ? N : 0, 0);
+  for (int v = lo; inside && v < B; ++v) {
     const int cs[2] = {f->h_child0[v], f->h_child1[v]};
     for (int c : cs)
       if (c >= f->F.num_leaves && c != f->h_heavy[v])
@@ -1450,27 +1456,29 @@ static const laml::ChainPlan* chain_plan(laml_forest* f, int hs) {
   cp.pack_cap = f->chain_pack;
   std::vector<int2> ch;
   std::vector<int32_t> nodes, off_of(N, -1), round_off;
-  std::vector<std::tuple<int, int, int>> in_heads;  // (inside round, -len, -head)
   ch.reserve(heads.size());
   nodes.reserve(B - lo);
-  for (const auto& hd : heads) {
-    const int r = std::get<0>(hd), v = -std::get<2>(hd);
-    while ((int)round_off.size() <= r) round_off.push_back((int32_t)ch.size());
-    off_of[v] = (int32_t)nodes.size();
-    ch.push_back(make_int2((int)nodes.size(), -std::get<1>(hd)));
-    for (int w = v; w >= 0; w = f->h_heavy[w]) nodes.push_back(w);
-    in_heads.emplace_back(in_round[v], std::get<1>(hd), std::get<2>(hd));
+  for (const Head& hd : heads) {
+    while ((int)round_off.size() <= hd.round) round_off.push_back((int32_t)ch.size());
+    off_of[hd.v] = (int32_t)nodes.size();
+    ch.push_back(make_int2((int)nodes.size(), hd.len));
+    for (int w = hd.v; w >= 0; w = f->h_heavy[w]) nodes.push_back(w);
   }
   round_off.push_back((int32_t)ch.size());
-  std::sort(in_heads.begin(), in_heads.end());
   std::vector<int2> ich;
-  ich.reserve(in_heads.size());
-  for (const auto& hd : in_heads) {
-    const int r = std::get<0>(hd), v = -std::get<2>(hd);
-    while ((int)cp.in_round_off.size() <= r) cp.in_round_off.push_back((int32_t)ich.size());
-    ich.push_back(make_int2(off_of[v], -std::get<1>(hd)));
+  cp.inside = inside;
+  if (inside) {
+    for (Head& hd : heads) hd.round = in_round[hd.v];
+    std::sort(heads.begin(), heads.end(), [](const Head& a, const Head& b) {
+      return a.round != b.round ? a.round < b.round : (a.len != b.len ? a.len > b.len : a.v > b.v);
+    });
+    ich.reserve(heads.size());
+    for (const Head& hd : heads) {
+      while ((int)cp.in_round_off.size() <= hd.round) cp.in_round_off.push_back((int32_t)ich.size());
+      ich.push_back(make_int2(off_of[hd.v], hd.len));
+    }
+    cp.in_round_off.push_back((int32_t)ich.size());
   }
-  cp.in_round_off.push_back((int32_t)ich.size());
   std::vector<laml::ChainStep> steps(nodes.size());
   for (size_t i = 0; i < nodes.size(); ++i) {
     const int v = nodes[i];
@@ -1495,8 +1503,7 @@ static const laml::ChainPlan* chain_plan(laml_forest* f, int hs) {
   phro.reserve(steps.size());
   {
     struct Pack {
-      int len;
-      std::vector<int32_t> members;
+      int len, first, members;  // members of `order`
     };
     for (size_t r = 0; r + 1 < round_off.size(); ++r) {
       cp.pack_round_off.push_back((int32_t)packs.size());
@@ -1514,22 +1521,23 @@ static const laml::ChainPlan* chain_plan(laml_forest* f, int hs) {
       });
       std::vector<Pack> rp;
       int cur_tree = -1;
-      for (const int i : order) {
-        const int tr = f->h_tree_of[nodes[ch[i].x]];
+      for (size_t q = 0; q < order.size(); ++q) {
+        const int i = order[q], tr = f->h_tree_of[nodes[ch[i].x]];
         if (tr != cur_tree || rp.back().len + ch[i].y > cap) {
-          rp.push_back(Pack{0, {}});
+          rp.push_back(Pack{0, (int)q, 0});
           cur_tree = tr;
         }
         rp.back().len += ch[i].y;
-        rp.back().members.push_back(i);
+        ++rp.back().members;
       }
       std::stable_sort(rp.begin(), rp.end(), [](const Pack& a, const Pack& b) { return a.len > b.len; });
       bool packed = false;
-      for (const Pack& pk : rp) packed = packed || pk.members.size() > 1;
+      for (const Pack& pk : rp) packed = packed || pk.members > 1;
       cp.round_packed.push_back(packed ? 1 : 0);
       for (const Pack& pk : rp) {
         packs.push_back(make_int2((int)psteps.size(), pk.len));
-        for (const int i : pk.members) {
+        for (int q = pk.first; q < pk.first + pk.members; ++q) {
+          const int i = order[q];
           for (int j = 0; j < ch[i].y; ++j) {
             laml::ChainStep rec = steps[ch[i].x + j];
             if (j == 0) {
@@ -1545,7 +1553,8 @@ static const laml::ChainPlan* chain_plan(laml_forest* f, int hs) {
     }
     cp.pack_round_off.push_back((int32_t)packs.size());
   }
-  if (f->upload(&cp.in_chains, ich.data(), ich.size()) || f->upload(&cp.nodes, nodes.data(), nodes.size()) ||
+  if ((inside && (f->upload(&cp.in_chains, ich.data(), ich.size()) ||
+                  f->upload(&cp.nodes, nodes.data(), nodes.size()))) ||
       f->upload(&cp.packs, packs.data(), packs.size()) || f->upload(&cp.pack_steps, psteps.data(), psteps.size()) ||
       f->upload(&cp.pack_head_ro, phro.data(), phro.size()))
     return nullptr;

@@ -278,6 +278,7 @@ struct ChainStep {
 struct ChainPlan {
   int32_t h_split = -1;
   int32_t pack_cap = 0;              // most steps per outside pack the plan was built for
+  bool inside = false;               // with the inside rounds (only where inside chains are asked for)
   const int2* in_chains = nullptr;
   const int32_t* nodes = nullptr;
   // outside packs: (offset into pack_steps, steps), each one or more chains
