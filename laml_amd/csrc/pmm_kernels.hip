@@ -1303,19 +1303,14 @@ __device__ __forceinline__ void out_write_partials(const DevForest& F, int u, co
     }
     v[10] = rt;
     v[11] = 0.0;
-    wave_sum12(v);
-    // lane 16r + j (j < 3) stores total 3r + j: counts 0..4 of child 0,
-    // counts 0..4 of child 1, the dropout sum
-    const int r = lane >> 4, j = lane & 15;
-    const int vi = 3 * r + j;
-    if (j < 3 && vi < 11) {
-      const double x = j == 0 ? v[0] : (j == 1 ? v[1] : v[2]);
-      if (vi < 10) {
-        const int i = vi >= 5 ? 1 : 0;
-        F.cpart[((int64_t)ch[i] * F.max_chunks + slot) * 5 + (vi - 5 * i)] = x;
-      } else {
-        F.rt_part[(int64_t)u * F.max_chunks + slot] = x;
-      }
+    const double x = wave_sum12(v);
+    // totals 0..4: counts of child 0, 5..9: of child 1, 10: the dropout sum
+    const int vi = sum12_value(lane);
+    if (vi >= 0 && vi < 10) {
+      const int i = vi >= 5 ? 1 : 0;
+      F.cpart[((int64_t)ch[i] * F.max_chunks + slot) * 5 + (vi - 5 * i)] = x;
+    } else if (vi == 10) {
+      F.rt_part[(int64_t)u * F.max_chunks + slot] = x;
     }
     const int nz = slot_end - slot - 1;
     if (nz > 0) {
@@ -1699,6 +1694,7 @@ __global__ void __launch_bounds__(256) k_outside_chain(DevForest F, const int2* 
   int touch = 0;  // first word of the record four steps ahead (brings its line into the scalar cache)
   if (len > 2) touch = uniform_load(&cs[min(len - 1, 4)].u);
 
+  const int vi = sum12_value(lane);
   double* pp = nullptr;  // partial count held back from the previous step
   double pv = 0.0;
   for (int j = 0;;) {
@@ -1759,9 +1755,8 @@ __global__ void __launch_bounds__(256) k_outside_chain(DevForest F, const int2* 
         chain_compute<kInternal, kInternal>(F, lds, lane, cf, phi, hv, raw, ro, kk, on, stream, stage, a0, aX, lu,
                                             o);
     }
-    // partial counts: one butterfly sum of the eleven values; lane 16r + i
-    // (i < 3) holds total 3r + i (counts 0..4 of child 0, of child 1, the
-    // dropout sum), stored at the top of the next step
+    // partial counts (0..4 of child 0, of child 1, the dropout sum), stored at
+    // the top of the next step
     double v[12];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
@@ -1770,18 +1765,13 @@ __global__ void __launch_bounds__(256) k_outside_chain(DevForest F, const int2* 
     }
     v[10] = o.rt;
     v[11] = 0.0;
-    wave_sum12(v);
-    {
-      const int rr = lane >> 4, i = lane & 15;
-      const int vi = 3 * rr + i;
-      pv = i == 0 ? v[0] : (i == 1 ? v[1] : v[2]);
-      pp = nullptr;
-      if (i < 3 && vi < 10) {
-        const int c = vi >= 5 ? 1 : 0;
-        pp = F.cpart + ((int64_t)(c ? r0.ch1 : r0.ch0) * F.max_chunks + chunk) * 5 + (vi - 5 * c);
-      } else if (i < 3 && vi == 10) {
-        pp = F.rt_part + (int64_t)u * F.max_chunks + chunk;
-      }
+    pv = wave_sum12(v);
+    pp = nullptr;
+    if (vi >= 0 && vi < 10) {
+      const int c = vi >= 5 ? 1 : 0;
+      pp = F.cpart + ((int64_t)(c ? r0.ch1 : r0.ch0) * F.max_chunks + chunk) * 5 + (vi - 5 * c);
+    } else if (vi == 10) {
+      pp = F.rt_part + (int64_t)u * F.max_chunks + chunk;
     }
     if (!more) break;
     ++j;
@@ -1796,9 +1786,9 @@ __global__ void __launch_bounds__(256) k_outside_chain(DevForest F, const int2* 
 // clade's root.  The children's inside rows, labels and codes of the next step
 // are copied to the slice during the step, as in k_outside_chain; prior
 // weights come from the chunk's piece in LDS and the coefficients in walking
-// order, as in k_inside_clade.  Sixteen trees of 10,000 leaves x 300 sites: 337
-// us and 150 in the rounds above, where the chain rounds and the levels above
-// took 675 us; 50,000 x 500: 178 and 82, 325.  Bound by instruction issue (93 %
+// order, as in k_inside_clade.  Sixteen trees of 10,000 leaves x 300 sites: 333
+// us and 125 in the rounds above, where the chain rounds and the levels above
+// took 675 us; 50,000 x 500: 175 and 91, 325.  Bound by instruction issue (93 %
 // of the VALU cycles at six wavefronts a SIMD).
 constexpr int kOutLdsBeta = 0;     // [2][64] double2
 constexpr int kOutLdsE = 2048;     // [2][64] int32
@@ -1903,6 +1893,7 @@ __global__ void __launch_bounds__(64 * kCladeOutWaves)
     aX = a.y;
   }
   clade_stage(F, r, (unsigned)k0, lane, lds, stream);
+  const int vi = sum12_value(lane);
   double* pp = nullptr;  // partial count held back from the previous step
   double pv = 0.0;
   for (;; --j) {
@@ -1941,18 +1932,13 @@ __global__ void __launch_bounds__(64 * kCladeOutWaves)
     }
     v[10] = o.rt;
     v[11] = 0.0;
-    wave_sum12(v);
-    {
-      const int rr = lane >> 4, i = lane & 15;
-      const int vi = 3 * rr + i;
-      pv = i == 0 ? v[0] : (i == 1 ? v[1] : v[2]);
-      pp = nullptr;
-      if (i < 3 && vi < 10) {
-        const int c = vi >= 5 ? 1 : 0;
-        pp = F.cpart + ((int64_t)(c ? r.ch[1] : r.ch[0]) * F.max_chunks + chunk) * 5 + (vi - 5 * c);
-      } else if (i < 3 && vi == 10) {
-        pp = F.rt_part + (int64_t)r.u * F.max_chunks + chunk;
-      }
+    pv = wave_sum12(v);
+    pp = nullptr;
+    if (vi >= 0 && vi < 10) {
+      const int c = vi >= 5 ? 1 : 0;
+      pp = F.cpart + ((int64_t)(c ? r.ch[1] : r.ch[0]) * F.max_chunks + chunk) * 5 + (vi - 5 * c);
+    } else if (vi == 10) {
+      pp = F.rt_part + (int64_t)r.u * F.max_chunks + chunk;
     }
     if (!more) break;
     r = r1;
@@ -3099,22 +3085,21 @@ __global__ void __launch_bounds__(64 * NW) k_quartet_em(DevForest F, const int32
       cf[j].msil = uniform_double(scf[j].msil);
       cf[j].esil = __builtin_amdgcn_readfirstlane(scf[j].esil);
     }
-    const int r = lane >> 4, i = lane & 15;
+    const int vi = sum12_value(lane);
     for (int k0 = 0; k0 < K; k0 += 64 * NW) {
       const int k = k0 + tid;
       const bool on = k < K;
       if (on && (it == 0 || K > 64 * NW)) q_load(F, n, k, x);
-      // totals over the wavefront, a dozen values at a time: row r gets
-      // values 3 r .. 3 r + 2; added to the earlier turns'
+      // totals over the wavefront, a dozen values at a time, added to the
+      // earlier turns'
       double v[12];
       int nv = 0, base = 0;
       auto put = [&](double s) {
         v[nv++] = on ? s : 0.0;
         if (nv < 12) return;
-        wave_sum12(v);
-        if (i < 3) {
-          double* o = &sh[wave][base + 3 * r + i];
-          const double y = i == 0 ? v[0] : (i == 1 ? v[1] : v[2]);
+        const double y = wave_sum12(v);
+        if (vi >= 0) {
+          double* o = &sh[wave][base + vi];
           *o = k0 == 0 ? y : *o + y;
         }
         nv = 0;
@@ -3501,7 +3486,6 @@ __device__ __forceinline__ void lds_cells(const LdsCtx& x, const LdsItem& it) {
     else lds_outside_cells<false>(x, it, v);
   }
   // sums over the lanes of the group: row r ends with values 3 r .. 3 r + 2
-  // (as wave_sum12)
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
     swap32(v[j], v[j + 6]);
