@@ -7,6 +7,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "pmm_solve.hpp"
+
 namespace laml {
 
 // value = m * 2^e
@@ -102,14 +104,6 @@ __device__ __forceinline__ int exp_of(double m) {
   int ex;
   (void)frexp(m, &ex);
   return ex;
-}
-
-// 1 / x where x and 1 / x are normal numbers: the hardware estimate and two
-// Newton steps (no scaling for extreme arguments)
-__device__ __forceinline__ double rcp_normal(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = fma(fma(-x, r, 1.0), r, r);
-  return fma(fma(-x, r, 1.0), r, r);
 }
 
 // 64-bit DPP move of a double (rows not in ROW_MASK read 0)
