@@ -100,10 +100,14 @@ struct laml_forest {
   // problem fits it; taken while the launch plan is the one the forest was
   // created with (any other plan asks for its own kernels).  They leave no
   // rows in global memory: rows_ok says whether the rows hold the inside
-  // state of the last call.
+  // state of the last call.  A call that is being captured runs again without
+  // this code when its graph is replayed: once one that leaves no inside rows,
+  // or not all outside rows, has been captured, rows_ok and alpha_complete
+  // are not trusted any more (rows_unsure, alpha_unsure).  The branch
+  // coefficients are always those of the last call, replayed or not.
   bool pb_ok = false;
   laml::LdsPlan pb{};
-  bool rows_ok = true;
+  bool rows_ok = true, rows_unsure = false, alpha_unsure = false;
   struct {
     int pass_mode, h_top, chains, chain_top_in, chain_top_out;
     bool fuse;
@@ -1876,13 +1880,40 @@ static void pass_outside(laml_forest* f, const DevForest& F, bool with_root, con
   f->alpha_complete = !cp && !cl;
 }
 
-// the inside rows of the last call's parameters, where it left none (its
-// branch coefficients are resident; not in a clade plan's steps: F names none)
-static void ensure_rows(laml_forest* f, const DevForest& F, hipStream_t s) {
-  if (f->rows_ok) return;
+// whether s is being captured (or may be: the query failed)
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// after a call on s that leaves no rows
+static void left_no_rows(laml_forest* f, hipStream_t s) {
+  f->rows_ok = f->alpha_complete = f->inside_fused = false;
+  if (!f->rows_unsure && capturing(s)) f->rows_unsure = f->alpha_unsure = true;
+}
+// after a call on s with an outside pass
+static void left_outside(laml_forest* f, hipStream_t s) {
+  if (!f->alpha_complete && !f->alpha_unsure && capturing(s)) f->alpha_unsure = true;
+}
+
+// the inside rows of the last call's parameters, where it left none or may
+// have left none (from its branch coefficients; not those in a clade plan's
+// steps: F names none).  Returns whether it formed them.
+static bool ensure_rows(laml_forest* f, const DevForest& F, hipStream_t s) {
+  if (f->rows_ok && !f->rows_unsure) return false;
   pass_inside_root(f, F, nullptr, nullptr, s);
-  f->rows_ok = true;
-  f->alpha_complete = false;
+  return true;
+}
+
+// every node's inside and outside rows, for a call that reads them: what the
+// last call kept out of memory is formed again.  A call that is being captured
+// may be replayed after an E-step that leaves fewer rows than the last one.
+static void ensure_all_rows(laml_forest* f, const DevForest& F, hipStream_t s) {
+  const bool formed = ensure_rows(f, F, s);
+  if (formed || !f->alpha_complete || f->alpha_unsure || ((chains_now(f) || out_clades(f)) && capturing(s)))
+    pass_outside(f, F, true, nullptr, s, false);
 }
 
 int laml_nll(laml_forest* f, const double* d, const double* nu, const double* phi, double* nll, double* site_llh,
@@ -1896,7 +1927,7 @@ int laml_nll(laml_forest* f, const double* d, const double* nu, const double* ph
   if (problem_now(f)) {
     laml::run_problem(lds_view(F, f->pb), f->pb, f->TW, const_cast<double*>(d), const_cast<double*>(nu),
                       const_cast<double*>(phi), nll, site_llh, nullptr, none, 1, 0, 0.0, laml::kPbCoef, s);
-    f->rows_ok = f->alpha_complete = f->inside_fused = false;
+    left_no_rows(f, s);
     return check_launch();
   }
   int rc = prepare_chains(f, s);
@@ -1916,15 +1947,10 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
   DevForest F = f->F;
   F.phi = phi;
   EmState none{};
-  if (problem_now(f)) {
-    const DevForest G = lds_view(F, f->pb);
-    laml::run_problem(G, f->pb, f->TW, const_cast<double*>(d), const_cast<double*>(nu), const_cast<double*>(phi), nll,
-                      nullptr, nullptr, none, 1, 0, 0.0, laml::kPbCoef | laml::kPbOut, s);
-    f->rows_ok = f->alpha_complete = f->inside_fused = false;
-    laml::run_counts(G, counts, s);
-    laml::run_rtilde(G, rtilde, nullptr, s);
-    return check_launch();
-  }
+  // Not in whole-problem blocks, also where the other calls take them: what
+  // follows an E-step reads its rows (posteriors, quartet EM), and forming them
+  // again costs more than the blocks save.  E-step and posteriors of one 250 x
+  // 30 problem 173 us, 221 with a block's E-step (E-step alone 79 and 58).
   pass_coef(f, F, d, nu, nullptr, s);
   int rc = prepare_chains(f, s);
   if (rc) return rc;
@@ -1943,6 +1969,7 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
     pass_inside_root(f, F, nullptr, nullptr, s);
     pass_outside(f, F, false, nullptr, s);
   }
+  left_outside(f, s);
   laml::run_llh(F, nll, none, 0, 0.0, s);
   laml::run_counts(F, counts, s);
   laml::run_rtilde(F, rtilde, nullptr, s);
@@ -1950,10 +1977,11 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
 }
 
 // the outside pass over the state of the last call: from its rows, or with
-// the inside pass again where it left none.  Returns the view of F that holds
-// the partial counts.
+// the inside pass again where it left none (a captured call may be replayed
+// after another one that did).  Returns the view of F that holds the partial
+// counts.
 static DevForest outside_again(laml_forest* f, const DevForest& F, const double* phi, hipStream_t s) {
-  if (!f->rows_ok && problem_now(f)) {
+  if (problem_now(f) && (!f->rows_ok || f->rows_unsure || capturing(s))) {
     const DevForest G = lds_view(F, f->pb);
     EmState none{};
     laml::run_problem(G, f->pb, f->TW, nullptr, nullptr, const_cast<double*>(phi), nullptr, nullptr, nullptr, none, 1,
@@ -1970,6 +1998,7 @@ static DevForest outside_again(laml_forest* f, const DevForest& F, const double*
     if (out_clades(f)) laml::run_clade_coef(G, s);
   }
   pass_outside(f, G, true, nullptr, s);
+  left_outside(f, s);
   return F;
 }
 
@@ -2067,6 +2096,7 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
     constexpr int kPbSteps = 128;
     const DevForest G = lds_view(F, f->pb);
     laml::run_em_reset(em, P, s);
+    left_no_rows(f, s);
     std::vector<int32_t> done_h(P);
     for (int64_t step = 0; step <= max_iter; step += kPbSteps) {
       const int steps = (int)std::min<int64_t>(kPbSteps, (int64_t)max_iter + 1 - step);
@@ -2082,7 +2112,6 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
         if (all) break;
       }
     }
-    f->rows_ok = f->alpha_complete = f->inside_fused = false;
     return LAML_OK;
   }
   int prc = prepare_chains(f, s);
@@ -2139,7 +2168,7 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
   // captured step's pass
   f->rows_ok = !problem_now(f);
   if (!f->rows_ok)
-    f->alpha_complete = f->inside_fused = false;
+    left_no_rows(f, s);
   else if (max_iter > 0 && f->pass_mode != LAML_PASS_TREES)
     f->alpha_complete = !out_clades(f) && !pass_chains(f, false, hybrid_split(f)) && !fuse_now(f);
   LAML_HIP(hipMemcpyAsync(iters, em.iters, sizeof(int32_t) * P, hipMemcpyDeviceToDevice, s));
@@ -2161,11 +2190,7 @@ int laml_posteriors(laml_forest* f, const double* phi, double* post0_host, doubl
   hipStream_t s = static_cast<hipStream_t>(stream);
   DevForest F = f->F;
   F.phi = phi;
-  // the last outside pass kept heavy children's outside states in
-  // registers: form every node's outside row again from the resident inside
-  // state (one outside pass in level launches)
-  ensure_rows(f, F, s);
-  if (!f->alpha_complete) pass_outside(f, F, true, nullptr, s, false);
+  ensure_all_rows(f, F, s);
   double* p0 = nullptr;
   if (hipMalloc(&p0, 2 * sizeof(double) * std::max<int64_t>(need, 1)) != hipSuccess)
     return fail(LAML_ENOMEM, "hipMalloc posteriors");
@@ -2199,8 +2224,7 @@ int laml_posteriors_noalloc(laml_forest* f, const double* phi, double* post0_hos
   hipStream_t s = static_cast<hipStream_t>(stream);
   DevForest F = f->F;
   F.phi = phi;
-  ensure_rows(f, F, s);
-  if (!f->alpha_complete) pass_outside(f, F, true, nullptr, s, false);
+  ensure_all_rows(f, F, s);
   double* o0 = f->post_scratch;
   double* oS = o0 + need;
   laml::run_node_post(F, f->W, f->d_desc_off, f->leaf_sites, o0, oS, s);
@@ -2230,8 +2254,7 @@ int laml_quartet_em(laml_forest* f, int32_t num_candidates, const int32_t* quart
   hipStream_t s = static_cast<hipStream_t>(stream);
   DevForest F = f->F;
   F.phi = phi;
-  ensure_rows(f, F, s);
-  if (!f->alpha_complete) pass_outside(f, F, true, nullptr, s, false);
+  ensure_all_rows(f, F, s);
   laml::run_quartet_em(f->F, num_candidates, quartet_nodes, lengths_in, optimise, llh_const, nu, phi, max_iter, tol,
                        lengths_out, nll, iters, s);
   return check_launch();

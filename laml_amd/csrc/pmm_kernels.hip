@@ -3560,8 +3560,9 @@ __device__ __forceinline__ void lds_sum(double (&v)[kN], double* sh) {
   }
 }
 
-// Whole problems of one tree, a block each: likelihood, E-step, or the EM
-// loop, for problems of at most kPbMaxSites sites whose state fits LDS.  The
+// Whole problems of one tree, a block each: likelihood, outside pass (the
+// inside pass again first), or the EM loop, for problems of at most
+// kPbMaxSites sites whose state fits LDS.  The
 // loop needs no launch, no host and no other block between EM steps.  A
 // thread keeps to the same branches throughout; the M-step reads their counts
 // from LDS.  One 250 x 30 problem: 43 us an EM step (inside 16, outside 19,
@@ -3610,14 +3611,19 @@ __global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
   const int hn = lds_first_narrow(x);
   const int nbr = 2 * x.nint + 1;
   for (int it = 0; it < pb_args().max_steps; ++it) {
-    if (what & kPbCoef) {
+    {
       const PbArgs& A = pb_args();
       const DevForest& F = A.F;
       const int ib = uniform_at(A.L.int_base, t);
       for (int r = (int)threadIdx.x; r < nbr; r += kLdsThreads) {
         const int v = lds_branch_node(F, x, t, r);
-        const Coef c = branch_coef(A.d[v], nv);
-        F.coef[v] = c;
+        Coef c;
+        if (what & kPbCoef) {
+          c = branch_coef(A.d[v], nv);
+          F.coef[v] = c;
+        } else {
+          c = F.coef[v];  // (those of the last call, whichever kernels ran it)
+        }
         if (r < nbr - 1) lds_set_coef(A.L, ib, r, c);
       }
       __syncthreads();
