@@ -1799,12 +1799,13 @@ static void pass_coef(laml_forest* f, DevForest& F, const double* d, const doubl
 
 // inside levels [1, hs) of the level and hybrid passes: chains below the
 // chain region's top, level launches above it
-static void inside_below(laml_forest* f, const DevForest& F, int hs, const int32_t* done, hipStream_t s) {
+static void inside_below(laml_forest* f, const DevForest& F, int hs, const int32_t* done, hipStream_t s,
+                         bool allow_chains = true) {
   if (const laml::CladePlan* cl = F.clade_coef ? pass_clades(f) : nullptr) {
     laml::run_inside_clades(F, *cl, done, s);
     return;
   }
-  const laml::ChainPlan* cp = pass_chains(f, true, hs);
+  const laml::ChainPlan* cp = allow_chains ? pass_chains(f, true, hs) : nullptr;
   if (cp) laml::run_inside_chains(F, *cp, done, s);
   laml::run_inside_levels(F, f->level_off, f->W, cp ? cp->h_split : 1, hs, f->in_cpw, done, s);
 }
@@ -1823,21 +1824,23 @@ static void outside_below(laml_forest* f, const DevForest& F, int hs, const int3
   f->alpha_complete = cp == nullptr;
 }
 
-// inside pass and root step (site likelihoods) in the forest's pass mode
+// inside pass and root step (site likelihoods) in the forest's pass mode.
+// plain: every node's rows, in level launches below the walk (no fused
+// cherries, and no chains, whose plan this call might have to build)
 static void pass_inside_root(laml_forest* f, const DevForest& F, double* site_llh, const int32_t* done,
-                             hipStream_t s) {
+                             hipStream_t s, bool plain = false) {
   if (f->pass_mode == LAML_PASS_HYBRID) {
     f->inside_fused = false;
     const int hs = hybrid_split(f);
-    inside_below(f, F, hs, done, s);
+    inside_below(f, F, hs, done, s, !plain);
     laml::run_tree_walk(F, f->TW, f->W, 3, site_llh, done, s, hs);
   } else if (f->pass_mode == 1) {
     f->inside_fused = false;
     laml::run_tree_walk(F, f->TW, f->W, 3, site_llh, done, s);
   } else {
-    f->inside_fused = fuse_now(f);
+    f->inside_fused = fuse_now(f) && !plain;
     const DevForest G = with_cherries(f, F, f->inside_fused);
-    const laml::ChainPlan* cp = pass_chains(f, true, hybrid_split(f));
+    const laml::ChainPlan* cp = plain ? nullptr : pass_chains(f, true, hybrid_split(f));
     const laml::CladePlan* cl = F.clade_coef ? pass_clades(f) : nullptr;
     laml::run_inside(G, f->level_off, f->W, f->h_top, f->in_cpw, done, s, f->inside_fused ? &f->split : nullptr, cp,
                      cl);
@@ -1903,7 +1906,7 @@ static void left_outside(laml_forest* f, hipStream_t s) {
 // steps: F names none).  Returns whether it formed them.
 static bool ensure_rows(laml_forest* f, const DevForest& F, hipStream_t s) {
   if (f->rows_ok && !f->rows_unsure) return false;
-  pass_inside_root(f, F, nullptr, nullptr, s);
+  pass_inside_root(f, F, nullptr, nullptr, s, true);
   return true;
 }
 
