@@ -195,6 +195,18 @@ int32_t laml_forest_fusion(laml_forest* f);
 #define LAML_CHAINS_OUTSIDE 1
 #define LAML_CHAINS_INSIDE 2
 int laml_forest_set_chains(laml_forest* f, int32_t which, int32_t inside_top, int32_t outside_top);
+
+/* How the next passes run, and what has been laid out for them so far (tests
+ * ask for it; no counterpart in the reference). */
+typedef struct {
+  int32_t blocks;          /* 1: likelihoods and EM steps in whole-problem blocks */
+  int32_t walk_level;      /* first level of the tree walk or the fused top-level kernel */
+  int32_t inside_clades;   /* clades of the inside pass (0: none, or not laid out yet) */
+  int32_t outside_clades;  /* clades of the outside pass */
+  int32_t largest_clade;   /* internal nodes of the largest of them */
+  int32_t chain_plans;     /* chain plans laid out */
+} laml_pass_plan;
+int laml_forest_pass_plan(laml_forest* f, laml_pass_plan* out);
 int laml_forest_get_chains(laml_forest* f, int32_t* which, int32_t* inside_top, int32_t* outside_top);
 int32_t laml_forest_chains(laml_forest* f);
 

@@ -80,6 +80,11 @@ class UltraDesc(ctypes.Structure):
     ]
 
 
+class PassPlan(ctypes.Structure):
+    _fields_ = [(x, ctypes.c_int32) for x in ("blocks", "walk_level", "inside_clades", "outside_clades",
+                                              "largest_clade", "chain_plans")]
+
+
 # name -> (restype, argtypes); every symbol include/laml_pmm.h declares
 SIGNATURES = {
     "laml_forest_create": (ctypes.c_int, [ctypes.POINTER(ForestDesc), ctypes.c_int,
@@ -107,6 +112,7 @@ SIGNATURES = {
     "laml_forest_set_chains": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32]),
     "laml_forest_get_chains": (ctypes.c_int, [ctypes.c_void_p] + [ctypes.POINTER(ctypes.c_int32)] * 3),
     "laml_forest_chains": (ctypes.c_int32, [ctypes.c_void_p]),
+    "laml_forest_pass_plan": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(PassPlan)]),
     "laml_posteriors": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, _f64p, _f64p, ctypes.c_int64,
                                          ctypes.c_void_p]),
     "laml_posteriors_noalloc": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, _f64p, _f64p, ctypes.c_int64,

@@ -1589,6 +1589,19 @@ static const laml::CladePlan* out_clades(const laml_forest* f) {
              : nullptr;
 }
 
+int laml_forest_pass_plan(laml_forest* f, laml_pass_plan* out) {
+  if (!f || !out) return fail(LAML_EINVAL, "null argument");
+  const laml::CladePlan *in = pass_clades(f), *oc = out_clades(f);
+  *out = laml_pass_plan{};
+  out->blocks = problem_now(f);
+  out->walk_level = f->pass_mode == LAML_PASS_TREES ? 1 : hybrid_split(f);
+  out->inside_clades = in ? in->count : 0;
+  out->outside_clades = oc ? oc->count : 0;
+  out->largest_clade = in ? in->largest : 0;
+  out->chain_plans = (int32_t)f->chain_plans.size();
+  return LAML_OK;
+}
+
 // Builds the clade plan of the internal nodes below the current split, if
 // there is none yet (kept for the forest's life).  A call that is being
 // captured, or that finds no memory, runs level launches.
@@ -1718,6 +1731,8 @@ static void prepare_clades(laml_forest* f, hipStream_t s) {
     }
     clades.back().w = (int)(leaf_row.size() / laml::kCladeBatch) - batch0;
   }
+  cl.count = (int)clades.size();
+  for (const int4& c : clades) cl.largest = std::max(cl.largest, c.y);
   cl.num = (int)blocks.size();
   cl.out_num = (int)oblocks.size();
   // one allocation

@@ -329,6 +329,7 @@ struct CladeCoef {
 };
 struct CladePlan {
   int32_t h_split = -1, cap = 0;
+  int32_t count = 0, largest = 0;  // clades, internal nodes of the largest
   int32_t num = 0;               // blocks
   int32_t q_bytes = 0;           // LDS for the prior weights of a chunk
   const int4* blocks = nullptr;  // first clade, clades, tree

@@ -561,6 +561,12 @@ class Forest(ForestLayout):
         """The chain flags the next passes use (0: none)."""
         return int(self._lib.laml_forest_chains(self.handle))
 
+    def pass_plan(self):
+        """How the next passes run (see laml_pass_plan), as a dict."""
+        p = _lib.PassPlan()
+        _lib.check(self._lib.laml_forest_pass_plan(self.handle, ctypes.byref(p)))
+        return {k: getattr(p, k) for k, _ in p._fields_}
+
     def get_shapes(self):
         """Launch shapes: (inside_cpw, outside_cpw, top_level); the cpw arrays
         hold, per level, the 64-site chunks one wavefront walks (all 0 when

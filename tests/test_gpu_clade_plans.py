@@ -1,0 +1,62 @@
+"""Clade passes where the plan is known to take them: the plan in use is
+asserted, so that a comparison with level launches cannot pass on level
+launches.  Splits near the root (LAML_TOP_MAX_NODES) give clades as large as
+their cap allows: long one-child walks over many batches of leaf codes
+(caterpillars), two pending states (Yule and balanced trees), clades that are
+whole trees.  Same bits as level launches, in the E-step, EM and posteriors."""
+import numpy as np
+import pytest
+import torch
+
+from laml_amd import sim
+from laml_amd._lib import PASS_HYBRID, PASS_LEVELS
+from laml_amd.forest import Forest
+from test_gpu_clades import _problem
+
+pytestmark = pytest.mark.gpu
+
+# kind, leaves and sites of the first tree, trees, and the largest clade at caps 1, 7 and 64
+CASES = [("caterpillar", 100, 130, 3, (1, 7, 64)), ("caterpillar", 70, 200, 2, (1, 7, 64)),
+         ("yule", 260, 100, 3, None), ("balanced", 256, 70, 2, (1, 7, 8)), ("yule", 2, 70, 4, (1, 1, 1)),
+         ("yule", 40, 129, 30, None)]
+
+
+def _dev(F, x):
+    return torch.tensor(np.asarray(x, dtype=np.float64), device=F.device)
+
+
+@pytest.mark.parametrize("kind,n,K,P,largest", CASES, ids=lambda x: str(x).replace(" ", ""))
+@pytest.mark.parametrize("cap", [1, 7, 64])
+def test_clades_in_use_equal_levels(kind, n, K, P, largest, cap, monkeypatch):
+    monkeypatch.setenv("LAML_TOP_MAX_NODES", "1")
+    probs = [_problem(kind, n + (0 if n == 2 else 9 * i), K - 5 * (i % 9), 300 + i) for i in range(P)]
+    specs = [sim.problem_spec(*p) for p in probs]
+    got = {}
+    for clades in (cap, 0):
+        monkeypatch.setenv("LAML_CLADES", str(clades))
+        F = Forest(specs, device=torch.cuda.current_device())
+        d = _dev(F, F.lengths_to_level([np.maximum(t.length, 0.005) for t, _, _ in probs]))
+        nu, phi = _dev(F, [0.2] * P), _dev(F, [0.3] * P)
+        for mode in (PASS_HYBRID, PASS_LEVELS):
+            F.set_pass_mode(mode)
+            print("clade plan", kind, n, K, P, clades, mode, flush=True)
+            counts, rt, nll = [x.cpu().numpy().copy() for x in F.estep(d, nu, phi)]
+            plan = F.pass_plan()
+            if clades:
+                assert plan["inside_clades"] > 0 and plan["outside_clades"] == plan["inside_clades"], plan
+                assert plan["walk_level"] > 1 and plan["blocks"] == 0 and plan["chain_plans"] == 0, plan
+                if largest is not None:
+                    assert plan["largest_clade"] == largest[(1, 7, 64).index(cap)], plan
+                elif cap == 64:
+                    assert plan["largest_clade"] > 7, plan
+            else:
+                assert plan["inside_clades"] == plan["outside_clades"] == 0, plan
+            em = [x.clone() for x in (d, nu, phi)]
+            F.em(*em, 3, 0.0)
+            F.estep(d, nu, phi)
+            post = [x.copy() for pair in F.posteriors(phi) for x in pair]
+            got[clades, mode] = [nll, counts, rt] + [x.cpu().numpy() for x in em] + post
+        F.close()
+    for mode in (PASS_HYBRID, PASS_LEVELS):
+        for a, b in zip(got[cap, mode], got[0, mode]):
+            np.testing.assert_array_equal(a, b)
