@@ -1969,10 +1969,10 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
   // follows an E-step reads its rows (posteriors, quartet EM), and forming them
   // again costs more than the blocks save.  E-step and posteriors of one 250 x
   // 30 problem 173 us, 221 with a block's E-step (E-step alone 79 and 58).
-  pass_coef(f, F, d, nu, nullptr, s);
   int rc = prepare_chains(f, s);
   if (rc) return rc;
   f->rows_ok = true;
+  pass_coef(f, F, d, nu, nullptr, s);
   if (f->pass_mode == 1) {
     f->inside_fused = false;
     laml::run_tree_walk(F, f->TW, f->W, 7, nullptr, nullptr, s);

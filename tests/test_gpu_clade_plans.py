@@ -3,7 +3,8 @@ asserted, so that a comparison with level launches cannot pass on level
 launches.  Splits near the root (LAML_TOP_MAX_NODES) give clades as large as
 their cap allows: long one-child walks over many batches of leaf codes
 (caterpillars), two pending states (Yule and balanced trees), clades that are
-whole trees.  Same bits as level launches, in the E-step, EM and posteriors."""
+whole trees.  Same bits as level launches, in the E-step, EM and posteriors.
+And the first call on a forest, whichever it is, takes the plan it lays out."""
 import numpy as np
 import pytest
 import torch
@@ -60,3 +61,24 @@ def test_clades_in_use_equal_levels(kind, n, K, P, largest, cap, monkeypatch):
     for mode in (PASS_HYBRID, PASS_LEVELS):
         for a, b in zip(got[cap, mode], got[0, mode]):
             np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("first", ["estep", "nll", "em"])
+def test_first_call_takes_the_plan_it_lays_out(first, monkeypatch):
+    """7,000 leaves x 300 sites, whose outside pass would run chains without
+    clades: no chain plan is laid out when it runs clades."""
+    monkeypatch.setenv("LAML_CLADES", "32")
+    t, Q, codes, _ = sim.make_problem(7000, 300, 3, 12, 1.0, 0.1, 0.1, 8)
+    F = Forest([sim.problem_spec(t, Q, codes)], device=torch.cuda.current_device())
+    prm = [_dev(F, F.lengths_to_level([np.maximum(t.length, 0.005)])), _dev(F, [0.2]), _dev(F, [0.1])]
+    print("first call", first, flush=True)
+    if first == "em":
+        F.em(*[x.clone() for x in prm], 1, 0.0)
+    elif first == "nll":
+        F.nll(*prm)
+        F.grad(*prm)
+    else:
+        F.estep(*prm)
+    plan = F.pass_plan()
+    assert plan["outside_clades"] > 0 and plan["chain_plans"] == 0, plan
+    F.close()
