@@ -798,13 +798,11 @@ def main():
 
     plan_desc = {}
 
-    from laml_amd.autotune import current_plan
 
     def run(problems, steps, warmup, tune=False):
         specs = [sim.problem_spec(t, q, c) for (t, q, c, _) in problems]
         t0 = time.perf_counter()
         F = Forest(specs, device=0)
-        F.created_plan = current_plan(F).describe()
         torch.cuda.synchronize()
         setup = time.perf_counter() - t0
         dev = F.device
@@ -900,16 +898,11 @@ def main():
     flags = F.chains()
     _, top_in, top_out = F.get_chains()
     region = lambda t: split if t <= 0 else min(t, split)
-    # the plan the forest was created with runs the passes of a large forest
-    # over clades below the walk's level
-    pairs = (F.num_nodes - F.num_leaves) * -(-int(F.tree_K.max()) // 64)
-    clades = None
-    if current_plan(F).describe() == F.created_plan and F.tree_K.max() > 32 and pairs >= 57344:
-        sizes, T = np.diff(F.level_off), F.num_trees
-        walk = 48 if T * -(-int(F.tree_K.max()) // 64) > 1024 else max(24, 10 * T)
-        clades = F.num_levels
-        while clades > 1 and sizes[clades - 1] <= walk:
-            clades -= 1
+    # the passes of a large forest run over clades below the walk's level
+    F.nll(d, nu, phi)
+    F.outside(phi)
+    passes = F.pass_plan()
+    clades = passes["walk_level"] if passes["outside_clades"] else None
     inside_b, outside_b = algorithmic_bytes(F, fused=F.fusion(), state=16, clade_split=clades,
                                             chain_split=region(top_out) if flags & 1 and clades is None else None,
                                             in_chain_split=region(top_in) if flags & 2 else None)

@@ -119,8 +119,11 @@ int64_t laml_forest_inside_rows(laml_forest* f);
  * more than 32 sites, each level runs one wavefront per node over
  * inside_cpw[h] / outside_cpw[h] consecutive chunks of 64 sites; otherwise
  * the entries read 0 and are ignored.  top_level is the first level that the
- * fused top-level kernel runs (num_levels: none); level checkpointing
- * disables the fused kernel while it is on.  Shapes change the order of
+ * fused top-level kernel (LAML_PASS_LEVELS) or the tree walk
+ * (LAML_PASS_HYBRID) runs (num_levels: none); level checkpointing disables the
+ * fused kernel while it is on.  A forest is created with a top_level of its
+ * own for either mode, and laml_forest_get_shapes reports that of the current
+ * one; laml_forest_set_shapes sets both.  Shapes change the order of
  * floating-point sums over sites only.
  * No counterpart in the reference (its passes are Python loops); the values
  * come from the default heuristic or from laml_amd.autotune. */
@@ -190,7 +193,8 @@ int32_t laml_forest_fusion(laml_forest* f);
  * subtrees of up to 64 nodes that one wavefront walks as a whole (environment
  * LAML_CLADES sets that cap at forest creation, 0 turns them off), the same
  * bits again; other shapes or chains ask for their own kernels.
- * laml_forest_chains reports the flags the next passes use.
+ * laml_forest_chains reports the flags the next passes use (not
+ * LAML_CHAINS_OUTSIDE where the outside pass runs over clades).
  * No counterpart in the reference. */
 #define LAML_CHAINS_OUTSIDE 1
 #define LAML_CHAINS_INSIDE 2

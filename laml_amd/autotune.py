@@ -98,6 +98,9 @@ def autotune(F, d, nu, phi, reps=3, max_levels=8, verbose=False):
     the fastest.  Returns (plan, log) where log lists (description, ms)."""
     H = F.num_levels
     base = current_plan(F)
+    F.set_pass_mode(PASS_LEVELS)
+    top0 = F.get_shapes()[2]  # where level mode's fused top-level kernel starts
+    F.set_pass_mode(base.mode)
     log = []
 
     def measure(plan, tag):
@@ -110,7 +113,6 @@ def autotune(F, d, nu, phi, reps=3, max_levels=8, verbose=False):
 
     best = base
     best_ms = measure(base, "default")
-    top0 = base.top_level
     cands = [("levels, fused top", Plan(PASS_LEVELS, base.inside_cpw, base.outside_cpw, top0, False)),
              ("levels", Plan(PASS_LEVELS, base.inside_cpw, base.outside_cpw, H, False)),
              ("tree walk", Plan(PASS_TREES, base.inside_cpw, base.outside_cpw, top0, False))]

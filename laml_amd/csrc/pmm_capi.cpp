@@ -67,7 +67,7 @@ struct laml_forest {
   int W = 64;
   int h_top = 1 << 30;  // first level handled by the fused top-level kernels
   int h_top_default = 1 << 30;
-  int h_walk = 1 << 30;  // first level of the hybrid passes' walk, in the launch plan the forest was created with
+  int h_walk = 1 << 30;  // first level of the hybrid passes' walk
   int ckpt_L = 0;       // level-checkpoint segment length (0: all inside vectors stored)
   // per level: 64-site chunks one wavefront of the row kernels walks (W == 64)
   std::vector<int32_t> in_cpw, out_cpw;
@@ -109,7 +109,7 @@ struct laml_forest {
   laml::LdsPlan pb{};
   bool rows_ok = true, rows_unsure = false, alpha_unsure = false;
   struct {
-    int pass_mode, h_top, chains, chain_top_in, chain_top_out;
+    int pass_mode, h_top, h_walk, chains, chain_top_in, chain_top_out;
     bool fuse;
     std::vector<int32_t> in_cpw, out_cpw;
   } def{};
@@ -845,6 +845,7 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   F.rt_c = 1;
   f->def.pass_mode = f->pass_mode;
   f->def.h_top = f->h_top_default;
+  f->def.h_walk = f->h_walk;
   f->def.chains = f->chains;
   f->def.chain_top_in = f->chain_top_in;
   f->def.chain_top_out = f->chain_top_out;
@@ -1043,7 +1044,7 @@ int laml_forest_get_shapes(laml_forest* f, int32_t* inside_cpw, int32_t* outside
     if (inside_cpw) inside_cpw[h] = f->in_cpw.empty() ? 0 : f->in_cpw[h];
     if (outside_cpw) outside_cpw[h] = f->out_cpw.empty() ? 0 : f->out_cpw[h];
   }
-  if (top_level) *top_level = f->h_top_default;
+  if (top_level) *top_level = f->pass_mode == LAML_PASS_HYBRID ? f->h_walk : f->h_top_default;
   return LAML_OK;
 }
 
@@ -1090,7 +1091,11 @@ int laml_forest_get_chains(laml_forest* f, int32_t* which, int32_t* inside_top, 
 }
 
 static int chains_now(const laml_forest* f);
-int32_t laml_forest_chains(laml_forest* f) { return f ? chains_now(f) : -1; }
+static bool clades_now(const laml_forest* f);
+static bool out_clades_now(const laml_forest* f);
+int32_t laml_forest_chains(laml_forest* f) {
+  return f ? chains_now(f) & ~(clades_now(f) && out_clades_now(f) ? LAML_CHAINS_OUTSIDE : 0) : -1;
+}
 
 int laml_forest_set_shapes(laml_forest* f, const int32_t* inside_cpw, const int32_t* outside_cpw, int32_t top_level) {
   if (!f) return fail(LAML_EINVAL, "null forest");
@@ -1107,7 +1112,7 @@ int laml_forest_set_shapes(laml_forest* f, const int32_t* inside_cpw, const int3
       if (outside_cpw) f->out_cpw[h] = outside_cpw[h];
     }
   }
-  f->h_top_default = top_level;
+  f->h_top_default = f->h_walk = top_level;
   f->plan_version++;
   if (f->ckpt_L == 0) f->h_top = top_level;
   return LAML_OK;
@@ -1375,8 +1380,8 @@ static DevForest with_cherries(const laml_forest* f, const DevForest& F, bool fu
 // whether the passes run as k_problem: the forest was planned for it and its
 // launch plan is untouched
 static bool problem_now(const laml_forest* f) {
-  return f->pb_ok && f->ckpt_L == 0 && f->pass_mode == f->def.pass_mode && f->h_top_default == f->def.h_top &&
-         f->chains == f->def.chains && f->chain_top_in == f->def.chain_top_in &&
+  const bool top = f->pass_mode == LAML_PASS_HYBRID ? f->h_walk == f->def.h_walk : f->h_top_default == f->def.h_top;
+  return f->pb_ok && f->ckpt_L == 0 && f->pass_mode == f->def.pass_mode && top && f->chains == f->def.chains && f->chain_top_in == f->def.chain_top_in &&
          f->chain_top_out == f->def.chain_top_out && f->fuse == f->def.fuse && f->in_cpw == f->def.in_cpw &&
          f->out_cpw == f->def.out_cpw;
 }
@@ -1399,8 +1404,7 @@ static DevForest lds_view(const DevForest& F, const laml::LdsPlan& L) {
 // (a block per tree and site chunk) for the levels from it up
 static int hybrid_split(const laml_forest* f) {
   const int H = (int)f->level_off.size() - 1;
-  const bool def = f->pass_mode == LAML_PASS_HYBRID && f->h_top == f->def.h_top;
-  return std::max(1, std::min(def ? f->h_walk : f->h_top, H));
+  return std::max(1, std::min(f->pass_mode == LAML_PASS_HYBRID ? f->h_walk : f->h_top, H));
 }
 
 // which passes run the levels below their split as heavy-path chains
@@ -1582,12 +1586,11 @@ static const laml::CladePlan* pass_clades(const laml_forest* f) {
 
 // The same for the outside pass, whose chains and shapes must be the default
 // ones as well.
-static const laml::CladePlan* out_clades(const laml_forest* f) {
+static bool out_clades_now(const laml_forest* f) {
   return f->out_clades && f->chains == f->def.chains && f->chain_top_out == f->def.chain_top_out &&
-                 f->out_cpw == f->def.out_cpw
-             ? pass_clades(f)
-             : nullptr;
+         f->out_cpw == f->def.out_cpw;
 }
+static const laml::CladePlan* out_clades(const laml_forest* f) { return out_clades_now(f) ? pass_clades(f) : nullptr; }
 
 int laml_forest_pass_plan(laml_forest* f, laml_pass_plan* out) {
   if (!f || !out) return fail(LAML_EINVAL, "null argument");

@@ -568,9 +568,9 @@ class Forest(ForestLayout):
         return {k: getattr(p, k) for k, _ in p._fields_}
 
     def get_shapes(self):
-        """Launch shapes: (inside_cpw, outside_cpw, top_level); the cpw arrays
-        hold, per level, the 64-site chunks one wavefront walks (all 0 when
-        the rows hold at most 32 sites)."""
+        """Launch shapes: (inside_cpw, outside_cpw, top_level of the current
+        pass mode); the cpw arrays hold, per level, the 64-site chunks one
+        wavefront walks (all 0 when the rows hold at most 32 sites)."""
         H = self.num_levels
         a = np.zeros(H, dtype=np.int32)
         b = np.zeros(H, dtype=np.int32)
