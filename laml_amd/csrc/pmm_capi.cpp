@@ -1093,8 +1093,13 @@ int laml_forest_get_chains(laml_forest* f, int32_t* which, int32_t* inside_top, 
 static int chains_now(const laml_forest* f);
 static bool clades_now(const laml_forest* f);
 static bool out_clades_now(const laml_forest* f);
+static const laml::CladePlan* pass_clades(const laml_forest* f);
 int32_t laml_forest_chains(laml_forest* f) {
-  return f ? chains_now(f) & ~(clades_now(f) && out_clades_now(f) ? LAML_CHAINS_OUTSIDE : 0) : -1;
+  if (!f) return -1;
+  // (before its first call a forest has laid out no clades)
+  const laml::CladePlan* cl = pass_clades(f);
+  const bool out = clades_now(f) && out_clades_now(f) && (!cl || cl->out_num > 0);
+  return chains_now(f) & ~(out ? LAML_CHAINS_OUTSIDE : 0);
 }
 
 int laml_forest_set_shapes(laml_forest* f, const int32_t* inside_cpw, const int32_t* outside_cpw, int32_t top_level) {
@@ -1590,7 +1595,10 @@ static bool out_clades_now(const laml_forest* f) {
   return f->out_clades && f->chains == f->def.chains && f->chain_top_out == f->def.chain_top_out &&
          f->out_cpw == f->def.out_cpw;
 }
-static const laml::CladePlan* out_clades(const laml_forest* f) { return out_clades_now(f) ? pass_clades(f) : nullptr; }
+static const laml::CladePlan* out_clades(const laml_forest* f) {
+  const laml::CladePlan* cl = out_clades_now(f) ? pass_clades(f) : nullptr;
+  return cl && cl->out_num > 0 ? cl : nullptr;
+}
 
 int laml_forest_pass_plan(laml_forest* f, laml_pass_plan* out) {
   if (!f || !out) return fail(LAML_EINVAL, "null argument");
@@ -1737,7 +1745,7 @@ static void prepare_clades(laml_forest* f, hipStream_t s) {
   cl.count = (int)clades.size();
   for (const int4& c : clades) cl.largest = std::max(cl.largest, c.y);
   cl.num = (int)blocks.size();
-  cl.out_num = (int)oblocks.size();
+  cl.out_num = cl.count > laml::kCladeOutFill * (int)oblocks.size() || f->clade_cap > 0 ? (int)oblocks.size() : 0;
   // one allocation
   size_t bytes = 0;
   auto place = [&](size_t n) {

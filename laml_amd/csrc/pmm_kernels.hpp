@@ -336,7 +336,7 @@ struct CladePlan {
   const int4* clades = nullptr;  // offset into steps, steps, first batch, batches
   const CladeStep* steps = nullptr;
   CladeCoef* coef = nullptr;     // by step
-  int32_t out_num = 0;           // blocks of the outside pass
+  int32_t out_num = 0;           // blocks of the outside pass (0: it takes none, see kCladeOutFill)
   const int4* out_blocks = nullptr;
   const CladeOut* out_steps = nullptr;
   const int32_t* pos = nullptr;  // [N] place of a branch's coefficients: 2 step + child, -1 none
@@ -361,6 +361,13 @@ constexpr int64_t kCladeForest = 12288;
 // 300 leaves x 300 (60k pairs) 172 us, 203 by chains; of 10,000 x 300 (50k) 216
 // and 221, but its gradient, whose launches are not in a graph, 291 and 267.
 constexpr int64_t kCladeOutForest = 57344;
+// Nor where a block holds at most this many clades on average: its wavefronts
+// walk clades of one tree, and with few of them the CU idles.  E-step by clades
+// a block, clades / chains: 1 (2,048 trees of 20 leaves x 300) 794 / 472 us,
+// 1.5 (2,048 of 40 x 70) 538 / 328, 4 (1,024 of 60 x 70) 290 / 241, 5.5 (500 of
+// 100 x 130) 294 / 266, 7.4 (300 of 300 x 300) 576 / 612, 8 (300 of 100 x 70)
+// 169 / 176, 9.7 (100 of 400 x 200) 270 / 286.
+constexpr int kCladeOutFill = 6;
 // most LDS for a chunk's prior weights: 64 sites of 62 edit states (up to 21 KB
 // three blocks fit a CU)
 constexpr int kCladeMaxQ = 31 * 1024;

@@ -82,3 +82,29 @@ def test_first_call_takes_the_plan_it_lays_out(first, monkeypatch):
     plan = F.pass_plan()
     assert plan["outside_clades"] > 0 and plan["chain_plans"] == 0, plan
     F.close()
+
+
+@pytest.mark.parametrize("n,K,P,outside", [(40, 70, 1000, False), (20, 300, 640, False), (300, 300, 60, True)])
+def test_outside_clades_only_where_blocks_fill(n, K, P, outside, monkeypatch):
+    """Forests of many trees with few clades each keep outside chains; the
+    counts are those of level launches either way."""
+    base = [_problem("yule", n, K, 500 + i) for i in range(10)]
+    specs = [sim.problem_spec(*base[i % 10]) for i in range(P)]
+    got = []
+    for env in (None, "0"):
+        if env is not None:
+            monkeypatch.setenv("LAML_CLADES", env)
+        F = Forest(specs, device=torch.cuda.current_device())
+        d = _dev(F, F.lengths_to_level([np.maximum(base[i % 10][0].length, 0.005) for i in range(P)]))
+        nu, phi = _dev(F, [0.2] * P), _dev(F, [0.3] * P)
+        assert (F.num_nodes - F.num_leaves) * -(-K // 64) >= 57344
+        print("outside clades", n, K, P, env, flush=True)
+        counts, rt, nll = F.estep(d, nu, phi)
+        plan = F.pass_plan()
+        if env is None:
+            assert plan["inside_clades"] > 0 and bool(plan["outside_clades"]) == outside, plan
+            assert F.chains() == (0 if outside else 1) and plan["chain_plans"] == (0 if outside else 1), plan
+        got.append([x.cpu().numpy().copy() for x in (nll, counts, rt)])
+        F.close()
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
