@@ -533,16 +533,20 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
     while (ht - 1 >= 1 && d->level_off[ht] - d->level_off[ht - 1] <= top_max) --ht;
     f->h_top = ht;
     f->h_top_default = ht;
-    // The hybrid passes' walk takes more, the levels where each of its blocks
-    // (a tree and a site chunk, 16 wavefronts) meets few nodes: it then runs a
-    // level in 2 us, a launch in 4.6.  E-step by the largest such level (nodes
-    // a tree): 10,000 x 300 220 us at 24, 225 at 48; sixteen such trees 884 at
-    // 10, 908 at 3; 50 trees of 50-500 x 100 126 at 8, 128 at 16, 154 at 1; 300
-    // of 20-200 x 100 156 at 8, 168 at 16, 177 at 1.  With more blocks than the
-    // chip holds the launches are better (3,000 trees x 20: 604 and 823).
+    // The hybrid passes' walk takes the levels where each of its blocks (a tree
+    // and a site chunk, 16 wavefronts) meets few nodes: it then runs a level in
+    // 2 us, a launch in 4.6.  E-step (likelihood) by the largest such level:
+    // 300 x 30 78 us (34) at 32, 78 (35) at 24, 83 (34) at 64; 2,000 x 150 129
+    // (59) at 32, 132 (62) at 16, 136 (60) at 64; 10,000 x 300 220 at 24, 225
+    // at 48; two trees of 600 x 100 100 (48) at 48, 107 (51) at 24; four of 300
+    // x 70 87 (42) at 48, 91 (44) at 32.  With more trees, nodes a tree:
+    // sixteen of 10,000 x 300 884 at 10, 908 at 3; 50 of 50-500 x 100 126 at 8,
+    // 128 at 16, 154 at 1; 300 of 20-200 x 100 156 at 8, 168 at 16, 177 at 1.
+    // With more blocks than the chip holds the launches are better (3,000 trees
+    // x 20: 604 and 823).
     int hh = d->num_levels;
     const int64_t T = d->num_trees, chunks = (max_k + f->W - 1) / f->W;
-    const int walk_max = env || T * chunks > 1024 ? top_max : (int)std::max<int64_t>(24, 10 * T);
+    const int walk_max = env || T * chunks > 1024 ? top_max : T == 1 ? 32 : (int)std::max<int64_t>(48, 10 * T);
     while (hh - 1 >= 1 && d->level_off[hh] - d->level_off[hh - 1] <= walk_max) --hh;
     f->h_walk = hh;
     const char* pm = getenv("LAML_PASS_MODE");
