@@ -120,6 +120,7 @@ struct laml_forest {
   int clade_cap = 0;
   bool out_clades = false;          // and of the outside pass
   int64_t clade_q = 0;              // most prior weights of a 64-site chunk
+  int64_t clade_wait = 0;           // what the calls before the first clade plan earn towards it (see prepare_clades)
   std::deque<laml::CladePlan> clade_plans;
   std::deque<laml::ChainPlan> chain_plans;  // a deque: plans stay put when more are added
   std::vector<int32_t> h_heavy;  // heavy child of each node (-1: no internal child)
@@ -371,6 +372,33 @@ int validate(const laml_forest_desc* d, Derived& D) {
 
 }  // namespace
 
+// Arrays laid out for one allocation: those placed come from the host in one
+// copy, those reserved follow.  (An allocation and a synchronous copy each take
+// some 10 us, the time of a small forest's likelihood.)
+struct Packed {
+  std::vector<char> host;
+  size_t bytes = 0;
+  template <typename T>
+  size_t place(const std::vector<T>& v) {
+    const size_t at = host.size(), n = v.size() * sizeof(T);
+    host.resize(at + (n + 255) / 256 * 256);
+    if (n > 0) std::memcpy(host.data() + at, v.data(), n);
+    bytes = host.size();
+    return at;
+  }
+  size_t reserve(size_t n) {
+    const size_t at = bytes;
+    bytes += (n + 255) / 256 * 256;
+    return at;
+  }
+  int upload(laml_forest* f, char** m) const {
+    const int rc = f->alloc(m, bytes);
+    if (rc) return rc;
+    if (!host.empty()) LAML_HIP(hipMemcpy(*m, host.data(), host.size(), hipMemcpyHostToDevice));
+    return LAML_OK;
+  }
+};
+
 extern "C" {
 
 const char* laml_last_error(void) { return g_err.c_str(); }
@@ -436,14 +464,28 @@ static int upload_lds_plan(laml_forest* f, laml::LdsPlan& L, const std::vector<l
   }
   L.num_blocks = (int32_t)blks.size();
   L.slots = slots;
-  int rc;
-  if ((rc = f->upload(&L.blk, blks.data(), blks.size())) ||
-      (rc = f->upload(&L.int_base, int_base.data(), int_base.size())) ||
-      (rc = f->upload(&L.rec, rec.data(), rec.size())) ||
-      (rc = f->upload(&L.lvl_off, lvl_off.data(), lvl_off.size())) || (rc = f->alloc(&L.lcoef, (size_t)recs)) || (rc = f->alloc(&L.w, (size_t)entries)) ||
-      (rc = f->alloc(&L.q, (size_t)entries)) || (rc = f->alloc(&L.cpart, (size_t)N * 5 * slots)) ||
-      (rc = f->alloc(&L.rt_part, (size_t)N * slots)))
-    return rc;
+  Packed m;
+  const size_t o[9] = {m.place(blks),
+                       m.place(int_base),
+                       m.place(rec),
+                       m.place(lvl_off),
+                       m.reserve((size_t)recs * sizeof(laml::LdsCoef)),
+                       m.reserve((size_t)entries * sizeof(uint4)),
+                       m.reserve((size_t)entries * sizeof(double4)),
+                       m.reserve((size_t)N * 5 * slots * sizeof(double)),
+                       m.reserve((size_t)N * slots * sizeof(double))};
+  char* d = nullptr;
+  const int rc = m.upload(f, &d);
+  if (rc) return rc;
+  L.blk = reinterpret_cast<const laml::LdsBlk*>(d + o[0]);
+  L.int_base = reinterpret_cast<const int32_t*>(d + o[1]);
+  L.rec = reinterpret_cast<const laml::LdsRec*>(d + o[2]);
+  L.lvl_off = reinterpret_cast<const int2*>(d + o[3]);
+  L.lcoef = reinterpret_cast<laml::LdsCoef*>(d + o[4]);
+  L.w = reinterpret_cast<uint4*>(d + o[5]);
+  L.q = reinterpret_cast<double4*>(d + o[6]);
+  L.cpart = reinterpret_cast<double*>(d + o[7]);
+  L.rt_part = reinterpret_cast<double*>(d + o[8]);
   return LAML_OK;
 }
 
@@ -1617,13 +1659,27 @@ int laml_forest_pass_plan(laml_forest* f, laml_pass_plan* out) {
   return LAML_OK;
 }
 
+// whether s is being captured (or may be: the query failed)
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 // Builds the clade plan of the internal nodes below the current split, if
 // there is none yet (kept for the forest's life).  A call that is being
-// captured, or that finds no memory, runs level launches.
-static void prepare_clades(laml_forest* f, hipStream_t s) {
+// captured, or that finds no memory, runs level launches, and so do the first
+// calls on a forest below kCladeEager pairs: the plan takes longer than such a
+// call, so it is laid out once it would have paid for itself.  earns: what the
+// call would save, in likelihoods (kCladeEarn).
+static void prepare_clades(laml_forest* f, hipStream_t s, int64_t earns) {
   if (!clades_now(f) || pass_clades(f)) return;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return;
+  if (f->clade_cap <= 0 && (int64_t)(f->F.num_nodes - f->F.num_leaves) * f->F.max_chunks < laml::kCladeEager) {
+    f->clade_wait += earns;
+    if (f->clade_wait < laml::kCladeEarn) return;
+  }
+  if (capturing(s)) return;
   const int hs = hybrid_split(f);
   std::lock_guard<std::mutex> legacy_lock(g_legacy_mu);  // (as chain_plan)
   const int n = f->F.num_leaves, B = f->level_off[hs];
@@ -1750,34 +1806,13 @@ static void prepare_clades(laml_forest* f, hipStream_t s) {
   for (const int4& c : clades) cl.largest = std::max(cl.largest, c.y);
   cl.num = (int)blocks.size();
   cl.out_num = cl.count > laml::kCladeOutFill * (int)oblocks.size() || f->clade_cap > 0 ? (int)oblocks.size() : 0;
-  // one allocation
-  size_t bytes = 0;
-  auto place = [&](size_t n) {
-    const size_t o = bytes;
-    bytes += (n + 255) / 256 * 256;
-    return o;
-  };
-  const size_t o[9] = {place(blocks.size() * sizeof(int4)),
-                       place(clades.size() * sizeof(int4)),
-                       place(steps.size() * sizeof(laml::CladeStep)),
-                       place(pos.size() * sizeof(int32_t)),
-                       place(leaf_row.size() * sizeof(int32_t)),
-                       place(rest.size() * sizeof(int32_t)),
-                       place(steps.size() * sizeof(laml::CladeCoef)),
-                       place(oblocks.size() * sizeof(int4)),
-                       place(osteps.size() * sizeof(laml::CladeOut))};
+  Packed pk;
+  pk.host.reserve(steps.size() * 40 + pos.size() * 4 + leaf_row.size() * 4 + (clades.size() + rest.size()) * 48 + 4096);
+  const size_t o[9] = {pk.place(blocks),  pk.place(clades), pk.place(steps),
+                       pk.place(pos),     pk.place(leaf_row), pk.place(rest),
+                       pk.place(oblocks), pk.place(osteps), pk.reserve(steps.size() * sizeof(laml::CladeCoef))};
   char* m = nullptr;
-  auto up = [&](size_t at, const void* src, size_t n) {
-    return n == 0 || hipMemcpy(m + at, src, n, hipMemcpyHostToDevice) == hipSuccess;
-  };
-  if (f->alloc(&m, bytes) || !up(o[0], blocks.data(), blocks.size() * sizeof(int4)) ||
-      !up(o[1], clades.data(), clades.size() * sizeof(int4)) ||
-      !up(o[2], steps.data(), steps.size() * sizeof(laml::CladeStep)) ||
-      !up(o[3], pos.data(), pos.size() * sizeof(int32_t)) ||
-      !up(o[4], leaf_row.data(), leaf_row.size() * sizeof(int32_t)) ||
-      !up(o[5], rest.data(), rest.size() * sizeof(int32_t)) ||
-      !up(o[7], oblocks.data(), oblocks.size() * sizeof(int4)) ||
-      !up(o[8], osteps.data(), osteps.size() * sizeof(laml::CladeOut))) {
+  if (pk.upload(f, &m)) {
     (void)hipGetLastError();
     f->clades = false;
     return;
@@ -1788,9 +1823,9 @@ static void prepare_clades(laml_forest* f, hipStream_t s) {
   cl.pos = reinterpret_cast<const int32_t*>(m + o[3]);
   cl.leaf_row = reinterpret_cast<const int32_t*>(m + o[4]);
   cl.rest = reinterpret_cast<const int32_t*>(m + o[5]);
-  cl.coef = reinterpret_cast<laml::CladeCoef*>(m + o[6]);
-  cl.out_blocks = reinterpret_cast<const int4*>(m + o[7]);
-  cl.out_steps = reinterpret_cast<const laml::CladeOut*>(m + o[8]);
+  cl.out_blocks = reinterpret_cast<const int4*>(m + o[6]);
+  cl.out_steps = reinterpret_cast<const laml::CladeOut*>(m + o[7]);
+  cl.coef = reinterpret_cast<laml::CladeCoef*>(m + o[8]);
   f->clade_plans.push_back(std::move(cl));
 }
 
@@ -1804,8 +1839,8 @@ static const laml::ChainPlan* pass_chains(laml_forest* f, bool inside, int hs) {
 }
 
 // builds the chain plans the next passes use, outside any stream capture
-static int prepare_chains(laml_forest* f, hipStream_t s) {
-  prepare_clades(f, s);
+static int prepare_chains(laml_forest* f, hipStream_t s, int64_t earns) {
+  prepare_clades(f, s, earns);
   const int hs = hybrid_split(f);
   for (const bool inside : {true, false}) {
     if (!inside && out_clades(f)) continue;
@@ -1913,14 +1948,6 @@ static void pass_outside(laml_forest* f, const DevForest& F, bool with_root, con
   f->alpha_complete = !cp && !cl;
 }
 
-// whether s is being captured (or may be: the query failed)
-static bool capturing(hipStream_t s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
-  (void)hipGetLastError();
-  return true;
-}
-
 // after a call on s that leaves no rows
 static void left_no_rows(laml_forest* f, hipStream_t s) {
   f->rows_ok = f->alpha_complete = f->inside_fused = false;
@@ -1963,7 +1990,7 @@ int laml_nll(laml_forest* f, const double* d, const double* nu, const double* ph
     left_no_rows(f, s);
     return check_launch();
   }
-  int rc = prepare_chains(f, s);
+  int rc = prepare_chains(f, s, 1);
   if (rc) return rc;
   f->rows_ok = true;
   pass_coef(f, F, d, nu, nullptr, s);
@@ -1984,7 +2011,7 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
   // follows an E-step reads its rows (posteriors, quartet EM), and forming them
   // again costs more than the blocks save.  E-step and posteriors of one 250 x
   // 30 problem 173 us, 221 with a block's E-step (E-step alone 79 and 58).
-  int rc = prepare_chains(f, s);
+  int rc = prepare_chains(f, s, 2);
   if (rc) return rc;
   f->rows_ok = true;
   pass_coef(f, F, d, nu, nullptr, s);
@@ -2039,7 +2066,7 @@ int laml_outside(laml_forest* f, const double* phi, double* counts, double* rtil
   if (!f || !phi || !counts || !rtilde) return fail(LAML_EINVAL, "null argument");
   DeviceGuard guard(f->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rc = prepare_chains(f, s);
+  int rc = prepare_chains(f, s, 1);
   if (rc) return rc;
   DevForest F = f->F;
   F.phi = phi;
@@ -2054,7 +2081,7 @@ int laml_grad(laml_forest* f, const double* d, const double* nu, const double* p
   if (!f || !d || !nu || !phi || !grad_d || !grad_nu || !grad_phi) return fail(LAML_EINVAL, "null argument");
   DeviceGuard guard(f->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rc = prepare_chains(f, s);
+  int rc = prepare_chains(f, s, 1);
   if (rc) return rc;
   DevForest F = f->F;
   F.phi = phi;
@@ -2147,7 +2174,7 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
     }
     return LAML_OK;
   }
-  int prc = prepare_chains(f, s);
+  int prc = prepare_chains(f, s, 4 * ((int64_t)max_iter + 1));
   if (prc) return prc;
   laml::run_em_reset(em, P, s);
   // The EM step is captured once into a HIP graph and replayed: its kernel

@@ -357,6 +357,13 @@ constexpr int kCladeMin = 16, kCladeCap = 64;
 // 500 (16k pairs) 63 us, 76 by levels; 1,000 x 500 (8k) 48 and 53, but a forest
 // that is solved once and dropped does not earn its plan back.
 constexpr int64_t kCladeForest = 12288;
+// Forests below kCladeEager pairs lay clades out once their calls would have
+// saved the time: the plan takes 0.11 ms (4,000 leaves x 300, 20k pairs), a
+// likelihood saves 12 us of 82 there, an E-step 30, an EM step 55.  From
+// kCladeEager pairs on (where outside chains had their plan to lay out) at
+// once.
+constexpr int64_t kCladeEager = 32768;
+constexpr int64_t kCladeEarn = 10;
 // And of at least this many in the outside pass as well: E-step of 300 trees of
 // 300 leaves x 300 (60k pairs) 172 us, 203 by chains; of 10,000 x 300 (50k) 216
 // and 221, but its gradient, whose launches are not in a graph, 291 and 267.

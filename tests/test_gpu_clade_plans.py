@@ -108,3 +108,37 @@ def test_outside_clades_only_where_blocks_fill(n, K, P, outside, monkeypatch):
         F.close()
     for a, b in zip(*got):
         np.testing.assert_array_equal(a, b)
+
+
+def test_clades_of_middle_forests_once_they_pay():
+    """A forest of 12,288 to 32,768 (node, chunk) pairs lays its clades out when
+    its calls would have saved the time, and gives the same bits before and
+    after; a call under capture lays out nothing."""
+    t, Q, codes = _problem("yule", 4000, 300, 9)
+    spec = sim.problem_spec(t, Q, codes)
+    F = Forest([spec], device=torch.cuda.current_device())
+    assert 12288 <= (F.num_nodes - F.num_leaves) * 5 < 32768
+    d, nu, phi = _dev(F, F.lengths_to_level([np.maximum(t.length, 0.005)])), _dev(F, [0.2]), _dev(F, [0.3])
+
+    def likelihood():
+        out = F.nll(d, nu, phi, site_llh=True).cpu().numpy().copy()
+        return np.concatenate([out, F.site_llh.cpu().numpy()])
+
+    first = likelihood()
+    assert F.pass_plan()["inside_clades"] == 0
+    counts = [x.cpu().numpy().copy() for x in F.estep(d, nu, phi)]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        for _ in range(12):
+            F.nll(d, nu, phi)
+    assert F.pass_plan()["inside_clades"] == 0
+    for _ in range(12):
+        np.testing.assert_array_equal(likelihood(), first)
+    assert F.pass_plan()["inside_clades"] > 0
+    for a, b in zip(F.estep(d, nu, phi), counts):
+        np.testing.assert_array_equal(a.cpu().numpy(), b)
+    F.close()
+    F = Forest([spec], device=torch.cuda.current_device())
+    F.em(d.clone(), nu.clone(), phi.clone(), 3, 0.0)
+    assert F.pass_plan()["inside_clades"] > 0
+    F.close()
