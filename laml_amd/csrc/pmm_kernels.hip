@@ -3590,7 +3590,7 @@ __device__ __forceinline__ const PbArgs& pb_args() {
 }
 __global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
   extern __shared__ __align__(16) char lds[];
-  __shared__ double sh[2][5 * (kLdsThreads / 64)];
+  __shared__ double sh[2][6 * (kLdsThreads / 64)];
   const int p = (int)blockIdx.x;
   const int t = p;  // one tree a problem
   const int what = pb_args().what;
@@ -3699,18 +3699,22 @@ __global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
           nu_term(F.nu_a[pos], F.nu_b[pos], F.nu_d[pos], xx, n);
         }
       }
-      double third = evals == 0 ? (bad != 0.0 ? INFINITY : rt) : 0.0;
-      double v[5] = {n.g, n.g1, n.g2, n.g3, third};
-      lds_sum<5>(v, sh[1 - (evals & 1)]);
-      n = NuSum{v[0], v[1], v[2], v[3]};
-      third = v[4];
+      double* const s = sh[1 - (evals & 1)];
       if (evals == 0) {
-        bad = isfinite(third) ? 0.0 : 1.0;
+        double v[6] = {n.g, n.g1, n.g2, n.g3, rt, bad};
+        lds_sum<6>(v, s);
+        n = NuSum{v[0], v[1], v[2], v[3]};
+        rt = v[4];
+        bad = v[5];
         if (flags & 1u) {
-          pv = third / (F.prob_nobs[p] + third);
+          pv = rt / (F.prob_nobs[p] + rt);
           if (fabs(pv) < F.prob_phimin[p]) pv = 0.0;
         }
         if (!opt_nu) break;
+      } else {
+        double v[4] = {n.g, n.g1, n.g2, n.g3};
+        lds_sum<4>(v, s);
+        n = NuSum{v[0], v[1], v[2], v[3]};
       }
       double xn;
       fin = nu_step(xx, n, lo, hi, xn);
