@@ -2188,7 +2188,7 @@ __device__ __forceinline__ double branch_length(const DevForest& F, double (&s)[
 // branch lengths (EM_solver.py:392-407); its derivative
 // h'(x) = sum_v d_v (b_v / expm1(x d_v) - a_v) sums over every branch of the
 // problem.  Warm-started solves take one evaluation of h' and its derivatives,
-// two when nu moves by more than kTaylorDone (Newton steps to 1e-12 took three
+// two when nu moves by more than kNuDone x (Newton steps to 1e-12 took three
 // to five).  Each problem's branches are split into spans of kNuThreads, a
 // block each, in two launches of an evaluation each, which write their spans'
 // sums; the next kernel's blocks all add the sums of their problem (in an

@@ -17,8 +17,11 @@ __device__ __forceinline__ double rcp_normal(double x) {
 
 // 1 / expm1(y) for y > 0.  Past 700 the quotient is below 1e-304, which no sum
 // of the solves resolves, and from 709.8 on expm1 is infinite, of which the
-// Newton steps of rcp_normal make inf * 0: 0 there, as the division gives.
-__device__ __forceinline__ double rcp_expm1(double y) { return y > 700.0 ? 0.0 : rcp_normal(expm1(y)); }
+// Newton steps of rcp_normal would make inf * 0: the value at 700 there.
+// (fmin drops a NaN; every caller has one beside it then, from a count, a
+// length or nu itself.  A comparison and a selection in its place cost an EM
+// step of 250 x 30 3 %.)
+__device__ __forceinline__ double rcp_expm1(double y) { return rcp_normal(expm1(fmin(y, 700.0))); }
 
 constexpr double kEpsNu = 1e-5;   // EM_solver.py:307 eps_nu
 constexpr double kEpsS = 1e-6;    // EM_solver.py:307 eps_s
@@ -28,11 +31,15 @@ constexpr double kEpsS = 1e-6;    // EM_solver.py:307 eps_s
 // nearly linear.  From g and its first three derivatives at x: the root of G's
 // cubic Taylor polynomial, as a step from x (a plain Newton step where the
 // polynomial gives none near).  The step's own error is of the fourth order:
-// one of at most kTaylorDone x ends a solve (the functions vary on the scale
-// of 2 pi in d and in nu d, so the error is below 1e-15 x).  A warm-started
-// solve takes one or two evaluations where Newton steps to 1e-13 x took four
+// one of at most kBranchDone x or kNuDone x ends a solve.  Over two million
+// random branch objectives the roots are then within 4.7e-16 of the true ones
+// in the default box and 2.3e-15 in [1e-6, 1000], Newton steps to 1e-13 x
+// within 4.7e-16 and 4.7e-14 (ending at 1e-4 x: 1.9e-15 and 1.3e-14); over
+// 20,000 nu problems within 3.3e-16, Newton steps to 1e-12 x within 3.6e-16.  A
+// warm-started solve takes one or two evaluations where Newton steps took four
 // to seven.
-constexpr double kTaylorDone = 1e-4;
+constexpr double kBranchDone = 6e-5;
+constexpr double kNuDone = 1e-4;
 __device__ __forceinline__ double taylor_step(double x, double g, double g1, double g2, double g3) {
   const double c0 = x * g, c1 = fma(x, g1, g), c2 = fma(0.5 * x, g2, g1), c3 = fma(x * (1.0 / 6.0), g3, 0.5 * g2);
   const double t0 = -c0 / c1;
@@ -102,7 +109,7 @@ __device__ double solve_branch(const BranchObj& o, double dmin, double dmax, dou
     }
     const double step = taylor_step(x, b.g, b.g1, b.g2, b.g3);
     double xn = x + step;
-    if (fabs(step) <= kTaylorDone * x && xn >= dmin && xn <= dmax) return xn;
+    if (fabs(step) <= kBranchDone * x && xn >= dmin && xn <= dmax) return xn;
     if (!(xn > lo && xn < hi)) {
       // out of the bracket: the optimum is at a bound whose slope points out
       if (!lo_known) {
@@ -146,7 +153,7 @@ __device__ __forceinline__ bool nu_step(double x, const NuSum& n, double& lo, do
   const double step = taylor_step(x, n.g, n.g1, n.g2, n.g3);
   const double top = fmin(hi, 1.0);
   xn = x + step;
-  if (fabs(step) <= kTaylorDone * x) {
+  if (fabs(step) <= kNuDone * x) {
     xn = fmin(fmax(xn, 0.0), 1.0);
     return true;
   }

@@ -44,7 +44,7 @@ void branches(int n, const double* A, const double* S1, const double* B, const d
     LD lo = dmin, hi = dmax;
     if (!(slope(o, lo) > 0)) { want[i] = dmin; continue; }
     if (!(slope(o, hi) < 0)) { want[i] = dmax; continue; }
-    for (int k = 0; k < 200; ++k) {
+    for (int k = 0; k < 120; ++k) {
       const LD m = 0.5L * (lo + hi);
       if (slope(o, m) > 0) lo = m; else hi = m;
     }

@@ -43,6 +43,21 @@ def test_branch_from_the_lower_bound_of_the_fastem_box():
         np.testing.assert_allclose(got, want, rtol=1e-12)
 
 
+@pytest.mark.parametrize("spread", [0.02, 1.0])
+def test_branch_solve_to_rounding(spread):
+    """Warm starts in the default box: within eight roundings (2^-53 each) of the
+    true root, whose slope times length is at least the objective's constant
+    term (an error in either is not amplified): three in the reciprocal, two in
+    the slope, one in the step, one in the result, one in the reference."""
+    A, S1, B, nu = _objectives(60000, 11)
+    _, want = ref.branches(A, S1, B, nu, 0.005, 10.0, 0.05)
+    sel = (want > 0.005) & (want < 10.0)
+    A, S1, B, nu, want = (np.ascontiguousarray(x[sel]) for x in (A, S1, B, nu, want))
+    rng = np.random.default_rng(12)
+    got, _ = ref.branches(A, S1, B, nu, 0.005, 10.0, want * np.exp(rng.uniform(-spread, spread, len(want))))
+    np.testing.assert_allclose(got, want, rtol=8 * 2.0 ** -53)
+
+
 @pytest.mark.parametrize("long_length", [0.5, 600.0, 709.0, 712.0, 1e3, 1e5])
 @pytest.mark.parametrize("nu0", [0.0, 1e-6, 0.3, 0.999, 1.0])
 def test_nu_solve_with_a_long_branch(long_length, nu0):
