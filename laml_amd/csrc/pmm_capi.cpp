@@ -2036,43 +2036,44 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
   return check_launch();
 }
 
-// the outside pass over the state of the last call: from its rows, or with
-// the inside pass again where it left none (a captured call may be replayed
-// after another one that did).  Returns the view of F that holds the partial
-// counts.
-static DevForest outside_again(laml_forest* f, const DevForest& F, const double* phi, hipStream_t s) {
-  if (problem_now(f) && (!f->rows_ok || f->rows_unsure || capturing(s))) {
-    const DevForest G = lds_view(F, f->pb);
-    EmState none{};
-    laml::run_problem(G, f->pb, f->TW, nullptr, nullptr, const_cast<double*>(phi), nullptr, nullptr, nullptr, none, 1,
-                      0, 0.0, laml::kPbOut, s);
-    return G;
-  }
+// whether an outside pass of its own runs in blocks, the inside pass again
+// first: where the last call left no rows (a captured call may be replayed
+// after another one that did)
+static bool outside_in_blocks(const laml_forest* f, hipStream_t s) {
+  return problem_now(f) && (!f->rows_ok || f->rows_unsure || capturing(s));
+}
+
+// the outside pass over the state of the last call, from its rows
+static void outside_again(laml_forest* f, DevForest F, hipStream_t s) {
   ensure_rows(f, F, s);
-  DevForest G = F;
   if (const laml::CladePlan* cl = pass_clades(f)) {
-    G.clade_coef = cl->coef;
-    G.clade_pos = cl->pos;
+    F.clade_coef = cl->coef;
+    F.clade_pos = cl->pos;
     // (the resident coefficients are those of any earlier call, a captured one
     // included)
-    if (out_clades(f)) laml::run_clade_coef(G, s);
+    if (out_clades(f)) laml::run_clade_coef(F, s);
   }
-  pass_outside(f, G, true, nullptr, s);
+  pass_outside(f, F, true, nullptr, s);
   left_outside(f, s);
-  return F;
 }
 
 int laml_outside(laml_forest* f, const double* phi, double* counts, double* rtilde, void* stream) {
   if (!f || !phi || !counts || !rtilde) return fail(LAML_EINVAL, "null argument");
   DeviceGuard guard(f->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rc = prepare_chains(f, s, 1);
-  if (rc) return rc;
   DevForest F = f->F;
   F.phi = phi;
-  const DevForest G = outside_again(f, F, phi, s);
-  laml::run_counts(G, counts, s);
-  laml::run_rtilde(G, rtilde, nullptr, s);
+  if (outside_in_blocks(f, s)) {
+    F = lds_view(F, f->pb);
+    laml::run_problem(F, f->pb, f->TW, nullptr, nullptr, const_cast<double*>(phi), nullptr, nullptr, nullptr,
+                      EmState{}, 1, 0, 0.0, laml::kPbOut, s);
+  } else {
+    int rc = prepare_chains(f, s, 1);
+    if (rc) return rc;
+    outside_again(f, F, s);
+  }
+  laml::run_counts(F, counts, s);
+  laml::run_rtilde(F, rtilde, nullptr, s);
   return check_launch();
 }
 
@@ -2081,12 +2082,18 @@ int laml_grad(laml_forest* f, const double* d, const double* nu, const double* p
   if (!f || !d || !nu || !phi || !grad_d || !grad_nu || !grad_phi) return fail(LAML_EINVAL, "null argument");
   DeviceGuard guard(f->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rc = prepare_chains(f, s, 1);
-  if (rc) return rc;
   DevForest F = f->F;
   F.phi = phi;
-  const DevForest G = outside_again(f, F, phi, s);
-  laml::run_grad(G, d, nu, phi, grad_d, grad_nu, grad_phi, s);
+  if (outside_in_blocks(f, s)) {
+    laml::run_problem(F, f->pb, f->TW, const_cast<double*>(d), const_cast<double*>(nu), const_cast<double*>(phi),
+                      nullptr, nullptr, nullptr, EmState{}, 1, 0, 0.0, laml::kPbOut | laml::kPbGrad, s,
+                      laml::GradOut{grad_d, grad_nu, grad_phi});
+    return check_launch();
+  }
+  int rc = prepare_chains(f, s, 1);
+  if (rc) return rc;
+  outside_again(f, F, s);
+  laml::run_grad(F, d, nu, phi, grad_d, grad_nu, grad_phi, s);
   return check_launch();
 }
 

@@ -2438,6 +2438,20 @@ __global__ void __launch_bounds__(kNuFinishThreads) k_nu_finish(DevForest F, con
 // n_obs counts leaf entries observed as 0 or an edit (an explicit -1 entry
 // does not depend on phi); Rt sums P(leaf not silenced | D) over '?' entries.
 // ---------------------------------------------------------------------------
+// a branch of length dv with counts s: dlogL/dd, and its part of dlogL/dnu but
+// -dv (S0 + S1 + S3)
+__device__ __forceinline__ double grad_length(const double (&s)[5], double dv, double x) {
+  double g = -(1.0 + x) * s[0] + s[1] * (1.0 / expm1(dv) - x) - x * s[3];
+  if (s[2] + s[4] != 0.0) g += (s[2] + s[4]) * x / expm1(x * dv);
+  return g;
+}
+__device__ __forceinline__ double grad_nu_part(double b, double dv, double x) {
+  return b != 0.0 ? b * dv / expm1(x * dv) : 0.0;
+}
+__device__ __forceinline__ double grad_phi_of(double nobs, double rt, double ph) {
+  return nobs / (1.0 - ph) - (rt != 0.0 ? rt / ph : 0.0);
+}
+
 __global__ void k_grad_branch(DevForest F, const double* __restrict__ d, const double* __restrict__ nu,
                               double* __restrict__ grad_d) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2449,10 +2463,8 @@ __global__ void k_grad_branch(DevForest F, const double* __restrict__ d, const d
   for (int c = 0; c < C; ++c)
 #pragma unroll
     for (int j = 0; j < 5; ++j) s[j] += F.cpart[v * F.cp_v + c * F.cp_c + j];
-  const double dv = d[v], x = nu[p];
-  double g = -(1.0 + x) * s[0] + s[1] * (1.0 / expm1(dv) - x) - x * s[3];
-  if (s[2] + s[4] != 0.0) g += (s[2] + s[4]) * x / expm1(x * dv);
-  grad_d[v] = -g;
+  const double dv = d[v];
+  grad_d[v] = -grad_length(s, dv, nu[p]);
   F.nu_a[F.node_pos[v]] = s[0] + s[1] + s[3];
   F.nu_b[F.node_pos[v]] = s[2] + s[4];
   F.nu_d[F.node_pos[v]] = dv;
@@ -2468,16 +2480,14 @@ __global__ void __launch_bounds__(kRedThreads) k_grad_problem(DevForest F, const
   double g = 0.0;
   for (int i = F.prob_node_off[p] + threadIdx.x; i < F.prob_node_off[p + 1]; i += kRedThreads) {
     const double dv = F.nu_d[i];
-    const double b = F.nu_b[i];
     g -= dv * F.nu_a[i];
-    if (b != 0.0) g += b * dv / expm1(x * dv);
+    g += grad_nu_part(F.nu_b[i], dv, x);
   }
   g = block_sum<kRedThreads>(g, sh);
   const double rt = problem_rtilde(F, p, sh);
   if (threadIdx.x == 0) {
     grad_nu[p] = -g;
-    const double ph = phi[p];
-    grad_phi[p] = F.prob_nobs_phi[p] / (1.0 - ph) - (rt != 0.0 ? rt / ph : 0.0);
+    grad_phi[p] = grad_phi_of(F.prob_nobs_phi[p], rt, phi[p]);
   }
 }
 
@@ -3578,6 +3588,7 @@ struct PbArgs {
   int max_steps, max_iter;
   double tol;
   int what;
+  GradOut grad;
 };
 // The kernel's arguments, read where they are used: from an address that the
 // compiler cannot tell from the last one, so that it loads again instead of
@@ -3637,7 +3648,26 @@ __global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
     const DevForest& F = A.F;
     if (!(what & kPbEm)) {
       if (threadIdx.x == 0 && A.nll) A.nll[p] = -llh;
-      if (out) lds_flush(F, x, t, 0);
+      if (what & kPbGrad) {
+        double g[2] = {0.0, 0.0};  // dlogL/dnu, the dropout sum
+        for (int r = (int)threadIdx.x; r < nbr; r += kLdsThreads) {
+          const int v = lds_branch_node(F, x, t, r);
+          const double dv = A.d[v];
+          double s[5];
+          lds_branch_counts(x, r, s);
+          A.grad.d[v] = -grad_length(s, dv, nv);
+          g[0] -= dv * (s[0] + s[1] + s[3]);
+          g[0] += grad_nu_part(s[2] + s[4], dv, nv);
+          if (r < nbr - 1 && !(r & 1)) g[1] += lds_slot(x, r >> 1, 0)[10];
+        }
+        lds_sum<2>(g, sh[1]);
+        if (threadIdx.x == 0) {
+          A.grad.nu[p] = -g[0];
+          A.grad.phi[p] = grad_phi_of(F.prob_nobs_phi[p], g[1], pv);
+        }
+      } else if (out) {
+        lds_flush(F, x, t, 0);
+      }
       return;
     }
     const EmState& em = A.em;
@@ -3787,10 +3817,10 @@ void run_lds_tables(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, hi
 
 void run_problem(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, double* d, double* nu, double* phi,
                  double* nll, double* site_llh_out, int32_t* iters_out, const EmState& em, int max_steps,
-                 int max_iter, double tol, int what, hipStream_t s) {
+                 int max_iter, double tol, int what, hipStream_t s, GradOut grad) {
   static const bool once = (allow_lds(k_problem), true);
   (void)once;
-  const PbArgs a{F, L, TW, d, nu, phi, nll, site_llh_out, iters_out, em, max_steps, max_iter, tol, what};
+  const PbArgs a{F, L, TW, d, nu, phi, nll, site_llh_out, iters_out, em, max_steps, max_iter, tol, what, grad};
   hipLaunchKernelGGL(k_problem, dim3(F.num_problems), dim3(kLdsThreads), L.lds_bytes, s, a);
 }
 

@@ -231,11 +231,14 @@ void run_lds_tables(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, hi
 // What k_problem does, a block per problem: branch coefficients from d and nu
 // (else those of the last call), the outside pass with counts (else inside
 // and likelihood alone), EM steps (at most max_steps, of the max_iter that
-// the run has in all)
-constexpr int kPbCoef = 1, kPbOut = 2, kPbEm = 4;
+// the run has in all), the gradient from the counts
+constexpr int kPbCoef = 1, kPbOut = 2, kPbEm = 4, kPbGrad = 8;
+struct GradOut {
+  double *d, *nu, *phi;
+};
 void run_problem(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, double* d, double* nu, double* phi,
                  double* nll, double* site_llh_out, int32_t* iters_out, const EmState& em, int max_steps,
-                 int max_iter, double tol, int what, hipStream_t s);
+                 int max_iter, double tol, int what, hipStream_t s, GradOut grad = {});
 void run_labels(const DevForest& F, const std::vector<int32_t>& lvl, int W, hipStream_t s);
 // the prior-weight rows qleaf / qint from the codes and labels (after run_labels)
 void run_qrows(const DevForest& F, double* qleaf, double* qint, hipStream_t s);
