@@ -203,7 +203,7 @@ int laml_forest_set_chains(laml_forest* f, int32_t which, int32_t inside_top, in
 /* How the next passes run, and what has been laid out for them so far (tests
  * ask for it; no counterpart in the reference). */
 typedef struct {
-  int32_t blocks;          /* 1: likelihoods and EM steps in whole-problem blocks */
+  int32_t blocks;          /* 1: EM steps, and likelihoods of up to 1,024 problems, in whole-problem blocks */
   int32_t walk_level;      /* first level of the tree walk or the fused top-level kernel */
   int32_t inside_clades;   /* clades of the inside pass (0: none, or not laid out yet) */
   int32_t outside_clades;  /* clades of the outside pass */

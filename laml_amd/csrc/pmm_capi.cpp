@@ -1984,7 +1984,7 @@ int laml_nll(laml_forest* f, const double* d, const double* nu, const double* ph
   DevForest F = f->F;
   F.phi = phi;
   EmState none{};
-  if (problem_now(f)) {
+  if (problem_now(f) && f->F.num_problems <= laml::kPbMaxSingle) {
     laml::run_problem(lds_view(F, f->pb), f->pb, f->TW, const_cast<double*>(d), const_cast<double*>(nu),
                       const_cast<double*>(phi), nll, site_llh, nullptr, none, 1, 0, 0.0, laml::kPbCoef, s);
     left_no_rows(f, s);

@@ -224,8 +224,13 @@ constexpr int kLdsSlotSites = 8;
 // the general passes overtake it when blocks are many and tiny (EM step, block
 // / general: 256 problems of 250 x 30 89 / 308 us, 1,024 of them 308 / 658,
 // 2,048 of 100 x 20 373 / 576, 4,096 of 60 x 16 720 / 588).
+// A likelihood (with its gradient) goes through blocks up to kPbMaxSingle: 1,024
+// problems of 10 x 8 44 (122) us, 45 (113) in the general passes, of 60 x 40
+// 70 (213) and 108 (264), of 120 x 60 96 (301) and 149 (370); 1,280 of them 55
+// (151) and 45 (106), 85 (259) and 85 (216), 136 (411) and 118 (334).
 constexpr int kPbMaxSites = 64;
 constexpr int kPbMaxProblems = 2048;
+constexpr int kPbMaxSingle = 1024;
 // the cell tables of an LDS plan (after run_labels)
 void run_lds_tables(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, hipStream_t s);
 // What k_problem does, a block per problem: branch coefficients from d and nu
