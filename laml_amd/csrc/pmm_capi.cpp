@@ -584,11 +584,14 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
     // x 70 87 (42) at 48, 91 (44) at 32.  With more trees, nodes a tree:
     // sixteen of 10,000 x 300 884 at 10, 908 at 3; 50 of 50-500 x 100 126 at 8,
     // 128 at 16, 154 at 1; 300 of 20-200 x 100 156 at 8, 168 at 16, 177 at 1.
-    // With more blocks than the chip holds the launches are better (3,000 trees
-    // x 20: 604 and 823).
+    // With more blocks than the chip holds (two a CU) the launches are better:
+    // at 768 blocks 185 us by launches, 233 by the walk (256 trees of 100 x
+    // 130), at 640 172 and 178 (213 of them), at 510 161 and 148; rows of at
+    // most 32 sites 169 and 159 at 768 (60 x 16), 188 and 199 at 1,024.
     int hh = d->num_levels;
     const int64_t T = d->num_trees, chunks = (max_k + f->W - 1) / f->W;
-    const int walk_max = env || T * chunks > 1024 ? top_max : T == 1 ? 32 : (int)std::max<int64_t>(48, 10 * T);
+    const bool many = T * chunks > (f->W == 64 ? 512 : 768);
+    const int walk_max = env || many ? top_max : T == 1 ? 32 : (int)std::max<int64_t>(48, 10 * T);
     while (hh - 1 >= 1 && d->level_off[hh] - d->level_off[hh - 1] <= walk_max) --hh;
     f->h_walk = hh;
     const char* pm = getenv("LAML_PASS_MODE");
