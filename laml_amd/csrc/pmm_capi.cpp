@@ -106,6 +106,7 @@ struct laml_forest {
   // are not trusted any more (rows_unsure, alpha_unsure).  The branch
   // coefficients are always those of the last call, replayed or not.
   bool pb_ok = false;
+  int lds_max = 0;  // LDS that a block of the LDS kernels may take
   laml::LdsPlan pb{};
   bool rows_ok = true, rows_unsure = false, alpha_unsure = false;
   struct {
@@ -505,7 +506,7 @@ static int plan_problems(laml_forest* f, int max_k, const std::vector<int32_t>& 
     b.k0 = 0;
     b.sb = (f->tree_nsites[t] + R - 1) / R * R;
     for (int i = lvl_base[t] + 1; i < lvl_base[t + 1]; ++i) b.nint += lvl_cnt[i];
-    if (b.nint < 1 || lds_need(b, lvl_base) > laml::kLdsMaxBytes) return LAML_OK;
+    if (b.nint < 1 || lds_need(b, lvl_base) > f->lds_max) return LAML_OK;
     b.tab = tab;
     tab += lds_entries(b, lvl_base, lvl_cnt);
     blks.push_back(b);
@@ -558,6 +559,7 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   {
     const char* env = getenv("LAML_EM_GRAPH");
     f->use_graph = !(env && env[0] == '0');
+    f->lds_max = laml::max_lds(device);
     // private capture stream (default priority)
     if (hipStreamCreateWithFlags(&f->cap_stream, hipStreamNonBlocking) != hipSuccess) {
       delete f;
@@ -849,7 +851,7 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
         qmax = std::max<int64_t>(qmax, qo[std::min(k + 64, d->tree_nsites[t])] - qo[k]);
       }
     f->clade_q = qmax;
-    f->out_clades = !env && (cenv || units >= laml::kCladeOutForest);
+    f->out_clades = !env && f->lds_max > 0 && (cenv || units >= laml::kCladeOutForest);
     f->clades = f->W == 64 && qmax * 8 <= laml::kCladeMaxQ && (cenv ? f->clade_cap > 0 : units >= laml::kCladeForest);
   }
   f->h_row_off = row_off;
@@ -1319,7 +1321,8 @@ int laml_forest_set_ultrametric(laml_forest* f, const laml_ultra_desc* u) {
     // without the packed model every solve is the barrier method's
     if (odd) std::fill(cls_off.begin(), cls_off.end(), 0);
     U.lds_bytes = (int32_t)std::min<int64_t>(odd ? 0 : max_lds, std::numeric_limits<int32_t>::max());
-    const bool big = U.lds_bytes > laml::kLdsMaxBytes;
+    const bool big = U.lds_bytes > f->lds_max;
+    if (big) U.lds_bytes = std::numeric_limits<int32_t>::max();
     if ((rc = f->uupload(&U.pk_cls_off, cls_off.data(), cls_off.size())) ||
         (rc = f->uupload(&U.pk_cls, cls.data(), cls.size())) || (rc = f->uupload(&U.pk_lvl, lvl.data(), lvl.size())) ||
         (rc = f->uupload(&U.pk_link, link.data(), link.size())) ||

@@ -31,13 +31,6 @@ __device__ __forceinline__ Coef branch_coef(double dv, double nv) {
   return c;
 }
 
-// a block may use all of a CU's LDS
-template <typename K>
-static void allow_lds(K kernel) {
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            kLdsMaxBytes);
-}
-
 // branch v's coefficients to its place in the steps of the clade plan
 __device__ __forceinline__ void clade_coef(const DevForest& F, int v, const Coef& c) {
   const int q = F.clade_pos[v];
@@ -3818,8 +3811,6 @@ void run_lds_tables(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, hi
 void run_problem(const DevForest& F, const LdsPlan& L, const TreeWalk& TW, double* d, double* nu, double* phi,
                  double* nll, double* site_llh_out, int32_t* iters_out, const EmState& em, int max_steps,
                  int max_iter, double tol, int what, hipStream_t s, GradOut grad) {
-  static const bool once = (allow_lds(k_problem), true);
-  (void)once;
   const PbArgs a{F, L, TW, d, nu, phi, nll, site_llh_out, iters_out, em, max_steps, max_iter, tol, what, grad};
   hipLaunchKernelGGL(k_problem, dim3(F.num_problems), dim3(kLdsThreads), L.lds_bytes, s, a);
 }
@@ -4085,8 +4076,6 @@ __global__ void __launch_bounds__(kUltraThreads) k_ultra(DevForest F, UltraDev U
 
 void run_ultra(const DevForest& F, const UltraDev& U, double* d, const double* nu, const int32_t* done,
                hipStream_t s) {
-  static const bool once = (allow_lds(k_ultra<true>), true);
-  (void)once;
   if (U.lds_bytes <= kLdsMaxBytes)
     hipLaunchKernelGGL(k_ultra<true>, dim3(F.num_problems), dim3(kUltraThreads), U.lds_bytes, s, F, U, d, nu, done);
   else
@@ -4311,8 +4300,6 @@ void run_outside_clades(const DevForest& F, const CladePlan& cl, const int32_t* 
   }
   if (cl.out_num == 0) return;
   const size_t lds = (size_t)kCladeOutWaves * kOutLdsBytes + cl.q_bytes;
-  static const bool once = (allow_lds(k_outside_clade), true);
-  (void)once;
   hipLaunchKernelGGL(k_outside_clade, dim3((unsigned)((cl.out_num + 7) / 8 * 8 * F.max_chunks)),
                      dim3(64 * kCladeOutWaves), lds, s, F, cl.out_blocks, cl.clades, cl.out_steps, cl.out_num, done);
 }
@@ -4449,6 +4436,23 @@ int post_scratch(int device, double** out) {
   }
   *out = it->second;
   return 0;
+}
+
+int max_lds(int device) {
+  static std::mutex mu;
+  static std::map<int, int> by_device;
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = by_device.find(device);
+  if (it == by_device.end()) {
+    // kernel attributes are the current device's, as `device` is
+    bool ok = true;
+    for (const void* k : {reinterpret_cast<const void*>(k_problem), reinterpret_cast<const void*>(k_ultra<true>),
+                          reinterpret_cast<const void*>(k_outside_clade)})
+      ok = ok && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMaxBytes) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+    it = by_device.emplace(device, ok ? kLdsMaxBytes : 0).first;
+  }
+  return it->second;
 }
 
 void run_counts(const DevForest& F, double* counts, hipStream_t s) {

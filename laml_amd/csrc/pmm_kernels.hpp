@@ -216,6 +216,10 @@ int seg_width(int max_k);
 // dynamic LDS a block of the LDS passes may take (160 KiB less their static
 // arrays)
 constexpr int kLdsMaxBytes = 160 * 1024 - 1024;
+// what they may take on `device` (which must be current), set up once per
+// device: kLdsMaxBytes, or 0 where the runtime refuses it (the passes then run
+// without these kernels)
+int max_lds(int device);
 // sites of a block that share a partial-count slot in its LDS (a block's
 // sites are a multiple)
 constexpr int kLdsSlotSites = 8;
