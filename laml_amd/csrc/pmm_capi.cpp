@@ -512,6 +512,11 @@ static int plan_problems(laml_forest* f, int max_k, const std::vector<int32_t>& 
     blks.push_back(b);
   }
   const int rc = upload_lds_plan(f, f->pb, blks, 1, lvl_base, lvl_beg, lvl_cnt);
+  if (rc == LAML_ENOMEM) {
+    // the forest may still fit without these tables
+    (void)hipGetLastError();
+    return LAML_OK;
+  }
   if (rc) return rc;
   f->pb_ok = true;
   return LAML_OK;

@@ -50,11 +50,33 @@ def segment_width(max_k):
 FOREST_FIXED_BYTES = 48 << 20
 
 
+# LDS a block of the whole-problem kernel may take, and what a cell's state
+# takes of it
+_LDS_BYTES, _LDS_CELL_BYTES = 160 * 1024 - 1024, 20
+
+
+def _block_plan_bytes(p):
+    """Device bytes of a problem's tables for the whole-problem kernel (0:
+    several trees, more than 64 sites or too large for it): 48 B per pair of
+    (internal node, site) cells, each level padded to 64 pairs; 104 B per
+    internal node and 48 per node."""
+    if len(p.trees) != 1 or p.sites.K > 64:
+        return 0
+    t = p.trees[0]
+    sb = -(-p.sites.K // 8) * 8
+    n_int = t.n_nodes - t.n_leaves
+    if n_int * sb * _LDS_CELL_BYTES > _LDS_BYTES:
+        return 0
+    pairs = 64 * -(-np.bincount(t.height)[1:] * sb // 128).sum()
+    return 48 * int(pairs) + 104 * n_int + 48 * t.n_nodes
+
+
 def estimate_forest_bytes(specs):
     """Device bytes of a forest of these problems that grow with it (rows
     padded to the segment width; per node metadata, records, chain plans,
-    partials and parameters; per site tables); with FOREST_FIXED_BYTES, an
-    upper bound on what its creation and an EM call take."""
+    partials and parameters; per site tables; the whole-problem kernel's
+    tables); with FOREST_FIXED_BYTES, an upper bound on what its creation and
+    an EM call take."""
     K = [p.sites.K for p in specs]
     W = segment_width(max(K))
     chunks = -(-max(K) // W)
@@ -70,6 +92,7 @@ def estimate_forest_bytes(specs):
             q = 8 if W == 64 else 0
             total += n_leaf * kp * (2 + q) + n_int * kp * (60 + q)
             nodes += t.n_nodes
+        total += _block_plan_bytes(p)
         total += p.sites.K * (8 + 4 + 8 + 4 + 4) + 8 * int(p.sites.qoff[-1])
     # per node: coefficients 40, counts 40, nu solve 24, node record 64,
     # ids and offsets 48, chain plan 48; per 64-site chunk: partial counts 40
