@@ -1073,6 +1073,12 @@ __device__ __forceinline__ void out_node_rec(const DevForest& F, const NodeRec& 
 // And a node with label 'z' is unedited given the data below it: a0 = 1 / b0
 // and aX = 0 whatever lies outside, so its row is not read (and may hold
 // anything).
+// Range: the scale sc of u's vector goes to the siblings' edge values and not
+// to the state, since 1 / B0 alone leaves a double's range where two unedited
+// children hang on branches of 300 or more.  a0 is at most 1 / b0, so it stays
+// finite while a node's unedited value is within 1e-308 of its edited one; the
+// ratio is at least (edit probability x prior weight) ^ 2 of one branch, 0
+// below that (then a0 counts for nothing).
 // A row is 16 bytes where the unconditional state (three more values, an
 // exponent and a specific state) took 38, and a step needs about half the
 // arithmetic: on 16 trees of 10,000 leaves x 300 sites the chain rounds below
@@ -1102,8 +1108,8 @@ __device__ __forceinline__ void cond_post(int lu, double a0, double aX, double p
   const double BA = z ? 0.0 : ep[0].eA * ep[1].eA;
   // the power of two that the inside pass scaled u's vector by
   const double sc = ldexp(1.0, min(-exp_of(fmax(B0, BA)), 1000));
-  const double f0 = z ? rcp_normal(B0 * sc) * sc : a0 * sc;
-  const double fX = z ? 0.0 : aX * sc;
+  const double f0 = z ? rcp_normal(B0 * sc) : a0;
+  const double fX = z ? 0.0 : aX;
   o.rt = 0.0;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -1111,8 +1117,8 @@ __device__ __forceinline__ void cond_post(int lu, double a0, double aX, double p
     const Coef& cf = cfs[i];
     // A, G: the data outside the child's branch joint with u unedited / in
     // an allowed edit state, over L and on the child's edge exponent
-    const double A = f0 * ep[w].e0;
-    const double G = fX * ep[w].eA;
+    const double A = f0 * (ep[w].e0 * sc);
+    const double G = fX * (ep[w].eA * sc);
     const double As = A * ep[i].s0, Gs = G * ep[i].s0;
     const double m = cf.mut * q[i] * As;
     const double pg = cf.pn * Gs;
@@ -2741,8 +2747,8 @@ __device__ __forceinline__ QTop q_node(const QTop& t, const Coef& cf, int lv, do
 // of two the parent's vector was scaled by) and the sibling's edge values
 __device__ __forceinline__ QTop q_top(const QTop& a, double sc, const Eps& ew) {
   QTop t;
-  t.A = a.A * sc * ew.e0;
-  t.G = a.G * sc * ew.eA;
+  t.A = a.A * (sc * ew.e0);
+  t.G = a.G * (sc * ew.eA);
   return t;
 }
 
@@ -3291,17 +3297,17 @@ __device__ __forceinline__ void lds_outside_cells(const LdsCtx& x, const LdsItem
     const double B0 = ep[0].e0 * ep[1].e0;
     const double BA = z ? 0.0 : ep[0].eA * ep[1].eA;
     const int sh = min(-exp_of(fmax(B0, BA)), 1000);
-    const double f0 = z ? rcp_normal(B0) : ldexp(a[c].x, sh);
-    const double fX = z ? 0.0 : ldexp(a[c].y, sh);
+    const double f0 = z ? rcp_normal(ldexp(B0, sh)) : a[c].x;
+    const double fX = z ? 0.0 : a[c].y;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const Eps& ew = ep[1 - i];
-      double k0 = ew.e0, kX = ew.eA;
+      double k0 = ldexp(ew.e0, sh), kX = ldexp(ew.eA, sh);
       if (kQ) {
+        v[5 * i + 2] = fma(f0, ep[i].s1 * k0, v[5 * i + 2]);
+        v[5 * i + 4] = fma(fX, ep[i].s1 * kX, v[5 * i + 4]);
         k0 *= ep[i].s0;
         kX *= ep[i].s0;
-        v[5 * i + 2] = fma(f0, ep[i].s1 * ew.e0, v[5 * i + 2]);
-        v[5 * i + 4] = fma(fX, ep[i].s1 * ew.eA, v[5 * i + 4]);
       }
       const double a0 = f0 * (it.cf.p1n[i] * k0);
       const double m = f0 * (mq[i] * k0);
