@@ -354,8 +354,9 @@ typedef struct {
 int laml_forest_set_ultrametric(laml_forest* f, const laml_ultra_desc* u);
 
 /* Starting heights of the variable classes (host [num_classes]); they must
- * give every free branch a length strictly inside (dmin, dmax).  Later
- * ultrametric M-steps warm-start from the previous solution. */
+ * give every free branch a length strictly inside (dmin, dmax).  An
+ * ultrametric M-step starts from the previous solution drawn a tenth towards
+ * them, which keeps the start inside the bounds. */
 int laml_forest_set_heights(laml_forest* f, const double* heights_host);
 
 /* Per-problem status of the last ultrametric M-step (0 ok, 1 line search

@@ -429,14 +429,13 @@ static int64_t lds_entries(const laml::LdsBlk& b, const std::vector<int32_t>& lv
   return n;
 }
 
-// The LDS plan whose block b runs tree blks[b].tree at its sites, a tree's
-// blocks writing one partial-count slot each.  Level tables as the tree
+// The LDS plan whose block b runs tree blks[b].tree.  Level tables as the tree
 // walk's.
 static int upload_lds_plan(laml_forest* f, laml::LdsPlan& L, const std::vector<laml::LdsBlk>& blks,
-                           int slots, const std::vector<int32_t>& lvl_base, const std::vector<int32_t>& lvl_beg,
+                           const std::vector<int32_t>& lvl_base, const std::vector<int32_t>& lvl_beg,
                            const std::vector<int32_t>& lvl_cnt) {
   const int N = f->F.num_nodes, n = f->F.num_leaves, T = f->F.num_trees;
-  std::vector<int32_t> tree_sb(T, 0);  // (the same for all blocks of a tree)
+  std::vector<int32_t> tree_sb(T, 0);
   for (const laml::LdsBlk& b : blks) tree_sb[b.tree] = b.sb;
   std::vector<int32_t> int_base(T, 0), local(N, -1);
   std::vector<int2> lvl_off(lvl_base[T], make_int2(0, 0));
@@ -464,7 +463,6 @@ static int upload_lds_plan(laml_forest* f, laml::LdsPlan& L, const std::vector<l
     L.lds_bytes = (int32_t)std::max<int64_t>(L.lds_bytes, lds_need(b, lvl_base));
   }
   L.num_blocks = (int32_t)blks.size();
-  L.slots = slots;
   Packed m;
   const size_t o[9] = {m.place(blks),
                        m.place(int_base),
@@ -473,8 +471,8 @@ static int upload_lds_plan(laml_forest* f, laml::LdsPlan& L, const std::vector<l
                        m.reserve((size_t)recs * sizeof(laml::LdsCoef)),
                        m.reserve((size_t)entries * sizeof(uint4)),
                        m.reserve((size_t)entries * sizeof(double4)),
-                       m.reserve((size_t)N * 5 * slots * sizeof(double)),
-                       m.reserve((size_t)N * slots * sizeof(double))};
+                       m.reserve((size_t)N * 5 * sizeof(double)),
+                       m.reserve((size_t)N * sizeof(double))};
   char* d = nullptr;
   const int rc = m.upload(f, &d);
   if (rc) return rc;
@@ -503,7 +501,6 @@ static int plan_problems(laml_forest* f, int max_k, const std::vector<int32_t>& 
   for (int t = 0; t < T; ++t) {
     laml::LdsBlk b{};
     b.tree = t;
-    b.k0 = 0;
     b.sb = (f->tree_nsites[t] + R - 1) / R * R;
     for (int i = lvl_base[t] + 1; i < lvl_base[t + 1]; ++i) b.nint += lvl_cnt[i];
     if (b.nint < 1 || lds_need(b, lvl_base) > f->lds_max) return LAML_OK;
@@ -511,7 +508,7 @@ static int plan_problems(laml_forest* f, int max_k, const std::vector<int32_t>& 
     tab += lds_entries(b, lvl_base, lvl_cnt);
     blks.push_back(b);
   }
-  const int rc = upload_lds_plan(f, f->pb, blks, 1, lvl_base, lvl_beg, lvl_cnt);
+  const int rc = upload_lds_plan(f, f->pb, blks, lvl_base, lvl_beg, lvl_cnt);
   if (rc == LAML_ENOMEM) {
     // the forest may still fit without these tables
     (void)hipGetLastError();
@@ -771,8 +768,8 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   double *pS, *site_llh, *rt_part, *cpart, *nu_a, *nu_b, *nu_d, *nu_part;
   int32_t* mstep_status;
   AL(labels, int16_t, int_rows);
-  // prior-weight rows: read by the chain kernels only, which need 64-site
-  // segments
+  // prior-weight rows: read by the chain kernels and the tree walk, where
+  // segments hold 64 sites
   double *qleaf = nullptr, *qint = nullptr;
   if (f->W == 64) {
     AL(qleaf, double, leaf_rows);
@@ -896,9 +893,7 @@ int laml_forest_create(const laml_forest_desc* d, int device, laml_forest** out)
   F.mstep_status = mstep_status;
   F.phi = nullptr;
   F.cp_v = (int64_t)F.max_chunks * 5;
-  F.cp_c = 5;
   F.rt_v = F.max_chunks;
-  F.rt_c = 1;
   f->def.pass_mode = f->pass_mode;
   f->def.h_top = f->h_top_default;
   f->def.h_walk = f->h_walk;
@@ -1451,14 +1446,11 @@ static bool problem_now(const laml_forest* f) {
 // F with the partial counts of an LDS plan
 static DevForest lds_view(const DevForest& F, const laml::LdsPlan& L) {
   DevForest G = F;
-  // one slot per block of a tree's sites
-  G.chunk_w = 1 << 24;
+  G.chunk_w = 1 << 24;  // (one chunk of sites)
   G.cpart = L.cpart;
   G.rt_part = L.rt_part;
   G.cp_v = 5;
-  G.cp_c = (int64_t)F.num_nodes * 5;
   G.rt_v = 1;
-  G.rt_c = F.num_nodes;
   return G;
 }
 

@@ -2056,7 +2056,7 @@ __global__ void __launch_bounds__(256) k_counts(DevForest F, double* __restrict_
   const int C = (F.tree_nsites[F.tree_of[v]] + F.chunk_w - 1) / F.chunk_w;
   const double* src = F.cpart + v * F.cp_v + j;
   double s = 0.0;
-  for (int c = 0; c < C; ++c) s += src[c * F.cp_c];
+  for (int c = 0; c < C; ++c) s += src[c * 5];
   counts[idx] = s;
 }
 
@@ -2125,12 +2125,12 @@ __device__ __forceinline__ void add_node_rt(const DevForest& F, int64_t v, int C
   if (C <= kC) {
     double x[kC];
 #pragma unroll
-    for (int c = 0; c < kC; ++c) x[c] = c < C ? src[c * F.rt_c] : 0.0;
+    for (int c = 0; c < kC; ++c) x[c] = c < C ? src[c] : 0.0;
 #pragma unroll
     for (int c = 0; c < kC; ++c)
       if (c < C) s += x[c];
   } else {
-    for (int c = 0; c < C; ++c) s += src[c * F.rt_c];
+    for (int c = 0; c < C; ++c) s += src[c];
   }
 }
 
@@ -2316,7 +2316,7 @@ __global__ void __launch_bounds__(kNuThreads) k_branch(DevForest F, const double
       } else {
         for (int c = 0; c < C; ++c)
 #pragma unroll
-          for (int j = 0; j < 5; ++j) s[j] += F.cpart[v * F.cp_v + c * F.cp_c + j];
+          for (int j = 0; j < 5; ++j) s[j] += F.cpart[v * F.cp_v + c * 5 + j];
       }
       if (kUltra) {
         const BranchObj o = branch_obj(s, (double)Kt, nu0);
@@ -2461,7 +2461,7 @@ __global__ void k_grad_branch(DevForest F, const double* __restrict__ d, const d
   double s[5] = {0, 0, 0, 0, 0};
   for (int c = 0; c < C; ++c)
 #pragma unroll
-    for (int j = 0; j < 5; ++j) s[j] += F.cpart[v * F.cp_v + c * F.cp_c + j];
+    for (int j = 0; j < 5; ++j) s[j] += F.cpart[v * F.cp_v + c * 5 + j];
   const double dv = d[v];
   grad_d[v] = -grad_length(s, dv, nu[p]);
   F.nu_a[F.node_pos[v]] = s[0] + s[1] + s[3];
@@ -3102,7 +3102,7 @@ struct LdsItem {
 
 // one block's tree
 struct LdsCtx {
-  int sb, nint, H, k0, K;
+  int sb, nint, H, K;
   unsigned magic;          // floor(i / sb) = umulhi(i, magic) for i < 2^20
   const uint4* w;
   const double4* q;
@@ -3137,7 +3137,6 @@ __device__ __forceinline__ LdsCtx lds_ctx(const DevForest& F, const LdsPlan& L, 
   LdsCtx x;
   x.sb = B.sb;
   x.nint = B.nint;
-  x.k0 = B.k0;
   x.K = uniform_at(F.tree_nsites, B.tree);
   const int lb = uniform_at(TW.lvl_base, B.tree);
   x.H = uniform_at(TW.lvl_base, B.tree + 1) - lb;
@@ -3448,9 +3447,8 @@ __device__ __forceinline__ double lds_root(const DevForest& F, const LdsCtx& x, 
   if (s < x.sb) {
     const int r = uniform_at(F.tree_root, t);
     const int pl = lds_place((x.nint - 1) * x.sb + s);
-    const int k = x.k0 + s;
-    const bool real = k < x.K;
-    const int kc = min(k, x.K - 1);
+    const bool real = s < x.K;
+    const int kc = min(s, x.K - 1);
     const int sk = uniform_at(F.tree_site_base, t) + kc;
     const int lab = F.labels[F.row_off[r] + kc];
     const double q = lab > 0 ? F.prior[F.site_qoff[sk] - 1 + lab] : F.site_qsum[sk];
@@ -3527,16 +3525,15 @@ __device__ __forceinline__ void lds_branch_counts(const LdsCtx& x, int r, double
 #pragma unroll
   for (int m = 0; m < 5; ++m) s[m] = stem && m > 2 ? 0.0 : c[m];
 }
-// the folded counts into slot `slot` of F's partials
-__device__ __forceinline__ void lds_flush(const DevForest& F, const LdsCtx& x, int t, int64_t slot) {
-  double* cp = F.cpart + slot * F.cp_c;
+// the folded counts into F's partials
+__device__ __forceinline__ void lds_flush(const DevForest& F, const LdsCtx& x, int t) {
   for (int r = (int)threadIdx.x; r <= 2 * x.nint; r += kLdsThreads) {
     double s[5];
     lds_branch_counts(x, r, s);
-    double* c = cp + lds_branch_node(F, x, t, r) * F.cp_v;
+    double* c = F.cpart + lds_branch_node(F, x, t, r) * F.cp_v;
 #pragma unroll
     for (int m = 0; m < 5; ++m) c[m] = s[m];
-    if (r < 2 * x.nint && !(r & 1)) F.rt_part[slot * F.rt_c + x.rec[r >> 1].v * F.rt_v] = lds_slot(x, r >> 1, 0)[10];
+    if (r < 2 * x.nint && !(r & 1)) F.rt_part[x.rec[r >> 1].v * F.rt_v] = lds_slot(x, r >> 1, 0)[10];
   }
 }
 
@@ -3665,7 +3662,7 @@ __global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
           A.grad.phi[p] = grad_phi_of(F.prob_nobs_phi[p], g[1], pv);
         }
       } else if (out) {
-        lds_flush(F, x, t, 0);
+        lds_flush(F, x, t);
       }
       return;
     }
@@ -3691,7 +3688,7 @@ __global__ void __launch_bounds__(kLdsThreads) k_problem(PbArgs) {
     const uint32_t flags = uniform_at(F.prob_flags, p);
     const bool opt_nu = (flags & 2u) && uniform_at(F.prob_nfree, p) > 0;
     const double K = (double)x.K;
-    // M-step: branch lengths (as branch_update), the dropout sum on the way
+    // M-step: branch lengths (as k_branch), the dropout sum on the way
     double a0 = 0.0, b0 = 0.0, d0 = 0.0;  // the thread's first branch, as nu_a, nu_b, nu_d
     double rt = 0.0, bad = 0.0;
     for (int r = (int)threadIdx.x; r < nbr; r += kLdsThreads) {
@@ -3776,7 +3773,7 @@ __global__ void __launch_bounds__(256) k_lds_tables(DevForest F, LdsPlan L, Tree
         const int i = lds_pair((unsigned)e) + c2;
         uint32_t pl[2] = {3, 3}, fl = kLdsLeaf0 | kLdsLeaf1;
         q[2 * c2] = q[2 * c2 + 1] = 0.0;
-        const int j = l0 + i / B.sb, s = i % B.sb, k = B.k0 + s;
+        const int j = l0 + i / B.sb, s = i % B.sb, k = s;
         if (i < n) {
           const LdsRec r = recs[j];
           int lab[2] = {0, 0};

@@ -93,9 +93,9 @@ struct DevForest {
   double* rt_part;  // [N * max_chunks] dropout sums of leaf children per chunk
   double* cpart;    // [N * max_chunks * 5] per-chunk branch count partials
   // where the readers of the partials find node v's chunk c: cpart + v cp_v +
-  // c cp_c (5 values), rt_part + v rt_v + c rt_c.  The row kernels write a
-  // node's chunks side by side, the LDS kernels a chunk's nodes.
-  int64_t cp_v, cp_c, rt_v, rt_c;
+  // 5 c, rt_part + v rt_v + c (a node's chunks side by side; one chunk holds
+  // all sites of the problems that k_problem runs)
+  int64_t cp_v, rt_v;
   double* nu_a;     // [N] by position in prob_nodes: S0+S1+S3 of the branch
   double* nu_b;     // [N] S2+S4 (0 for fixed branches)
   double* nu_d;     // [N] new branch length
@@ -167,13 +167,13 @@ struct TreeWalk {
   const int32_t* lvl_cnt;
 };
 
-// Plan of the LDS passes (k_problem, k_lds_pass): block b runs tree
-// blk[b].tree at sites [k0, k0 + sb) (sb a multiple of the reduction width),
-// the state of every internal node at those sites in LDS.  Internal nodes are
-// numbered within their tree in level order ("local"), so the root is last.
+// Plan of k_problem: block b runs tree blk[b].tree at all its sites (sb: their
+// number rounded up to a multiple of the reduction width), the state of every
+// internal node in LDS.  Internal nodes are numbered within their tree in level
+// order ("local"), so the root is last.
 struct LdsBlk {
-  int32_t tree, k0, sb, nint;  // nint: internal nodes of the tree
-  int64_t tab;                 // first entry of the block's cell tables
+  int32_t tree, sb, nint, pad;  // nint: internal nodes of the tree
+  int64_t tab;                  // first entry of the block's cell tables
 };
 // an internal node: its children's local numbers (-1: leaf) and node ids, its
 // own id
@@ -188,7 +188,7 @@ struct LdsCoef {
   int32_t pad[2];
 };
 struct LdsPlan {
-  int32_t num_blocks, slots;   // slots: partial counts per node (blocks of its tree)
+  int32_t num_blocks;
   int32_t lds_bytes;           // dynamic LDS of a block
   const LdsBlk* blk;
   const int32_t* int_base;     // [T] first record of each tree
@@ -200,7 +200,7 @@ struct LdsPlan {
   // the children's prior weights; fixed for the forest's life
   uint4* w;
   double4* q;
-  double* cpart;               // partials, chunk-major
+  double* cpart;               // partials
   double* rt_part;
 };
 
