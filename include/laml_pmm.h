@@ -189,10 +189,12 @@ int32_t laml_forest_fusion(laml_forest* f);
  * MI355X, outside chains below level 10 beat level launches on forests of
  * that size; inside chains were slower on every forest tried (opt-in).
  * In the launch plan a forest is created with, large forests (inside pass
- * from 12,288 pairs, outside pass from 57,344) run over clades instead:
- * subtrees of up to 64 nodes that one wavefront walks as a whole (environment
- * LAML_CLADES sets that cap at forest creation, 0 turns them off), the same
- * bits again; other shapes or chains ask for their own kernels.
+ * from 12,288 pairs, below 32,768 once a few calls have earned the layout;
+ * outside pass from 57,344, unless its trees hold too few clades to fill
+ * blocks) run over clades instead: subtrees of up to 64 nodes that one
+ * wavefront walks as a whole (environment LAML_CLADES sets that cap at forest
+ * creation, 0 turns them off), the same bits again; other shapes or chains ask
+ * for their own kernels.
  * laml_forest_chains reports the flags the next passes use (not
  * LAML_CHAINS_OUTSIDE where the outside pass runs over clades).
  * No counterpart in the reference. */

@@ -148,12 +148,11 @@ __device__ __forceinline__ void swap16(double& x, double& y) {
 // (12 -> 6 -> 3 values; row r of 16 lanes then holds values 3r .. 3r + 2), 8
 // apart (the first two share a register), mirrored within 8 lanes (the third
 // joins them), then two steps within quads.  50 instructions instead of 12
-// separate reductions; without the last two halvings, 67 (the outside pass
-// over clades of 16 x 10,000 leaves x 300 sites: 337 us, 333
-// now).  On the
-// matrix cores, with a column of ones and four values to a register, the sums
-// take 15 instructions of 16 cycles and 6 more, but hold up the other
-// wavefronts' arithmetic (426 us).
+// separate reductions; without the last two halvings, 67 (the outside walk over
+// clades in an EM step of 16 x 10,000 leaves x 300 sites: 337 us, and 333 with
+// them).  On the matrix cores, with a column of ones and four values to a
+// register, the sums take 15 instructions of 16 cycles and 6 more, but hold up
+// the other wavefronts' arithmetic (426 us).
 // Returns the total of value sum12_value(lane) in that lane.
 __device__ __forceinline__ int sum12_value(int lane) {
   const int i = lane & 15;

@@ -1785,10 +1785,10 @@ __global__ void __launch_bounds__(256) k_outside_chain(DevForest F, const int2* 
 // clade's root.  The children's inside rows, labels and codes of the next step
 // are copied to the slice during the step, as in k_outside_chain; prior
 // weights come from the chunk's piece in LDS and the coefficients in walking
-// order, as in k_inside_clade.  Sixteen trees of 10,000 leaves x 300 sites: 333
-// us and 125 in the rounds above, where the chain rounds and the levels above
-// took 675 us; 50,000 x 500: 175 and 91, 325.  Bound by instruction issue (93 %
-// of the VALU cycles at six wavefronts a SIMD).
+// order, as in k_inside_clade.  EM step of sixteen trees of 10,000 leaves x 300
+// sites: 335 us and 126 in the rounds above, where the chain rounds and the
+// levels above took 675 us; 50,000 x 500: 178 and 86, 325.  Bound by instruction
+// issue (82 % of the VALU cycles at six wavefronts a SIMD).
 constexpr int kOutLdsBeta = 0;     // [2][64] double2
 constexpr int kOutLdsE = 2048;     // [2][64] int32
 constexpr int kOutLdsCode = 2560;  // [2][64] int16

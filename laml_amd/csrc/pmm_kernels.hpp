@@ -229,8 +229,9 @@ constexpr int kLdsSlotSites = 8;
 // / general: 256 problems of 250 x 30 89 / 308 us, 1,024 of them 308 / 658,
 // 2,048 of 100 x 20 373 / 576, 4,096 of 60 x 16 720 / 588).
 // A likelihood (with its gradient) goes through blocks up to kPbMaxSingle: 1,024
-// problems of 10 x 8 44 (122) us, 45 (113) in the general passes, of 60 x 40
-// 70 (213) and 108 (264), of 120 x 60 96 (301) and 149 (370); 1,280 of them 55
+// problems of 10 x 8 41 (115) us, 46 (104) in the general passes, of 60 x 40
+// 67 (204) and 73 (188), of 120 x 60 89 (286) and 97 (281); 768 of them 30 (84)
+// and 35 (89), 51 (154) and 69 (172), 70 (221) and 90 (243); 1,280 of them 55
 // (151) and 45 (106), 85 (259) and 85 (216), 136 (411) and 118 (334).
 constexpr int kPbMaxSites = 64;
 constexpr int kPbMaxProblems = 2048;
