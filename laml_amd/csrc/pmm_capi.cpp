@@ -103,12 +103,13 @@ struct laml_forest {
   // state of the last call.  A call that is being captured runs again without
   // this code when its graph is replayed: once one that leaves no inside rows,
   // or not all outside rows, has been captured, rows_ok and alpha_complete
-  // are not trusted any more (rows_unsure, alpha_unsure).  The branch
+  // are not trusted any more (rows_unsure, alpha_unsure); nor the rows of
+  // cherries, once one that fuses them has been (cherries_unsure).  The branch
   // coefficients are always those of the last call, replayed or not.
   bool pb_ok = false;
   int lds_max = 0;  // LDS that a block of the LDS kernels may take
   laml::LdsPlan pb{};
-  bool rows_ok = true, rows_unsure = false, alpha_unsure = false;
+  bool rows_ok = true, rows_unsure = false, alpha_unsure = false, cherries_unsure = false;
   struct {
     int pass_mode, h_top, h_walk, chains, chain_top_in, chain_top_out;
     bool fuse;
@@ -1956,6 +1957,10 @@ static void left_no_rows(laml_forest* f, hipStream_t s) {
   f->rows_ok = f->alpha_complete = f->inside_fused = false;
   if (!f->rows_unsure && capturing(s)) f->rows_unsure = f->alpha_unsure = true;
 }
+// after a call on s with an inside pass
+static void left_inside(laml_forest* f, hipStream_t s) {
+  if (f->inside_fused && !f->cherries_unsure && capturing(s)) f->cherries_unsure = true;
+}
 // after a call on s with an outside pass
 static void left_outside(laml_forest* f, hipStream_t s) {
   if (!f->alpha_complete && !f->alpha_unsure && capturing(s)) f->alpha_unsure = true;
@@ -1965,7 +1970,7 @@ static void left_outside(laml_forest* f, hipStream_t s) {
 // have left none (from its branch coefficients; not those in a clade plan's
 // steps: F names none).  Returns whether it formed them.
 static bool ensure_rows(laml_forest* f, const DevForest& F, hipStream_t s) {
-  if (f->rows_ok && !f->rows_unsure) return false;
+  if (f->rows_ok && !f->rows_unsure && (f->inside_fused || !f->cherries_unsure)) return false;
   pass_inside_root(f, F, nullptr, nullptr, s, true);
   return true;
 }
@@ -1998,6 +2003,7 @@ int laml_nll(laml_forest* f, const double* d, const double* nu, const double* ph
   f->rows_ok = true;
   pass_coef(f, F, d, nu, nullptr, s);
   pass_inside_root(f, F, site_llh, nullptr, s);
+  left_inside(f, s);
   laml::run_llh(F, nll, none, 0, 0.0, s);
   return check_launch();
 }
@@ -2032,6 +2038,7 @@ int laml_estep(laml_forest* f, const double* d, const double* nu, const double* 
     pass_inside_root(f, F, nullptr, nullptr, s);
     pass_outside(f, F, false, nullptr, s);
   }
+  left_inside(f, s);
   left_outside(f, s);
   laml::run_llh(F, nll, none, 0, 0.0, s);
   laml::run_counts(F, counts, s);

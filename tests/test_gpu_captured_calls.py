@@ -209,3 +209,27 @@ def test_outside_after_a_replay_in_another_plan(kind, monkeypatch):
     E.close()
     _same(got, want)
     c.F.close()
+
+
+def test_readers_after_a_replay_with_fused_cherries(monkeypatch):
+    """An E-step captured with fused cherries (whose rows it does not write),
+    replayed after an eager one without."""
+    c = Case("levels", monkeypatch)
+    prm = c.set(0)
+    c.F.set_pass_mode(PASS_LEVELS)
+    c.F.set_fusion(True)
+    assert c.F.fusion()
+    g = _capture(lambda: c.F.estep(*prm))
+    c.F.set_fusion(False)
+    other = tuple(x.clone() for x in c.set(3))
+    c.set(1)
+    c.F.estep(*other)
+    g.replay()
+    got = _post(c.F, c.phi) + _host(c.F.outside(c.phi)) + _host(c.F.grad(*prm))
+    E = c.forest()
+    E.set_pass_mode(PASS_LEVELS)
+    E.estep(*prm)
+    want = _post(E, c.phi) + _host(E.outside(c.phi)) + _host(E.grad(*prm))
+    E.close()
+    _same(got, want)
+    c.F.close()
