@@ -2248,6 +2248,8 @@ int laml_em(laml_forest* f, double* d, double* nu, double* phi, int32_t max_iter
     left_no_rows(f, s);
   else if (max_iter > 0 && f->pass_mode != LAML_PASS_TREES)
     f->alpha_complete = !out_clades(f) && !pass_chains(f, false, hybrid_split(f)) && !fuse_now(f);
+  left_inside(f, s);
+  left_outside(f, s);
   LAML_HIP(hipMemcpyAsync(iters, em.iters, sizeof(int32_t) * P, hipMemcpyDeviceToDevice, s));
   return check_launch();
 }

@@ -211,25 +211,29 @@ def test_outside_after_a_replay_in_another_plan(kind, monkeypatch):
     c.F.close()
 
 
-def test_readers_after_a_replay_with_fused_cherries(monkeypatch):
-    """An E-step captured with fused cherries (whose rows it does not write),
-    replayed after an eager one without."""
+@pytest.mark.parametrize("call", ["estep", "em"])
+def test_readers_after_a_replay_with_fused_cherries(call, monkeypatch):
+    """An E-step, or an EM of no steps (a likelihood), captured with fused
+    cherries (whose rows it does not write) and replayed after an eager E-step
+    without."""
     c = Case("levels", monkeypatch)
     prm = c.set(0)
     c.F.set_pass_mode(PASS_LEVELS)
     c.F.set_fusion(True)
     assert c.F.fusion()
-    g = _capture(lambda: c.F.estep(*prm))
+    g = _capture(lambda: c.F.estep(*prm) if call == "estep" else c.F.em(*prm, 0, 0.0))
     c.F.set_fusion(False)
     other = tuple(x.clone() for x in c.set(3))
     c.set(1)
     c.F.estep(*other)
     g.replay()
-    got = _post(c.F, c.phi) + _host(c.F.outside(c.phi)) + _host(c.F.grad(*prm))
+    got = _post(c.F, c.phi) if call == "estep" else []
+    got += _host(c.F.outside(c.phi)) + _host(c.F.grad(*prm))
     E = c.forest()
     E.set_pass_mode(PASS_LEVELS)
     E.estep(*prm)
-    want = _post(E, c.phi) + _host(E.outside(c.phi)) + _host(E.grad(*prm))
+    want = _post(E, c.phi) if call == "estep" else []
+    want += _host(E.outside(c.phi)) + _host(E.grad(*prm))
     E.close()
     _same(got, want)
     c.F.close()
