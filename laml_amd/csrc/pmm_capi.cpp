@@ -1831,6 +1831,7 @@ static void prepare_clades(laml_forest* f, hipStream_t s, int64_t earns) {
   cl.out_steps = reinterpret_cast<const laml::CladeOut*>(m + o[7]);
   cl.coef = reinterpret_cast<laml::CladeCoef*>(m + o[8]);
   f->clade_plans.push_back(std::move(cl));
+  f->plan_version++;  // (an EM step captured before takes them from the next call on)
 }
 
 // the chain plan of a pass below split level hs (nullptr: that pass runs
